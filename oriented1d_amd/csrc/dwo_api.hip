@@ -14,6 +14,7 @@
 #include "dwo_nhwc.h"
 #include "dwo_dispatch.h"
 #include "dwo_nhwc_tile.h"
+#include "dwo_window_dispatch.h"
 #include "dwo_fused.h"
 
 using namespace dwo;
@@ -155,6 +156,32 @@ int try_nhwc_plane_wgrad(const void *x, const void *dy, const void *taps, float 
     return -100;
 }
 
+// NCHW at stride 1, any extent, kernel sizes of DWO_WINDOW_KS: the window kernels
+bool window_covers(const ConvDims &d, int layout, size_t esize, WinDims &wd) {
+    return layout == DWO_NCHW && d.stride == 1 && win_dims(d.N, d.C, d.H, d.W, d.K, esize, wd);
+}
+template <typename T>
+int try_window_conv(const void *src, const float *w, const float *bias, const void *taps, void *dst,
+                    const ConvDims &d, int layout, int flip, hipStream_t st) {
+    WinDims wd;
+    if (!window_covers(d, layout, sizeof(T), wd)) return -100;
+#define DWO_MATCH(K_) \
+    if (d.K == K_) return launch_window_conv<T, K_>(src, w, bias, taps, dst, wd, flip, st);
+    DWO_WINDOW_KS(DWO_MATCH)
+#undef DWO_MATCH
+    return -100;
+}
+template <typename T>
+int try_window_wgrad(const void *x, const void *dy, const void *taps, float *part, float *dw, float *db,
+                     unsigned *tickets, const WinDims &wd, int K, int *groups, hipStream_t st) {
+#define DWO_MATCH(K_) \
+    if (K == K_)      \
+        return launch_window_wgrad<T, K_>(x, dy, taps, part, dw, db, tickets, wd, groups, st);
+    DWO_WINDOW_KS(DWO_MATCH)
+#undef DWO_MATCH
+    return -100;
+}
+
 // shapes the tile kernels take: NCHW always, NHWC with the channel count a multiple of 4; images
 // below 2 GB (32-bit offsets inside one)
 bool tile_covers(const ConvDims &d, int layout, size_t esize) {
@@ -172,6 +199,9 @@ int wgrad_max_partials(const ConvDims &d, int layout, size_t esize) {
         return nbatch < kMaxPlaneGroups ? nbatch : kMaxPlaneGroups;
     }
     const int PB = plane_batch(d, layout);
+    WinDims wd;
+    if (PB == 0 && window_covers(d, layout, esize, wd))
+        return wd.units < kMaxWinGroups ? wd.units : kMaxWinGroups;
     if (PB == 0 && tile_covers(d, layout, esize)) {
         int band_rows, nbands;
         return tile_wgrad_groups(d, &band_rows, &nbands);
@@ -239,6 +269,8 @@ int fprop_t(const void *x, const float *w, const float *bias, const void *taps, 
     if (fast != -100) return fast;
     const int sliced = try_nhwc_plane_conv<T>(OP_FPROP, x, w, bias, taps, y, d, layout, st);
     if (sliced != -100) return sliced;
+    const int windowed = try_window_conv<T>(x, w, bias, taps, y, d, layout, 0, st);
+    if (windowed != -100) return windowed;
     const int tiled = try_tile_conv<T>(x, w, bias, taps, y, d, layout, 0, st);
     if (tiled != -100) return tiled;
     const int nhwc = try_nhwc_conv<T, NHWC_FPROP>(x, w, bias, taps, y, d, layout, st);
@@ -262,6 +294,8 @@ int dgrad_t(const void *dy, const float *w, const void *taps, void *dx, const Co
     if (fast != -100) return fast;
     const int sliced = try_nhwc_plane_conv<T>(OP_DGRAD, dy, w, nullptr, taps, dx, d, layout, st);
     if (sliced != -100) return sliced;
+    const int windowed = try_window_conv<T>(dy, w, nullptr, taps, dx, d, layout, 1, st);
+    if (windowed != -100) return windowed;
     const int tiled = try_tile_conv<T>(dy, w, nullptr, taps, dx, d, layout, 1, st);
     if (tiled != -100) return tiled;
     const int nhwc = try_nhwc_conv<T, NHWC_DGRAD>(dy, w, nullptr, taps, dx, d, layout, st);
@@ -354,6 +388,7 @@ int wgrad_t(const void *dy, const void *x, const void *taps, float *dw, float *d
             const ConvDims &d, int layout, hipStream_t st) {
     float *part = (float *)scratch;
     int rc, NG = 0;
+    WinDims wd;
     bool direct = false;  // stage 1 wrote dw / db itself (one group per channel, or tickets)
     if (plane_batch(d, layout) != 0) {
         unsigned *tickets = ticket_row(d.C, st);
@@ -362,6 +397,10 @@ int wgrad_t(const void *dy, const void *x, const void *taps, float *dw, float *d
     } else if (nhwc_plane_batch(d, layout) != 0) {
         unsigned *tickets = ticket_row(d.C / kSliceCh, st);
         rc = try_nhwc_plane_wgrad<T>(x, dy, taps, part, dw, db, tickets, &NG, d, st);
+        direct = NG == 1 || tickets != nullptr;
+    } else if (window_covers(d, layout, sizeof(T), wd)) {
+        unsigned *tickets = ticket_row(d.C, st);
+        rc = try_window_wgrad<T>(x, dy, taps, part, dw, db, tickets, wd, d.K, &NG, st);
         direct = NG == 1 || tickets != nullptr;
     } else if (tile_covers(d, layout, sizeof(T))) {
         rc = launch_tile_wgrad<T>(x, dy, taps, part, &NG, d, layout == DWO_NCHW, st);
@@ -448,6 +487,15 @@ int init_type() {
     rc |= launch_nhwc_plane_wgrad<T, K_, H_, W_>(nullptr, nullptr, nullptr, nullptr, nullptr,     \
                                                  nullptr, nullptr, 0, kSliceCh, &ng, nullptr);
     DWO_PLANE_SHAPES(DWO_PREP)
+#undef DWO_PREP
+    WinDims wd;
+    (void)win_dims(1, 1, 64, 64, 31, sizeof(T), wd);
+    wd.N = 0;
+#define DWO_PREP(K_)                                                                           \
+    rc |= launch_window_conv<T, K_>(nullptr, nullptr, nullptr, nullptr, nullptr, wd, 0, nullptr); \
+    rc |= launch_window_wgrad<T, K_>(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, \
+                                     wd, &ng, nullptr);
+    DWO_WINDOW_KS(DWO_PREP)
 #undef DWO_PREP
     ConvDims d = make_dims(1, kSliceCh, 8, 8, 7, 2);
     d.N = 0;

@@ -535,11 +535,13 @@ struct ChannelTaps {
     unsigned wp[NPAIR];
     float bv;
 
+    // (reversed: the weights in reverse tap order as run-time data)
     __device__ __forceinline__ void load(const float *__restrict__ wt, const float *__restrict__ bias,
-                                         int c) {
-        const float *wc = wt + (size_t)c * K;
+                                         int c, int reversed = 0) {
+        const float *wc = wt + (size_t)c * K + (reversed ? K - 1 : 0);
+        const int step = reversed ? -1 : 1;
 #pragma unroll
-        for (int s = 0; s < K; s++) wv[s] = wc[OP == OP_DGRAD ? K - 1 - s : s];
+        for (int s = 0; s < K; s++) wv[s] = wc[step * (OP == OP_DGRAD ? K - 1 - s : s)];
         static_for<K>([&](auto s) {
             constexpr int r = G::plan.rep[s];
             if constexpr (r >= 0 && r != s) wv[r] += wv[s];

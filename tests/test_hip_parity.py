@@ -216,6 +216,21 @@ def test_nchw_large_planes_many_tiles(oracle, stride, H, W, K, dtype):
     _case(oracle, 3, 38, H, W, K, stride, dtype, False, theta, seed=H + W + K + 1)
 
 
+# Window kernels (NCHW, stride 1, any extent): the edges of their units.  Plane mode: one column more
+# or less than a four-column chunk, the smallest rows they take, the row-stride switch at 32 columns,
+# the largest plane, batches that do not fill a unit.  Tile mode: one row or column beyond a plane,
+# tiles cut by both edges, planes of one tile row or column.
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("N,C,H,W,K", [
+    (1, 9, 1, 4, 31), (5, 12, 7, 5, 7), (9, 17, 8, 12, 15), (11, 9, 18, 28, 27), (3, 16, 31, 32, 31),
+    (3, 9, 32, 33, 13), (2, 20, 37, 57, 27), (2, 9, 64, 63, 31), (1, 9, 65, 64, 31), (2, 9, 64, 65, 15),
+    (1, 16, 3, 200, 31), (1, 16, 131, 6, 31), (2, 9, 75, 113, 31), (1, 8, 128, 130, 7)])
+def test_window_kernels_unit_edges(oracle, N, C, H, W, K, dtype):
+    theta = canonical_theta(C)
+    theta[8:9] = 0.61  # one channel on the table-driven body
+    _case(oracle, N, C, H, W, K, 1, dtype, False, theta, seed=H * 1000 + W)
+
+
 @pytest.mark.parametrize("nhwc", [False, True], ids=["nchw", "nhwc"])
 def test_random_angles_ragged_shapes(oracle, nhwc):
     rng = np.random.default_rng(77)
