@@ -5,6 +5,7 @@ import os
 HERE = os.path.dirname(os.path.abspath(__file__))
 # DWOCONV1D_LIB overrides the library location (e.g. an instrumented build)
 LIB_PATH = os.environ.get("DWOCONV1D_LIB") or os.path.join(HERE, "libdwoconv1d_hip.so")
+HOST_PATH = os.path.join(HERE, "_host.so")
 
 F32, BF16, F16 = 0, 1, 2
 NCHW, NHWC = 0, 1
@@ -53,6 +54,27 @@ def load():
 
 
 _ready = set()
+_host = None
+
+
+def host(index):
+    """The native call path (csrc/dwo_host.cpp) with the kernels set up on CUDA device ``index``
+    (below zero for a tensor that is on no CUDA device: the call itself refuses those)."""
+    global _host
+    if index >= 0 and index not in _ready:
+        import torch
+
+        ready(torch.device("cuda", index))
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError("%s is not built; run `python -m oriented1d_amd.build`" % HOST_PATH)
+        import torch  # noqa: F401  (the extension links against its libraries)
+        from . import _host as native
+
+        native.bind(LIB_PATH)
+        _host = native
+    return _host
 
 
 def ready(device):

@@ -7,6 +7,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libdwoconv1d_hip.so")
+HOST_LIB = os.path.join(HERE, "_host.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -51,8 +52,24 @@ def _run(cmd, verbose):
         print(err)
 
 
+def host_command(out):
+    """Compiler line of the native call path: an extension module against PyTorch's libraries."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    dirs = cpp_extension.include_paths() + ["/opt/rocm/include", sysconfig.get_paths()["include"],
+                                            os.path.join(ROOT, "include")]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI] + [
+            "-I" + d for d in dirs] + [os.path.join(CSRC, "dwo_host.cpp")] + [
+            "-L" + d for d in cpp_extension.library_paths()] + [
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python", "-o", out]
+
+
 def build(verbose=False, jobs=None, only=None):
-    """Compile csrc/dwo_api.hip and one csrc/dwo_inst.hip object per (element type, plane
+    """Compile csrc/dwo_host.cpp (the extension module _host.so), csrc/dwo_api.hip and one csrc/dwo_inst.hip object per (element type, plane
     extent) in parallel, then link libdwoconv1d_hip.so into the package directory.  ``only``
     (substrings of object names, e.g. ``["dwo_api", "float_k31_56"]``) recompiles just those
     units and links them with the objects a previous full build left in place."""
@@ -76,6 +93,11 @@ def build(verbose=False, jobs=None, only=None):
                           os.path.join(objdir, "dwo_inst_%s_k%d_%dx%d.o" % (t, K, H, W)),
                           ["-DDWO_INST_T=" + t, "-DDWO_INST_K=%d" % K, "-DDWO_INST_H=%d" % H,
                            "-DDWO_INST_W=%d" % W]))
+    if not only or "dwo_host" in only:
+        _run(host_command(HOST_LIB + ".tmp"), verbose)
+        os.replace(HOST_LIB + ".tmp", HOST_LIB)
+        if only == ["dwo_host"]:
+            return HOST_LIB
     todo = units
     if only:
         todo = [u for u in units if any(tag in os.path.basename(u[1]) for tag in only)]

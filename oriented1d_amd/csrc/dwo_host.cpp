@@ -1,0 +1,256 @@
+// Python entry points of the operator on the host: argument checks, output and scratch allocation,
+// and the calls of libdwoconv1d_hip.so on the tensors' device and current stream.
+//
+// What bounds a call on small tensors is this path (the stage convolutions of ConvNeXt-T at batch
+// 64 take 240 us of GPU time in 12 kernels).  Kept in Python, with one ctypes call, one device query,
+// one stream object and up to four tensor constructions per kernel, forward and backward of one
+// layer took 90 to 170 us of host time, hence native code, without the GIL.  The autograd function
+// itself stays a Python one (its hooks, modes and refusals are PyTorch's own).
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <dlfcn.h>
+#include <torch/extension.h>
+
+#include <stdexcept>
+#include <string>
+#include <tuple>
+
+#include "dwoconv1d_hip.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+
+// the entry points of the library that the Python side has loaded
+struct Library {
+    decltype(&::dwo_status_string) status_string;
+    decltype(&::dwo_taps_bytes) taps_bytes;
+    decltype(&::dwo_fprop) fprop;
+    decltype(&::dwo_dgrad) dgrad;
+    decltype(&::dwo_wgrad_scratch_bytes) wgrad_scratch_bytes;
+    decltype(&::dwo_wgrad) wgrad;
+    decltype(&::dwo_layernorm_nhwc) layernorm_nhwc;
+    decltype(&::dwo_nchw_layernorm_nhwc) nchw_layernorm_nhwc;
+    decltype(&::dwo_nhwc_scale_add_nchw) nhwc_scale_add_nchw;
+} lib;
+
+[[noreturn]] void fail(const std::string &msg) { throw std::runtime_error(msg); }
+
+void bind_library(const std::string &path) {
+    void *h = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+    if (h == nullptr) fail(dlerror());
+    auto find = [h](auto &fn, const char *name) {
+        fn = reinterpret_cast<std::decay_t<decltype(fn)>>(dlsym(h, name));
+        if (fn == nullptr) fail(std::string("missing symbol ") + name);
+    };
+    find(lib.status_string, "dwo_status_string");
+    find(lib.taps_bytes, "dwo_taps_bytes");
+    find(lib.fprop, "dwo_fprop");
+    find(lib.dgrad, "dwo_dgrad");
+    find(lib.wgrad_scratch_bytes, "dwo_wgrad_scratch_bytes");
+    find(lib.wgrad, "dwo_wgrad");
+    find(lib.layernorm_nhwc, "dwo_layernorm_nhwc");
+    find(lib.nchw_layernorm_nhwc, "dwo_nchw_layernorm_nhwc");
+    find(lib.nhwc_scale_add_nchw, "dwo_nhwc_scale_add_nchw");
+}
+
+void check(int status, const char *what) {
+    if (status != 0)
+        fail(std::string(what) + " failed: " + lib.status_string(status) + " (status " +
+             std::to_string(status) + ")");
+}
+
+int dtype_code(const Tensor &t) {
+    switch (t.scalar_type()) {
+        case at::kFloat: return DWO_F32;
+        case at::kBFloat16: return DWO_BF16;
+        case at::kHalf: return DWO_F16;
+        default: return -1;
+    }
+}
+
+// models/dwoconv1d/kernels/kernels.cu:11-13,17-18
+void check_activation(const Tensor &t, const char *name) {
+    if (!t.is_cuda()) fail(std::string(name) + " must be a CUDA tensor");
+    if (!t.is_contiguous()) fail(std::string(name) + " must be contiguous");
+    if (dtype_code(t) < 0)
+        fail(std::string(name) + " has unsupported dtype " +
+             py::cast<std::string>(py::str(py::cast(t).attr("dtype"))));
+    if (t.dim() != 4) fail(std::string(name) + " must be a 4-d tensor");
+}
+
+void check_taps(const Tensor &taps, int64_t C, int64_t K) {
+    const int64_t want = (int64_t)lib.taps_bytes((int)C, (int)K);
+    if (taps.scalar_type() != at::kByte || taps.numel() != want)
+        fail("tap table does not match C=" + std::to_string(C) + ", K=" + std::to_string(K) + " (" +
+             std::to_string(taps.numel()) + " bytes, expected " + std::to_string(want) + ")");
+}
+
+// extents of the input side; sizes beyond int32 saturate, which the library refuses
+struct Dims {
+    int64_t n, c, h, w;
+    Dims(const Tensor &t, bool nhwc)
+        : n(t.size(0)), c(t.size(nhwc ? 3 : 1)), h(t.size(nhwc ? 1 : 2)), w(t.size(nhwc ? 2 : 3)) {}
+};
+int as_int(int64_t v) { return v > 0x7fffffff ? 0x7fffffff : (int)v; }
+int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+std::array<int64_t, 4> shape_of(int64_t n, int64_t c, int64_t h, int64_t w, bool nhwc) {
+    if (nhwc) return {n, h, w, c};
+    return {n, c, h, w};
+}
+
+void check_stride(int64_t stride) {
+    if (stride != 1 && stride != 2 && stride != 4) fail(lib.status_string(DWO_ERR_BAD_STRIDE));
+}
+
+// the weights as [C, K] fp32 rows
+Tensor rows_f32(const Tensor &w, int64_t C) {
+    if (w.scalar_type() == at::kFloat && w.is_contiguous() && C > 0 && w.numel() % C == 0 && w.numel() > 0)
+        return w;
+    return w.detach().reshape({C, -1}).to(at::kFloat).contiguous();
+}
+
+const void *ptr(const Tensor &t) { return t.const_data_ptr(); }
+const float *fptr(const OptTensor &t) {
+    return t.has_value() ? reinterpret_cast<const float *>(t->const_data_ptr()) : nullptr;
+}
+
+// the tensor's device made current, and the current stream there
+struct Place {
+    c10::OptionalDeviceGuard guard;
+    void *stream;
+    explicit Place(const Tensor &t) : guard(t.device()) {
+        stream = c10::hip::getCurrentHIPStream(t.device().index()).stream();
+    }
+};
+
+Tensor fprop(const Tensor &x, const Tensor &w, const Tensor &taps, int64_t stride, const OptTensor &bias,
+             bool nhwc) {
+    check_activation(x, "x");
+    check_stride(stride);
+    const Dims d(x, nhwc);
+    const Tensor w2 = rows_f32(w, d.c);
+    const int64_t K = w2.numel() / std::max<int64_t>(d.c, 1);
+    check_taps(taps, d.c, K);
+    py::gil_scoped_release nogil;
+    const Place at(x);
+    Tensor y = at::empty(shape_of(d.n, d.c, up(d.h, stride), up(d.w, stride), nhwc), x.options());
+    check(lib.fprop(ptr(x), (const float *)ptr(w2), fptr(bias), ptr(taps), y.data_ptr(), as_int(d.n),
+                    as_int(d.c), as_int(d.h), as_int(d.w), as_int(K), as_int(stride), dtype_code(x), nhwc,
+                    at.stream),
+          "dwo_fprop");
+    return y;
+}
+
+Tensor dgrad(const Tensor &dy, const Tensor &w, const Tensor &taps, int64_t H, int64_t W, int64_t stride,
+             bool nhwc) {
+    check_activation(dy, "dy");
+    check_stride(stride);
+    const Dims d(dy, nhwc);
+    if (d.h != up(H, stride) || d.w != up(W, stride)) fail("dy extent does not match the input extent and stride");
+    const Tensor w2 = rows_f32(w, d.c);
+    const int64_t K = w2.numel() / std::max<int64_t>(d.c, 1);
+    check_taps(taps, d.c, K);
+    py::gil_scoped_release nogil;
+    const Place at(dy);
+    Tensor dx = at::empty(shape_of(d.n, d.c, H, W, nhwc), dy.options());
+    check(lib.dgrad(ptr(dy), (const float *)ptr(w2), ptr(taps), dx.data_ptr(), as_int(d.n), as_int(d.c),
+                    as_int(H), as_int(W), as_int(K), as_int(stride), dtype_code(dy), nhwc, at.stream),
+          "dwo_dgrad");
+    return dx;
+}
+
+std::tuple<Tensor, OptTensor> wgrad(const Tensor &dy, const Tensor &x, const Tensor &taps, int64_t K,
+                                    int64_t stride, bool nhwc, bool with_bias) {
+    check_activation(dy, "dy");
+    check_activation(x, "x");
+    check_stride(stride);
+    if (dy.scalar_type() != x.scalar_type()) fail("dy and x must have the same dtype");
+    const Dims d(x, nhwc);
+    const auto want = shape_of(d.n, d.c, up(d.h, stride), up(d.w, stride), nhwc);
+    if (dy.sizes() != at::IntArrayRef(want)) fail("dy extent does not match the input extent and stride");
+    check_taps(taps, d.c, K);
+    py::gil_scoped_release nogil;
+    const Place at(x);
+    const int n = as_int(d.n), c = as_int(d.c), h = as_int(d.h), wd = as_int(d.w), k = as_int(K),
+              s = as_int(stride), dt = dtype_code(x);
+    const size_t nbytes = lib.wgrad_scratch_bytes(n, c, h, wd, k, s, dt, nhwc);
+    const Tensor scratch = at::empty({(int64_t)std::max<size_t>(nbytes, 16)}, x.options().dtype(at::kByte));
+    const auto f32 = x.options().dtype(at::kFloat);
+    Tensor dw = at::empty({d.c, 1, 1, K}, f32);
+    OptTensor db;
+    if (with_bias) db = at::empty({d.c}, f32);
+    check(lib.wgrad(ptr(dy), ptr(x), ptr(taps), (float *)dw.data_ptr(), db.has_value() ? (float *)db->data_ptr() : nullptr,
+                    scratch.data_ptr(), nbytes, n, c, h, wd, k, s, dt, nhwc, at.stream),
+          "dwo_wgrad");
+    return {dw, db};
+}
+
+void check_glue(const Tensor &t, const char *name) {
+    if (!t.is_cuda() || dtype_code(t) < 0)
+        fail(std::string(name) + " must be a CUDA tensor of type float32, bfloat16 or float16");
+}
+
+Tensor layernorm_nhwc(const Tensor &x_, const Tensor &g, const Tensor &b, double eps, bool gelu) {
+    check_glue(x_, "x");
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const Tensor x = x_.contiguous();
+    const int64_t C = x.size(-1);
+    Tensor out = at::empty_like(x);
+    check(lib.layernorm_nhwc(ptr(x), (const float *)ptr(g), (const float *)ptr(b), out.data_ptr(),
+                             (size_t)(x.numel() / std::max<int64_t>(C, 1)), as_int(C), (float)eps, gelu,
+                             dtype_code(x), at.stream),
+          "dwo_layernorm_nhwc");
+    return out;
+}
+
+Tensor nchw_layernorm_nhwc(const Tensor &x_, const Tensor &g, const Tensor &b, double eps) {
+    check_glue(x_, "x");
+    if (x_.dim() != 4) throw py::value_error("x must be a 4-d tensor");
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const Tensor x = x_.contiguous();
+    const Dims d(x, false);
+    Tensor out = at::empty({d.n, d.h, d.w, d.c}, x.options());
+    check(lib.nchw_layernorm_nhwc(ptr(x), (const float *)ptr(g), (const float *)ptr(b), out.data_ptr(),
+                                  as_int(d.n), as_int(d.c), as_int(d.h), as_int(d.w), (float)eps, dtype_code(x),
+                                  at.stream),
+          "dwo_nchw_layernorm_nhwc");
+    return out;
+}
+
+Tensor nhwc_scale_add_nchw(const Tensor &y_, const OptTensor &scale, const OptTensor &residual) {
+    check_glue(y_, "y");
+    if (y_.dim() != 4) throw py::value_error("y must be a 4-d tensor");
+    py::gil_scoped_release nogil;
+    const Place at(y_);
+    const Tensor y = y_.contiguous();
+    const Dims d(y, true);
+    Tensor res;
+    if (residual.has_value()) {
+        const std::array<int64_t, 4> want = {d.n, d.c, d.h, d.w};
+        if (residual->sizes() != at::IntArrayRef(want) || residual->scalar_type() != y.scalar_type())
+            fail("residual must be [N,C,H,W] of the same type as y");
+        res = residual->contiguous();
+    }
+    Tensor out = at::empty({d.n, d.c, d.h, d.w}, y.options());
+    check(lib.nhwc_scale_add_nchw(ptr(y), fptr(scale), res.defined() ? ptr(res) : nullptr, out.data_ptr(),
+                                  as_int(d.n), as_int(d.c), as_int(d.h), as_int(d.w), dtype_code(y), at.stream),
+          "dwo_nhwc_scale_add_nchw");
+    return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+    m.def("bind", &bind_library);
+    m.def("fprop", &fprop);
+    m.def("dgrad", &dgrad);
+    m.def("wgrad", &wgrad);
+    m.def("layernorm_nhwc", &layernorm_nhwc);
+    m.def("nchw_layernorm_nhwc", &nchw_layernorm_nhwc);
+    m.def("nhwc_scale_add_nchw", &nhwc_scale_add_nchw);
+}

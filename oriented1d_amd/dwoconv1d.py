@@ -35,10 +35,6 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else None
 
 
-def _stream(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
-
-
 def _check_activation(t, name):
     # models/dwoconv1d/kernels/kernels.cu:11-13,17-18
     if not t.is_cuda:
@@ -90,7 +86,7 @@ class _TapCache:
         self.entries = {}  # (id(theta), device, C, K) -> (state key, weak ref, device blob)
 
     def get(self, theta, C, K, device):
-        slot = (id(theta), str(device), C, K)
+        slot = (id(theta), device, C, K)
         state = (theta.data_ptr(), theta._version)
         hit = self.entries.get(slot)
         if hit is None or hit[0] != state or hit[1]() is not theta:
@@ -102,32 +98,12 @@ class _TapCache:
         return hit[2]
 
 
-def _check_taps(taps, C, K):
-    """The device kernels index the tap blob with the C and K they are launched with and cannot
-    see its header without a device read, so the size is checked here: a blob of
-    ``dwo_taps_bytes(C, K)`` bytes keeps every table read in range."""
-    want = _lib.load().dwo_taps_bytes(C, K)
-    if taps.dtype != torch.uint8 or taps.numel() != want:
-        raise RuntimeError("tap table does not match C=%d, K=%d (%d bytes, expected %d)"
-                           % (C, K, taps.numel(), want))
-
-
 def _dims(x, nhwc):
     if nhwc:
         N, H, W, C = x.shape
     else:
         N, C, H, W = x.shape
     return N, C, H, W
-
-
-def _out_shape(N, C, H, W, stride, nhwc):
-    P, Q = -(-H // stride), -(-W // stride)
-    return (N, P, Q, C) if nhwc else (N, C, P, Q)
-
-
-def _w2d(w, C):
-    w = w.detach().reshape(C, -1)
-    return w.to(torch.float32).contiguous()
 
 
 _F32_COPIES = {}  # id(parameter) -> (weak reference, state key, fp32 copy)
@@ -151,57 +127,19 @@ def f32_copy(p):
 
 def fprop(x, w, taps, stride=1, bias=None, nhwc=False):
     """y = fprop(x, w, theta) (+ bias).  x: [N,C,H,W] or [N,H,W,C]; w: [C,1,1,K]."""
-    _check_activation(x, "x")
-    lib = _lib.ready(x.device)
-    N, C, H, W = _dims(x, nhwc)
-    w2 = _w2d(w, C)
-    K = w2.shape[1]
-    _check_taps(taps, C, K)
     b = f32_copy(bias) if bias is not None else None
-    y = torch.empty(_out_shape(N, C, H, W, stride, nhwc), dtype=x.dtype, device=x.device)
-    _lib.check(_lib.launch(x.device, lib.dwo_fprop, _ptr(x), _ptr(w2), _ptr(b), _ptr(taps), _ptr(y),
-                           N, C, H, W, K, stride, _DTYPES[x.dtype], int(nhwc), _stream(x)),
-               "dwo_fprop")
-    return y
+    return _lib.host(x.get_device()).fprop(x, w, taps, stride, b, nhwc)
 
 
 def dgrad(dy, w, taps, in_hw, stride=1, nhwc=False):
     """dx = dgrad(dy, w, theta); ``in_hw`` is the (H, W) of the forward input."""
-    _check_activation(dy, "dy")
-    lib = _lib.ready(dy.device)
     H, W = in_hw
-    N, C, P, Q = _dims(dy, nhwc)
-    if (P, Q) != (-(-H // stride), -(-W // stride)):
-        raise RuntimeError("dy extent does not match the input extent and stride")
-    w2 = _w2d(w, C)
-    K = w2.shape[1]
-    _check_taps(taps, C, K)
-    dx = torch.empty((N, H, W, C) if nhwc else (N, C, H, W), dtype=dy.dtype, device=dy.device)
-    _lib.check(_lib.launch(dy.device, lib.dwo_dgrad, _ptr(dy), _ptr(w2), _ptr(taps), _ptr(dx), N, C,
-                           H, W, K, stride, _DTYPES[dy.dtype], int(nhwc), _stream(dy)), "dwo_dgrad")
-    return dx
+    return _lib.host(dy.get_device()).dgrad(dy, w, taps, H, W, stride, nhwc)
 
 
 def wgrad(dy, x, taps, K, stride=1, nhwc=False, with_bias=False):
     """(dw [C,1,1,K] fp32, db [C] fp32 or None) = wgrad(dy, x, theta)."""
-    _check_activation(dy, "dy")
-    _check_activation(x, "x")
-    lib = _lib.ready(x.device)
-    if dy.dtype != x.dtype:
-        raise RuntimeError("dy and x must have the same dtype")
-    N, C, H, W = _dims(x, nhwc)
-    if tuple(dy.shape) != _out_shape(N, C, H, W, stride, nhwc):
-        raise RuntimeError("dy extent does not match the input extent and stride")
-    _check_taps(taps, C, K)
-    dt, lay = _DTYPES[x.dtype], int(nhwc)
-    nbytes = lib.dwo_wgrad_scratch_bytes(N, C, H, W, K, stride, dt, lay)
-    scratch = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
-    dw = torch.empty((C, 1, 1, K), dtype=torch.float32, device=x.device)
-    db = torch.empty((C,), dtype=torch.float32, device=x.device) if with_bias else None
-    _lib.check(_lib.launch(x.device, lib.dwo_wgrad, _ptr(dy), _ptr(x), _ptr(taps), _ptr(dw), _ptr(db),
-                           _ptr(scratch), nbytes, N, C, H, W, K, stride, dt, lay, _stream(x)),
-               "dwo_wgrad")
-    return dw, db
+    return _lib.host(x.get_device()).wgrad(dy, x, taps, K, stride, nhwc, with_bias)
 
 
 class KernelTuple(tuple):
@@ -256,7 +194,7 @@ class _DepthwiseOrientedConv1d(torch.autograd.Function):
             w_eff = w_eff + resid.to(w_eff)
         x = x.contiguous()
         _check_activation(x, "x")
-        N, Cx, H, W = _dims(x, nhwc)
+        _, Cx, H, W = _dims(x, nhwc)
         if Cx != C:
             raise RuntimeError("input has %d channels, weight has %d" % (Cx, C))
         if not module.arbitrary_size and (H % stride != 0 or W % stride != 0):
@@ -319,9 +257,10 @@ class _DepthwiseOrientedConv1d(torch.autograd.Function):
         need_db = ctx.with_bias and ctx.needs_input_grad[3]
         if ctx.needs_input_grad[1]:
             dw, db32 = wgrad(dy, x, taps, ctx.K, ctx.stride, nhwc=ctx.nhwc, with_bias=need_db)
-            dw = dw.to(ctx.w_dtype)
+            if ctx.w_dtype != torch.float32:
+                dw = dw.to(ctx.w_dtype)
             if need_db:
-                db = db32.to(ctx.b_dtype)
+                db = db32 if ctx.b_dtype == torch.float32 else db32.to(ctx.b_dtype)
         elif need_db:
             red = [0, 1, 2] if ctx.nhwc else [0, 2, 3]
             db = dy.sum(dim=red, dtype=torch.float32).to(ctx.b_dtype)

@@ -36,49 +36,19 @@ def usable(x, C, tiled):
 
 def layernorm_nhwc(x, weight, bias, eps, gelu=False):
     """LayerNorm over the last dimension of a contiguous tensor (+ exact GELU)."""
-    if not x.is_cuda or x.dtype not in _DTYPES:
-        raise RuntimeError("x must be a CUDA tensor of type float32, bfloat16 or float16")
-    x = x.contiguous()
-    C = x.shape[-1]
-    out = torch.empty_like(x)
-    g, b = _f32(weight), _f32(bias)  # held until the launch is queued
-    _lib.check(_lib.load().dwo_layernorm_nhwc(
-        _ptr(x), _ptr(g), _ptr(b), _ptr(out), x.numel() // C, C, float(eps), int(gelu),
-        _DTYPES[x.dtype], _stream(x)), "dwo_layernorm_nhwc")
-    return out
+    return _lib.host(x.get_device()).layernorm_nhwc(x, _f32(weight), _f32(bias), eps, gelu)
 
 
 def nchw_layernorm_nhwc(x, weight, bias, eps):
     """[N,C,H,W] -> [N,H,W,C], LayerNorm over C: ``norm(x.permute(0, 2, 3, 1))`` in one pass."""
-    if not x.is_cuda or x.dtype not in _DTYPES:
-        raise RuntimeError("x must be a CUDA tensor of type float32, bfloat16 or float16")
-    x = x.contiguous()
-    N, C, H, W = x.shape
-    out = torch.empty((N, H, W, C), dtype=x.dtype, device=x.device)
-    g, b = _f32(weight), _f32(bias)
-    _lib.check(_lib.load().dwo_nchw_layernorm_nhwc(
-        _ptr(x), _ptr(g), _ptr(b), _ptr(out), N, C, H, W, float(eps), _DTYPES[x.dtype],
-        _stream(x)), "dwo_nchw_layernorm_nhwc")
-    return out
+    return _lib.host(x.get_device()).nchw_layernorm_nhwc(x, _f32(weight), _f32(bias), eps)
 
 
 def nhwc_scale_add_nchw(y, scale=None, residual=None):
     """[N,H,W,C] -> [N,C,H,W]: ``residual + (scale * y).permute(0, 3, 1, 2)`` in one pass
     (``scale`` [C] and ``residual`` [N,C,H,W] optional)."""
-    if not y.is_cuda or y.dtype not in _DTYPES:
-        raise RuntimeError("y must be a CUDA tensor of type float32, bfloat16 or float16")
-    y = y.contiguous()
-    N, H, W, C = y.shape
-    if residual is not None:
-        if tuple(residual.shape) != (N, C, H, W) or residual.dtype != y.dtype:
-            raise RuntimeError("residual must be [N,C,H,W] of the same type as y")
-        residual = residual.contiguous()
-    out = torch.empty((N, C, H, W), dtype=y.dtype, device=y.device)
     sc = _f32(scale) if scale is not None else None
-    _lib.check(_lib.load().dwo_nhwc_scale_add_nchw(
-        _ptr(y), _ptr(sc), _ptr(residual), _ptr(out), N, C, H, W, _DTYPES[y.dtype], _stream(y)),
-        "dwo_nhwc_scale_add_nchw")
-    return out
+    return _lib.host(y.get_device()).nhwc_scale_add_nchw(y, sc, residual)
 
 
 def pointwise_dwconv_nhwc(x, linear, conv):
