@@ -200,6 +200,17 @@ int dwo_nchw_layernorm_nhwc(const void *x, const float *gamma, const float *beta
 int dwo_nhwc_scale_add_nchw(const void *y, const float *scale, const void *res, void *out, int N,
                             int C, int H, int W, int dtype, void *stream);
 
+/*
+ * Parameter gradients of a pointwise layer with few inputs (the stem's first layer,
+ * models/convnext.py:143,177): dw[c,k] = sum_p dy[p,c] * x[p,k], db[c] = sum_p dy[p,c] (db may be
+ * null), fp32, for x [rows,Cin], dy [rows,C] of one type, Cin in {1,2,3,4}.  dy is 16-byte aligned and C a
+ * multiple of 16 bytes' worth of channels, at most 256 such pieces.  scratch holds at least
+ * dwo_pointwise_wgrad_scratch_bytes(Cin, C) bytes.
+ */
+size_t dwo_pointwise_wgrad_scratch_bytes(int Cin, int C);
+int dwo_pointwise_wgrad(const void *dy, const void *x, float *dw, float *db, void *scratch, size_t scratch_bytes,
+                        size_t rows, int Cin, int C, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -30,6 +30,8 @@ SIGNATURES = {
     "dwo_layernorm_nhwc": (_i, [_vp, _vp, _vp, _vp, _sz, _i, ctypes.c_float, _i, _i, _vp]),
     "dwo_nchw_layernorm_nhwc": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, ctypes.c_float, _i, _vp]),
     "dwo_nhwc_scale_add_nchw": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
+    "dwo_pointwise_wgrad_scratch_bytes": (_sz, [_i, _i]),
+    "dwo_pointwise_wgrad": (_i, [_vp] * 5 + [_sz, _sz] + [_i] * 3 + [_vp]),
 }
 
 _lib = None

@@ -96,13 +96,20 @@ class StochasticDepth(nn.Module):
         return x * keep / (1.0 - self.p)
 
 
+class PointwiseLinear(nn.Linear):
+    """The stem's first layer, 3 -> dim1 at every pixel of the image."""
+
+    def forward(self, x):
+        return fused.pointwise_linear(x, self)
+
+
 class Stem1D(nn.Module):
     """3 -> dim1 pointwise, two stride-2 oriented convs (NHWC) with LayerNorm + GELU, dim1 -> dim2
     pointwise, LayerNorm; NCHW in, NCHW out at 1/4 resolution (models/convnext.py:132-191)."""
 
     def __init__(self, dim0, dim1, dim2, kernel_size, arbitrary_size=False, wrapped=False):
         super().__init__()
-        self.pw1 = nn.Linear(dim0, dim1)
+        self.pw1 = PointwiseLinear(dim0, dim1)
         self.pw2 = nn.Linear(dim1, dim2)
         pad = (kernel_size - 2) // 2  # shapes the parent Conv2d only; compute pads K // 2
         self.dw1 = oriented_conv(dim1, kernel_size, stride=2, padding=pad, nhwc=True,

@@ -16,6 +16,7 @@
 #include "dwo_nhwc_tile.h"
 #include "dwo_window_dispatch.h"
 #include "dwo_fused.h"
+#include "dwo_pointwise.h"
 
 using namespace dwo;
 
@@ -438,6 +439,18 @@ int pointwise_fprop_t(const void *x, const float *pw_w, const float *pw_b, const
     }
 }
 
+template <typename T>
+int pointwise_wgrad_t(const void *dy, const void *x, float *dw, float *db, float *part, size_t rows, int Cin,
+                      int C, hipStream_t st) {
+    if (C % Piece<T>::N != 0 || C / Piece<T>::N > kPwThreads) return DWO_ERR_BAD_SHAPE;
+    switch (Cin) {
+        case 1: return launch_pointwise_wgrad<T, 1>(dy, x, dw, db, part, rows, C, st);
+        case 2: return launch_pointwise_wgrad<T, 2>(dy, x, dw, db, part, rows, C, st);
+        case 3: return launch_pointwise_wgrad<T, 3>(dy, x, dw, db, part, rows, C, st);
+        default: return launch_pointwise_wgrad<T, 4>(dy, x, dw, db, part, rows, C, st);
+    }
+}
+
 int wgrad_dispatch(const void *dy, const void *x, const void *taps, float *dw, float *db,
                    void *scratch, int N, int C, int H, int W, int K, int stride, int dtype,
                    int layout, hipStream_t st) {
@@ -712,6 +725,28 @@ int dwo_pointwise_fprop_nhwc(const void *x, const float *pw_w, const float *pw_b
         case DWO_F32: return pointwise_fprop_t<float>(x, pw_w, pw_b, w, bias, taps, y, Cin, d, st);
         case DWO_BF16: return pointwise_fprop_t<bf16_t>(x, pw_w, pw_b, w, bias, taps, y, Cin, d, st);
         default: return pointwise_fprop_t<f16_t>(x, pw_w, pw_b, w, bias, taps, y, Cin, d, st);
+    }
+}
+
+size_t dwo_pointwise_wgrad_scratch_bytes(int Cin, int C) {
+    if (Cin < 1 || Cin > kPwMaxCin || C < 1) return 0;
+    return (size_t)C * (Cin + 1) * kPwBlocks * sizeof(float);
+}
+
+int dwo_pointwise_wgrad(const void *dy, const void *x, float *dw, float *db, void *scratch, size_t scratch_bytes,
+                        size_t rows, int Cin, int C, int dtype, void *stream) {
+    if (!dy || !x || !dw || !scratch) return DWO_ERR_NULL_POINTER;
+    if (rows < 1 || rows > (size_t)1 << 40 || Cin < 1 || Cin > kPwMaxCin || C < 1 || (uintptr_t)dy % 16 != 0)
+        return DWO_ERR_BAD_SHAPE;
+    if (scratch_bytes < dwo_pointwise_wgrad_scratch_bytes(Cin, C)) return DWO_ERR_SCRATCH_TOO_SMALL;
+    hipStream_t st = (hipStream_t)stream;
+    float *part = (float *)scratch;
+    begin_call();
+    switch (dtype) {
+        case DWO_F32: return pointwise_wgrad_t<float>(dy, x, dw, db, part, rows, Cin, C, st);
+        case DWO_BF16: return pointwise_wgrad_t<bf16_t>(dy, x, dw, db, part, rows, Cin, C, st);
+        case DWO_F16: return pointwise_wgrad_t<f16_t>(dy, x, dw, db, part, rows, Cin, C, st);
+        default: return DWO_ERR_BAD_DTYPE;
     }
 }
 

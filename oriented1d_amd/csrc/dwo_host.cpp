@@ -33,6 +33,8 @@ struct Library {
     decltype(&::dwo_layernorm_nhwc) layernorm_nhwc;
     decltype(&::dwo_nchw_layernorm_nhwc) nchw_layernorm_nhwc;
     decltype(&::dwo_nhwc_scale_add_nchw) nhwc_scale_add_nchw;
+    decltype(&::dwo_pointwise_wgrad_scratch_bytes) pointwise_wgrad_scratch_bytes;
+    decltype(&::dwo_pointwise_wgrad) pointwise_wgrad;
 } lib;
 
 [[noreturn]] void fail(const std::string &msg) { throw std::runtime_error(msg); }
@@ -53,6 +55,8 @@ void bind_library(const std::string &path) {
     find(lib.layernorm_nhwc, "dwo_layernorm_nhwc");
     find(lib.nchw_layernorm_nhwc, "dwo_nchw_layernorm_nhwc");
     find(lib.nhwc_scale_add_nchw, "dwo_nhwc_scale_add_nchw");
+    find(lib.pointwise_wgrad_scratch_bytes, "dwo_pointwise_wgrad_scratch_bytes");
+    find(lib.pointwise_wgrad, "dwo_pointwise_wgrad");
 }
 
 void check(int status, const char *what) {
@@ -243,6 +247,31 @@ Tensor nhwc_scale_add_nchw(const Tensor &y_, const OptTensor &scale, const OptTe
     return out;
 }
 
+// dy [.., C] and x [.., Cin] of one type, contiguous
+std::tuple<Tensor, OptTensor> pointwise_wgrad(const Tensor &dy, const Tensor &x, bool with_bias) {
+    check_glue(dy, "dy");
+    if (!dy.is_contiguous() || !x.is_contiguous() || x.device() != dy.device() ||
+        dy.scalar_type() != x.scalar_type())
+        fail("dy and x must be contiguous, on one device and of one type");
+    if (dy.dim() < 1 || x.dim() != dy.dim() || x.sizes().slice(0, x.dim() - 1) != dy.sizes().slice(0, dy.dim() - 1))
+        fail("dy and x must have the same pixels");
+    const int64_t C = dy.size(-1), Cin = x.size(-1);
+    py::gil_scoped_release nogil;
+    const Place at(dy);
+    const size_t nbytes = lib.pointwise_wgrad_scratch_bytes(as_int(Cin), as_int(C));
+    const Tensor scratch = at::empty({(int64_t)std::max<size_t>(nbytes, 16)}, dy.options().dtype(at::kByte));
+    const auto f32 = dy.options().dtype(at::kFloat);
+    Tensor dw = at::empty({C, Cin}, f32);
+    OptTensor db;
+    if (with_bias) db = at::empty({C}, f32);
+    check(lib.pointwise_wgrad(ptr(dy), ptr(x), (float *)dw.data_ptr(),
+                              db.has_value() ? (float *)db->data_ptr() : nullptr, scratch.data_ptr(), nbytes,
+                              (size_t)(dy.numel() / std::max<int64_t>(C, 1)), as_int(Cin), as_int(C),
+                              dtype_code(dy), at.stream),
+          "dwo_pointwise_wgrad");
+    return {dw, db};
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -250,6 +279,7 @@ PYBIND11_MODULE(_host, m) {
     m.def("fprop", &fprop);
     m.def("dgrad", &dgrad);
     m.def("wgrad", &wgrad);
+    m.def("pointwise_wgrad", &pointwise_wgrad);
     m.def("layernorm_nhwc", &layernorm_nhwc);
     m.def("nchw_layernorm_nhwc", &nchw_layernorm_nhwc);
     m.def("nhwc_scale_add_nchw", &nhwc_scale_add_nchw);

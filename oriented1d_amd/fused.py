@@ -6,6 +6,7 @@ gradient is being recorded; with autograd on it composes the same values from Py
 import ctypes
 
 import torch
+import torch.nn.functional as F
 
 from . import _lib
 
@@ -49,6 +50,53 @@ def nhwc_scale_add_nchw(y, scale=None, residual=None):
     (``scale`` [C] and ``residual`` [N,C,H,W] optional)."""
     sc = _f32(scale) if scale is not None else None
     return _lib.host(y.get_device()).nhwc_scale_add_nchw(y, sc, residual)
+
+
+class _PointwiseLinear(torch.autograd.Function):
+    """``F.linear`` whose parameter gradients come from the library: with a few input channels
+    and every pixel of a batch as rows they are a reduction, not a matrix product."""
+
+    @staticmethod
+    def forward(ctx, x, w, b):
+        ctx.set_materialize_grads(False)
+        y = F.linear(x, w, b)
+        ctx.save_for_backward(x if x.dtype == y.dtype else x.to(y.dtype), w, b)
+        ctx.x_dtype = x.dtype
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        if dy is None:
+            return None, None, None
+        x, w, b = ctx.saved_tensors
+        dx = dw = db = None
+        if ctx.needs_input_grad[0]:
+            dx = torch.matmul(dy, w.to(dy.dtype)).to(ctx.x_dtype)
+        need_db = b is not None and ctx.needs_input_grad[2]
+        if ctx.needs_input_grad[1] or need_db:
+            dy, x = dy.contiguous(), x.contiguous()
+            if torch.is_grad_enabled() or dy.data_ptr() % 16 != 0 or dy.dtype != x.dtype:
+                # gradients of gradients, or a piece of another buffer
+                rows = dy.reshape(-1, dy.shape[-1])
+                dw = torch.matmul(rows.t(), x.reshape(-1, x.shape[-1]).to(rows.dtype))
+                db = rows.sum(0)
+            else:
+                dw, db = _lib.host(dy.get_device()).pointwise_wgrad(dy, x, need_db)
+            dw = dw.to(w.dtype) if ctx.needs_input_grad[1] else None
+            db = db.to(b.dtype) if need_db else None
+        return dx, dw, db
+
+
+def pointwise_linear(x, linear):
+    """``linear(x)`` of an ``nn.Linear`` with at most four inputs; where its parameters are being
+    trained on a GPU, with the parameter gradients of ``dwo_pointwise_wgrad``."""
+    w, b = linear.weight, linear.bias
+    dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
+    if (torch.is_grad_enabled() and w.requires_grad and x.is_cuda and w.device == x.device and x.numel() > 0
+            and dtype in _DTYPES and x.dtype in _DTYPES and 1 <= x.shape[-1] <= 4
+            and w.shape[0] * dtype.itemsize % 16 == 0 and w.shape[0] * dtype.itemsize <= 4096):
+        return _PointwiseLinear.apply(x, w, b)
+    return F.linear(x, w, b)
 
 
 def pointwise_dwconv_nhwc(x, linear, conv):

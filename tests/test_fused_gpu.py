@@ -151,3 +151,33 @@ def test_bf16_network_fused_equal_unfused_and_parameter_copies_refresh():
     y_plain2 = m(x).detach()
     _close(y_fused2, y_plain2, torch.bfloat16, "bf16 network after update")
     assert not torch.equal(y_fused, y_fused2)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("shape,cin", [((1, 1, 1, 8), 1), ((2, 9, 13, 64), 3), ((1, 40, 50, 24), 2),
+                                       ((2, 224, 224, 64), 3), ((1, 7, 5, 1024), 4)])
+def test_pointwise_linear_gradients(shape, cin, dtype):
+    """dw and db of a layer with few inputs; sums of P terms in fp32 in another order: the bound is
+    the rounding of the largest partial sums, sqrt(P) * 2^-24 relative to the sums' own spread
+    sqrt(P), far below 1e-5; 16-bit results are rounded once."""
+    torch.manual_seed(cin)
+    C = shape[-1]
+    x = torch.randn(*shape[:-1], cin, device="cuda").to(dtype)
+    lin = torch.nn.Linear(cin, C).cuda().to(dtype)
+    dy = torch.randn(*shape, device="cuda").to(dtype)
+    y = fused.pointwise_linear(x, lin)
+    assert torch.equal(y, lin(x)) and type(y.grad_fn).__name__ == "_PointwiseLinearBackward"
+    dw, db = torch.autograd.grad(y, (lin.weight, lin.bias), dy)
+    rows, xs = dy.double().reshape(-1, C), x.double().reshape(-1, cin)
+    _close(dw, rows.t() @ xs, dtype, "dw")
+    _close(db, rows.sum(0), dtype, "db")
+    # gradients of gradients, input gradients and a view of another buffer: as nn.Linear has them
+    xg, buf = x.clone().requires_grad_(), torch.cat([dy.reshape(-1)[:1], dy.reshape(-1)])
+    odd = buf[1:].view(shape)
+    for layer in (fused.pointwise_linear, lambda a, m: m(a)):
+        g = torch.autograd.grad(layer(xg, lin), (xg, lin.weight, lin.bias), odd, create_graph=True)
+        gg = torch.autograd.grad(g[1].double().sum(), xg)[0]
+        if layer is fused.pointwise_linear:
+            first = g + (gg,)
+    for a, b in zip(first, g + (gg,)):
+        _close(a.detach(), b.detach(), dtype, "second order")
