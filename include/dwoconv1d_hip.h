@@ -69,6 +69,11 @@ extern "C" {
 
 #define DWO_NCHW 0
 #define DWO_NHWC 1
+/* Added to DWO_NHWC: dwo_taps_grouped() returned 1 for the tap table and this element type, i.e. the channels
+ * of every aligned 16 bytes share one orientation.  Such calls may take kernels that work on whole
+ * pieces (other results' rounding, same precision); a table it does not hold for is slow, not wrong.  The
+ * scratch of dwo_wgrad is sized with the layout of the call. */
+#define DWO_GROUPED 2
 
 /* Library version (major*10000 + minor*100 + patch). */
 int dwo_version(void);
@@ -94,6 +99,10 @@ int dwo_init(void);
  */
 size_t dwo_taps_bytes(int C, int K);
 int dwo_build_taps(const float *theta_host, int C, int K, void *taps_host);
+
+/* 1 when every run of `channels` channels (aligned, C a multiple) of a host blob shares one of the eight
+ * compile-time orientations, else 0; channels = 16 / element size for DWO_GROUPED. */
+int dwo_taps_grouped(const void *taps_host, int channels);
 
 /* Debug/inspection helper: (dh,dw) of channel c, tap s from a host blob. */
 int dwo_taps_get(const void *taps_host, int c, int s, int *dh, int *dw);

@@ -8,7 +8,7 @@ LIB_PATH = os.environ.get("DWOCONV1D_LIB") or os.path.join(HERE, "libdwoconv1d_h
 HOST_PATH = os.path.join(HERE, "_host.so")
 
 F32, BF16, F16 = 0, 1, 2
-NCHW, NHWC = 0, 1
+NCHW, NHWC, GROUPED = 0, 1, 2
 
 _vp, _i, _sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t
 
@@ -19,6 +19,7 @@ SIGNATURES = {
     "dwo_init": (_i, []),
     "dwo_taps_bytes": (_sz, [_i, _i]),
     "dwo_build_taps": (_i, [_vp, _i, _i, _vp]),
+    "dwo_taps_grouped": (_i, [_vp, _i]),
     "dwo_taps_get": (_i, [_vp, _i, _i, ctypes.POINTER(_i), ctypes.POINTER(_i)]),
     "dwo_fprop": (_i, [_vp, _vp, _vp, _vp, _vp] + [_i] * 8 + [_vp]),
     "dwo_dgrad": (_i, [_vp, _vp, _vp, _vp] + [_i] * 8 + [_vp]),

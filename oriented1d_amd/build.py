@@ -37,7 +37,7 @@ PLANE_SHAPES = [(31, 56, 56), (31, 28, 28), (31, 14, 14), (31, 7, 7),
                 (7, 56, 56), (7, 28, 28), (7, 14, 14),
                 (31, 64, 64), (31, 32, 32), (31, 16, 16)]  # = DWO_PLANE_SHAPES
 PLANE_TYPES = ["float", "bf16_t", "f16_t"]
-WINDOW_KS = [7, 13, 15, 27, 31]  # = DWO_WINDOW_KS
+WINDOW_KS = [7, 13, 15, 27, 31]  # = DWO_WINDOW_KS = DWO_GROUPED_KS
 
 
 def _run(cmd, verbose):
@@ -82,9 +82,10 @@ def build(verbose=False, jobs=None, only=None):
     units = [(os.path.join(CSRC, "dwo_api.hip"), os.path.join(objdir, "dwo_api.o"), [])]
     for K in sorted(WINDOW_KS, reverse=True):
         for t in PLANE_TYPES:
-            units.append((os.path.join(CSRC, "dwo_inst_window.hip"),
-                          os.path.join(objdir, "dwo_window_%s_k%d.o" % (t, K)),
-                          ["-DDWO_INST_T=" + t, "-DDWO_INST_K=%d" % K]))
+            for family in ("window", "grouped"):
+                units.append((os.path.join(CSRC, "dwo_inst_%s.hip" % family),
+                              os.path.join(objdir, "dwo_%s_%s_k%d.o" % (family, t, K)),
+                              ["-DDWO_INST_T=" + t, "-DDWO_INST_K=%d" % K]))
     # longest translation units first (the register-plane extents, then the largest planes): the
     # build ends when the last worker does
     for K, H, W in sorted(PLANE_SHAPES, key=lambda s: (s[1] > 16, -s[0], -s[1] if s[1] > 16 else s[1])):

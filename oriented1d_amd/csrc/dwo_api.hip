@@ -15,6 +15,7 @@
 #include "dwo_dispatch.h"
 #include "dwo_nhwc_tile.h"
 #include "dwo_window_dispatch.h"
+#include "dwo_grouped_dispatch.h"
 #include "dwo_fused.h"
 #include "dwo_pointwise.h"
 
@@ -30,12 +31,15 @@ int check_common(int N, int C, int H, int W, int K, int stride, int dtype, int l
     if (K < 1 || K > DWO_MAX_K || (K & 1) == 0) return DWO_ERR_BAD_KERNEL;
     if (log2_stride(stride) < 0) return DWO_ERR_BAD_STRIDE;
     if (dtype != DWO_F32 && dtype != DWO_BF16 && dtype != DWO_F16) return DWO_ERR_BAD_DTYPE;
-    if (layout != DWO_NCHW && layout != DWO_NHWC) return DWO_ERR_BAD_LAYOUT;
+    if (layout != DWO_NCHW && layout != DWO_NHWC && layout != (DWO_NHWC | DWO_GROUPED)) return DWO_ERR_BAD_LAYOUT;
     return DWO_OK;
 }
 
-ConvDims make_dims(int N, int C, int H, int W, int K, int stride) {
+// (splits DWO_GROUPED off the layout)
+ConvDims make_dims(int N, int C, int H, int W, int K, int stride, int &layout) {
     ConvDims d;
+    d.grouped = layout & DWO_GROUPED ? 1 : 0;
+    layout &= ~DWO_GROUPED;
     d.N = N, d.C = C, d.H = H, d.W = W, d.K = K, d.stride = stride;
     d.shift = log2_stride(stride);
     d.P = (H + stride - 1) / stride;
@@ -183,6 +187,45 @@ int try_window_wgrad(const void *x, const void *dy, const void *taps, float *par
     return -100;
 }
 
+// NHWC at strides 1 and 2 with channels grouped by orientation, any extent: the grouped kernels
+bool grouped_shape(const ConvDims &d, int layout, size_t esize) {
+    if (!d.grouped || layout != DWO_NHWC || d.stride > 2 || d.C % grp_channels(esize) != 0) return false;
+    if ((size_t)d.H * d.W * d.C * esize >= 0x80000000ull) return false;
+#define DWO_MATCH(K_) if (d.K == K_) return true;
+    DWO_GROUPED_KS(DWO_MATCH)
+#undef DWO_MATCH
+    return false;
+}
+bool aligned16(const void *p) { return (uintptr_t)p % 16 == 0; }
+template <typename T>
+int try_grouped_conv(const void *src, const float *w, const float *bias, const void *taps, void *dst,
+                     const ConvDims &d, int layout, int flip, hipStream_t st) {
+    if (!grouped_shape(d, layout, sizeof(T)) || !aligned16(src) || !aligned16(dst)) return -100;
+    if (flip && d.stride != 1) return -100;
+    // planes of at most 16 x 16 run on the register planes, which read whole lines
+    if (nhwc_plane_batch(d, layout) != 0 && reg_plane_shape_rt(d.H, d.W)) return -100;
+#define DWO_MATCH(K_) \
+    if (d.K == K_) return launch_grouped_conv<T, K_>(src, w, bias, taps, dst, d, flip, st);
+    DWO_GROUPED_KS(DWO_MATCH)
+#undef DWO_MATCH
+    return -100;
+}
+bool grouped_wgrad_covers(const ConvDims &d, int layout, size_t esize) {
+    // (with fewer planes than half the slots the fixed cost of a workgroup's sums shows: 4 x 64 x 20 x 20 in
+    // bf16 takes 14.6 us, on the tile kernels 11.7; 16 x 256 x 16 x 16 22.9 against 25.7)
+    if ((long)d.N * d.C < (long)kGrpSlots / 2 * grp_channels(esize)) return false;
+    return grouped_shape(d, layout, esize) && !(nhwc_plane_batch(d, layout) != 0 && reg_plane_shape_rt(d.H, d.W));
+}
+template <typename T>
+int try_grouped_wgrad(const void *x, const void *dy, const void *taps, float *part, int *groups,
+                      const ConvDims &d, hipStream_t st) {
+#define DWO_MATCH(K_) \
+    if (d.K == K_) return launch_grouped_wgrad<T, K_>(x, dy, taps, part, d, groups, st);
+    DWO_GROUPED_KS(DWO_MATCH)
+#undef DWO_MATCH
+    return -100;
+}
+
 // shapes the tile kernels take: NCHW always, NHWC with the channel count a multiple of 4; images
 // below 2 GB (32-bit offsets inside one)
 bool tile_covers(const ConvDims &d, int layout, size_t esize) {
@@ -193,7 +236,15 @@ bool tile_covers(const ConvDims &d, int layout, size_t esize) {
     return layout == DWO_NCHW || d.C % kSliceCh == 0;
 }
 
-int wgrad_max_partials(const ConvDims &d, int layout, size_t esize) {
+int wgrad_max_partials(const ConvDims &d_, int layout, size_t esize) {
+    ConvDims d = d_;
+    if (grouped_wgrad_covers(d, layout, esize)) {
+        // (tensors that are not aligned take the path below)
+        const int G = grp_wgrad_groups(d, esize);
+        d.grouped = 0;
+        const int other = wgrad_max_partials(d, layout, esize);
+        return G > other ? G : other;
+    }
     const int PBI = nhwc_plane_batch(d, layout);
     if (PBI != 0) {
         const int nbatch = (d.N + PBI - 1) / PBI;
@@ -268,6 +319,8 @@ int fprop_t(const void *x, const float *w, const float *bias, const void *taps, 
             const ConvDims &d, int layout, hipStream_t st) {
     const int fast = try_plane_conv<T>(OP_FPROP, x, w, bias, taps, y, d, layout, st);
     if (fast != -100) return fast;
+    const int grouped = try_grouped_conv<T>(x, w, bias, taps, y, d, layout, 0, st);
+    if (grouped != -100) return grouped;
     const int sliced = try_nhwc_plane_conv<T>(OP_FPROP, x, w, bias, taps, y, d, layout, st);
     if (sliced != -100) return sliced;
     const int windowed = try_window_conv<T>(x, w, bias, taps, y, d, layout, 0, st);
@@ -293,6 +346,8 @@ int dgrad_t(const void *dy, const float *w, const void *taps, void *dx, const Co
             int layout, hipStream_t st) {
     const int fast = try_plane_conv<T>(OP_DGRAD, dy, w, nullptr, taps, dx, d, layout, st);
     if (fast != -100) return fast;
+    const int grouped = try_grouped_conv<T>(dy, w, nullptr, taps, dx, d, layout, 1, st);
+    if (grouped != -100) return grouped;
     const int sliced = try_nhwc_plane_conv<T>(OP_DGRAD, dy, w, nullptr, taps, dx, d, layout, st);
     if (sliced != -100) return sliced;
     const int windowed = try_window_conv<T>(dy, w, nullptr, taps, dx, d, layout, 1, st);
@@ -395,6 +450,8 @@ int wgrad_t(const void *dy, const void *x, const void *taps, float *dw, float *d
         unsigned *tickets = ticket_row(d.C, st);
         rc = try_plane_wgrad<T>(x, dy, taps, part, dw, db, tickets, &NG, d, st);
         direct = NG == 1 || tickets != nullptr;
+    } else if (grouped_wgrad_covers(d, layout, sizeof(T)) && aligned16(x) && aligned16(dy)) {
+        rc = try_grouped_wgrad<T>(x, dy, taps, part, &NG, d, st);
     } else if (nhwc_plane_batch(d, layout) != 0) {
         unsigned *tickets = ticket_row(d.C / kSliceCh, st);
         rc = try_nhwc_plane_wgrad<T>(x, dy, taps, part, dw, db, tickets, &NG, d, st);
@@ -454,7 +511,7 @@ int pointwise_wgrad_t(const void *dy, const void *x, float *dw, float *db, float
 int wgrad_dispatch(const void *dy, const void *x, const void *taps, float *dw, float *db,
                    void *scratch, int N, int C, int H, int W, int K, int stride, int dtype,
                    int layout, hipStream_t st) {
-    const ConvDims d = make_dims(N, C, H, W, K, stride);
+    const ConvDims d = make_dims(N, C, H, W, K, stride, layout);
     begin_call();
     switch (dtype) {
         case DWO_F32: return wgrad_t<float>(dy, x, taps, dw, db, scratch, d, layout, st);
@@ -510,8 +567,18 @@ int init_type() {
                                      wd, &ng, nullptr);
     DWO_WINDOW_KS(DWO_PREP)
 #undef DWO_PREP
-    ConvDims d = make_dims(1, kSliceCh, 8, 8, 7, 2);
+    int nhwc = DWO_NHWC;
+    ConvDims d = make_dims(1, 16, 8, 8, 7, 2, nhwc);
     d.N = 0;
+    for (int stride = 1; stride <= 2; stride++) {
+        ConvDims g = d;
+        g.stride = stride;
+#define DWO_PREP(K_)                                                                                       \
+    rc |= launch_grouped_conv<T, K_>(nullptr, nullptr, nullptr, nullptr, nullptr, g, 0, nullptr);          \
+    rc |= launch_grouped_wgrad<T, K_>(nullptr, nullptr, nullptr, nullptr, g, &ng, nullptr);
+        DWO_GROUPED_KS(DWO_PREP)
+#undef DWO_PREP
+    }
     rc |= launch_nchw_tile_fprop<T>(nullptr, nullptr, nullptr, nullptr, nullptr, d, 0, nullptr);
     rc |= launch_nhwc_tile_fprop<T>(nullptr, nullptr, nullptr, nullptr, nullptr, d, 0, nullptr);
     rc |= launch_tile_dgrad_strided<T>(nullptr, nullptr, nullptr, nullptr, d, true, nullptr);
@@ -637,6 +704,16 @@ int dwo_build_taps(const float *theta_host, int C, int K, void *taps_host) {
     return DWO_OK;
 }
 
+int dwo_taps_grouped(const void *taps_host, int channels) {
+    if (taps_host == nullptr || channels < 1) return 0;
+    const int32_t *hdr = (const int32_t *)taps_host;
+    if (hdr[0] != kTapsMagic || hdr[1] != kTapsVersion || hdr[2] % channels != 0) return 0;
+    const int32_t *cls = taps_class(taps_host, hdr[2], hdr[3]);
+    for (int c = 0; c < hdr[2]; c++)
+        if (cls[c] < 0 || cls[c] != cls[c / channels * channels]) return 0;
+    return 1;
+}
+
 int dwo_taps_get(const void *taps_host, int c, int s, int *dh, int *dw) {
     if (taps_host == nullptr || dh == nullptr || dw == nullptr) return DWO_ERR_NULL_POINTER;
     const int32_t *hdr = (const int32_t *)taps_host;
@@ -653,7 +730,7 @@ int dwo_fprop(const void *x, const float *w, const float *bias, const void *taps
     int rc = check_common(N, C, H, W, K, stride, dtype, layout);
     if (rc != DWO_OK) return rc;
     if (!x || !w || !taps || !y) return DWO_ERR_NULL_POINTER;
-    const ConvDims d = make_dims(N, C, H, W, K, stride);
+    const ConvDims d = make_dims(N, C, H, W, K, stride, layout);
     hipStream_t st = (hipStream_t)stream;
     begin_call();
     switch (dtype) {
@@ -668,7 +745,7 @@ int dwo_dgrad(const void *dy, const float *w, const void *taps, void *dx, int N,
     int rc = check_common(N, C, H, W, K, stride, dtype, layout);
     if (rc != DWO_OK) return rc;
     if (!dy || !w || !taps || !dx) return DWO_ERR_NULL_POINTER;
-    const ConvDims d = make_dims(N, C, H, W, K, stride);
+    const ConvDims d = make_dims(N, C, H, W, K, stride, layout);
     hipStream_t st = (hipStream_t)stream;
     begin_call();
     switch (dtype) {
@@ -681,7 +758,7 @@ int dwo_dgrad(const void *dy, const float *w, const void *taps, void *dx, int N,
 size_t dwo_wgrad_scratch_bytes(int N, int C, int H, int W, int K, int stride, int dtype,
                                int layout) {
     if (check_common(N, C, H, W, K, stride, dtype, layout) != DWO_OK) return 0;
-    const ConvDims d = make_dims(N, C, H, W, K, stride);
+    const ConvDims d = make_dims(N, C, H, W, K, stride, layout);
     return (size_t)C * (K + 1) * wgrad_max_partials(d, layout, dtype == DWO_F32 ? 4 : 2) * sizeof(float);
 }
 
@@ -718,7 +795,8 @@ int dwo_pointwise_fprop_nhwc(const void *x, const float *pw_w, const float *pw_b
     if (rc != DWO_OK) return rc;
     if (!x || !pw_w || !w || !taps || !y) return DWO_ERR_NULL_POINTER;
     if (Cin < 1 || Cin > 4 || C % kSliceCh != 0) return DWO_ERR_BAD_SHAPE;
-    const ConvDims d = make_dims(N, C, H, W, K, stride);
+    int layout = DWO_NHWC;
+    const ConvDims d = make_dims(N, C, H, W, K, stride, layout);
     hipStream_t st = (hipStream_t)stream;
     begin_call();
     switch (dtype) {

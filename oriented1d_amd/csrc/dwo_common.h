@@ -150,6 +150,7 @@ inline int per_device_once(int *cache, F make) {
 
 struct ConvDims {
     int N, C, H, W, P, Q, K, stride, shift;  // shift = log2(stride)
+    int grouped;  // the caller's DWO_GROUPED
 };
 
 }  // namespace dwo

@@ -1,0 +1,54 @@
+// Which calls the grouped kernels of dwo_grouped.h cover, how an image is cut into tiles, and the
+// launchers compiled per (element type, kernel size).
+#pragma once
+
+#include "dwo_common.h"
+#include "dwo_plan.h"
+
+// X(K): the kernel sizes of the networks and of the reference's layer benchmark
+#define DWO_GROUPED_KS(X) X(7) X(13) X(15) X(27) X(31)
+
+namespace dwo {
+
+constexpr int kGrpThreads = 512;
+constexpr int kGrpPixels = 4960;  // staged pixels of 16 bytes: two workgroups per CU
+constexpr int kGrpSlots = 512;     // workgroups resident on the chip
+constexpr int kGrpLeastRows = 8;  // of a tile that is cut to fill the chip
+// channels of one 16-byte pixel piece: they share an orientation
+constexpr int grp_channels(size_t esize) { return 16 / (int)esize; }
+// widest tile, in outputs
+constexpr int grp_tile_cols(int S) { return S == 1 ? 64 : 32; }
+
+struct GrpTiles {
+    int th, tw, nth, ntw;  // tile extents and counts
+};
+
+// Partial sums per (channel, tap): a multiple of eight (unit u runs on XCD u % 8), about two rounds of the
+// chip's slots at most, and no more than there are tiles of 16 x 32 outputs (surplus groups
+// contribute zeros).
+inline int grp_wgrad_groups(const ConvDims &d, size_t esize) {
+    const long units = (long)d.N * ((d.P + 15) / 16) * ((d.Q + 31) / 32), ngroups = d.C / grp_channels(esize);
+    long G = 1024 / ngroups;
+    if (G > units) G = units;
+    return (int)((G < 1 ? 1 : G) + 7) / 8 * 8;
+}
+
+template <typename T, int K>
+int launch_grouped_conv(const void *src, const float *w, const float *bias, const void *taps, void *dst,
+                        const ConvDims &d, int flip, hipStream_t st);
+template <typename T, int K>
+int launch_grouped_wgrad(const void *x, const void *dy, const void *taps, float *part, const ConvDims &d,
+                         int *groups_out, hipStream_t st);
+
+#define DWO_DECLARE(T, K)                                                                                \
+    extern template int launch_grouped_conv<T, K>(const void *, const float *, const float *,           \
+                                                  const void *, void *, const ConvDims &, int,          \
+                                                  hipStream_t);                                         \
+    extern template int launch_grouped_wgrad<T, K>(const void *, const void *, const void *, float *,   \
+                                                   const ConvDims &, int *, hipStream_t);
+#define DWO_DECLARE_ALL(K) DWO_DECLARE(float, K) DWO_DECLARE(bf16_t, K) DWO_DECLARE(f16_t, K)
+DWO_GROUPED_KS(DWO_DECLARE_ALL)
+#undef DWO_DECLARE_ALL
+#undef DWO_DECLARE
+
+}  // namespace dwo

@@ -131,7 +131,8 @@ struct Place {
 };
 
 Tensor fprop(const Tensor &x, const Tensor &w, const Tensor &taps, int64_t stride, const OptTensor &bias,
-             bool nhwc) {
+             int64_t layout) {
+    const bool nhwc = layout & DWO_NHWC;
     check_activation(x, "x");
     check_stride(stride);
     const Dims d(x, nhwc);
@@ -142,14 +143,15 @@ Tensor fprop(const Tensor &x, const Tensor &w, const Tensor &taps, int64_t strid
     const Place at(x);
     Tensor y = at::empty(shape_of(d.n, d.c, up(d.h, stride), up(d.w, stride), nhwc), x.options());
     check(lib.fprop(ptr(x), (const float *)ptr(w2), fptr(bias), ptr(taps), y.data_ptr(), as_int(d.n),
-                    as_int(d.c), as_int(d.h), as_int(d.w), as_int(K), as_int(stride), dtype_code(x), nhwc,
+                    as_int(d.c), as_int(d.h), as_int(d.w), as_int(K), as_int(stride), dtype_code(x), (int)layout,
                     at.stream),
           "dwo_fprop");
     return y;
 }
 
 Tensor dgrad(const Tensor &dy, const Tensor &w, const Tensor &taps, int64_t H, int64_t W, int64_t stride,
-             bool nhwc) {
+             int64_t layout) {
+    const bool nhwc = layout & DWO_NHWC;
     check_activation(dy, "dy");
     check_stride(stride);
     const Dims d(dy, nhwc);
@@ -161,13 +163,14 @@ Tensor dgrad(const Tensor &dy, const Tensor &w, const Tensor &taps, int64_t H, i
     const Place at(dy);
     Tensor dx = at::empty(shape_of(d.n, d.c, H, W, nhwc), dy.options());
     check(lib.dgrad(ptr(dy), (const float *)ptr(w2), ptr(taps), dx.data_ptr(), as_int(d.n), as_int(d.c),
-                    as_int(H), as_int(W), as_int(K), as_int(stride), dtype_code(dy), nhwc, at.stream),
+                    as_int(H), as_int(W), as_int(K), as_int(stride), dtype_code(dy), (int)layout, at.stream),
           "dwo_dgrad");
     return dx;
 }
 
 std::tuple<Tensor, OptTensor> wgrad(const Tensor &dy, const Tensor &x, const Tensor &taps, int64_t K,
-                                    int64_t stride, bool nhwc, bool with_bias) {
+                                    int64_t stride, int64_t layout, bool with_bias) {
+    const bool nhwc = layout & DWO_NHWC;
     check_activation(dy, "dy");
     check_activation(x, "x");
     check_stride(stride);
@@ -180,14 +183,14 @@ std::tuple<Tensor, OptTensor> wgrad(const Tensor &dy, const Tensor &x, const Ten
     const Place at(x);
     const int n = as_int(d.n), c = as_int(d.c), h = as_int(d.h), wd = as_int(d.w), k = as_int(K),
               s = as_int(stride), dt = dtype_code(x);
-    const size_t nbytes = lib.wgrad_scratch_bytes(n, c, h, wd, k, s, dt, nhwc);
+    const size_t nbytes = lib.wgrad_scratch_bytes(n, c, h, wd, k, s, dt, (int)layout);
     const Tensor scratch = at::empty({(int64_t)std::max<size_t>(nbytes, 16)}, x.options().dtype(at::kByte));
     const auto f32 = x.options().dtype(at::kFloat);
     Tensor dw = at::empty({d.c, 1, 1, K}, f32);
     OptTensor db;
     if (with_bias) db = at::empty({d.c}, f32);
     check(lib.wgrad(ptr(dy), ptr(x), ptr(taps), (float *)dw.data_ptr(), db.has_value() ? (float *)db->data_ptr() : nullptr,
-                    scratch.data_ptr(), nbytes, n, c, h, wd, k, s, dt, nhwc, at.stream),
+                    scratch.data_ptr(), nbytes, n, c, h, wd, k, s, dt, (int)layout, at.stream),
           "dwo_wgrad");
     return {dw, db};
 }

@@ -181,6 +181,16 @@ constexpr int round_up(int v, int m) { return (v + m - 1) / m * m; }
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 constexpr int cmin(int a, int b) { return a < b ? a : b; }
 
+// largest |dh| (h) or |dw| of an orientation's taps
+constexpr int win_extent(int o, int K, bool h) {
+    int m = 0;
+    for (int s = 0; s < K; s++) {
+        const int v = h ? canon_dh(o, K, s) : canon_dw(o, K, s);
+        m = cmax(m, cmax(v, -v));
+    }
+    return m;
+}
+
 // Smallest r >= need with (mult * r - target) divisible by 32, or need rounded to odd when
 // no such r exists within one period.  Used to pick LDS row strides for which the flattened
 // item -> address map is linear modulo the 32 banks.

@@ -40,14 +40,6 @@ struct WinMode {
 };
 
 // LDS layout of one orientation (the interface of Geo that the plans use).
-constexpr int win_extent(int o, int K, bool h) {
-    int m = 0;
-    for (int s = 0; s < K; s++) {
-        const int v = h ? canon_dh(o, K, s) : canon_dw(o, K, s);
-        m = cmax(m, cmax(v, -v));
-    }
-    return m;
-}
 template <int CLS_, int DH_, int DW_, int P0_, int Q0_, int EH_, int WM, bool TILE>
 struct WinLayout {
     static constexpr int CLS = CLS_, DH = DH_, DW = DW_, P0 = P0_, Q0 = Q0_, EH = EH_;

@@ -83,19 +83,29 @@ class _TapCache:
     KEEP = 8
 
     def __init__(self):
-        self.entries = {}  # (id(theta), device, C, K) -> (state key, weak ref, device blob)
+        # (id(theta), device, C, K) -> (state key, weak ref, device blob, layouts by element size)
+        self.entries = {}
 
     def get(self, theta, C, K, device):
+        """The device tap table."""
+        return self.lookup(theta, C, K, device)[0]
+
+    def lookup(self, theta, C, K, device):
+        """(device tap table, {element size: layout code of an NHWC call}): ``GROUPED`` is added
+        where every 16 bytes of channels share an orientation."""
         slot = (id(theta), device, C, K)
         state = (theta.data_ptr(), theta._version)
         hit = self.entries.get(slot)
         if hit is None or hit[0] != state or hit[1]() is not theta:
             if len(self.entries) >= self.KEEP:
                 self.entries.pop(next(iter(self.entries)))
-            blob = build_taps(theta, C, K).to(device)
-            hit = (state, weakref.ref(theta), blob)
+            blob = build_taps(theta, C, K)
+            grouped = _lib.load().dwo_taps_grouped
+            layouts = {size: _lib.NHWC + (_lib.GROUPED if grouped(_ptr(blob), 16 // size) else 0)
+                       for size in (2, 4)}
+            hit = (state, weakref.ref(theta), blob.to(device), layouts)
             self.entries[slot] = hit
-        return hit[2]
+        return hit[2], hit[3]
 
 
 def _dims(x, nhwc):
@@ -126,20 +136,21 @@ def f32_copy(p):
 
 
 def fprop(x, w, taps, stride=1, bias=None, nhwc=False):
-    """y = fprop(x, w, theta) (+ bias).  x: [N,C,H,W] or [N,H,W,C]; w: [C,1,1,K]."""
+    """y = fprop(x, w, theta) (+ bias).  x: [N,C,H,W] or [N,H,W,C]; w: [C,1,1,K].  ``nhwc`` is a
+    truth value or, here and below, a layout code of ``_TapCache.lookup``."""
     b = f32_copy(bias) if bias is not None else None
-    return _lib.host(x.get_device()).fprop(x, w, taps, stride, b, nhwc)
+    return _lib.host(x.get_device()).fprop(x, w, taps, stride, b, int(nhwc))
 
 
 def dgrad(dy, w, taps, in_hw, stride=1, nhwc=False):
     """dx = dgrad(dy, w, theta); ``in_hw`` is the (H, W) of the forward input."""
     H, W = in_hw
-    return _lib.host(dy.get_device()).dgrad(dy, w, taps, H, W, stride, nhwc)
+    return _lib.host(dy.get_device()).dgrad(dy, w, taps, H, W, stride, int(nhwc))
 
 
 def wgrad(dy, x, taps, K, stride=1, nhwc=False, with_bias=False):
     """(dw [C,1,1,K] fp32, db [C] fp32 or None) = wgrad(dy, x, theta)."""
-    return _lib.host(x.get_device()).wgrad(dy, x, taps, K, stride, nhwc, with_bias)
+    return _lib.host(x.get_device()).wgrad(dy, x, taps, K, stride, int(nhwc), with_bias)
 
 
 class KernelTuple(tuple):
@@ -200,14 +211,15 @@ class _DepthwiseOrientedConv1d(torch.autograd.Function):
         if not module.arbitrary_size and (H % stride != 0 or W % stride != 0):
             # models/dwoconv1d/kernels/kernels.cu:20
             raise RuntimeError("Invalid input size: H,W not divisible by stride")
-        taps = module.taps.get(theta, C, K, x.device)
+        taps, layouts = module.taps.lookup(theta, C, K, x.device)
+        layout = layouts[x.element_size()] if nhwc else _lib.NCHW
 
-        ctx.stride, ctx.nhwc, ctx.K = stride, nhwc, K
+        ctx.stride, ctx.nhwc, ctx.K = stride, layout, K
         ctx.with_bias = bias is not None
         ctx.w_dtype = w.dtype
         ctx.b_dtype = bias.dtype if bias is not None else None
         ctx.save_for_backward(x, w_eff, taps)
-        return fprop(x, w_eff, taps, stride, bias=bias, nhwc=nhwc)
+        return fprop(x, w_eff, taps, stride, bias=bias, nhwc=layout)
 
     @staticmethod
     def _forward_plain(ctx, x, w, theta, bias, module, nhwc, resid):

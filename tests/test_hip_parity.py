@@ -231,6 +231,46 @@ def test_window_kernels_unit_edges(oracle, N, C, H, W, K, dtype):
     _case(oracle, N, C, H, W, K, 1, dtype, False, theta, seed=H * 1000 + W)
 
 
+# tile edges (one tile of 32 x 64 outputs or less and one more row or column; 16 x 32 at stride 2), odd
+# extents, extents below an item's four outputs, more units than slots, kernel sizes
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("N,C,H,W,K,stride", [
+    (2, 64, 28, 28, 31, 1), (1, 64, 32, 64, 31, 1), (1, 64, 33, 65, 31, 1), (3, 64, 56, 56, 31, 1),
+    (2, 64, 17, 3, 31, 1), (2, 128, 70, 19, 13, 1), (1, 64, 40, 130, 7, 1), (2, 64, 21, 66, 27, 1),
+    (2, 64, 56, 56, 31, 2), (1, 64, 65, 131, 31, 2), (3, 64, 33, 63, 15, 2), (2, 64, 5, 18, 7, 2),
+    (9, 64, 66, 66, 13, 2), (40, 64, 34, 30, 15, 1),
+    # (wgrad: enough planes for the grouped kernel)
+    (2, 1024, 28, 28, 31, 1), (2, 1024, 33, 65, 31, 1), (2, 1024, 17, 3, 13, 1), (2, 1024, 21, 18, 27, 1),
+    (2, 1024, 33, 67, 31, 2), (2, 1024, 5, 18, 7, 2), (2, 1024, 35, 31, 15, 2)])
+def test_grouped_nhwc_kernels(oracle, N, C, H, W, K, stride, dtype):
+    """Channels grouped by angle, as the networks have them: whole 16-byte pieces per orientation."""
+    for offset in (0.0, 0.5):
+        theta = grouped_theta(C, offset)
+        layouts = op._TapCache().lookup(torch.from_numpy(theta), C, K, torch.device("cuda"))[1]
+        assert layouts == {2: 3, 4: 3}
+        _case(oracle, N, C, H, W, K, stride, dtype, 3, theta, seed=H + W + K)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("stride", [1, 2])
+def test_grouped_claim_that_does_not_hold(oracle, stride, dtype):
+    """Mixed orientations behind DWO_GROUPED, and a tensor off its 16-byte alignment: same values."""
+    C = 1024  # (enough planes for the grouped wgrad)
+    theta = canonical_theta(C)
+    theta[8:16] = 0.3  # a run of one angle that is none of the eight
+    layouts = op._TapCache().lookup(torch.from_numpy(theta), C, 15, torch.device("cuda"))[1]
+    assert layouts == {2: 1, 4: 1}
+    _case(oracle, 2, C, 20, 23, 15, stride, dtype, 3, theta, seed=5)
+    taps = op.build_taps(torch.from_numpy(grouped_theta(C)), C, 15).cuda()
+    buf = torch.randn(1 + 2 * 24 * 24 * C, device="cuda").to(dtype)
+    x, w = buf[1:].view(2, 24, 24, C), torch.randn(C, 1, 1, 15, device="cuda")
+    dy = torch.randn(2, 24 // stride, 24 // stride, C, device="cuda").to(dtype)
+    assert x.data_ptr() % 16 != 0
+    for a, b in ((op.fprop(x, w, taps, stride, nhwc=3), op.fprop(x.clone(), w, taps, stride, nhwc=1)),
+                 (op.wgrad(dy, x, taps, 15, stride, nhwc=3)[0], op.wgrad(dy, x, taps, 15, stride, nhwc=1)[0])):
+        assert_close(host(a), host(b), dtype, "misaligned")
+
+
 @pytest.mark.parametrize("nhwc", [False, True], ids=["nchw", "nhwc"])
 def test_random_angles_ragged_shapes(oracle, nhwc):
     rng = np.random.default_rng(77)
