@@ -201,7 +201,6 @@ template <typename T>
 int try_grouped_conv(const void *src, const float *w, const float *bias, const void *taps, void *dst,
                      const ConvDims &d, int layout, int flip, hipStream_t st) {
     if (!grouped_shape(d, layout, sizeof(T)) || !aligned16(src) || !aligned16(dst)) return -100;
-    if (flip && d.stride != 1) return -100;
     // planes of at most 16 x 16 run on the register planes, which read whole lines
     if (nhwc_plane_batch(d, layout) != 0 && reg_plane_shape_rt(d.H, d.W)) return -100;
 #define DWO_MATCH(K_) \
@@ -575,6 +574,7 @@ int init_type() {
         g.stride = stride;
 #define DWO_PREP(K_)                                                                                       \
     rc |= launch_grouped_conv<T, K_>(nullptr, nullptr, nullptr, nullptr, nullptr, g, 0, nullptr);          \
+    rc |= launch_grouped_conv<T, K_>(nullptr, nullptr, nullptr, nullptr, nullptr, g, 1, nullptr);          \
     rc |= launch_grouped_wgrad<T, K_>(nullptr, nullptr, nullptr, nullptr, g, &ng, nullptr);
         DWO_GROUPED_KS(DWO_PREP)
 #undef DWO_PREP

@@ -1,6 +1,6 @@
 // NHWC kernels for channel groups of one orientation (the networks give contiguous channels the same
-// angle): fprop at strides 1 and 2, dgrad at stride 1 (reversed weights), wgrad at strides 1 and 2,
-// any extent.
+// angle): fprop, dgrad and wgrad at strides 1 and 2, any extent (dgrad at stride 1 is fprop with reversed
+// weights).
 //
 // A workgroup owns one 16-byte piece of a pixel (8 channels of a 16-bit type, 4 of fp32) over a tile of
 // outputs.  It stages the tile's window as it lies in memory, pixel by pixel, and four lanes
@@ -88,27 +88,103 @@ struct GrpGeo {
         return t;
     }
 };
-template <int K, int S, int... Os>
+// Plan of dgrad at stride 2.  The dx pixels come in quads, (2 i + a, 2 j + b) for a, b in {0, 1}; tap
+// (dh, dw) feeds the quad's pixel of its own parities from dy(i - floor(dh / 2), j - floor(dw / 2)), so a
+// quad takes every tap once, and an item of L neighbouring quads shares its sources as outputs do.
+struct QuadPlan {
+    int nsrc = 0, nfma = 0;
+    int16_t sh[kMaxSrc] = {}, sw[kMaxSrc] = {};
+    int8_t user[kMaxSrc][2][4] = {};  // [quad][2 a + b]: first tap with that offset, or -1
+    int8_t rep[64] = {};
+};
+constexpr int floor_half(int v) { return v >= 0 ? v / 2 : -((1 - v) / 2); }
+constexpr QuadPlan make_quad_plan(int o, int K, int L) {
+    QuadPlan p{};
+    const int eh = step_h(o), ew = step_w(o);
+    constexpr int G = 24, GS = 2 * G + 1;
+    int16_t at[GS][GS] = {};
+    for (int i = 0; i < GS; i++)
+        for (int j = 0; j < GS; j++) at[i][j] = -1;
+    for (int s = 0; s < K; s++) {
+        const int dh = canon_dh(o, K, s), dw = canon_dw(o, K, s);
+        int r = 0;
+        while (canon_dh(o, K, r) != dh || canon_dw(o, K, r) != dw) r++;
+        p.rep[s] = (int8_t)r;
+        if (r != s) continue;
+        for (int l = 0; l < L; l++) {
+            const int h = l * eh - floor_half(dh), w = l * ew - floor_half(dw);
+            int16_t &m = at[h + G][w + G];
+            if (m < 0) {
+                m = (int16_t)p.nsrc++;
+                p.sh[m] = (int16_t)h, p.sw[m] = (int16_t)w;
+                for (int q = 0; q < 2; q++)
+                    for (int k = 0; k < 4; k++) p.user[m][q][k] = -1;
+            }
+            p.user[m][l][2 * (dh - 2 * floor_half(dh)) + dw - 2 * floor_half(dw)] = (int8_t)s;
+            p.nfma++;
+        }
+    }
+    return p;
+}
+// its window of dy: the interface of GrpGeo, in quads, at stride 1
+template <int O, int K>
+struct GrpQuadGeo {
+    static constexpr int CLS = orient_class(O), L = 2, EH = step_h(O);
+    static constexpr int DH = (win_extent(O, K, true) + 1) / 2, DW = (win_extent(O, K, false) + 1) / 2;
+    static constexpr int SR = 1, SC = 1;
+    static constexpr int LR = CLS == CLS_H ? 1 : L;
+    static constexpr int P0 = CLS == CLS_D && EH < 0 ? L - 1 : 0;
+    static constexpr int PADL = CLS == CLS_D ? L - 1 : 0;
+    static constexpr int EXTRA = 2 * DW + 2 * PADL;
+    static constexpr int WIDTH = grp_tile_cols(1) + EXTRA;
+    static constexpr int M = L, SUB = (WIDTH + M - 1) / M;
+    static constexpr int RS = CLS == CLS_H ? M * SUB : WIDTH;
+    static constexpr int col(int u) { return CLS == CLS_H ? (u % M) * SUB + u / M : u; }
+    static constexpr QuadPlan plan = make_quad_plan(O, K, L);
+    static constexpr int imm(int sh, int sw) { return (sh + P0 + DH) * RS + col(sw + DW); }
+    static constexpr int rows(int th) { return (th + LR - 1) / LR * LR + 2 * DH; }
+    static constexpr int pixels(int th) { return rows(th) * RS; }
+    static constexpr int max_rows() {
+        int t = 64;
+        while (pixels(t) > kGrpPixels) t--;
+        return t;
+    }
+};
+
+// the geometries of a kernel for all orientations
+template <int K, int S>
+struct ConvSet {
+    static constexpr int TW = grp_tile_cols(S);
+    template <int O>
+    using Geo = GrpGeo<O, K, S>;
+};
+template <int K>
+struct QuadSet {
+    static constexpr int TW = grp_tile_cols(1);
+    template <int O>
+    using Geo = GrpQuadGeo<O, K>;
+};
+template <class Set, int... Os>
 constexpr int grp_max_rows_impl(std::integer_sequence<int, Os...>) {
     int m = 64;
-    ((m = cmin(m, GrpGeo<Os, K, S>::max_rows())), ...);
+    ((m = cmin(m, Set::template Geo<Os>::max_rows())), ...);
     return m;
 }
 // most output rows per tile, whatever the orientation (one tile grid for all of them keeps the groups
 // of a tile together)
-template <int K, int S>
+template <class Set>
 constexpr int grp_max_rows() {
-    return grp_max_rows_impl<K, S>(std::make_integer_sequence<int, 8>{});
+    return grp_max_rows_impl<Set>(std::make_integer_sequence<int, 8>{});
 }
-template <int K, int S, int... Os>
+template <class Set, int... Os>
 constexpr int grp_pixels_impl(int th, std::integer_sequence<int, Os...>) {
     int m = 0;
-    ((m = cmax(m, GrpGeo<Os, K, S>::pixels(th))), ...);
+    ((m = cmax(m, Set::template Geo<Os>::pixels(th))), ...);
     return m;
 }
-template <int K, int S>
+template <class Set>
 constexpr int grp_pixels(int th) {
-    return grp_pixels_impl<K, S>(th, std::make_integer_sequence<int, 8>{});
+    return grp_pixels_impl<Set>(th, std::make_integer_sequence<int, 8>{});
 }
 
 typedef unsigned grp_u4 __attribute__((ext_vector_type(4)));
@@ -150,7 +226,7 @@ template <class G, int S, typename T>
 __device__ __forceinline__ void grp_stage(grp_u4 *lds, const T *xn, const ConvDims &d, const GrpTile &t, int c0) {
     const __amdgpu_buffer_rsrc_t rsrc =
         win_rsrc(xn, xn + (size_t)d.H * d.W * d.C - c0);
-    const unsigned ww = (((t.tw + 3) & ~3) - 1) * G::SC + 1 + G::EXTRA;
+    const unsigned ww = (((t.tw + G::L - 1) / G::L * G::L) - 1) * G::SC + 1 + G::EXTRA;
     const unsigned nwin = G::rows(t.th) * ww, magic = win_magic(ww);
     const int r0 = t.p * S - G::DH, q0 = t.q * S - G::DW - G::PADL;
     const unsigned pix = (unsigned)d.C * (unsigned)sizeof(T);
@@ -179,7 +255,7 @@ template <class G>
 struct GrpItems {
     unsigned ipr, magic, count;
     __device__ __forceinline__ explicit GrpItems(const GrpTile &t) {
-        ipr = G::CLS == CLS_H ? (t.tw + 3) / 4 : (G::CLS == CLS_V ? t.tw : t.tw + G::L - 1);
+        ipr = G::CLS == CLS_H ? (t.tw + G::L - 1) / G::L : (G::CLS == CLS_V ? t.tw : t.tw + G::L - 1);
         count = (G::CLS == CLS_H ? t.th : (t.th + G::L - 1) / G::L) * ipr;
         magic = win_magic(ipr);
     }
@@ -187,7 +263,7 @@ struct GrpItems {
         const unsigned rb = win_div(item, magic), j = item - rb * ipr;
         word = (rb * (G::LR * G::SR * G::RS) + (G::CLS == CLS_H ? j : j * G::SC)) * 4 + threadIdx.x % 4;
         row = (int)rb * G::LR + G::P0;
-        col = G::CLS == CLS_H ? (int)j * 4 : (int)j - (G::CLS == CLS_D ? G::L - 1 : 0);
+        col = G::CLS == CLS_H ? (int)j * G::L : (int)j - (G::CLS == CLS_D ? G::L - 1 : 0);
     }
     // output l of the item
     static __device__ __forceinline__ int row_of(int row, int l) {
@@ -336,6 +412,136 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
         DWO_CASE(6)
         DWO_CASE(7)
         default: grp_conv_any<S, T, K>(xn, yn, wt, bias, taps_dhdw(blob), d, t, c0, flip);
+    }
+#undef DWO_CASE
+}
+
+// ---------------------------------------------------------------------------------------------
+// dgrad at stride 2 (QuadPlan).  `d` describes dy as both the source and the plane of quads (H = P,
+// W = Q); dx is dxh x dxw.  64 x 64 x 224 x 224 bf16, K = 31: 249 us, bound by the writes in 16-byte
+// pieces (the residue classes one after the other from a sorted tap table, dwo_nhwc_tile.h: 542).
+template <int O, typename T, int K>
+__device__ __forceinline__ void grp_dgrad2_body(grp_u4 *lds, float *lw, const T *dyn, T *dxn, const ConvDims &d,
+                                                const GrpTile &t, int c0, int dxh, int dxw) {
+    using G = GrpQuadGeo<O, K>;
+    constexpr int N = Word<T>::N, L = G::L;
+    grp_stage<G, 1>(lds, dyn, d, t, c0);
+    __syncthreads();
+    const int ch = (int)(threadIdx.x % 4) * N;
+    float wv[K][N];
+#pragma unroll
+    for (int e = 0; e < N; e++) {
+        const float *row = lw + (ch + e) * K;
+#pragma unroll
+        for (int s = 0; s < K; s++) wv[s][e] = row[s];
+        static_for<K>([&](auto s) {
+            constexpr int r = G::plan.rep[s];
+            if constexpr (r != s) wv[r][e] += wv[s][e];
+        });
+    }
+    const __amdgpu_buffer_rsrc_t out = win_rsrc(dxn, dxn + (size_t)dxh * dxw * d.C - c0);
+    const unsigned *words = reinterpret_cast<const unsigned *>(lds);
+    const unsigned pix = (unsigned)d.C * (unsigned)sizeof(T);
+    const GrpItems<G> items(t);
+    for (unsigned it = threadIdx.x / 4; it < items.count; it += kGrpThreads / 4) {
+        unsigned word;
+        int row, col;
+        items.at(it, word, row, col);
+        float acc[L][4][N];
+#pragma unroll
+        for (int l = 0; l < L; l++)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int e = 0; e < N; e++) acc[l][k][e] = 0.f;
+        const unsigned *base = words + word;
+        static_for<G::plan.nsrc>([&](auto m) {
+            constexpr int off = G::imm(G::plan.sh[m], G::plan.sw[m]) * 4;
+            const unsigned v = base[off];
+#pragma unroll
+            for (int e = 0; e < N; e++) {
+                const float x = Word<T>::get(v, e);
+                static_for<4 * L>([&](auto i) {
+                    constexpr int l = i / 4, k = i % 4, s = G::plan.user[m][l][k];
+                    if constexpr (s >= 0) acc[l][k][e] = __builtin_fmaf(x, wv[s][e], acc[l][k][e]);
+                });
+            }
+        });
+        pipeline_reads_and_fmas<G::plan.nsrc, N * G::plan.nfma + (N - 1) * 2 * G::plan.nsrc>();
+#pragma unroll
+        for (int l = 0; l < L; l++)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int e = 0; e < N; e++) asm volatile("" : "+v"(acc[l][k][e]));  // (as in grp_conv_body)
+#pragma unroll
+        for (int l = 0; l < L; l++) {
+            const int r = GrpItems<G>::row_of(row, l), c = GrpItems<G>::col_of(col, l);
+            const int h = 2 * (t.p + r), w = 2 * (t.q + c);
+            const bool in = ((unsigned)r < (unsigned)t.vh) & ((unsigned)c < (unsigned)t.vw);
+            const unsigned o = ((unsigned)h * dxw + (unsigned)w) * pix + threadIdx.x % 4 * 4;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const bool ok = in & (h + k / 2 < dxh) & (w + k % 2 < dxw);
+                __builtin_amdgcn_raw_buffer_store_b32(Word<T>::pack(acc[l][k]), out,
+                                                      ok ? o + (k / 2 * dxw + k % 2) * pix : kWinNowhere, 0, 0);
+            }
+        }
+    }
+}
+
+// the claim did not hold: one dx pixel and channel per thread
+template <typename T, int K>
+__device__ void grp_dgrad2_any(const T *dyn, T *dxn, const float *wt, const int8_t *dhdw, const ConvDims &d,
+                               const GrpTile &t, int c0, int dxh, int dxw) {
+    constexpr int CG = grp_channels(sizeof(T));
+    for (int f = threadIdx.x; f < 4 * t.vh * t.vw * CG; f += kGrpThreads) {
+        const int k = f % CG, o = f / CG, c = c0 + k;
+        const int h = 2 * t.p + o / (2 * t.vw), w = 2 * t.q + o % (2 * t.vw);
+        if (h >= dxh || w >= dxw) continue;
+        float a = 0.f;
+        for (int s = 0; s < K; s++) {
+            const int ph = h - dhdw[((size_t)c * K + s) * 2], pw = w - dhdw[((size_t)c * K + s) * 2 + 1];
+            if (((ph | pw) & 1) == 0 && (unsigned)(ph / 2) < (unsigned)d.H && (unsigned)(pw / 2) < (unsigned)d.W &&
+                ph >= 0 && pw >= 0)
+                a = __builtin_fmaf(to_float(dyn[((size_t)(ph / 2) * d.W + pw / 2) * d.C + k]),
+                                   wt[(size_t)c * K + s], a);
+        }
+        dxn[((size_t)h * dxw + w) * d.C + k] = from_float<T>(a);
+    }
+}
+
+template <typename T, int K>
+__global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void grouped_dgrad2_kernel(
+    const T *__restrict__ dy, const float *__restrict__ wt, const void *__restrict__ blob, T *__restrict__ dx,
+    ConvDims d, GrpTiles tiles, int pixels, int dxh, int dxw) {
+    extern __shared__ float lds_f[];
+    grp_u4 *lds = reinterpret_cast<grp_u4 *>(lds_f);
+    float *lw = lds_f + 4 * pixels;
+    constexpr int CG = grp_channels(sizeof(T));
+    int unit, group;
+    grp_task(d.C / CG, unit, group);
+    if (unit >= d.N * tiles.nth * tiles.ntw) return;
+    const int c0 = group * CG;
+    GrpTile t;
+    t.set(d, tiles, unit);
+    const T *dyn = dy + (size_t)t.n * d.H * d.W * d.C + c0;
+    T *dxn = dx + (size_t)t.n * dxh * dxw * d.C + c0;
+    if (threadIdx.x < CG * K) lw[threadIdx.x] = wt[(size_t)c0 * K + threadIdx.x];
+#define DWO_CASE(O)                                                     \
+    case O:                                                             \
+        grp_dgrad2_body<O, T, K>(lds, lw, dyn, dxn, d, t, c0, dxh, dxw); \
+        break;
+    switch (grp_class<CG>(taps_class(blob, d.C, K) + c0)) {
+        DWO_CASE(0)
+        DWO_CASE(1)
+        DWO_CASE(2)
+        DWO_CASE(3)
+        DWO_CASE(4)
+        DWO_CASE(5)
+        DWO_CASE(6)
+        DWO_CASE(7)
+        default: grp_dgrad2_any<T, K>(dyn, dxn, wt, taps_dhdw(blob), d, t, c0, dxh, dxw);
     }
 #undef DWO_CASE
 }
@@ -491,9 +697,9 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
 
 // Tiles of a P x Q output plane, even in size (the last is no sliver); planes x groups that would leave
 // workgroup slots empty are cut into lower tiles.
-template <int K, int S>
+template <class Set>
 GrpTiles grp_tiles(int P, int Q, long planes) {
-    constexpr int TH = grp_max_rows<K, S>(), TW = grp_tile_cols(S);
+    constexpr int TH = grp_max_rows<Set>(), TW = Set::TW;
     static_assert(TH >= 4, "a window of four output rows must fit");
     GrpTiles t;
     t.nth = (P + TH - 1) / TH, t.ntw = (Q + TW - 1) / TW;
@@ -521,8 +727,8 @@ int launch_grouped_conv_s(const void *src, const float *w, const float *bias, co
     });
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
-    const GrpTiles t = grp_tiles<K, S>(d.P, d.Q, (long)d.N * ngroups);
-    const int pixels = grp_pixels<K, S>(t.th);
+    const GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, (long)d.N * ngroups);
+    const int pixels = grp_pixels<ConvSet<K, S>>(t.th);
     const long grid = 8L * (((long)d.N * t.nth * t.ntw + 7) / 8) * ngroups;
     if (grid > 0x7fffffffL) return DWO_ERR_BAD_SHAPE;
     grouped_conv_kernel<S, T, K><<<dim3((unsigned)grid), dim3(kGrpThreads), (pixels * 4 + CG * K) * sizeof(float),
@@ -532,8 +738,33 @@ int launch_grouped_conv_s(const void *src, const float *w, const float *bias, co
 }
 
 template <typename T, int K>
+int launch_grouped_dgrad2(const void *dy, const float *w, const void *taps, void *dx, const ConvDims &d_,
+                          hipStream_t st) {
+    using Set = QuadSet<K>;
+    constexpr int CG = grp_channels(sizeof(T));
+    static int cache[kMaxDevices];
+    per_device_once(cache, [&] {
+        allow_large_lds(grouped_dgrad2_kernel<T, K>, (kGrpPixels * 4 + CG * K) * sizeof(float));
+        return 1;
+    });
+    if (d_.N == 0) return 0;  // set-up only
+    ConvDims d = d_;
+    d.H = d.P, d.W = d.Q;
+    const int ngroups = d.C / CG;
+    const GrpTiles t = grp_tiles<Set>(d.P, d.Q, (long)d.N * ngroups);
+    const int pixels = grp_pixels<Set>(t.th);
+    const long grid = 8L * (((long)d.N * t.nth * t.ntw + 7) / 8) * ngroups;
+    if (grid > 0x7fffffffL) return DWO_ERR_BAD_SHAPE;
+    grouped_dgrad2_kernel<T, K><<<dim3((unsigned)grid), dim3(kGrpThreads), (pixels * 4 + CG * K) * sizeof(float),
+                                  st>>>((const T *)dy, w, taps, (T *)dx, d, t, pixels, d_.H, d_.W);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : (int)e;
+}
+
+template <typename T, int K>
 int launch_grouped_conv(const void *src, const float *w, const float *bias, const void *taps, void *dst,
                         const ConvDims &d, int flip, hipStream_t st) {
+    if (flip && d.stride == 2) return launch_grouped_dgrad2<T, K>(src, w, taps, dst, d, st);
     return d.stride == 1 ? launch_grouped_conv_s<T, K, 1>(src, w, bias, taps, dst, d, flip, st)
                          : launch_grouped_conv_s<T, K, 2>(src, w, bias, taps, dst, d, flip, st);
 }
@@ -551,8 +782,8 @@ int launch_grouped_wgrad_s(const void *x, const void *dy, const void *taps, floa
     });
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
-    const GrpTiles t = grp_tiles<K, S>(d.P, d.Q, kGrpSlots);  // (lower tiles would cost more partial sums)
-    const int floats = cmax(grp_pixels<K, S>(t.th) * 4, kRed);
+    const GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, kGrpSlots);  // (lower tiles would cost more partial sums)
+    const int floats = cmax(grp_pixels<ConvSet<K, S>>(t.th) * 4, kRed);
     if ((long)NG * ngroups > 0x7fffffffL) return DWO_ERR_BAD_SHAPE;
     grouped_wgrad_kernel<S, T, K><<<dim3(NG * ngroups), dim3(kGrpThreads), floats * sizeof(float), st>>>(
         (const T *)x, (const T *)dy, taps, part, d, t, NG);
