@@ -181,3 +181,16 @@ def test_pointwise_linear_gradients(shape, cin, dtype):
             first = g + (gg,)
     for a, b in zip(first, g + (gg,)):
         _close(a.detach(), b.detach(), dtype, "second order")
+
+
+def test_pointwise_linear_second_order_under_autocast():
+    """d(sum of dw) / dx under autocast: dw is linear in x, so it is the upstream gradient's channel sum."""
+    torch.manual_seed(0)
+    x = torch.randn(2, 5, 7, 3, device="cuda", requires_grad=True)
+    lin = torch.nn.Linear(3, 64).cuda()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = fused.pointwise_linear(x, lin)
+    dy = torch.randn(y.shape, device="cuda").to(torch.bfloat16).requires_grad_()
+    dw = torch.autograd.grad(y, lin.weight, dy, create_graph=True)[0]
+    gx = torch.autograd.grad(dw.sum(), x)[0]
+    _close(gx, dy.detach().double().sum(-1, keepdim=True).expand(x.shape), torch.bfloat16, "autocast second order")
