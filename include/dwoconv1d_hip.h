@@ -187,6 +187,10 @@ int dwo_set_wgrad_reduction(int in_kernel);
 int dwo_pointwise_fprop_nhwc(const void *x, const float *pw_w, const float *pw_b, const float *w,
                              const float *bias, const void *taps, void *y, int N, int Cin, int C,
                              int H, int W, int K, int stride, int dtype, void *stream);
+/* The same with a layout code: DWO_NHWC, or DWO_NHWC | DWO_GROUPED as dwo_fprop takes it. */
+int dwo_pointwise_fprop(const void *x, const float *pw_w, const float *pw_b, const float *w,
+                        const float *bias, const void *taps, void *y, int N, int Cin, int C, int H,
+                        int W, int K, int stride, int dtype, int layout, void *stream);
 
 /*
  * Forward-only glue of a ConvNeXt-1D block, each one pass over HBM in place of the PyTorch

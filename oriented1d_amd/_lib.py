@@ -28,6 +28,7 @@ SIGNATURES = {
     "dwo_wgrad_static": (_i, [_vp, _vp, _vp, _vp, _vp] + [_i] * 8 + [_vp]),
     "dwo_set_wgrad_reduction": (_i, [_i]),
     "dwo_pointwise_fprop_nhwc": (_i, [_vp] * 7 + [_i] * 8 + [_vp]),
+    "dwo_pointwise_fprop": (_i, [_vp] * 7 + [_i] * 9 + [_vp]),
     "dwo_layernorm_nhwc": (_i, [_vp, _vp, _vp, _vp, _sz, _i, ctypes.c_float, _i, _i, _vp]),
     "dwo_nchw_layernorm_nhwc": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, ctypes.c_float, _i, _vp]),
     "dwo_nhwc_scale_add_nchw": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),

@@ -487,6 +487,15 @@ template <typename T>
 int pointwise_fprop_t(const void *x, const float *pw_w, const float *pw_b, const float *w,
                       const float *bias, const void *taps, void *y, int Cin, const ConvDims &d,
                       hipStream_t st) {
+    // (the input is read element by element: only the output's alignment matters)
+    if (Cin == kGrpProjected && d.stride == 2 && grouped_shape(d, DWO_NHWC, sizeof(T)) && aligned16(y)) {
+        int rc = -100;
+#define DWO_MATCH(K_) \
+    if (d.K == K_) rc = launch_grouped_projected<T, K_>(x, pw_w, pw_b, w, bias, taps, y, d, st);
+        DWO_GROUPED_KS(DWO_MATCH)
+#undef DWO_MATCH
+        if (rc != -100) return rc;
+    }
     switch (Cin) {
         case 1: return launch_nhwc_tile_pointwise_fprop<T, 1>(x, pw_w, pw_b, w, bias, taps, y, d, st);
         case 2: return launch_nhwc_tile_pointwise_fprop<T, 2>(x, pw_w, pw_b, w, bias, taps, y, d, st);
@@ -575,6 +584,7 @@ int init_type() {
 #define DWO_PREP(K_)                                                                                       \
     rc |= launch_grouped_conv<T, K_>(nullptr, nullptr, nullptr, nullptr, nullptr, g, 0, nullptr);          \
     rc |= launch_grouped_conv<T, K_>(nullptr, nullptr, nullptr, nullptr, nullptr, g, 1, nullptr);          \
+    rc |= launch_grouped_projected<T, K_>(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, g, nullptr); \
     rc |= launch_grouped_wgrad<T, K_>(nullptr, nullptr, nullptr, nullptr, g, &ng, nullptr);
         DWO_GROUPED_KS(DWO_PREP)
 #undef DWO_PREP
@@ -788,14 +798,14 @@ int dwo_wgrad_static(const void *dy, const void *x, const void *taps, float *dw,
                           (hipStream_t)stream);
 }
 
-int dwo_pointwise_fprop_nhwc(const void *x, const float *pw_w, const float *pw_b, const float *w,
+int dwo_pointwise_fprop(const void *x, const float *pw_w, const float *pw_b, const float *w,
                              const float *bias, const void *taps, void *y, int N, int Cin, int C,
-                             int H, int W, int K, int stride, int dtype, void *stream) {
-    int rc = check_common(N, C, H, W, K, stride, dtype, DWO_NHWC);
+                             int H, int W, int K, int stride, int dtype, int layout, void *stream) {
+    int rc = check_common(N, C, H, W, K, stride, dtype, layout);
+    if (rc == DWO_OK && !(layout & DWO_NHWC)) rc = DWO_ERR_BAD_LAYOUT;
     if (rc != DWO_OK) return rc;
     if (!x || !pw_w || !w || !taps || !y) return DWO_ERR_NULL_POINTER;
     if (Cin < 1 || Cin > 4 || C % kSliceCh != 0) return DWO_ERR_BAD_SHAPE;
-    int layout = DWO_NHWC;
     const ConvDims d = make_dims(N, C, H, W, K, stride, layout);
     hipStream_t st = (hipStream_t)stream;
     begin_call();
@@ -804,6 +814,12 @@ int dwo_pointwise_fprop_nhwc(const void *x, const float *pw_w, const float *pw_b
         case DWO_BF16: return pointwise_fprop_t<bf16_t>(x, pw_w, pw_b, w, bias, taps, y, Cin, d, st);
         default: return pointwise_fprop_t<f16_t>(x, pw_w, pw_b, w, bias, taps, y, Cin, d, st);
     }
+}
+
+int dwo_pointwise_fprop_nhwc(const void *x, const float *pw_w, const float *pw_b, const float *w,
+                             const float *bias, const void *taps, void *y, int N, int Cin, int C,
+                             int H, int W, int K, int stride, int dtype, void *stream) {
+    return dwo_pointwise_fprop(x, pw_w, pw_b, w, bias, taps, y, N, Cin, C, H, W, K, stride, dtype, DWO_NHWC, stream);
 }
 
 size_t dwo_pointwise_wgrad_scratch_bytes(int Cin, int C) {

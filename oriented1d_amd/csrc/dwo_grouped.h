@@ -280,12 +280,12 @@ __device__ __forceinline__ unsigned grp_offset(const GrpTile &t, const ConvDims 
     return in ? o + threadIdx.x % 4 * 4 : kWinNowhere;
 }
 
+// outputs of a staged window
 template <int O, int S, typename T, int K>
-__device__ __forceinline__ void grp_conv_body(grp_u4 *lds, float *lw, const T *xn, T *yn, const float *bias,
-                                              const ConvDims &d, const GrpTile &t, int c0) {
+__device__ __forceinline__ void grp_conv_items(const grp_u4 *lds, const float *lw, T *yn, const float *bias,
+                                               const ConvDims &d, const GrpTile &t, int c0) {
     using G = GrpGeo<O, K, S>;
     constexpr int N = Word<T>::N, L = G::L;
-    grp_stage<G, S>(lds, xn, d, t, c0);
     __syncthreads();
     // this lane's weights, taps at one offset added up
     const int ch = (int)(threadIdx.x % 4) * N;
@@ -339,6 +339,13 @@ __device__ __forceinline__ void grp_conv_body(grp_u4 *lds, float *lw, const T *x
                 Word<T>::pack(acc[l]), out,
                 grp_offset<T>(t, d, GrpItems<G>::row_of(row, l), GrpItems<G>::col_of(col, l)), 0, 0);
     }
+}
+
+template <int O, int S, typename T, int K>
+__device__ __forceinline__ void grp_conv_body(grp_u4 *lds, float *lw, const T *xn, T *yn, const float *bias,
+                                              const ConvDims &d, const GrpTile &t, int c0) {
+    grp_stage<GrpGeo<O, K, S>, S>(lds, xn, d, t, c0);
+    grp_conv_items<O, S, T, K>(lds, lw, yn, bias, d, t, c0);
 }
 
 // A group whose channels do not share a canonical orientation (the caller's claim did not hold):
@@ -412,6 +419,134 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
         DWO_CASE(6)
         DWO_CASE(7)
         default: grp_conv_any<S, T, K>(xn, yn, wt, bias, taps_dhdw(blob), d, t, c0, flip);
+    }
+#undef DWO_CASE
+}
+
+// ---------------------------------------------------------------------------------------------
+// fprop behind a pointwise layer of CIN inputs (the stem's dw1(pw1(x)) at inference): a workgroup
+// projects the window's pixels to its group's channels while it stages them, rounded to T as the
+// layer's own output would be.  The image is read once per channel group (eight times at 64 channels of a
+// 16-bit type), and the C-channel tensor never exists.
+template <typename T>
+__device__ __forceinline__ float grp_value(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    else return Word<T>::get((unsigned)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0), 0);
+}
+
+template <typename T, int CIN>
+struct Projection {
+    static constexpr int CG = grp_channels(sizeof(T));
+    float w[CG][CIN], b[CG];  // uniform: scalar registers
+    __device__ __forceinline__ Projection(const float *pw_w, const float *pw_b, int c0) {
+#pragma unroll
+        for (int c = 0; c < CG; c++) {
+            b[c] = pw_b != nullptr ? pw_b[c0 + c] : 0.f;
+#pragma unroll
+            for (int k = 0; k < CIN; k++) w[c][k] = pw_w[(size_t)(c0 + c) * CIN + k];
+        }
+    }
+    __device__ __forceinline__ float channel(const float (&x)[CIN], int c) const {
+        float a = b[c];
+#pragma unroll
+        for (int k = 0; k < CIN; k++) a = __builtin_fmaf(x[k], w[c][k], a);
+        return a;
+    }
+};
+
+template <class G, int S, typename T, int CIN>
+__device__ __forceinline__ void grp_stage_projected(grp_u4 *lds, const T *img, const Projection<T, CIN> &pw,
+                                                    const ConvDims &d, const GrpTile &t) {
+    constexpr int N = Word<T>::N;
+    const __amdgpu_buffer_rsrc_t rsrc = win_rsrc(img, img + (size_t)d.H * d.W * CIN);
+    const unsigned ww = (((t.tw + G::L - 1) / G::L * G::L) - 1) * G::SC + 1 + G::EXTRA;
+    const unsigned nwin = G::rows(t.th) * ww, magic = win_magic(ww);
+    const int r0 = t.p * S - G::DH, q0 = t.q * S - G::DW - G::PADL;
+    constexpr int U = 4;
+    for (unsigned f0 = threadIdx.x; f0 < nwin; f0 += U * kGrpThreads) {
+        float v[U][CIN];
+        unsigned at[U];
+        bool in[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const unsigned f = f0 + u * kGrpThreads, i = win_div(f, magic), j = f - i * ww;
+            const int r = r0 + (int)i * (S / G::SR), q = q0 + (int)j * (S / G::SC);
+            in[u] = f < nwin && (unsigned)r < (unsigned)d.H && (unsigned)q < (unsigned)d.W;
+            at[u] = i * G::RS + G::col(j);
+            const unsigned o = ((unsigned)r * d.W + (unsigned)q) * (unsigned)(CIN * sizeof(T));
+#pragma unroll
+            for (int k = 0; k < CIN; k++)
+                v[u][k] = grp_value<T>(rsrc, in[u] ? o + k * (unsigned)sizeof(T) : kWinNowhere);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            grp_u4 px;
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                float a[N];
+#pragma unroll
+                for (int e = 0; e < N; e++) a[e] = pw.channel(v[u], m * N + e);
+                px[m] = in[u] ? Word<T>::pack(a) : 0u;
+            }
+            if (f0 + u * kGrpThreads < nwin) lds[at[u]] = px;
+        }
+    }
+}
+
+template <int S, typename T, int K, int CIN>
+__device__ void grp_projected_any(const T *img, T *yn, const float *wt, const float *bias, const float *pw_w,
+                                  const float *pw_b, const int8_t *dhdw, const ConvDims &d, const GrpTile &t, int c0) {
+    constexpr int CG = grp_channels(sizeof(T));
+    for (int f = threadIdx.x; f < t.vh * t.vw * CG; f += kGrpThreads) {
+        const int k = f % CG, o = f / CG, p = t.p + o / t.vw, q = t.q + o % t.vw, c = c0 + k;
+        float a = bias != nullptr ? bias[c] : 0.f;
+        for (int s = 0; s < K; s++) {
+            const int h = p * S + dhdw[((size_t)c * K + s) * 2], w = q * S + dhdw[((size_t)c * K + s) * 2 + 1];
+            if ((unsigned)h >= (unsigned)d.H || (unsigned)w >= (unsigned)d.W) continue;
+            float v = pw_b != nullptr ? pw_b[c] : 0.f;
+            for (int i = 0; i < CIN; i++)
+                v = __builtin_fmaf(to_float(img[((size_t)h * d.W + w) * CIN + i]), pw_w[(size_t)c * CIN + i], v);
+            a = __builtin_fmaf(to_float(from_float<T>(v)), wt[(size_t)c * K + s], a);
+        }
+        yn[((size_t)p * d.Q + q) * d.C + k] = from_float<T>(a);
+    }
+}
+
+template <int S, typename T, int K, int CIN>
+__global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void grouped_projected_kernel(
+    const T *__restrict__ x, const float *__restrict__ pw_w, const float *__restrict__ pw_b,
+    const float *__restrict__ wt, const float *__restrict__ bias, const void *__restrict__ blob, T *__restrict__ y,
+    ConvDims d, GrpTiles tiles, int pixels) {
+    extern __shared__ float lds_f[];
+    grp_u4 *lds = reinterpret_cast<grp_u4 *>(lds_f);
+    float *lw = lds_f + 4 * pixels;
+    constexpr int CG = grp_channels(sizeof(T));
+    int unit, group;
+    grp_task(d.C / CG, unit, group);
+    if (unit >= d.N * tiles.nth * tiles.ntw) return;
+    const int c0 = group * CG;
+    GrpTile t;
+    t.set(d, tiles, unit);
+    const T *img = x + (size_t)t.n * d.H * d.W * CIN;
+    T *yn = y + (size_t)t.n * d.P * d.Q * d.C + c0;
+    if (threadIdx.x < CG * K) lw[threadIdx.x] = wt[(size_t)c0 * K + threadIdx.x];
+    const Projection<T, CIN> pw(pw_w, pw_b, c0);
+#define DWO_CASE(O)                                                              \
+    case O:                                                                      \
+        grp_stage_projected<GrpGeo<O, K, S>, S, T, CIN>(lds, img, pw, d, t);     \
+        grp_conv_items<O, S, T, K>(lds, lw, yn, bias, d, t, c0);                 \
+        break;
+    switch (grp_class<CG>(taps_class(blob, d.C, K) + c0)) {
+        DWO_CASE(0)
+        DWO_CASE(1)
+        DWO_CASE(2)
+        DWO_CASE(3)
+        DWO_CASE(4)
+        DWO_CASE(5)
+        DWO_CASE(6)
+        DWO_CASE(7)
+        default:
+            grp_projected_any<S, T, K, CIN>(img, yn, wt, bias, pw_w, pw_b, taps_dhdw(blob), d, t, c0);
     }
 #undef DWO_CASE
 }
@@ -798,6 +933,28 @@ int launch_grouped_wgrad(const void *x, const void *dy, const void *taps, float 
     *groups_out = NG;
     return d.stride == 1 ? launch_grouped_wgrad_s<T, K, 1>(x, dy, taps, part, d, NG, st)
                          : launch_grouped_wgrad_s<T, K, 2>(x, dy, taps, part, d, NG, st);
+}
+
+template <typename T, int K>
+int launch_grouped_projected(const void *x, const float *pw_w, const float *pw_b, const float *w, const float *bias,
+                             const void *taps, void *y, const ConvDims &d, hipStream_t st) {
+    constexpr int CG = grp_channels(sizeof(T));
+    static int cache[kMaxDevices];
+    per_device_once(cache, [&] {
+        allow_large_lds(grouped_projected_kernel<2, T, K, kGrpProjected>, (kGrpPixels * 4 + CG * K) * sizeof(float));
+        return 1;
+    });
+    if (d.N == 0) return 0;  // set-up only
+    const int ngroups = d.C / CG;
+    const GrpTiles t = grp_tiles<ConvSet<K, 2>>(d.P, d.Q, (long)d.N * ngroups);
+    const int pixels = grp_pixels<ConvSet<K, 2>>(t.th);
+    const long grid = 8L * (((long)d.N * t.nth * t.ntw + 7) / 8) * ngroups;
+    if (grid > 0x7fffffffL) return -100;
+    grouped_projected_kernel<2, T, K, kGrpProjected>
+        <<<dim3((unsigned)grid), dim3(kGrpThreads), (pixels * 4 + CG * K) * sizeof(float), st>>>(
+            (const T *)x, pw_w, pw_b, w, bias, taps, (T *)y, d, t, pixels);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : (int)e;
 }
 
 }  // namespace dwo

@@ -16,6 +16,8 @@ constexpr int kGrpSlots = 512;     // workgroups resident on the chip
 constexpr int kGrpLeastRows = 8;  // of a tile that is cut to fill the chip
 // channels of one 16-byte pixel piece: they share an orientation
 constexpr int grp_channels(size_t esize) { return 16 / (int)esize; }
+// inputs of the pointwise layer that the projecting kernel is compiled for: the channels of an image
+constexpr int kGrpProjected = 3;
 // widest tile, in outputs
 constexpr int grp_tile_cols(int S) { return S == 1 ? 64 : 32; }
 
@@ -39,13 +41,20 @@ int launch_grouped_conv(const void *src, const float *w, const float *bias, cons
 template <typename T, int K>
 int launch_grouped_wgrad(const void *x, const void *dy, const void *taps, float *part, const ConvDims &d,
                          int *groups_out, hipStream_t st);
+// fprop at stride 2 behind a pointwise layer of kGrpProjected inputs
+template <typename T, int K>
+int launch_grouped_projected(const void *x, const float *pw_w, const float *pw_b, const float *w, const float *bias,
+                             const void *taps, void *y, const ConvDims &d, hipStream_t st);
 
 #define DWO_DECLARE(T, K)                                                                                \
     extern template int launch_grouped_conv<T, K>(const void *, const float *, const float *,           \
                                                   const void *, void *, const ConvDims &, int,          \
                                                   hipStream_t);                                         \
     extern template int launch_grouped_wgrad<T, K>(const void *, const void *, const void *, float *,   \
-                                                   const ConvDims &, int *, hipStream_t);
+                                                   const ConvDims &, int *, hipStream_t);              \
+    extern template int launch_grouped_projected<T, K>(const void *, const float *, const float *,      \
+                                                       const float *, const float *, const void *,      \
+                                                       void *, const ConvDims &, hipStream_t);
 #define DWO_DECLARE_ALL(K) DWO_DECLARE(float, K) DWO_DECLARE(bf16_t, K) DWO_DECLARE(f16_t, K)
 DWO_GROUPED_KS(DWO_DECLARE_ALL)
 #undef DWO_DECLARE_ALL

@@ -8,4 +8,7 @@ template int launch_grouped_conv<DWO_INST_T, DWO_INST_K>(const void *, const flo
                                                          hipStream_t);
 template int launch_grouped_wgrad<DWO_INST_T, DWO_INST_K>(const void *, const void *, const void *, float *,
                                                           const ConvDims &, int *, hipStream_t);
+template int launch_grouped_projected<DWO_INST_T, DWO_INST_K>(const void *, const float *, const float *,
+                                                              const float *, const float *, const void *, void *,
+                                                              const ConvDims &, hipStream_t);
 }  // namespace dwo

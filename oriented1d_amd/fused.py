@@ -113,14 +113,14 @@ def pointwise_dwconv_nhwc(x, linear, conv):
     w = _f32(conv.weight)
     if conv.resid is not None:
         w = w + conv.resid.to(w)
-    taps = conv._taps.get(conv.theta, C, K, x.device)  # cached per theta version
+    taps, layouts = conv._taps.lookup(conv.theta, C, K, x.device)  # cached per theta version
     P, Q = -(-H // stride), -(-W // stride)
     y = torch.empty((N, P, Q, C), dtype=x.dtype, device=x.device)
     pw_w = _f32(linear.weight)
     pw_b = _f32(linear.bias) if linear.bias is not None else None
     w2 = w.reshape(C, K)
     cb = _f32(conv.bias) if conv.bias is not None else None
-    _lib.check(_lib.ready(x.device).dwo_pointwise_fprop_nhwc(
+    _lib.check(_lib.ready(x.device).dwo_pointwise_fprop(
         _ptr(x), _ptr(pw_w), _ptr(pw_b), _ptr(w2), _ptr(cb), _ptr(taps), _ptr(y), N, Cin, C, H, W,
-        K, stride, _DTYPES[x.dtype], _stream(x)), "dwo_pointwise_fprop_nhwc")
+        K, stride, _DTYPES[x.dtype], layouts[x.element_size()], _stream(x)), "dwo_pointwise_fprop")
     return y

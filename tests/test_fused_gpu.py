@@ -194,3 +194,30 @@ def test_pointwise_linear_second_order_under_autocast():
     dw = torch.autograd.grad(y, lin.weight, dy, create_graph=True)[0]
     gx = torch.autograd.grad(dw.sum(), x)[0]
     _close(gx, dy.detach().double().sum(-1, keepdim=True).expand(x.shape), torch.bfloat16, "autocast second order")
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("C,H,W,K", [(64, 1, 1, 7), (64, 33, 66, 31), (64, 65, 131, 15), (128, 18, 5, 13),
+                                     (64, 97, 70, 27), (64, 2, 200, 31)])
+def test_projected_stem_tile_edges(C, H, W, K, dtype):
+    """The projecting kernel at the edges of its tiles, and where the claim of common orientations does
+    not hold (mixed angles behind it), against the two separate layers."""
+    from parity_util import canonical_theta, grouped_theta
+    from oriented1d_amd.dwoconv1d import DepthwiseOrientedConv1d
+
+    torch.manual_seed(H)
+    lin = torch.nn.Linear(3, C).cuda()
+    x = torch.randn(2, H, W, 3, device="cuda").to(dtype)
+    for theta, claimed in ((grouped_theta(C), False), (canonical_theta(C), True)):
+        conv = DepthwiseOrientedConv1d(C, C, K, groups=C, stride=2, padding=K // 2, bias=True, angle=theta.tolist(),
+                                       nhwc=True, arbitrary_size=True).cuda()
+        torch.nn.init.normal_(conv.bias, std=0.3)
+        if claimed:
+            look = conv._taps.lookup
+            conv._taps.lookup = lambda *a: (look(*a)[0], {2: 3, 4: 3})
+        with torch.no_grad():
+            got = fused.pointwise_dwconv_nhwc(x, lin, conv)
+            if claimed:
+                conv._taps.lookup = look
+            mid = torch.nn.functional.linear(x.double(), lin.weight.double(), lin.bias.double()).to(dtype)
+            _close(got, conv(mid), dtype, "projected")
