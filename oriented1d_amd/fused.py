@@ -95,7 +95,8 @@ def pointwise_linear(x, linear):
     # (an input that autocast converts is saved converted, without its history: one that is
     # differentiated itself stays with PyTorch, whose gradients of gradients reach it)
     if (torch.is_grad_enabled() and w.requires_grad and x.is_cuda and w.device == x.device and x.numel() > 0
-            and (x.dtype == dtype or not x.requires_grad) and dtype in _DTYPES and x.dtype in _DTYPES and 1 <= x.shape[-1] <= 4
+            and (x.dtype == dtype or not x.requires_grad) and dtype in _DTYPES and x.dtype in _DTYPES
+            and 1 <= x.shape[-1] <= 4
             and w.shape[0] * dtype.itemsize % 16 == 0 and w.shape[0] * dtype.itemsize <= 4096):
         return _PointwiseLinear.apply(x, w, b)
     return F.linear(x, w, b)
