@@ -59,8 +59,15 @@ class _PointwiseLinear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, b):
         ctx.set_materialize_grads(False)
-        y = F.linear(x, w, b)
-        ctx.save_for_backward(x if x.dtype == y.dtype else x.to(y.dtype), w, b)
+        xc, wc, bc = x, w, b
+        if torch.is_autocast_enabled(x.device.type):
+            # the conversions of autocast, but not its own: gradients are off here, and the copies that
+            # it keeps for the rest of the region would be cut off from the parameters
+            dtype = torch.get_autocast_dtype(x.device.type)
+            xc, wc, bc = (t if t is None else t.to(dtype) for t in (x, w, b))
+        with torch.autocast(x.device.type, enabled=False):
+            y = F.linear(xc, wc, bc)
+        ctx.save_for_backward(xc, w, b)
         ctx.x_dtype = x.dtype
         return y
 
@@ -95,7 +102,8 @@ def pointwise_linear(x, linear):
     # (an input that autocast converts is saved converted, without its history: one that is
     # differentiated itself stays with PyTorch, whose gradients of gradients reach it)
     if (torch.is_grad_enabled() and w.requires_grad and x.is_cuda and w.device == x.device and x.numel() > 0
-            and (x.dtype == dtype or not x.requires_grad) and dtype in _DTYPES and x.dtype in _DTYPES
+            and (x.dtype == dtype or not x.requires_grad) and dtype in _DTYPES
+            and all(t is None or t.dtype in _DTYPES for t in (x, w, b))
             and 1 <= x.shape[-1] <= 4
             and w.shape[0] * dtype.itemsize % 16 == 0 and w.shape[0] * dtype.itemsize <= 4096):
         return _PointwiseLinear.apply(x, w, b)

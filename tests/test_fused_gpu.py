@@ -221,3 +221,25 @@ def test_projected_stem_tile_edges(C, H, W, K, dtype):
                 conv._taps.lookup = look
             mid = torch.nn.functional.linear(x.double(), lin.weight.double(), lin.bias.double()).to(dtype)
             _close(got, conv(mid), dtype, "projected")
+
+
+@pytest.mark.parametrize("dtype", DTYPES[1:], ids=["bf16", "f16"])
+def test_pointwise_linear_leaves_the_autocast_cache_alone(dtype):
+    """Two passes of one autocast region, the second on an input that is differentiated itself (it stays
+    with PyTorch, which takes the region's cached low-precision parameters): both give the parameters
+    their gradients, as nn.Linear does, in either order."""
+    torch.manual_seed(1)
+    lin = torch.nn.Linear(3, 64).cuda()
+    x, xg = torch.randn(2, 2, 9, 11, 3, device="cuda").unbind(0)
+    xg = xg.clone().requires_grad_()
+    dy = torch.randn(2, 9, 11, 64, device="cuda").to(dtype)
+    for inputs in ((x, xg), (xg, x)):
+        grads = []
+        for layer in (fused.pointwise_linear, lambda a, m: m(a)):
+            with torch.autocast("cuda", dtype=dtype):
+                ys = [layer(a, lin) for a in inputs]
+            grads.append([torch.autograd.grad(y, (lin.weight, lin.bias), dy, allow_unused=True) for y in ys])
+        for got, want in zip(*grads):
+            for a, b in zip(got, want):
+                assert a is not None
+                _close(a, b, dtype, "autocast cache")
