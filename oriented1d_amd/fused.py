@@ -67,19 +67,21 @@ class _PointwiseLinear(torch.autograd.Function):
             xc, wc, bc = (t if t is None else t.to(dtype) for t in (x, w, b))
         with torch.autocast(x.device.type, enabled=False):
             y = F.linear(xc, wc, bc)
-        ctx.save_for_backward(xc, w, b)
-        ctx.x_dtype = x.dtype
+        # (only what backward reads: parameters may be updated between the passes where the input takes
+        # no gradient)
+        ctx.save_for_backward(xc, w if ctx.needs_input_grad[0] else None)
+        ctx.w_dtype, ctx.b_dtype = w.dtype, b.dtype if b is not None else None
         return y
 
     @staticmethod
     def backward(ctx, dy):
         if dy is None:
             return None, None, None
-        x, w, b = ctx.saved_tensors
+        x, w = ctx.saved_tensors
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
-            dx = torch.matmul(dy, w.to(dy.dtype)).to(ctx.x_dtype)
-        need_db = b is not None and ctx.needs_input_grad[2]
+            dx = torch.matmul(dy, w)
+        need_db = ctx.b_dtype is not None and ctx.needs_input_grad[2]
         if ctx.needs_input_grad[1] or need_db:
             dy, x = dy.contiguous(), x.contiguous()
             if torch.is_grad_enabled() or dy.data_ptr() % 16 != 0 or dy.dtype != x.dtype:
@@ -89,8 +91,8 @@ class _PointwiseLinear(torch.autograd.Function):
                 db = rows.sum(0)
             else:
                 dw, db = _lib.host(dy.get_device()).pointwise_wgrad(dy, x, need_db)
-            dw = dw.to(w.dtype) if ctx.needs_input_grad[1] else None
-            db = db.to(b.dtype) if need_db else None
+            dw = dw.to(ctx.w_dtype) if ctx.needs_input_grad[1] else None
+            db = db.to(ctx.b_dtype) if need_db else None
         return dx, dw, db
 
 
@@ -99,10 +101,10 @@ def pointwise_linear(x, linear):
     trained on a GPU, with the parameter gradients of ``dwo_pointwise_wgrad``."""
     w, b = linear.weight, linear.bias
     dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
-    # (an input that autocast converts is saved converted, without its history: one that is
-    # differentiated itself stays with PyTorch, whose gradients of gradients reach it)
+    # (what autocast converts is saved converted, without its history: an input that is differentiated
+    # itself stays with PyTorch then, whose gradients of gradients reach it and the weights)
     if (torch.is_grad_enabled() and w.requires_grad and x.is_cuda and w.device == x.device and x.numel() > 0
-            and (x.dtype == dtype or not x.requires_grad) and dtype in _DTYPES
+            and (x.dtype == w.dtype == dtype or not x.requires_grad) and dtype in _DTYPES
             and all(t is None or t.dtype in _DTYPES for t in (x, w, b))
             and 1 <= x.shape[-1] <= 4
             and w.shape[0] * dtype.itemsize % 16 == 0 and w.shape[0] * dtype.itemsize <= 4096):

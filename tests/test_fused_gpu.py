@@ -243,3 +243,21 @@ def test_pointwise_linear_leaves_the_autocast_cache_alone(dtype):
             for a, b in zip(got, want):
                 assert a is not None
                 _close(a, b, dtype, "autocast cache")
+
+
+def test_pointwise_linear_with_parameters_updated_before_backward():
+    """Images take no gradient, so backward needs no weights: an update between the passes (two losses,
+    stepped one after the other) is allowed, as with nn.Linear."""
+    torch.manual_seed(2)
+    lin = torch.nn.Linear(3, 64).cuda()
+    x, dy = torch.randn(2, 5, 7, 3, device="cuda"), torch.randn(2, 5, 7, 64, device="cuda")
+    for context in (torch.autocast("cuda", enabled=False), torch.autocast("cuda", dtype=torch.bfloat16)):
+        with context:
+            y = fused.pointwise_linear(x, lin)
+        assert type(y.grad_fn).__name__ == "_PointwiseLinearBackward"
+        with torch.no_grad():
+            lin.weight.mul_(0.5)
+            lin.bias.add_(1.0)
+        dw, db = torch.autograd.grad(y, (lin.weight, lin.bias), dy.to(y.dtype))
+        _close(dw, dy.double().reshape(-1, 64).t() @ x.double().reshape(-1, 3), y.dtype, "dw")
+        _close(db, dy.double().reshape(-1, 64).sum(0), y.dtype, "db")
