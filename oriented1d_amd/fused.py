@@ -6,6 +6,7 @@ gradient is being recorded; with autograd on it composes the same values from Py
 import ctypes
 
 import torch
+import torch.autograd.forward_ad as fwd
 import torch.nn.functional as F
 
 from . import _lib
@@ -96,6 +97,17 @@ class _PointwiseLinear(torch.autograd.Function):
         return dx, dw, db
 
 
+def _eager(*tensors):
+    """True for ordinary tensors in ordinary execution: no compilation, tracing, torch.func transform,
+    forward-mode derivative or tensor subclass, all of which an autograd function around native code would
+    hide the layer from."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._are_functorch_transforms_active()):
+        return False
+    return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter)
+                             and fwd.unpack_dual(t).tangent is None) for t in tensors)
+
+
 def pointwise_linear(x, linear):
     """``linear(x)`` of an ``nn.Linear`` with at most four inputs; where its parameters are being
     trained on a GPU, with the parameter gradients of ``dwo_pointwise_wgrad``."""
@@ -103,7 +115,8 @@ def pointwise_linear(x, linear):
     dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
     # (what autocast converts is saved converted, without its history: an input that is differentiated
     # itself stays with PyTorch then, whose gradients of gradients reach it and the weights)
-    if (torch.is_grad_enabled() and w.requires_grad and x.is_cuda and w.device == x.device and x.numel() > 0
+    if (torch.is_grad_enabled() and _eager(x, w, b)
+            and w.requires_grad and x.is_cuda and w.device == x.device and x.numel() > 0
             and (x.dtype == w.dtype == dtype or not x.requires_grad) and dtype in _DTYPES
             and all(t is None or t.dtype in _DTYPES for t in (x, w, b))
             and 1 <= x.shape[-1] <= 4

@@ -261,3 +261,44 @@ def test_pointwise_linear_with_parameters_updated_before_backward():
         dw, db = torch.autograd.grad(y, (lin.weight, lin.bias), dy.to(y.dtype))
         _close(dw, dy.double().reshape(-1, 64).t() @ x.double().reshape(-1, 3), y.dtype, "dw")
         _close(db, dy.double().reshape(-1, 64).sum(0), y.dtype, "db")
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("use", ["forward_mode", "func_grad", "vmap", "trace", "compile", "subclass"])
+def test_pointwise_linear_inside_transforms(use):
+    """What nn.Linear takes part in and an autograd function with a native backward cannot: forward-mode
+    derivatives, torch.func transforms, tracing, compilation and tensor subclasses."""
+    from oriented1d_amd.convnext1d import PointwiseLinear
+
+    torch.manual_seed(3)
+    lin = PointwiseLinear(3, 64).cuda()
+    plain = torch.nn.Linear(3, 64).cuda()
+    plain.load_state_dict(lin.state_dict())
+    x, t = torch.randn(2, 4, 5, 6, 3, device="cuda").unbind(0)
+
+    def results(layer):
+        if use == "forward_mode":
+            import torch.autograd.forward_ad as fw
+            with fw.dual_level():
+                dual = fw.unpack_dual(layer(fw.make_dual(x, t)))
+                return [dual.primal.detach(), dual.tangent.detach()]
+        if use == "func_grad":
+            p = {k: v.detach() for k, v in layer.named_parameters()}
+            return list(torch.func.grad(lambda q: torch.func.functional_call(layer, q, x).square().sum())(p).values())
+        if use == "vmap":
+            return [torch.vmap(layer)(x).detach()]
+        if use == "trace":
+            traced = torch.jit.trace(layer, x)
+            assert "PythonOp" not in str(traced.graph)
+            return [traced(t).detach()]
+        if use == "compile":
+            return [torch.compile(layer, backend="eager", fullgraph=True)(x).detach()]
+        y = layer(x.as_subclass(_Sub))
+        assert type(y) is _Sub and type(y.grad_fn).__name__ != "_PointwiseLinearBackward"
+        return [y.detach().as_subclass(torch.Tensor)]
+
+    for a, b in zip(results(lin), results(plain)):
+        _close(a, b, torch.float32, use)
