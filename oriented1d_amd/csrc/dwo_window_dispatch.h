@@ -38,7 +38,8 @@ inline bool win_has_k(int K) {
 }
 
 // Cuts a launch into units; false when the window kernels do not take the shape (rows shorter than
-// a four-column chunk, units beyond 32-bit byte offsets).
+// a four-column chunk, units beyond 32-bit byte offsets: a tile's window begins up to `pad` rows above the
+// image, and its offsets count from there).
 inline bool win_dims(int N, int C, int H, int W, int K, size_t esize, WinDims &d) {
     if (!win_has_k(K) || W < 4 || (double)H * W * esize >= 2147483648.0 || H > 32767) return false;
     d.N = N, d.C = C, d.H = H, d.W = W;
@@ -66,6 +67,8 @@ inline bool win_dims(int N, int C, int H, int W, int K, size_t esize, WinDims &d
         d.units = (N + d.PB - 1) / d.PB;
         return true;
     }
+    const int window_rows = (H < kWinMaxTile + pad ? H : kWinMaxTile + pad) + pad;
+    if ((double)window_rows * W * esize >= 2147483648.0) return false;
     // tiles of at most 64 x 64: the split with the least estimated work, per tile the rounds over
     // its row-blocks, the staging of its window and a fixed charge
     double best = 1e30;

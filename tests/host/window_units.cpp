@@ -1,0 +1,52 @@
+// Host-side checks of how the window kernels' launches are cut (dwo_window_dispatch.h), over the shapes that
+// they accept.  Prints one line per violation; exit status 0 when there is none.
+#include <cstdio>
+#include <cstring>
+
+#include "dwo_window_dispatch.h"
+
+using namespace dwo;
+
+static int failures = 0;
+#define EXPECT(cond, ...)                          \
+    do {                                           \
+        if (!(cond)) {                             \
+            if (failures++ < 20) printf(__VA_ARGS__); \
+        }                                          \
+    } while (0)
+
+// Byte offsets of a tile's window count from its corner, which may lie a halo above the image: those of the
+// rows and columns inside the image must stay below the descriptor's 2^31 - 1 bytes.
+static void check_offsets(int H, int W, int K, int es) {
+    WinDims d;
+    if (!win_dims(1, 8, H, W, K, es, d) || !d.tiled()) return;
+    for (int halo = 0; halo <= K / 2; halo++)
+        for (int a = 0; a < d.nth; a += d.nth > 3 && a == 1 ? d.nth - 2 : 1) {
+            const long corner = (long)a * d.th - halo, q_lo = (K / 2 + 3) & ~3;
+            for (long i = 0; i < d.th + 2 * halo; i++) {
+                if (corner + i < 0 || corner + i >= H) continue;
+                const long cols = cmin(W, d.tw + 2 * (int)q_lo + 4);
+                const long end = (i * W + cols) * es;
+                EXPECT(end <= 0x7fffffffL, "offset %ld: %d x %d, K %d, %d bytes, halo %d, tile row %d\n", end, H, W, K,
+                       es, halo, a);
+            }
+        }
+}
+
+int main() {
+    for (int K : {7, 13, 15, 27, 31})
+        for (int es : {2, 4})
+            for (int H : {1, 2, 4, 5, 16, 17, 48, 63, 64, 65, 100, 128, 200})
+                for (int rows = 1; rows <= 130; rows++)
+                    for (int extra : {-8, -1, 0, 1, 3, 8}) {
+                        const double W = 2147483648.0 / es / rows + extra;
+                        if (W * H * es < 2147483648.0) check_offsets(H, (int)W, K, es);
+                    }
+    for (int K : {7, 31}) {
+        WinDims d;
+        EXPECT(win_dims(1, 8, 64, 4000000, K, 4, d) && d.tiled(), "4 million columns are refused\n");
+        EXPECT(win_dims(1, 8, 1, 20000000, K, 4, d) && d.tiled(), "a row of 20 million columns is refused\n");
+    }
+    printf("%d violations\n", failures);
+    return failures != 0;
+}
