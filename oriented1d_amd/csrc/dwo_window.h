@@ -645,7 +645,11 @@ __device__ __forceinline__ void win_wgrad(const T *__restrict__ x, const T *__re
     float acc[K + 1];  // acc[s] for representative taps s, acc[K] = sum of dy (bias gradient)
 #pragma unroll
     for (int s = 0; s <= K; s++) acc[s] = 0.f;
+    // (item i of the unit.  Beyond its last item lie planes beyond its last: those are not behind the
+    // descriptor's bound, which covers the per-lane part of an address only.  In tile mode they are rows
+    // beyond its last, which load() leaves out)
     auto fetch = [&](const WinUnit<TILE> &u, unsigned i) {
+        if (!TILE && i >= u.planes(d) * grp.per_plane) return;  // uniform
         const T *at = dy + ((size_t)u.n * d.C + c) * plane + (size_t)u.p * d.W + u.q;
         const __amdgpu_buffer_rsrc_t rsrc = win_rsrc(at, dy + (size_t)d.N * d.C * plane);
         g.load(rsrc, rt, win_item(grp, rt, lds, i), (unsigned)d.W, u.rows(d), u.cols(d), grp.plane_elems);

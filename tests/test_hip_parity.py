@@ -224,7 +224,9 @@ def test_nchw_large_planes_many_tiles(oracle, stride, H, W, K, dtype):
 @pytest.mark.parametrize("N,C,H,W,K", [
     (1, 9, 1, 4, 31), (5, 12, 7, 5, 7), (9, 17, 8, 12, 15), (11, 9, 18, 28, 27), (3, 16, 31, 32, 31),
     (3, 9, 32, 33, 13), (2, 20, 37, 57, 27), (2, 9, 64, 63, 31), (1, 9, 65, 64, 31), (2, 9, 64, 65, 15),
-    (1, 16, 3, 200, 31), (1, 16, 131, 6, 31), (2, 9, 75, 113, 31), (1, 8, 128, 130, 7)])
+    (1, 16, 3, 200, 31), (1, 16, 131, 6, 31), (2, 9, 75, 113, 31), (1, 8, 128, 130, 7),
+    # (fewer items than waves: one plane, and a last unit of fewer planes than the others)
+    (1, 64, 20, 20, 31), (10, 40, 9, 11, 15)])
 def test_window_kernels_unit_edges(oracle, N, C, H, W, K, dtype):
     theta = canonical_theta(C)
     theta[8:9] = 0.61  # one channel on the table-driven body
