@@ -251,8 +251,10 @@ int wgrad_max_partials(const ConvDims &d_, int layout, size_t esize) {
     }
     const int PB = plane_batch(d, layout);
     WinDims wd;
-    if (PB == 0 && window_covers(d, layout, esize, wd))
-        return wd.units < kMaxWinGroups ? wd.units : kMaxWinGroups;
+    if (PB == 0 && window_covers(d, layout, esize, wd)) {
+        const int most = win_wgrad_groups(d.C, d.K);
+        return wd.units < most ? wd.units : most;
+    }
     if (PB == 0 && tile_covers(d, layout, esize)) {
         int band_rows, nbands;
         return tile_wgrad_groups(d, &band_rows, &nbands);

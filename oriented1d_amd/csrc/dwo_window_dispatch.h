@@ -25,7 +25,13 @@ struct WinDims {
 
 constexpr int kWinMaxTile = 64;
 constexpr int kWinMaxPlanes = 8;
-constexpr int kMaxWinGroups = 64;  // image groups per channel in wgrad (partial sums per tap)
+constexpr int kMaxWinGroups = 64;  // image groups per channel in wgrad (partial sums per tap), at most
+// and no more than dwo_wgrad_static has room for (C x (K + 1) sums each).  The bound starts at C = 1024
+// (K = 31), where a chip's slots make at most two groups per channel: no launch is cut differently for it.
+inline int win_wgrad_groups(int C, int K) {
+    const long fit = (long)(DWO_STATIC_SCRATCH_BYTES / sizeof(float)) / ((long)C * (K + 1));
+    return fit < 1 ? 1 : (fit < kMaxWinGroups ? (int)fit : kMaxWinGroups);
+}
 // Threads per workgroup, and staged four-column chunks per thread at most (plane and tile mode).
 constexpr int kWinThreads = 512;
 constexpr int win_slots_per_thread(bool tile) { return tile ? 5 : 2; }

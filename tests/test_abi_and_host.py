@@ -199,3 +199,15 @@ def test_state_dict_with_16_bit_theta_loads_as_fp32_values():
     m.load_state_dict(sd)
     assert m.theta.dtype == torch.float32
     assert torch.equal(m.theta.detach(), torch.tensor(angles).to(torch.bfloat16).float())
+
+
+def test_window_partial_sums_fit_the_static_scratch():
+    """NCHW wgrad at any extent bounds its image groups by DWO_STATIC_SCRATCH_BYTES, so dwo_wgrad_static
+    takes every channel count for which one group's sums fit: 64 x 1152 x 48 x 48 is 4.5 MiB in the tile
+    kernels' split."""
+    lib = _lib.load()
+    for C in (3, 96, 1024, 1025, 1152, 4096, 16384, 65536):
+        for N, H, W in ((64, 48, 48), (64, 5, 5), (1, 130, 130)):
+            if N * C * H * W < 2 ** 31:
+                got = lib.dwo_wgrad_scratch_bytes(N, C, H, W, 31, 1, 0, 0)
+                assert 0 < got <= 8 << 20, (N, C, H, W, got)

@@ -85,6 +85,7 @@ def test_two_calls_in_a_row_second_one_smaller():
     (2, 5, 33, 17, 7, 1, torch.float32, True),         # lane = channel kernel (C % 4 != 0)
     (1, 8, 40, 37, 63, 1, torch.float32, False),       # generic kernel (K = 63 at fp32)
     (2, 768, 7, 7, 31, 1, torch.float32, False),       # a single image group: no reduction pass
+    (64, 1152, 48, 48, 31, 1, torch.bfloat16, False),  # NCHW window kernel, its groups bounded by the array
 ])
 def test_kernel_families_share_the_static_scratch(N, C, H, W, K, stride, dtype, nhwc):
     _equal(_both(N, C, H, W, K, stride, dtype, nhwc, grouped_theta(C, 0.5), N + C, with_bias=N % 2 == 0))
