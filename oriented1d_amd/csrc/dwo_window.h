@@ -732,18 +732,6 @@ int win_slots(Kern kern, int threads, int *cache, size_t lds, int &cus) {
     const int by_regs = (packed & 0xffff) / cus, by_lds = (int)(160 * 1024 / lds);
     return cus * (by_lds < 1 ? 1 : (by_regs < by_lds ? by_regs : by_lds));
 }
-// units are dealt to as many workgroups per channel as the chip holds at once, or two rounds of
-// them where one would leave a quarter idle (plane_groups)
-inline int win_groups(const WinDims &d, int slots, int most) {
-    int g = slots / d.C;
-    if (g < 1) g = 1;
-    if ((long)d.C * g * 4 < (long)slots * 3) g = (2 * slots + d.C - 1) / d.C;
-    if (g > d.units) g = d.units;
-    if (g > most) g = most;
-    // workgroups of equal length: the launch ends with its slowest
-    const int per = (d.units + g - 1) / g;
-    return (d.units + per - 1) / per;
-}
 template <typename T, int K, int WM, bool TILE>
 int launch_window_conv_v(const void *src, const float *w, const float *bias, const void *taps, void *dst,
                          const WinDims &d, int flip, hipStream_t st) {
@@ -753,7 +741,7 @@ int launch_window_conv_v(const void *src, const float *w, const float *bias, con
     int cus = 0;
     const int slots = win_slots(window_kernel<T, K, WM, TILE>, WinMode<WM, TILE>::NT, cache, lds, cus);
     if (d.N == 0) return 0;  // set-up only
-    const int groups = win_groups(d, slots, kMaxWinGroups);
+    const int groups = win_groups(d, slots, cus, d.units);
     window_kernel<T, K, WM, TILE><<<dim3(d.C * groups), dim3(WinMode<WM, TILE>::NT), lds, st>>>(
         (const T *)src, w, bias, taps, (T *)dst, d, words, groups, flip);
     const hipError_t e = hipGetLastError();
@@ -779,7 +767,7 @@ int launch_window_wgrad_v(const void *x, const void *dy, const void *taps, float
     int cus = 0;
     const int slots = win_slots(window_wgrad_kernel<T, K, WM, TILE>, NT, cache, lds, cus);
     if (d.N == 0) return 0;
-    const int groups = win_groups(d, slots, win_wgrad_groups(d.C, K));
+    const int groups = win_groups(d, slots, cus, win_wgrad_groups(d.C, K));
     *groups_out = groups;
     window_wgrad_kernel<T, K, WM, TILE><<<dim3(plane_grid(d.C, groups, cus)), dim3(NT), lds, st>>>(
         (const T *)x, (const T *)dy, taps, WgradOut{part, dw, db, groups, tickets}, d, words, cus);

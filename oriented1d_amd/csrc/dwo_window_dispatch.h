@@ -95,6 +95,27 @@ inline bool win_dims(int N, int C, int H, int W, int K, size_t esize, WinDims &d
     return true;
 }
 
+// Workgroups per channel, at most `most`: as many as the chip holds at once (`slots` over all channels), or two
+// rounds of them where one would leave a quarter idle (plane_groups).  With few channels these are many short
+// workgroups; more than kMaxWinGroups of them only where that gives the busiest CU no more units than
+// kMaxWinGroups do (8 channels of 64 x 128 x 128, any angle: nine units 26.1 us, eight 24.8; 3 channels: three
+// 12.7, four 18.7).
+inline int win_groups(const WinDims &d, int slots, int cus, int most) {
+    // workgroups of equal length: the launch ends with its slowest
+    auto even = [&d](int g) {
+        const int per = (d.units + g - 1) / g;
+        return (d.units + per - 1) / per;
+    };
+    auto busiest = [&d, cus](int g) { return ((long)d.C * g + cus - 1) / cus * ((d.units + g - 1) / g); };
+    int g = slots / d.C;
+    if (g < 1) g = 1;
+    if ((long)d.C * g * 4 < (long)slots * 3) g = (2 * slots + d.C - 1) / d.C;
+    if (g > d.units) g = d.units;
+    if (g > most) g = most;
+    g = even(g);
+    if (g > kMaxWinGroups && busiest(g) > busiest(even(kMaxWinGroups))) g = even(kMaxWinGroups);
+    return g;
+}
 template <typename T, int K>
 int launch_window_conv(const void *src, const float *w, const float *bias, const void *taps, void *dst,
                        const WinDims &d, int flip, hipStream_t st);

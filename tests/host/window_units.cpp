@@ -47,6 +47,19 @@ int main() {
         EXPECT(win_dims(1, 8, 64, 4000000, K, 4, d) && d.tiled(), "4 million columns are refused\n");
         EXPECT(win_dims(1, 8, 1, 20000000, K, 4, d) && d.tiled(), "a row of 20 million columns is refused\n");
     }
+    // few channels: the workgroups fill the chip's slots where there are units for them, in wgrad within
+    // its partial sums
+    for (int C : {1, 2, 3, 5, 8, 11, 12, 64, 96})
+        for (int slots : {512, 768, 1024}) {
+            WinDims d;
+            const int N = 4096 / C;
+            EXPECT(win_dims(N, C, 128, 128, 31, 4, d), "128 x 128 is refused\n");
+            const int groups = win_groups(d, slots, 256, d.units);
+            const int sums = win_groups(d, slots, 256, win_wgrad_groups(C, 31));
+            EXPECT((C * groups >= 512 || C * groups * 4 >= slots * 3) && groups <= d.units,
+                   "%d groups of %d channels in %d slots\n", groups, C, slots);
+            EXPECT(sums >= 1 && sums <= kMaxWinGroups, "%d groups of sums\n", sums);
+        }
     printf("%d violations\n", failures);
     return failures != 0;
 }
