@@ -377,14 +377,6 @@ __device__ __forceinline__ int grp_class(const int32_t *cls) {
     return __builtin_amdgcn_readfirstlane(o);
 }
 
-// Workgroup -> (unit, channel group): the groups of a unit, which share its lines, get ids of one XCD
-// (consecutive ids go to the eight XCDs in turn) at about the same time.
-__device__ __forceinline__ void grp_task(int ngroups, int &unit, int &group) {
-    const int k = blockIdx.x / 8;
-    unit = blockIdx.x % 8 + 8 * (k / ngroups);
-    group = k % ngroups;
-}
-
 template <int S, typename T, int K>
 __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void grouped_conv_kernel(
     const T *__restrict__ x, const float *__restrict__ wt, const float *__restrict__ bias,
@@ -394,8 +386,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
     float *lw = lds_f + 4 * pixels;  // the group's weights
     constexpr int CG = grp_channels(sizeof(T));
     int unit, group;
-    grp_task(d.C / CG, unit, group);
-    if (unit >= d.N * tiles.nth * tiles.ntw) return;
+    if (!grp_task(blockIdx.x, d.N * tiles.nth * tiles.ntw, d.C / CG, unit, group)) return;
     const int c0 = group * CG;
     GrpTile t;
     t.set(d, tiles, unit);
@@ -524,8 +515,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
     float *lw = lds_f + 4 * pixels;
     constexpr int CG = grp_channels(sizeof(T));
     int unit, group;
-    grp_task(d.C / CG, unit, group);
-    if (unit >= d.N * tiles.nth * tiles.ntw) return;
+    if (!grp_task(blockIdx.x, d.N * tiles.nth * tiles.ntw, d.C / CG, unit, group)) return;
     const int c0 = group * CG;
     GrpTile t;
     t.set(d, tiles, unit);
@@ -657,8 +647,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
     float *lw = lds_f + 4 * pixels;
     constexpr int CG = grp_channels(sizeof(T));
     int unit, group;
-    grp_task(d.C / CG, unit, group);
-    if (unit >= d.N * tiles.nth * tiles.ntw) return;
+    if (!grp_task(blockIdx.x, d.N * tiles.nth * tiles.ntw, d.C / CG, unit, group)) return;
     const int c0 = group * CG;
     GrpTile t;
     t.set(d, tiles, unit);
@@ -812,7 +801,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
     grp_u4 *lds = reinterpret_cast<grp_u4 *>(lds_f);
     constexpr int CG = grp_channels(sizeof(T));
     int g, group;
-    grp_task(d.C / CG, g, group);
+    if (!grp_task(blockIdx.x, NG, d.C / CG, g, group)) return;
     const int c0 = group * CG;
 #define DWO_CASE(O)                                                               \
     case O:                                                                       \
@@ -866,7 +855,7 @@ int launch_grouped_conv_s(const void *src, const float *w, const float *bias, co
     const int ngroups = d.C / CG;
     const GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, (long)d.N * ngroups);
     const int pixels = grp_pixels<ConvSet<K, S>>(t.th);
-    const long grid = 8L * (((long)d.N * t.nth * t.ntw + 7) / 8) * ngroups;
+    const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (grid > 0x7fffffffL) return DWO_ERR_BAD_SHAPE;
     grouped_conv_kernel<S, T, K><<<dim3((unsigned)grid), dim3(kGrpThreads), (pixels * 4 + CG * K) * sizeof(float),
                                    st>>>((const T *)src, w, bias, taps, (T *)dst, d, t, pixels, flip);
@@ -890,7 +879,7 @@ int launch_grouped_dgrad2(const void *dy, const float *w, const void *taps, void
     const int ngroups = d.C / CG;
     const GrpTiles t = grp_tiles<Set>(d.P, d.Q, (long)d.N * ngroups);
     const int pixels = grp_pixels<Set>(t.th);
-    const long grid = 8L * (((long)d.N * t.nth * t.ntw + 7) / 8) * ngroups;
+    const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (grid > 0x7fffffffL) return DWO_ERR_BAD_SHAPE;
     grouped_dgrad2_kernel<T, K><<<dim3((unsigned)grid), dim3(kGrpThreads), (pixels * 4 + CG * K) * sizeof(float),
                                   st>>>((const T *)dy, w, taps, (T *)dx, d, t, pixels, d_.H, d_.W);
@@ -921,8 +910,9 @@ int launch_grouped_wgrad_s(const void *x, const void *dy, const void *taps, floa
     const int ngroups = d.C / CG;
     const GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, kGrpSlots);  // (lower tiles would cost more partial sums)
     const int floats = cmax(grp_pixels<ConvSet<K, S>>(t.th) * 4, kRed);
-    if ((long)NG * ngroups > 0x7fffffffL) return DWO_ERR_BAD_SHAPE;
-    grouped_wgrad_kernel<S, T, K><<<dim3(NG * ngroups), dim3(kGrpThreads), floats * sizeof(float), st>>>(
+    const long grid = grp_grid(NG, ngroups);
+    if (grid > 0x7fffffffL) return DWO_ERR_BAD_SHAPE;
+    grouped_wgrad_kernel<S, T, K><<<dim3((unsigned)grid), dim3(kGrpThreads), floats * sizeof(float), st>>>(
         (const T *)x, (const T *)dy, taps, part, d, t, NG);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : (int)e;
@@ -950,7 +940,7 @@ int launch_grouped_projected(const void *x, const float *pw_w, const float *pw_b
     const int ngroups = d.C / CG;
     const GrpTiles t = grp_tiles<ConvSet<K, 2>>(d.P, d.Q, (long)d.N * ngroups);
     const int pixels = grp_pixels<ConvSet<K, 2>>(t.th);
-    const long grid = 8L * (((long)d.N * t.nth * t.ntw + 7) / 8) * ngroups;
+    const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (grid > 0x7fffffffL) return -100;
     grouped_projected_kernel<2, T, K, kGrpProjected>
         <<<dim3((unsigned)grid), dim3(kGrpThreads), (pixels * 4 + CG * K) * sizeof(float), st>>>(

@@ -21,6 +21,25 @@ constexpr int kGrpProjected = 3;
 // widest tile, in outputs
 constexpr int grp_tile_cols(int S) { return S == 1 ? 64 : 32; }
 
+// Workgroup -> (unit, channel group) of a launch's units x ngroups tasks.  The groups of a unit share its lines, so
+// they get ids of one XCD (consecutive ids go to the eight XCDs in turn) at about the same time: unit u runs on
+// XCD u % 8.  The tasks of the units beyond the last eight are dealt to all XCDs in runs of equal length instead:
+// two images of 1024 x 28 x 28 fp32 ran on two of the eight (fprop 27 us; now 9.2, on the slice kernels 9.4).
+// False for the ids that fill up the last run.
+constexpr long grp_grid(long units, int ngroups) { return 8 * (units / 8 * ngroups + (units % 8 * ngroups + 7) / 8); }
+__host__ __device__ inline bool grp_task(unsigned block, int units, int ngroups, int &unit, int &group) {
+    const unsigned xcd = block % 8, k = block / 8, full = (unsigned)(units / 8 * ngroups);
+    if (k < full) {
+        unit = (int)(k / (unsigned)ngroups * 8 + xcd);
+        group = (int)(k % (unsigned)ngroups);
+        return true;
+    }
+    const unsigned t = xcd * (unsigned)((units % 8 * ngroups + 7) / 8) + (k - full);
+    unit = units / 8 * 8 + (int)(t / (unsigned)ngroups);
+    group = (int)(t % (unsigned)ngroups);
+    return unit < units;
+}
+
 struct GrpTiles {
     int th, tw, nth, ntw;  // tile extents and counts
 };

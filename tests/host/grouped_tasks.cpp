@@ -1,0 +1,33 @@
+// Host-side check of the grouped kernels' task map (dwo_grouped_dispatch.h): every (unit, channel group) once, the
+// eight XCDs within one task of each other.  Prints one line per violation; exit status 0 when there is none.
+#include <algorithm>
+#include <cstdio>
+#include <vector>
+
+#include "dwo_grouped_dispatch.h"
+
+using namespace dwo;
+
+int main() {
+    int failures = 0;
+    for (int units : {1, 2, 3, 7, 8, 9, 64, 257})
+        for (int ngroups : {1, 2, 3, 8, 12, 24, 100, 512}) {
+            std::vector<int> seen((size_t)units * ngroups, 0), per_xcd(8, 0);
+            const unsigned grid = (unsigned)grp_grid(units, ngroups);
+            for (unsigned b = 0; b < grid; b++) {
+                int unit = 0, group = 0;
+                if (!grp_task(b, units, ngroups, unit, group)) continue;
+                if (unit < 0 || unit >= units || group < 0 || group >= ngroups) {
+                    printf("block %u of %u: unit %d, group %d\n", b, grid, unit, group), failures++;
+                    continue;
+                }
+                seen[(size_t)unit * ngroups + group]++, per_xcd[b % 8]++;
+            }
+            const bool once = std::all_of(seen.begin(), seen.end(), [](int n) { return n == 1; });
+            const int most = *std::max_element(per_xcd.begin(), per_xcd.end());
+            // (the last runs are short)
+            if (!once || most != (units * ngroups + 7) / 8)
+                printf("%d units, %d groups: %s, %d tasks on one XCD\n", units, ngroups, once ? "once" : "not once", most), failures++;
+        }
+    return failures != 0;
+}
