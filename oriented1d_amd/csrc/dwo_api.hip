@@ -191,6 +191,7 @@ int try_window_wgrad(const void *x, const void *dy, const void *taps, float *par
 bool grouped_shape(const ConvDims &d, int layout, size_t esize) {
     if (!d.grouped || layout != DWO_NHWC || d.stride > 2 || d.C % grp_channels(esize) != 0) return false;
     if ((size_t)d.H * d.W * d.C * esize >= 0x80000000ull) return false;
+    if (!grp_grid_fits(grp_grid(8, d.C / grp_channels(esize)))) return false;  // (wgrad's smallest launch)
 #define DWO_MATCH(K_) if (d.K == K_) return true;
     DWO_GROUPED_KS(DWO_MATCH)
 #undef DWO_MATCH

@@ -856,7 +856,7 @@ int launch_grouped_conv_s(const void *src, const float *w, const float *bias, co
     const GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, (long)d.N * ngroups);
     const int pixels = grp_pixels<ConvSet<K, S>>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
-    if (grid > 0x7fffffffL) return DWO_ERR_BAD_SHAPE;
+    if (!grp_grid_fits(grid)) return -100;
     grouped_conv_kernel<S, T, K><<<dim3((unsigned)grid), dim3(kGrpThreads), (pixels * 4 + CG * K) * sizeof(float),
                                    st>>>((const T *)src, w, bias, taps, (T *)dst, d, t, pixels, flip);
     const hipError_t e = hipGetLastError();
@@ -880,7 +880,7 @@ int launch_grouped_dgrad2(const void *dy, const float *w, const void *taps, void
     const GrpTiles t = grp_tiles<Set>(d.P, d.Q, (long)d.N * ngroups);
     const int pixels = grp_pixels<Set>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
-    if (grid > 0x7fffffffL) return DWO_ERR_BAD_SHAPE;
+    if (!grp_grid_fits(grid)) return -100;
     grouped_dgrad2_kernel<T, K><<<dim3((unsigned)grid), dim3(kGrpThreads), (pixels * 4 + CG * K) * sizeof(float),
                                   st>>>((const T *)dy, w, taps, (T *)dx, d, t, pixels, d_.H, d_.W);
     const hipError_t e = hipGetLastError();
@@ -910,9 +910,7 @@ int launch_grouped_wgrad_s(const void *x, const void *dy, const void *taps, floa
     const int ngroups = d.C / CG;
     const GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, kGrpSlots);  // (lower tiles would cost more partial sums)
     const int floats = cmax(grp_pixels<ConvSet<K, S>>(t.th) * 4, kRed);
-    const long grid = grp_grid(NG, ngroups);
-    if (grid > 0x7fffffffL) return DWO_ERR_BAD_SHAPE;
-    grouped_wgrad_kernel<S, T, K><<<dim3((unsigned)grid), dim3(kGrpThreads), floats * sizeof(float), st>>>(
+    grouped_wgrad_kernel<S, T, K><<<dim3((unsigned)grp_grid(NG, ngroups)), dim3(kGrpThreads), floats * sizeof(float), st>>>(
         (const T *)x, (const T *)dy, taps, part, d, t, NG);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : (int)e;
@@ -941,7 +939,7 @@ int launch_grouped_projected(const void *x, const float *pw_w, const float *pw_b
     const GrpTiles t = grp_tiles<ConvSet<K, 2>>(d.P, d.Q, (long)d.N * ngroups);
     const int pixels = grp_pixels<ConvSet<K, 2>>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
-    if (grid > 0x7fffffffL) return -100;
+    if (!grp_grid_fits(grid)) return -100;
     grouped_projected_kernel<2, T, K, kGrpProjected>
         <<<dim3((unsigned)grid), dim3(kGrpThreads), (pixels * 4 + CG * K) * sizeof(float), st>>>(
             (const T *)x, pw_w, pw_b, w, bias, taps, (T *)y, d, t, pixels);

@@ -27,6 +27,9 @@ constexpr int grp_tile_cols(int S) { return S == 1 ? 64 : 32; }
 // two images of 1024 x 28 x 28 fp32 ran on two of the eight (fprop 27 us; now 9.2, on the slice kernels 9.4).
 // False for the ids that fill up the last run.
 constexpr long grp_grid(long units, int ngroups) { return 8 * (units / 8 * ngroups + (units % 8 * ngroups + 7) / 8); }
+// A launch holds fewer than 2^32 threads; what needs more goes to the kernels that would take it otherwise (the slice
+// kernels walk any number of planes of 56 x 56 and 28 x 28 with the chip's slots).
+constexpr bool grp_grid_fits(long grid) { return grid * kGrpThreads < 1L << 32; }
 __host__ __device__ inline bool grp_task(unsigned block, int units, int ngroups, int &unit, int &group) {
     const unsigned xcd = block % 8, k = block / 8, full = (unsigned)(units / 8 * ngroups);
     if (k < full) {

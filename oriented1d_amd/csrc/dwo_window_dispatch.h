@@ -48,6 +48,8 @@ inline bool win_has_k(int K) {
 // image, and its offsets count from there).
 inline bool win_dims(int N, int C, int H, int W, int K, size_t esize, WinDims &d) {
     if (!win_has_k(K) || W < 4 || (double)H * W * esize >= 2147483648.0 || H > 32767) return false;
+    // (a launch holds fewer than 2^32 threads: a workgroup per channel at least, on a padded grid)
+    if (((long)C + 4096) * kWinThreads >= 1L << 32) return false;
     d.N = N, d.C = C, d.H = H, d.W = W;
     const int pad = K / 2;
     // a wave takes 64 lanes of row-blocks: rounds of the workgroup's waves over those of `planes`

@@ -29,5 +29,13 @@ int main() {
             if (!once || most != (units * ngroups + 7) / 8)
                 printf("%d units, %d groups: %s, %d tasks on one XCD\n", units, ngroups, once ? "once" : "not once", most), failures++;
         }
+    // launches of fewer than 2^32 threads
+    for (long units : {1L, 7L, 8L, 9L, 100L, 16384L, 131071L, 131072L, 131073L, 1L << 27})
+        for (int ngroups : {1, 8, 64, 512, 1 << 20, (1 << 20) + 1}) {
+            const long grid = grp_grid(units, ngroups);
+            const bool fits = grid * 512 <= 0xffffffffL;
+            if (grid < units * ngroups || grp_grid_fits(grid) != fits)
+                printf("%ld units, %d groups: %ld workgroups\n", units, ngroups, grid), failures++;
+        }
     return failures != 0;
 }

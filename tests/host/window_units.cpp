@@ -47,6 +47,13 @@ int main() {
         EXPECT(win_dims(1, 8, 64, 4000000, K, 4, d) && d.tiled(), "4 million columns are refused\n");
         EXPECT(win_dims(1, 8, 1, 20000000, K, 4, d) && d.tiled(), "a row of 20 million columns is refused\n");
     }
+    // a workgroup per channel, in launches of fewer than 2^32 threads
+    for (long C : {1L << 20, 8000000L, 8384511L, 8388607L, 8388608L, 20000000L}) {
+        WinDims d;
+        if (!win_dims(1, (int)C, 4, 4, 31, 2, d)) continue;
+        const long groups = win_groups(d, 1024, 256, d.units);
+        EXPECT((C * groups + 255) / 256 * 256 * kWinThreads < 1L << 32, "%ld channels in %ld groups\n", C, groups);
+    }
     // few channels: the workgroups fill the chip's slots where there are units for them, in wgrad within
     // its partial sums
     for (int C : {1, 2, 3, 5, 8, 11, 12, 64, 96})
