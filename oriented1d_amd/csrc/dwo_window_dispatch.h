@@ -75,6 +75,15 @@ inline bool win_dims(int N, int C, int H, int W, int K, size_t esize, WinDims &d
         d.units = (N + d.PB - 1) / d.PB;
         return true;
     }
+    // Thin planes.  A tile's waves stand for 32 rows of 64 columns, so of a plane of few rows or columns most
+    // of the issue slots are spent on nothing, where the tile kernels fit their windows to the plane.  Those
+    // take them from about the batch on at which they fill the chip (four channels of up to 32 rows per
+    // workgroup); below it the window kernels' shorter chains win.  fprop us, tile / window kernels, K = 31:
+    // 32 x 384 x 4 x 256 bf16 87 / 177, 64 x 200 x 7 x 256 fp32 160 / 224, 32 x 200 x 400 x 6 fp32 (any angle)
+    // 263 / 459; 2 x 384 x 8 x 400 fp32 73 / 26; K = 7 in narrow planes: 64 x 96 x 190 x 5 bf16 96 / 54.
+    const long planes = (long)N * C;
+    if (H <= 4 ? planes >= 768 : (H <= 8 && planes >= 1536)) return false;
+    if (W <= 8 && K > 7 && planes >= 6144) return false;
     const int window_rows = (H < kWinMaxTile + pad ? H : kWinMaxTile + pad) + pad;
     if ((double)window_rows * W * esize >= 2147483648.0) return false;
     // tiles of at most 64 x 64: the split with the least estimated work, per tile the rounds over

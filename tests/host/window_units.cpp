@@ -54,6 +54,16 @@ int main() {
         const long groups = win_groups(d, 1024, 256, d.units);
         EXPECT((C * groups + 255) / 256 * 256 * kWinThreads < 1L << 32, "%ld channels in %ld groups\n", C, groups);
     }
+    // thin planes of more than 64 rows or columns: small batches are taken, large ones left to the tile kernels
+    for (int large : {0, 1}) {
+        WinDims d;
+        EXPECT(win_dims(large ? 32 : 2, 200, 4, 400, 31, 2, d) == !large, "4 x 400, batch %d\n", large);
+        EXPECT(win_dims(large ? 64 : 2, 200, 8, 256, 31, 4, d) == !large, "8 x 256, batch %d\n", large);
+        EXPECT(win_dims(large ? 32 : 2, 200, 400, 6, 31, 4, d) == !large, "400 x 6, batch %d\n", large);
+        EXPECT(win_dims(large ? 64 : 2, 200, 400, 6, 7, 4, d) && win_dims(large ? 64 : 2, 200, 9, 400, 31, 2, d) &&
+                   win_dims(large ? 64 : 2, 200, 4, 64, 31, 4, d),
+               "a plane that is not thin, batch %d\n", large);
+    }
     // few channels: the workgroups fill the chip's slots where there are units for them, in wgrad within
     // its partial sums
     for (int C : {1, 2, 3, 5, 8, 11, 12, 64, 96})
