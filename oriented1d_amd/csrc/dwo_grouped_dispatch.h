@@ -47,14 +47,19 @@ struct GrpTiles {
     int th, tw, nth, ntw;  // tile extents and counts
 };
 
-// Partial sums per (channel, tap): a multiple of eight (unit u runs on XCD u % 8), about two rounds of the
-// chip's slots at most, and no more than there are tiles of 16 x 32 outputs (surplus groups
-// contribute zeros).
+// Partial sums per (channel, tap): about two rounds of the chip's slots at most, and no more than there are tiles of
+// 16 x 32 outputs; a multiple of eight (unit u runs on XCD u % 8) where there are as many tiles.  A workgroup's sums
+// over lanes and waves cost as much as a few hundred outputs, so it gets 256 of them, or four tiles where tiles are
+// that small (surplus groups would add zeros, at that cost).  K = 31, us, with a group per tile / like this:
+// 107 x 16 x 5 x 64 fp32 38 / 28, 64 x 64 x 17 x 17 bf16 stride 2 44 / 33, 53 x 32 x 4 x 84 fp32 33 / 25.
 inline int grp_wgrad_groups(const ConvDims &d, size_t esize) {
     const long units = (long)d.N * ((d.P + 15) / 16) * ((d.Q + 31) / 32), ngroups = d.C / grp_channels(esize);
+    long most = (long)d.N * d.P * d.Q / 256;
+    if (most < (units + 3) / 4) most = (units + 3) / 4;
     long G = 1024 / ngroups;
-    if (G > units) G = units;
-    return (int)((G < 1 ? 1 : G) + 7) / 8 * 8;
+    if (G > most) G = most;
+    G = ((G < 1 ? 1 : G) + 7) / 8 * 8;
+    return (int)(G < units ? G : units);
 }
 
 template <typename T, int K>

@@ -37,5 +37,19 @@ int main() {
             if (grid < units * ngroups || grp_grid_fits(grid) != fits)
                 printf("%ld units, %d groups: %ld workgroups\n", units, ngroups, grid), failures++;
         }
+    // wgrad's groups: each has a tile, and all of them fit a launch
+    for (int N : {1, 3, 64, 300})
+        for (int C : {16, 64, 272, 2048, 65536})
+            for (int P : {1, 2, 5, 17, 40, 112})
+                for (int Q : {1, 9, 33, 128})
+                    for (int es : {2, 4}) {
+                        ConvDims d{};
+                        d.N = N, d.C = C, d.P = P, d.Q = Q;
+                        const long units = (long)N * ((P + 15) / 16) * ((Q + 31) / 32);
+                        const int G = grp_wgrad_groups(d, es), ngroups = C / grp_channels(es);
+                        if (G < 1 || G > units || (G > 8 && (long)G * ngroups > 1024 + 8L * ngroups) ||
+                            !grp_grid_fits(grp_grid(G, ngroups)))
+                            printf("%d groups of %d x %d x %d x %d\n", G, N, C, P, Q), failures++;
+                    }
     return failures != 0;
 }
