@@ -582,13 +582,10 @@ struct WinDy {
         else return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, off, soff, 0);
     }
     __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rsrc, const WinRt &rt, const WinItem &it,
-                                         unsigned W, int planes, int rows, int cols, unsigned plane_elems) {
+                                         unsigned W, int rows, int cols, unsigned plane_elems) {
         constexpr unsigned ES = sizeof(T);
         const unsigned soff = (it.pl * plane_elems + (unsigned)it.row0 * W) * ES;
-        // (planes beyond the unit's last have no rows: the descriptor's bound covers the per-lane part of an
-        // address only, not soff.  A branch around the loads instead took 512 x 3 x 60 x 60 in bf16 from 31 to
-        // 43 us)
-        const int left = it.pl < (unsigned)planes ? rows - it.row0 : 0;  // uniform
+        const int left = rows - it.row0;
         if (rt.cls == CLS_H) {
             // (a quad that the unit's last column cuts is loaded from four columns before its end
             // and shifted: units are at least four columns wide)
@@ -648,11 +645,14 @@ __device__ __forceinline__ void win_wgrad(const T *__restrict__ x, const T *__re
     float acc[K + 1];  // acc[s] for representative taps s, acc[K] = sum of dy (bias gradient)
 #pragma unroll
     for (int s = 0; s <= K; s++) acc[s] = 0.f;
-    // (item i of the unit, or nothing beyond its last)
+    // (Item i of the unit.  A wave without one loads the last again and drops it: behind that lie planes that
+    // need not be there, and the descriptor's bound covers the per-lane part of an address only, not soff.  The
+    // loads sent nowhere instead, as rows that do not exist, took 19 x 829 x 35 x 35 in bf16 from 74 to 84 us.)
     auto fetch = [&](const WinUnit<TILE> &u, unsigned i) {
         const T *at = dy + ((size_t)u.n * d.C + c) * plane + (size_t)u.p * d.W + u.q;
         const __amdgpu_buffer_rsrc_t rsrc = win_rsrc(at, dy + (size_t)d.N * d.C * plane);
-        g.load(rsrc, rt, win_item(grp, rt, lds, i), (unsigned)d.W, u.planes(d), u.rows(d), u.cols(d), grp.plane_elems);
+        const WinItem it = win_item(grp, rt, lds, min(i, u.planes(d) * grp.per_plane - 1));
+        g.load(rsrc, rt, it, (unsigned)d.W, u.rows(d), u.cols(d), grp.plane_elems);
     };
     win_walk<T, WM, TILE>(
         x, lds, words, d, rt, grp.pls, c, u0, u1, [&](const WinUnit<TILE> &u) { fetch(u, wave); },
