@@ -241,6 +241,8 @@ def test_window_kernels_unit_edges(oracle, N, C, H, W, K, dtype):
     (2, 64, 17, 3, 31, 1), (2, 128, 70, 19, 13, 1), (1, 64, 40, 130, 7, 1), (2, 64, 21, 66, 27, 1),
     (2, 64, 56, 56, 31, 2), (1, 64, 65, 131, 31, 2), (3, 64, 33, 63, 15, 2), (2, 64, 5, 18, 7, 2),
     (9, 64, 66, 66, 13, 2), (40, 64, 34, 30, 15, 1),
+    # (fp32: thin planes that go to the tile kernels, and the next extents that do not)
+    (64, 64, 3, 70, 7, 1), (64, 64, 5, 70, 7, 2), (64, 64, 4, 65, 7, 1), (64, 64, 3, 64, 7, 1), (63, 64, 3, 70, 7, 1),
     # (wgrad: enough planes for the grouped kernel)
     (2, 1024, 28, 28, 31, 1), (2, 1024, 33, 65, 31, 1), (2, 1024, 17, 3, 13, 1), (2, 1024, 21, 18, 27, 1),
     (2, 1024, 33, 67, 31, 2), (2, 1024, 5, 18, 7, 2), (2, 1024, 35, 31, 15, 2)])
