@@ -99,10 +99,10 @@ class _PointwiseLinear(torch.autograd.Function):
 
 def _eager(*tensors):
     """True for ordinary tensors in ordinary execution: no compilation, tracing, torch.func transform,
-    forward-mode derivative or tensor subclass, all of which an autograd function around native code would
-    hide the layer from."""
+    dispatch mode, forward-mode derivative or tensor subclass, all of which an autograd function around native
+    code would hide the layer from."""
     if (torch.compiler.is_compiling() or torch.jit.is_tracing()
-            or torch._C._are_functorch_transforms_active()):
+            or torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack()):
         return False
     return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter)
                              and fwd.unpack_dual(t).tangent is None) for t in tensors)

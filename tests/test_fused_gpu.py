@@ -267,10 +267,10 @@ class _Sub(torch.Tensor):
     pass
 
 
-@pytest.mark.parametrize("use", ["forward_mode", "func_grad", "vmap", "trace", "compile", "subclass"])
+@pytest.mark.parametrize("use", ["forward_mode", "func_grad", "vmap", "trace", "compile", "subclass", "fx"])
 def test_pointwise_linear_inside_transforms(use):
     """What nn.Linear takes part in and an autograd function with a native backward cannot: forward-mode
-    derivatives, torch.func transforms, tracing, compilation and tensor subclasses."""
+    derivatives, torch.func transforms, tracing (of the backward pass too), compilation and tensor subclasses."""
     from oriented1d_amd.convnext1d import PointwiseLinear
 
     torch.manual_seed(3)
@@ -296,6 +296,11 @@ def test_pointwise_linear_inside_transforms(use):
             return [traced(t).detach()]
         if use == "compile":
             return [torch.compile(layer, backend="eager", fullgraph=True)(x).detach()]
+        if use == "fx":
+            from torch.fx.experimental.proxy_tensor import make_fx
+            dy = torch.randn(4, 5, 6, 64, device="cuda", generator=torch.Generator("cuda").manual_seed(4))
+            graph = make_fx(lambda a: torch.autograd.grad(layer(a), (layer.weight, layer.bias), dy))(x)
+            return list(graph(t))
         y = layer(x.as_subclass(_Sub))
         assert type(y) is _Sub and type(y.grad_fn).__name__ != "_PointwiseLinearBackward"
         return [y.detach().as_subclass(torch.Tensor)]
