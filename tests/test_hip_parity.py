@@ -266,12 +266,15 @@ def test_grouped_claim_that_does_not_hold(oracle, stride, dtype):
     assert layouts == {2: 1, 4: 1}
     _case(oracle, 2, C, 20, 23, 15, stride, dtype, 3, theta, seed=5)
     taps = op.build_taps(torch.from_numpy(grouped_theta(C)), C, 15).cuda()
+    P = 24 // stride
     buf = torch.randn(1 + 2 * 24 * 24 * C, device="cuda").to(dtype)
     x, w = buf[1:].view(2, 24, 24, C), torch.randn(C, 1, 1, 15, device="cuda")
-    dy = torch.randn(2, 24 // stride, 24 // stride, C, device="cuda").to(dtype)
-    assert x.data_ptr() % 16 != 0
+    dy = buf[1:1 + 2 * P * P * C].view(2, P, P, C)
+    assert x.data_ptr() % 16 != 0 and dy.data_ptr() % 16 != 0
     for a, b in ((op.fprop(x, w, taps, stride, nhwc=3), op.fprop(x.clone(), w, taps, stride, nhwc=1)),
-                 (op.wgrad(dy, x, taps, 15, stride, nhwc=3)[0], op.wgrad(dy, x, taps, 15, stride, nhwc=1)[0])):
+                 (op.dgrad(dy, w, taps, (24, 24), stride, nhwc=3), op.dgrad(dy.clone(), w, taps, (24, 24), stride, nhwc=1)),
+                 (op.wgrad(dy.clone(), x, taps, 15, stride, nhwc=3)[0], op.wgrad(dy, x, taps, 15, stride, nhwc=1)[0]),
+                 (op.wgrad(dy, x.clone(), taps, 15, stride, nhwc=3)[0], op.wgrad(dy, x, taps, 15, stride, nhwc=1)[0])):
         assert_close(host(a), host(b), dtype, "misaligned")
 
 
