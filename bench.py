@@ -426,11 +426,11 @@ def main():
             torch.cuda.empty_cache()
 
     # ------------------------------------------------------------------ shapes without planes
-    # Per-kernel times of shapes outside the sweep, bf16, the networks' contiguous-group angles:
-    # on the tile kernels (any extent, stride and layout) the two stem convolutions of the networks
-    # at batch 128 (NHWC, stride 2) and the stage shapes of a 512 x 512 input at batch 8 (NCHW); on
-    # the NHWC plane kernels the second convolution of the ConvNeXt-B-1D++ blocks at batch 64
-    # (4 x dim channels: the launches of the training configuration).
+    # Per-kernel times of shapes outside the sweep, bf16, the networks' contiguous-group angles: the
+    # two stem convolutions of the networks at batch 128 (NHWC, stride 2) on the grouped kernels,
+    # the stage shapes of a 512 x 512 input at batch 8 (NCHW; 128 x 128 on the window kernels) and the
+    # second convolution of the ConvNeXt-B-1D++ blocks at batch 64 (NHWC, 4 x dim channels: the
+    # launches of the training configuration; 56 x 56 and 28 x 28 on the grouped kernels).
     other_shapes = {}
     if not args.no_extra_sweeps and not args.only:
         for tag, (N_, C_, HW_, st_, lay_) in (
@@ -448,12 +448,15 @@ def main():
             x = torch.randn(xs, device=dev, generator=g).to(torch.bfloat16)
             dy = torch.randn(ys, device=dev, generator=g).to(torch.bfloat16)
             w2 = (torch.randn(C_, KSIZE, device=dev, generator=g) * 0.02).contiguous()
-            taps = op.build_taps(torch.from_numpy(theta_for(C_, "grouped")), C_, KSIZE).to(dev)
+            blob = op.build_taps(torch.from_numpy(theta_for(C_, "grouped")), C_, KSIZE)
+            # (the layout code the module passes)
+            lay = (_lib.NHWC + (_lib.GROUPED if lib.dwo_taps_grouped(vp(blob), 8) else 0)) if nhwc else _lib.NCHW
+            taps = blob.to(dev)
             y, dx = torch.empty_like(dy), torch.empty_like(x)
             dw = torch.empty(C_, KSIZE, device=dev)
-            nb = lib.dwo_wgrad_scratch_bytes(N_, C_, HW_, HW_, KSIZE, st_, 1, int(nhwc))
+            nb = lib.dwo_wgrad_scratch_bytes(N_, C_, HW_, HW_, KSIZE, st_, 1, lay)
             scr = torch.empty(max(nb, 16), dtype=torch.uint8, device=dev)
-            dims = (N_, C_, HW_, HW_, KSIZE, st_, 1, int(nhwc), stream_h)
+            dims = (N_, C_, HW_, HW_, KSIZE, st_, 1, lay, stream_h)
             fns = {"fprop": (lambda a=(vp(x), vp(w2), None, vp(taps), vp(y)) + dims: lib.dwo_fprop(*a)),
                    "dgrad": (lambda a=(vp(dy), vp(w2), vp(taps), vp(dx)) + dims: lib.dwo_dgrad(*a)),
                    "wgrad": (lambda a=(vp(dy), vp(x), vp(taps), vp(dw), None, vp(scr), nb) + dims:

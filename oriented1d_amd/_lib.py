@@ -95,19 +95,6 @@ def ready(device):
     return lib
 
 
-def launch(device, fn, *args):
-    """Calls a launching entry point with ``device`` current: the library keeps its per-device
-    state (occupancy figures, counters, the static scratch) under the current device, which
-    must be the one the tensors and the stream live on."""
-    import torch
-
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    if index == torch.cuda.current_device():
-        return fn(*args)
-    with torch.cuda.device(index):
-        return fn(*args)
-
-
 def check(status, what):
     if status != 0:
         msg = load().dwo_status_string(status).decode()

@@ -12,12 +12,14 @@
 // looked up by half as many workgroups; the price is a weight per lane in vector registers
 // (two channels: 62), and two shifts or masks per read.
 //
-// What bounds these kernels is the multiply-adds with those unpacking instructions (64 x 512 x 56 x 56: about
-// 110 us of the chip's issue slots) and, phase after phase, the cache lines moved from L2 to L1 for a
-// 16-byte piece each.  Two workgroups per CU (80 KB of LDS, 128 registers) overlap those phases.
-// Measured (us, fprop / wgrad, K = 31, angles of the networks): 64 x 512 x 56 x 56 bf16 234 / 257 (slice
-// kernels 335 / 428), 64 x 1024 x 28 x 28 bf16 115 / 125 (129 / 190), 64 x 384 x 56 x 56 fp32 299 / 354 (326 / 551);
-// stride 2, 64 x 64 x 224 x 224 bf16 308 / 454 (tile kernels 568 / 809).
+// What bounds them, from counters (K = 31): at stride 1 in bf16 the issue slots of the multiply-adds and those
+// unpacking instructions (64 x 512 x 56 x 56 fprop 151 of 233 us; L2 lookups 42 %, LDS 25 %); at stride 2 lines that cross
+// the fabric again, as the eight groups of a line come to it at different times (64 x 64 x 224 x 224: fprop reads x
+// 2.4 times, wgrad x and dy 5.4 times, at 6 TB/s; dgrad writes dx twice).  Two workgroups per CU (80 KB of LDS,
+// 128 registers) overlap staging and evaluation.
+// Measured (us, fprop / wgrad, K = 31, angles of the networks): 64 x 512 x 56 x 56 bf16 233 / 264 (slice
+// kernels 335 / 428), 64 x 1024 x 28 x 28 bf16 114 / 121 (129 / 190), 64 x 384 x 56 x 56 fp32 298 / 355 (326 / 551);
+// stride 2, 64 x 64 x 224 x 224 bf16 310 / 451 (tile kernels 574 / 817).
 #pragma once
 
 #include "dwo_grouped_dispatch.h"
@@ -419,8 +421,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
 // projects the window's pixels to its group's channels while it stages them, rounded to T as the
 // layer's own output would be.  The image is read once per channel group (eight times at 64 channels of a
 // 16-bit type), and the C-channel tensor never exists.  Compiled for stride 2 and the three channels of an
-// image: the stem.  Whole ConvNeXt-T inference of 128 images in bf16: 6986 us with the tile kernel here
-// (986 of them), 6440 with this one (647).
+// image: the stem.  In ConvNeXt-T inference of 128 images in bf16 647 us, with the tile kernel 986.
 template <typename T>
 __device__ __forceinline__ float grp_value(__amdgpu_buffer_rsrc_t r, unsigned off) {
     if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
@@ -545,8 +546,8 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
 
 // ---------------------------------------------------------------------------------------------
 // dgrad at stride 2 (QuadPlan).  `d` describes dy as both the source and the plane of quads (H = P,
-// W = Q); dx is dxh x dxw.  64 x 64 x 224 x 224 bf16, K = 31: 249 us, bound by the writes in 16-byte
-// pieces (the residue classes one after the other from a sorted tap table, dwo_nhwc_tile.h: 542).
+// W = Q); dx is dxh x dxw.  64 x 64 x 224 x 224 bf16, K = 31: 247 us, bound by the writes in 16-byte
+// pieces, twice dx (the residue classes one after the other from a sorted tap table, dwo_nhwc_tile.h: 544).
 template <int O, typename T, int K>
 __device__ __forceinline__ void grp_dgrad2_body(grp_u4 *lds, float *lw, const T *dyn, T *dxn, const ConvDims &d,
                                                 const GrpTile &t, int c0, int dxh, int dxw) {

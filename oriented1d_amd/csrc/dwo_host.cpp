@@ -2,7 +2,7 @@
 // and the calls of libdwoconv1d_hip.so on the tensors' device and current stream.
 //
 // What bounds a call on small tensors is this path (the stage convolutions of ConvNeXt-T at batch
-// 64 take 240 us of GPU time in 12 kernels).  Kept in Python, with one ctypes call, one device query,
+// 64 take 216 us of GPU time in 12 kernels).  Kept in Python, with one ctypes call, one device query,
 // one stream object and up to four tensor constructions per kernel, forward and backward of one
 // layer took 90 to 170 us of host time, hence native code, without the GIL.  The autograd function
 // itself stays a Python one (its hooks, modes and refusals are PyTorch's own).
