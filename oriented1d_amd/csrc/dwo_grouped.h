@@ -421,7 +421,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
 // projects the window's pixels to its group's channels while it stages them, rounded to T as the
 // layer's own output would be.  The image is read once per channel group (eight times at 64 channels of a
 // 16-bit type), and the C-channel tensor never exists.  Compiled for stride 2 and the three channels of an
-// image: the stem.  In ConvNeXt-T inference of 128 images in bf16 647 us, with the tile kernel 986.
+// image: the stem.  In ConvNeXt-T inference of 128 images in bf16 489 us, with the tile kernel 986.
 template <typename T>
 __device__ __forceinline__ float grp_value(__amdgpu_buffer_rsrc_t r, unsigned off) {
     if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
