@@ -224,6 +224,48 @@ size_t dwo_pointwise_wgrad_scratch_bytes(int Cin, int C);
 int dwo_pointwise_wgrad(const void *dy, const void *x, float *dw, float *db, void *scratch, size_t scratch_bytes,
                         size_t rows, int Cin, int C, int dtype, void *stream);
 
+/*
+ * The passes around the operator and the pointwise layers of a block (models/convnext.py:306-318) and of the stem
+ * (:176-190) with their backward passes; no counterpart in the reference's extension.  LayerNorm is over C with the
+ * biased variance; gamma, beta and scale are fp32 [C]; C is a multiple of 8 up to 1024; tensors are dense and 16-byte
+ * aligned; in_dtype and out_dtype are equal or one of them is DWO_F32; stats receives (mean, 1 / deviation) per row, what the
+ * backward pass takes (forward only: may be null); dgamma, dbeta and dscale are written as grad_dtype and may be null;
+ * scratch holds at least dwo_block_scratch_bytes(C) bytes.
+ *
+ * dwo_ln_rows:     out[r,:] = act(LN(x[r,:])) for rows of C channels (act = exact GELU when gelu != 0);
+ *                  _backward also takes dout [rows,C] (out_dtype) and writes dx (in_dtype).
+ * dwo_ln_tile:     x [N,C,H,W] -> out [N,H,W,C] = LN over C; _backward: dout [N,H,W,C] -> dx [N,C,H,W].
+ * dwo_block_tail:  out [N,C,H,W] = res + scale[c] * y for y [N,H,W,C] of y_dtype, res and out of dtype;
+ *                  _backward: dout [N,C,H,W] (dtype) -> dy [N,H,W,C] (y_dtype), dscale.  (The gradient of res is dout.)
+ */
+size_t dwo_block_scratch_bytes(int C);
+int dwo_ln_rows(const void *x, const float *gamma, const float *beta, void *out, float *stats, size_t rows, int C,
+                float eps, int gelu, int in_dtype, int out_dtype, void *stream);
+int dwo_ln_rows_backward(const void *dout, const void *x, const float *stats, const float *gamma, const float *beta,
+                         void *dx, void *dgamma, void *dbeta, void *scratch, size_t scratch_bytes, size_t rows, int C,
+                         int gelu, int in_dtype, int out_dtype, int grad_dtype, void *stream);
+int dwo_ln_tile(const void *x, const float *gamma, const float *beta, void *out, float *stats, int N, int C, int H,
+                int W, float eps, int in_dtype, int out_dtype, void *stream);
+int dwo_ln_tile_backward(const void *dout, const void *x, const float *stats, const float *gamma, void *dx,
+                         void *dgamma, void *dbeta, void *scratch, size_t scratch_bytes, int N, int C, int H, int W,
+                         int in_dtype, int out_dtype, int grad_dtype, void *stream);
+int dwo_block_tail(const void *y, const float *scale, const void *res, void *out, int N, int C, int H, int W,
+                   int y_dtype, int dtype, void *stream);
+int dwo_block_tail_backward(const void *dout, const void *y, const float *scale, void *dy, void *dscale, void *scratch,
+                            size_t scratch_bytes, int N, int C, int H, int W, int y_dtype, int dtype, int grad_dtype,
+                            void *stream);
+
+/*
+ * Parameter gradients of a pointwise layer K -> N over 16-bit activations (the blocks' linear layers,
+ * models/convnext.py:296-298): dw[n,k] = sum_m dy[m,n] * x[m,k], db[n] = sum_m dy[m,n] (db may be null), for
+ * dy [rows,N] and x [rows,K] of type dtype (DWO_BF16 or DWO_F16), summed in fp32 and written as grad_dtype.  N and
+ * K are multiples of 8 up to 65536, rows at most 2^31; dy, x and scratch are 16-byte aligned and scratch holds at least
+ * dwo_linear_wgrad_scratch_bytes(rows, N, K) bytes (0: sizes that are not accepted).
+ */
+size_t dwo_linear_wgrad_scratch_bytes(size_t rows, int N, int K);
+int dwo_linear_wgrad(const void *dy, const void *x, void *dw, void *db, void *scratch, size_t scratch_bytes,
+                     size_t rows, int N, int K, int dtype, int grad_dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

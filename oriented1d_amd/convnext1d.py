@@ -77,8 +77,10 @@ class ChannelsFirstLayerNorm(nn.Module):
         if fused.usable(x, x.shape[1], tiled=True):
             y = fused.nchw_layernorm_nhwc(x, self.weight, self.bias, self.eps)
         else:
-            y = F.layer_norm(x.permute(0, 2, 3, 1), self.weight.shape, self.weight, self.bias,
-                             self.eps)
+            y = fused.tile_norm(x, self)
+            if y is None:
+                y = F.layer_norm(x.permute(0, 2, 3, 1), self.weight.shape, self.weight, self.bias,
+                                 self.eps)
         return y.permute(0, 3, 1, 2)
 
 
@@ -110,7 +112,7 @@ class Stem1D(nn.Module):
     def __init__(self, dim0, dim1, dim2, kernel_size, arbitrary_size=False, wrapped=False):
         super().__init__()
         self.pw1 = PointwiseLinear(dim0, dim1)
-        self.pw2 = nn.Linear(dim1, dim2)
+        self.pw2 = fused.Linear(dim1, dim2)
         pad = (kernel_size - 2) // 2  # shapes the parent Conv2d only; compute pads K // 2
         self.dw1 = oriented_conv(dim1, kernel_size, stride=2, padding=pad, nhwc=True,
                                  layer_offset=_odd_layer_offset(0), arbitrary_size=arbitrary_size,
@@ -138,11 +140,17 @@ class Stem1D(nn.Module):
             x = fused.layernorm_nhwc(self.pw2(x), self.norm3.weight, self.norm3.bias,
                                      self.norm3.eps)
             return fused.nhwc_scale_add_nchw(x)
-        x = self.pw1(x)
-        x = F.gelu(self.norm1(self.dw1(x)))
-        x = F.gelu(self.norm2(self.dw2(x)))
-        x = self.norm3(self.pw2(x))
-        return x.permute(0, 3, 1, 2).contiguous()
+        x = self._norm_gelu(self.dw1(self.pw1(x)), self.norm1)
+        x = self._norm_gelu(self.dw2(x), self.norm2, self.pw2)
+        x = self.pw2(x)
+        y = fused.row_norm(x, self.norm3)
+        y = self.norm3(x) if y is None else y
+        return y.permute(0, 3, 1, 2).contiguous()
+
+    @staticmethod
+    def _norm_gelu(x, norm, consumer=None):
+        y = fused.row_norm(x, norm, gelu=True, consumer=consumer)
+        return F.gelu(norm(x)) if y is None else y
 
 
 class Block(nn.Module):
@@ -153,8 +161,8 @@ class Block(nn.Module):
                  layer_offset=0.0, n_dir=8, arbitrary_size=False, wrapped=False):
         super().__init__()
         self.norm = nn.LayerNorm(dim, eps=1e-6)
-        self.pwconv1 = nn.Linear(dim, 4 * dim)
-        self.pwconv2 = nn.Linear(4 * dim, dim)
+        self.pwconv1 = fused.Linear(dim, 4 * dim)
+        self.pwconv2 = fused.Linear(4 * dim, dim)
         self.gamma = (nn.Parameter(layer_scale_init_value * torch.ones(dim))
                       if layer_scale_init_value > 0 else None)
         self.drop_path = StochasticDepth(drop_path) if drop_path > 0.0 else nn.Identity()
@@ -174,8 +182,9 @@ class Block(nn.Module):
         fuse = fused.usable(y, y.shape[1], tiled=True) and not self.training
         if fuse:  # permute + LayerNorm as one pass
             y = fused.nchw_layernorm_nhwc(y, self.norm.weight, self.norm.bias, self.norm.eps)
-        else:
-            y = self.norm(y.permute(0, 2, 3, 1).contiguous())
+        else:  # (recorded by autograd: one pass each way as well)
+            z = fused.tile_norm(y, self.norm, self.pwconv1) if fused.plain(self.norm, nn.LayerNorm) else None
+            y = self.norm(y.permute(0, 2, 3, 1).contiguous()) if z is None else z
         y = F.gelu(self.pwconv1(y))
         if self.plus_plus:
             y = self.dwconv2(y)
@@ -183,8 +192,18 @@ class Block(nn.Module):
         if fuse:  # layer scale + permute + residual as one pass (no stochastic depth in eval)
             return fused.nhwc_scale_add_nchw(y, self.gamma, x)
         if self.gamma is not None:
+            if self._keeps_all():
+                out = fused.block_tail(y, self.gamma, x)
+                if out is not None:
+                    return out
             y = self.gamma * y
         return x + self.drop_path(y.permute(0, 3, 1, 2).contiguous())
+
+    def _keeps_all(self):
+        """True where ``drop_path`` returns what it is given."""
+        d = self.drop_path
+        return fused.plain(d, nn.Identity) or (fused.plain(d, StochasticDepth)
+                                               and (not d.training or d.p == 0.0))
 
 
 class ConvNeXt1D(nn.Module):

@@ -35,6 +35,15 @@ struct Library {
     decltype(&::dwo_nhwc_scale_add_nchw) nhwc_scale_add_nchw;
     decltype(&::dwo_pointwise_wgrad_scratch_bytes) pointwise_wgrad_scratch_bytes;
     decltype(&::dwo_pointwise_wgrad) pointwise_wgrad;
+    decltype(&::dwo_block_scratch_bytes) block_scratch_bytes;
+    decltype(&::dwo_ln_rows) ln_rows;
+    decltype(&::dwo_ln_rows_backward) ln_rows_backward;
+    decltype(&::dwo_ln_tile) ln_tile;
+    decltype(&::dwo_ln_tile_backward) ln_tile_backward;
+    decltype(&::dwo_block_tail) block_tail;
+    decltype(&::dwo_block_tail_backward) block_tail_backward;
+    decltype(&::dwo_linear_wgrad_scratch_bytes) linear_wgrad_scratch_bytes;
+    decltype(&::dwo_linear_wgrad) linear_wgrad;
 } lib;
 
 [[noreturn]] void fail(const std::string &msg) { throw std::runtime_error(msg); }
@@ -57,6 +66,15 @@ void bind_library(const std::string &path) {
     find(lib.nhwc_scale_add_nchw, "dwo_nhwc_scale_add_nchw");
     find(lib.pointwise_wgrad_scratch_bytes, "dwo_pointwise_wgrad_scratch_bytes");
     find(lib.pointwise_wgrad, "dwo_pointwise_wgrad");
+    find(lib.block_scratch_bytes, "dwo_block_scratch_bytes");
+    find(lib.ln_rows, "dwo_ln_rows");
+    find(lib.ln_rows_backward, "dwo_ln_rows_backward");
+    find(lib.ln_tile, "dwo_ln_tile");
+    find(lib.ln_tile_backward, "dwo_ln_tile_backward");
+    find(lib.block_tail, "dwo_block_tail");
+    find(lib.block_tail_backward, "dwo_block_tail_backward");
+    find(lib.linear_wgrad_scratch_bytes, "dwo_linear_wgrad_scratch_bytes");
+    find(lib.linear_wgrad, "dwo_linear_wgrad");
 }
 
 void check(int status, const char *what) {
@@ -65,14 +83,16 @@ void check(int status, const char *what) {
              std::to_string(status) + ")");
 }
 
-int dtype_code(const Tensor &t) {
-    switch (t.scalar_type()) {
+int dtype_code(at::ScalarType t) {
+    switch (t) {
         case at::kFloat: return DWO_F32;
         case at::kBFloat16: return DWO_BF16;
         case at::kHalf: return DWO_F16;
         default: return -1;
     }
 }
+
+int dtype_code(const Tensor &t) { return dtype_code(t.scalar_type()); }
 
 // models/dwoconv1d/kernels/kernels.cu:11-13,17-18
 void check_activation(const Tensor &t, const char *name) {
@@ -275,6 +295,167 @@ std::tuple<Tensor, OptTensor> pointwise_wgrad(const Tensor &dy, const Tensor &x,
     return {dw, db};
 }
 
+// dense and 16-byte aligned, as the block's kernels read and write (a gradient may be a piece of another buffer)
+Tensor dense(const Tensor &t) {
+    Tensor d = t.contiguous();
+    if (reinterpret_cast<uintptr_t>(d.const_data_ptr()) % 16 != 0) d = d.clone();
+    return d;
+}
+void check_pair(const Tensor &a, const Tensor &b) {
+    if (a.device() != b.device()) fail("tensors on different devices");
+}
+Tensor bytes(const Tensor &like, size_t n) {
+    return at::empty({(int64_t)std::max<size_t>(n, 16)}, like.options().dtype(at::kByte));
+}
+
+// dy [.., N] and x [.., K] of one 16-bit type -> dw [N, K], db [N] of grad_dtype
+std::tuple<Tensor, OptTensor> linear_wgrad(const Tensor &dy_, const Tensor &x_, bool with_bias,
+                                           at::ScalarType grad_dtype) {
+    check_glue(dy_, "dy");
+    check_glue(x_, "x");
+    check_pair(dy_, x_);
+    if (dy_.scalar_type() != x_.scalar_type()) fail("dy and x must have the same dtype");
+    if (dy_.dim() < 1 || x_.dim() != dy_.dim() ||
+        x_.sizes().slice(0, x_.dim() - 1) != dy_.sizes().slice(0, dy_.dim() - 1))
+        fail("dy and x must have the same rows");
+    py::gil_scoped_release nogil;
+    const Place at(dy_);
+    const Tensor dy = dense(dy_), x = dense(x_);
+    const int64_t N = dy.size(-1), K = x.size(-1), rows = dy.numel() / std::max<int64_t>(N, 1);
+    const size_t nbytes = lib.linear_wgrad_scratch_bytes((size_t)rows, as_int(N), as_int(K));
+    const Tensor scratch = bytes(dy, nbytes);
+    const auto opt = dy.options().dtype(grad_dtype);
+    Tensor dw = at::empty({N, K}, opt);
+    OptTensor db;
+    if (with_bias) db = at::empty({N}, opt);
+    check(lib.linear_wgrad(ptr(dy), ptr(x), dw.data_ptr(), db.has_value() ? db->data_ptr() : nullptr,
+                           scratch.data_ptr(), nbytes, (size_t)rows, as_int(N), as_int(K), dtype_code(dy),
+                           dtype_code(grad_dtype), at.stream),
+          "dwo_linear_wgrad");
+    return {dw, db};
+}
+
+// LayerNorm (+ GELU) over the last dimension; (out, stats)
+std::tuple<Tensor, Tensor> ln_rows(const Tensor &x_, const Tensor &g, const Tensor &b, double eps, bool gelu,
+                                   at::ScalarType out_dtype) {
+    check_glue(x_, "x");
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const Tensor x = dense(x_);
+    const int64_t C = x.size(-1), rows = x.numel() / std::max<int64_t>(C, 1);
+    Tensor out = at::empty(x.sizes(), x.options().dtype(out_dtype));
+    Tensor stats = at::empty({rows, 2}, x.options().dtype(at::kFloat));
+    check(lib.ln_rows(ptr(x), (const float *)ptr(g), (const float *)ptr(b), out.data_ptr(), (float *)stats.data_ptr(),
+                      (size_t)rows, as_int(C), (float)eps, gelu, dtype_code(x), dtype_code(out_dtype), at.stream),
+          "dwo_ln_rows");
+    return {out, stats};
+}
+
+std::tuple<Tensor, Tensor, Tensor> ln_rows_backward(const Tensor &dout_, const Tensor &x_, const Tensor &stats,
+                                                    const Tensor &g, const Tensor &b, bool gelu,
+                                                    at::ScalarType grad_dtype) {
+    check_glue(dout_, "dout");
+    check_glue(x_, "x");
+    check_pair(dout_, x_);
+    if (dout_.sizes() != x_.sizes()) fail("dout and x must have the same shape");
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const Tensor x = dense(x_), dout = dense(dout_);
+    const int64_t C = x.size(-1), rows = x.numel() / std::max<int64_t>(C, 1);
+    const size_t nbytes = lib.block_scratch_bytes(as_int(C));
+    const Tensor scratch = bytes(x, nbytes);
+    Tensor dx = at::empty(x.sizes(), x.options());
+    Tensor dg = at::empty({C}, x.options().dtype(grad_dtype)), db = at::empty({C}, dg.options());
+    check(lib.ln_rows_backward(ptr(dout), ptr(x), (const float *)ptr(stats), (const float *)ptr(g),
+                               (const float *)ptr(b), dx.data_ptr(), dg.data_ptr(), db.data_ptr(), scratch.data_ptr(),
+                               nbytes, (size_t)rows, as_int(C), gelu, dtype_code(x), dtype_code(dout),
+                               dtype_code(grad_dtype), at.stream),
+          "dwo_ln_rows_backward");
+    return {dx, dg, db};
+}
+
+// [N,C,H,W] -> LayerNorm over C -> [N,H,W,C]; (out, stats)
+std::tuple<Tensor, Tensor> ln_tile(const Tensor &x_, const Tensor &g, const Tensor &b, double eps,
+                                   at::ScalarType out_dtype) {
+    check_glue(x_, "x");
+    if (x_.dim() != 4) throw py::value_error("x must be a 4-d tensor");
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const Tensor x = dense(x_);
+    const Dims d(x, false);
+    Tensor out = at::empty({d.n, d.h, d.w, d.c}, x.options().dtype(out_dtype));
+    Tensor stats = at::empty({d.n * d.h * d.w, 2}, x.options().dtype(at::kFloat));
+    check(lib.ln_tile(ptr(x), (const float *)ptr(g), (const float *)ptr(b), out.data_ptr(), (float *)stats.data_ptr(),
+                      as_int(d.n), as_int(d.c), as_int(d.h), as_int(d.w), (float)eps, dtype_code(x),
+                      dtype_code(out_dtype), at.stream),
+          "dwo_ln_tile");
+    return {out, stats};
+}
+
+std::tuple<Tensor, Tensor, Tensor> ln_tile_backward(const Tensor &dout_, const Tensor &x_, const Tensor &stats,
+                                                    const Tensor &g, at::ScalarType grad_dtype) {
+    check_glue(dout_, "dout");
+    check_glue(x_, "x");
+    check_pair(dout_, x_);
+    const Dims d(x_, false);
+    const std::array<int64_t, 4> want = {d.n, d.h, d.w, d.c};
+    if (dout_.sizes() != at::IntArrayRef(want)) fail("dout must be [N,H,W,C]");
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const Tensor x = dense(x_), dout = dense(dout_);
+    const size_t nbytes = lib.block_scratch_bytes(as_int(d.c));
+    const Tensor scratch = bytes(x, nbytes);
+    Tensor dx = at::empty(x.sizes(), x.options());
+    Tensor dg = at::empty({d.c}, x.options().dtype(grad_dtype)), db = at::empty({d.c}, dg.options());
+    check(lib.ln_tile_backward(ptr(dout), ptr(x), (const float *)ptr(stats), (const float *)ptr(g), dx.data_ptr(),
+                               dg.data_ptr(), db.data_ptr(), scratch.data_ptr(), nbytes, as_int(d.n), as_int(d.c),
+                               as_int(d.h), as_int(d.w), dtype_code(x), dtype_code(dout), dtype_code(grad_dtype),
+                               at.stream),
+          "dwo_ln_tile_backward");
+    return {dx, dg, db};
+}
+
+// res + scale * y: y [N,H,W,C], res [N,C,H,W]
+Tensor block_tail(const Tensor &y_, const Tensor &scale, const Tensor &res_) {
+    check_glue(y_, "y");
+    check_glue(res_, "res");
+    check_pair(y_, res_);
+    if (y_.dim() != 4) throw py::value_error("y must be a 4-d tensor");
+    const Dims d(y_, true);
+    const std::array<int64_t, 4> want = {d.n, d.c, d.h, d.w};
+    if (res_.sizes() != at::IntArrayRef(want)) fail("res must be [N,C,H,W]");
+    py::gil_scoped_release nogil;
+    const Place at(y_);
+    const Tensor y = dense(y_), res = dense(res_);
+    Tensor out = at::empty(res.sizes(), res.options());
+    check(lib.block_tail(ptr(y), (const float *)ptr(scale), ptr(res), out.data_ptr(), as_int(d.n), as_int(d.c),
+                         as_int(d.h), as_int(d.w), dtype_code(y), dtype_code(res), at.stream),
+          "dwo_block_tail");
+    return out;
+}
+
+std::tuple<Tensor, Tensor> block_tail_backward(const Tensor &dout_, const Tensor &y_, const Tensor &scale,
+                                               at::ScalarType grad_dtype) {
+    check_glue(dout_, "dout");
+    check_glue(y_, "y");
+    check_pair(dout_, y_);
+    const Dims d(y_, true);
+    const std::array<int64_t, 4> want = {d.n, d.c, d.h, d.w};
+    if (dout_.sizes() != at::IntArrayRef(want)) fail("dout must be [N,C,H,W]");
+    py::gil_scoped_release nogil;
+    const Place at(y_);
+    const Tensor y = dense(y_), dout = dense(dout_);
+    const size_t nbytes = lib.block_scratch_bytes(as_int(d.c));
+    const Tensor scratch = bytes(y, nbytes);
+    Tensor dy = at::empty(y.sizes(), y.options());
+    Tensor ds = at::empty({d.c}, y.options().dtype(grad_dtype));
+    check(lib.block_tail_backward(ptr(dout), ptr(y), (const float *)ptr(scale), dy.data_ptr(), ds.data_ptr(),
+                                  scratch.data_ptr(), nbytes, as_int(d.n), as_int(d.c), as_int(d.h), as_int(d.w),
+                                  dtype_code(y), dtype_code(dout), dtype_code(grad_dtype), at.stream),
+          "dwo_block_tail_backward");
+    return {dy, ds};
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -286,4 +467,11 @@ PYBIND11_MODULE(_host, m) {
     m.def("layernorm_nhwc", &layernorm_nhwc);
     m.def("nchw_layernorm_nhwc", &nchw_layernorm_nhwc);
     m.def("nhwc_scale_add_nchw", &nhwc_scale_add_nchw);
+    m.def("linear_wgrad", &linear_wgrad);
+    m.def("ln_rows", &ln_rows);
+    m.def("ln_rows_backward", &ln_rows_backward);
+    m.def("ln_tile", &ln_tile);
+    m.def("ln_tile_backward", &ln_tile_backward);
+    m.def("block_tail", &block_tail);
+    m.def("block_tail_backward", &block_tail_backward);
 }

@@ -1,18 +1,21 @@
-"""Forward-only glue of a ConvNeXt-1D block on the GPU, one pass each, in place of the PyTorch
-passes the reference spends around the operator (``models/convnext.py:306-318``: permute +
-LayerNorm before the pointwise layers, layer scale + permute + residual after them; the
-channels-last LayerNorm + GELU of the stem, ``:176-190``).  The harness uses them when no
-gradient is being recorded; with autograd on it composes the same values from PyTorch ops."""
+"""Glue of a ConvNeXt-1D block on the GPU, one pass each, in place of the PyTorch passes the
+reference spends around the operator (``models/convnext.py:306-318``: permute + LayerNorm before the
+pointwise layers, layer scale + permute + residual after them; the channels-last LayerNorm + GELU
+of the stem, ``:176-190``).  The first functions are forward only, for calls under ``no_grad``; the
+autograd functions below them are what a training pass runs, for ordinary tensors and modules (no
+transforms, tracing, subclasses or hooks: those compose the same values from PyTorch ops)."""
 import ctypes
 
 import torch
 import torch.autograd.forward_ad as fwd
 import torch.nn.functional as F
+import torch.nn.modules.module as _mod
 
 from . import _lib
 
 _DTYPES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 MAX_C_ROWS, MAX_C_TILE = 2048, 1536
+MAX_C_TRAIN = 1024
 
 
 def _ptr(t):
@@ -123,6 +126,220 @@ def pointwise_linear(x, linear):
             and w.shape[0] * dtype.itemsize % 16 == 0 and w.shape[0] * dtype.itemsize <= 4096):
         return _PointwiseLinear.apply(x, w, b)
     return F.linear(x, w, b)
+
+
+def plain(module, *types):
+    """True where calling the module is calling its class's own forward: no subclass, no hooks."""
+    return (type(module) in types and not (module._forward_hooks or module._forward_pre_hooks
+                                           or module._backward_hooks or module._backward_pre_hooks)
+            and not (_mod._global_forward_hooks or _mod._global_forward_pre_hooks
+                     or _mod._global_backward_hooks or _mod._global_backward_pre_hooks)
+            and "forward" not in module.__dict__)
+
+
+def _recording(*tensors):
+    """True where the training kernels may stand for a composition of PyTorch ops on these tensors (None for
+    an absent one): gradients are being recorded, on one GPU, for ordinary non-empty tensors of a known type."""
+    x = tensors[0]
+    return (torch.is_grad_enabled() and x.is_cuda and x.numel() > 0 and _eager(*tensors)
+            and all(t is None or (t.device == x.device and t.dtype in _DTYPES) for t in tensors))
+
+
+def _autocast(x):
+    """The type that autocast converts a pointwise layer's tensors to here, or None."""
+    return torch.get_autocast_dtype(x.device.type) if torch.is_autocast_enabled(x.device.type) else None
+
+
+def _norm_type(x, C, norm, consumer):
+    """Output type of LayerNorm over C channels of x: fp32 under autocast, or what autocast makes of it for ``consumer``
+    where nothing but that plain pointwise layer sees it; None where the kernels do not cover the call."""
+    w, b = norm.weight, norm.bias
+    if w is None or b is None or w.shape != (C,) or b.shape != (C,) or C % 8 != 0 or C > MAX_C_TRAIN:
+        return None
+    ac = _autocast(x)
+    if ac is None:
+        return x.dtype if x.dtype == w.dtype == b.dtype else None
+    out = ac if ac in _DTYPES and consumer is not None and plain(consumer, Linear) else torch.float32
+    return out if x.dtype == out or torch.float32 in (x.dtype, out) else None
+
+
+def _second_order(value, inputs, dout):
+    """Gradients of ``value(*inputs)`` with their own history (a backward pass that is being recorded)."""
+    needed = [t for t in inputs if t.requires_grad]
+    with torch.autocast(dout.device.type, enabled=False):
+        y = value(*inputs)
+        got = iter(torch.autograd.grad(y, needed, dout, create_graph=True, allow_unused=True))
+    return [next(got) if t.requires_grad else None for t in inputs]
+
+
+class _TileNorm(torch.autograd.Function):
+    """LayerNorm over dim 1 of an NCHW tensor, as [N,H,W,C]."""
+
+    @staticmethod
+    def forward(ctx, x, w, b, eps, dtype):
+        ctx.set_materialize_grads(False)
+        x = x.contiguous()
+        out, stats = _lib.host(x.get_device()).ln_tile(x, _f32(w), _f32(b), eps, dtype)
+        ctx.save_for_backward(x, w, b, stats)
+        ctx.eps, ctx.dtype = eps, dtype
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        if dout is None:
+            return None, None, None, None, None
+        x, w, b, stats = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            def value(x, w, b):
+                y = F.layer_norm(x.permute(0, 2, 3, 1).float(), w.shape, w.float(), b.float(), ctx.eps)
+                return y.to(ctx.dtype)
+            return (*_second_order(value, (x, w, b), dout), None, None)
+        dx, dw, db = _lib.host(x.get_device()).ln_tile_backward(dout, x, stats, _f32(w), w.dtype)
+        return dx, dw, db.to(b.dtype), None, None
+
+
+class _RowNorm(torch.autograd.Function):
+    """LayerNorm over the last dimension (+ exact GELU)."""
+
+    @staticmethod
+    def forward(ctx, x, w, b, eps, gelu, dtype):
+        ctx.set_materialize_grads(False)
+        x = x.contiguous()
+        out, stats = _lib.host(x.get_device()).ln_rows(x, _f32(w), _f32(b), eps, gelu, dtype)
+        ctx.save_for_backward(x, w, b, stats)
+        ctx.eps, ctx.gelu, ctx.dtype = eps, gelu, dtype
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        if dout is None:
+            return None, None, None, None, None, None
+        x, w, b, stats = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            def value(x, w, b):
+                y = F.layer_norm(x.float(), w.shape, w.float(), b.float(), ctx.eps)
+                return (F.gelu(y) if ctx.gelu else y).to(ctx.dtype)
+            return (*_second_order(value, (x, w, b), dout), None, None, None)
+        dx, dw, db = _lib.host(x.get_device()).ln_rows_backward(dout, x, stats, _f32(w), _f32(b), ctx.gelu, w.dtype)
+        return dx, dw, db.to(b.dtype), None, None, None
+
+
+class _BlockTail(torch.autograd.Function):
+    """``x + (gamma * y).permute(0, 3, 1, 2)`` for y [N,H,W,C] and x [N,C,H,W]."""
+
+    @staticmethod
+    def forward(ctx, y, gamma, x):
+        ctx.set_materialize_grads(False)
+        y = y.contiguous()
+        out = _lib.host(y.get_device()).block_tail(y, _f32(gamma), x)
+        ctx.save_for_backward(y, gamma)
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        if dout is None:
+            return None, None, None
+        y, gamma = ctx.saved_tensors
+        dx = dout if ctx.needs_input_grad[2] else None
+        if not (ctx.needs_input_grad[0] or ctx.needs_input_grad[1]):
+            return None, None, dx
+        if torch.is_grad_enabled():
+            def value(y, gamma):
+                return (gamma * y).permute(0, 3, 1, 2).to(dout.dtype)
+            return (*_second_order(value, (y, gamma), dout), dx)
+        dy, dg = _lib.host(y.get_device()).block_tail_backward(dout, y, _f32(gamma), gamma.dtype)
+        return dy, dg, dx
+
+
+class _Linear(torch.autograd.Function):
+    """``F.linear`` over 16-bit activations whose parameter gradients come from ``dwo_linear_wgrad``, in the parameters'
+    own type."""
+
+    @staticmethod
+    def forward(ctx, x, w, b):
+        ctx.set_materialize_grads(False)
+        # (conversions as autocast makes them, but not kept for the rest of its region: gradients are off here, and
+        # such copies would be cut off from the parameters)
+        wc, bc = w.to(x.dtype), b if b is None else b.to(x.dtype)
+        y = F.linear(x, wc, bc)
+        # (only what backward reads: the parameters themselves may be updated between the passes where the input
+        # takes no gradient, and always where they were converted)
+        need = ctx.needs_input_grad[0]
+        ctx.save_for_backward(x, wc if need else None)
+        ctx.weight = w if need and wc is not w else None
+        ctx.w_dtype, ctx.b_dtype = w.dtype, b.dtype if b is not None else None
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        if dy is None:
+            return None, None, None
+        x, wc = ctx.saved_tensors
+        dx = dw = db = None
+        need_db = ctx.b_dtype is not None and ctx.needs_input_grad[2]
+        if torch.is_grad_enabled():  # gradients of gradients: with the history of x and of the weights themselves
+            if ctx.needs_input_grad[0]:
+                dx = torch.matmul(dy, wc if ctx.weight is None else ctx.weight.to(dy.dtype))
+            rows = dy.reshape(-1, dy.shape[-1])
+            if ctx.needs_input_grad[1]:
+                dw = torch.matmul(rows.t(), x.reshape(-1, x.shape[-1])).to(ctx.w_dtype)
+            if need_db:
+                db = rows.sum(0).to(ctx.b_dtype)
+            return dx, dw, db
+        if ctx.needs_input_grad[0]:
+            dx = torch.matmul(dy, wc)
+        if ctx.needs_input_grad[1] or need_db:
+            dw, db = _lib.host(x.get_device()).linear_wgrad(dy, x, need_db, ctx.w_dtype)
+            if need_db and ctx.b_dtype != ctx.w_dtype:
+                db = db.to(ctx.b_dtype)
+        return dx, dw if ctx.needs_input_grad[1] else None, db
+
+
+class Linear(torch.nn.Linear):
+    """``nn.Linear``; where it is trained over 16-bit activations on a GPU, its parameter gradients are one pass
+    over them (``dwo_linear_wgrad``)."""
+
+    def forward(self, x):
+        w, b = self.weight, self.bias
+        if (w.requires_grad and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and max(w.shape) <= 65536
+                and x.dim() >= 1 and x.shape[-1] == w.shape[1] and _recording(x, w, b)
+                and x.numel() // w.shape[1] <= 1 << 31):
+            ac = _autocast(x)
+            dtype = ac or x.dtype
+            if dtype in (torch.bfloat16, torch.float16) and (
+                    ac is not None or (x.dtype == w.dtype and (b is None or b.dtype == w.dtype))):
+                return _Linear.apply(x.to(dtype), w, b)
+        return F.linear(x, w, b)
+
+
+def tile_norm(x, norm, consumer=None):
+    """LayerNorm (the parameters and eps of ``norm``) over dim 1 of an NCHW tensor as [N,H,W,C], recorded by autograd, in
+    the type that ``consumer`` (the pointwise layer that alone reads it) takes; None where the kernels do not cover the
+    call."""
+    if not (_recording(x, norm.weight, norm.bias) and x.dim() == 4 and x.numel() < 1 << 31):
+        return None
+    dtype = _norm_type(x, x.shape[1], norm, consumer)
+    return None if dtype is None else _TileNorm.apply(x, norm.weight, norm.bias, norm.eps, dtype)
+
+
+def row_norm(x, norm, gelu=False, consumer=None):
+    """``norm(x)`` of an ``nn.LayerNorm`` over the last dimension (then exact GELU), as ``tile_norm``."""
+    if not (_recording(x, norm.weight, norm.bias) and plain(norm, torch.nn.LayerNorm) and x.dim() >= 2
+            and x.numel() // max(x.shape[-1], 1) < 1 << 31):
+        return None
+    dtype = _norm_type(x, x.shape[-1], norm, consumer)
+    return None if dtype is None else _RowNorm.apply(x, norm.weight, norm.bias, norm.eps, gelu, dtype)
+
+
+def block_tail(y, gamma, x):
+    """``x + (gamma * y).permute(0, 3, 1, 2)`` recorded by autograd; None where the kernels do not cover the call."""
+    if not (_recording(y, gamma, x) and y.dim() == 4 and gamma.shape == y.shape[-1:] and y.shape[-1] % 8 == 0
+            and y.shape[-1] <= MAX_C_TRAIN and y.numel() < 1 << 31
+            and x.shape == (y.shape[0], y.shape[3], y.shape[1], y.shape[2])
+            and torch.promote_types(torch.promote_types(gamma.dtype, y.dtype), x.dtype) == x.dtype
+            and x.dtype in (y.dtype, torch.float32)):
+        return None
+    return _BlockTail.apply(y, gamma, x)
 
 
 def pointwise_dwconv_nhwc(x, linear, conv):

@@ -1,0 +1,205 @@
+"""The training passes of the block and the stem (LayerNorm in both layouts, GELU, layer scale + residual, the
+pointwise layers' parameter gradients) against the same compositions in fp64 PyTorch.
+
+Tolerances: tensors and sums of fp32 are good to 1e-5 as the operator's; what is rounded to a 16-bit type on the way out
+carries that type's rounding, 2^-9 (bf16) or 2^-12 (fp16) of the value at most, and 1e-2 is the operator's own bound for them.
+Parameter gradients are fp32 sums of exact products of the inputs: 1e-5 whatever the inputs' type, except where
+they are asked for in 16 bits."""
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from parity_util import TOL, rel_err
+
+from oriented1d_amd import fused
+
+pytestmark = pytest.mark.gpu
+F32, BF16, F16 = torch.float32, torch.bfloat16, torch.float16
+TYPES = [(F32, F32), (F32, BF16), (F32, F16), (BF16, BF16), (BF16, F32), (F16, F16), (F16, F32)]
+
+
+def close(got, ref, tol, what):
+    e = rel_err(got.detach().float().cpu().numpy(), ref.detach().double().cpu().numpy())
+    assert max(e) <= tol, (what, e)
+
+
+def run_norm(x, w, b, dout, native, reference, tol_out, tol_dx):
+    leaves = [t.detach().clone().requires_grad_(True) for t in (x, w, b)]
+    out = native(*leaves)
+    got = torch.autograd.grad(out, leaves, dout)
+    ref_leaves = [t.detach().double().requires_grad_(True) for t in (x, w, b)]
+    ref = reference(*ref_leaves)
+    want = torch.autograd.grad(ref, ref_leaves, dout.double())
+    close(out, ref, tol_out, "out")
+    close(got[0], want[0], tol_dx, "dx")
+    close(got[1], want[1], 1e-5, "dw")
+    close(got[2], want[2], 1e-5, "db")
+
+
+@pytest.mark.parametrize("types", TYPES, ids=str)
+@pytest.mark.parametrize("N,C,H,W", [(2, 96, 9, 8), (1, 8, 1, 1), (3, 64, 5, 13), (2, 72, 16, 16), (1, 128, 33, 2),
+                                     (2, 256, 7, 7), (2, 520, 3, 4), (1, 1024, 7, 7), (40, 96, 56, 56)])
+def test_tile_norm(N, C, H, W, types):
+    if N == 40 and types != (F32, BF16):
+        pytest.skip("one type at the size where workgroups take several tiles")
+    tin, tout = types
+    torch.manual_seed(C + H)
+    x = (torch.randn(N, C, H, W, device="cuda") * 2 + 0.5).to(tin)
+    w, b = torch.randn(C, device="cuda") * 0.5 + 1, torch.randn(C, device="cuda") * 0.1
+    dout = torch.randn(N, H, W, C, device="cuda").to(tout)
+    run_norm(x, w, b, dout, lambda x, w, b: fused._TileNorm.apply(x, w, b, 1e-6, tout),
+             lambda x, w, b: F.layer_norm(x.permute(0, 2, 3, 1), (C,), w, b, 1e-6), TOL[tout], TOL[tin])
+
+
+@pytest.mark.parametrize("types", TYPES, ids=str)
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("shape", [(2, 11, 5, 64), (1, 8), (37, 72), (9, 9, 128), (130, 256), (33, 520), (5, 1024),
+                                   (9000, 64)])
+def test_row_norm(shape, gelu, types):
+    tin, tout = types
+    C = shape[-1]
+    torch.manual_seed(C)
+    x = (torch.randn(*shape, device="cuda") * 2 - 0.25).to(tin)
+    w, b = torch.randn(C, device="cuda") * 0.5 + 1, torch.randn(C, device="cuda") * 0.1
+    dout = torch.randn(*shape, device="cuda").to(tout)
+
+    def reference(x, w, b):
+        y = F.layer_norm(x, (C,), w, b, 1e-6)
+        return F.gelu(y) if gelu else y
+    run_norm(x, w, b, dout, lambda x, w, b: fused._RowNorm.apply(x, w, b, 1e-6, gelu, tout), reference,
+             TOL[tout], TOL[tin])
+
+
+@pytest.mark.parametrize("ty,tr", [(F32, F32), (BF16, F32), (F16, F32), (BF16, BF16), (F16, F16)], ids=str)
+@pytest.mark.parametrize("N,C,H,W", [(2, 96, 9, 8), (1, 8, 1, 1), (3, 64, 5, 13), (2, 136, 16, 16), (2, 768, 7, 7),
+                                     (70, 64, 56, 56)])
+def test_block_tail(N, C, H, W, ty, tr):
+    torch.manual_seed(C + W)
+    y = torch.randn(N, H, W, C, device="cuda").to(ty).requires_grad_(True)
+    g = (torch.randn(C, device="cuda") * 0.5).requires_grad_(True)
+    x = torch.randn(N, C, H, W, device="cuda").to(tr).requires_grad_(True)
+    dout = torch.randn(N, C, H, W, device="cuda").to(tr)
+    out = fused._BlockTail.apply(y, g, x)
+    got = torch.autograd.grad(out, (y, g, x), dout)
+    leaves = [t.detach().double().requires_grad_(True) for t in (y, g, x)]
+    ref = leaves[2] + (leaves[1] * leaves[0]).permute(0, 3, 1, 2)
+    want = torch.autograd.grad(ref, leaves, dout.double())
+    close(out, ref, TOL[tr], "out")
+    close(got[0], want[0], TOL[ty], "dy")
+    close(got[1], want[1], 1e-5, "dgamma")
+    assert torch.equal(got[2], dout)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16], ids=str)
+@pytest.mark.parametrize("M,K,N", [(1, 8, 8), (63, 96, 384), (64, 128, 128), (65, 136, 120), (4096, 64, 72), (777, 768, 192),
+                                   (20000, 96, 136), (300, 1024, 264)])
+def test_linear_gradients(M, K, N, dtype):
+    torch.manual_seed(M + K)
+    m = fused.Linear(K, N).cuda()
+    x = torch.randn(M, K, device="cuda", requires_grad=True)
+    dy = torch.randn(M, N, device="cuda").to(dtype)
+    with torch.autocast("cuda", dtype=dtype):
+        y = m(x)
+    assert type(y.grad_fn).__name__ == "_LinearBackward" and y.dtype == dtype
+    dx, dw, db = torch.autograd.grad(y, (x, m.weight, m.bias), dy)
+    xq, wq = x.detach().to(dtype).double(), m.weight.detach().to(dtype).double()
+    close(dx, dy.double() @ wq, TOL[dtype], "dx")
+    assert dw.dtype == F32 and db.dtype == F32
+    close(dw, dy.double().t() @ xq, 1e-5, "dw")
+    close(db, dy.double().sum(0), 1e-5, "db")
+
+
+def test_linear_covers_batches_views_and_second_order():
+    torch.manual_seed(0)
+    m = fused.Linear(64, 128).cuda().bfloat16()
+    x = torch.randn(2, 3, 5, 64, device="cuda").to(BF16)
+    buf = torch.randn(2 * 3 * 5 * 128 + 1, device="cuda").to(BF16)
+    dy = buf[1:].view(2, 3, 5, 128)  # a gradient that is a misaligned piece of another buffer
+    y = m(x)
+    dw, db = torch.autograd.grad(y, (m.weight, m.bias), dy)
+    assert dw.dtype == BF16
+    close(dw, dy.double().reshape(-1, 128).t() @ x.double().reshape(-1, 64), TOL[BF16], "dw")
+    close(db, dy.double().sum((0, 1, 2)), TOL[BF16], "db")
+    m = fused.Linear(64, 64).cuda()
+    x = torch.randn(7, 64, device="cuda", requires_grad=True)
+    with torch.autocast("cuda", dtype=BF16):
+        y = m(x)
+    gx, gw = torch.autograd.grad(y.float().square().sum(), (x, m.weight), create_graph=True)
+    hx, hw = torch.autograd.grad(gx.square().sum() + gw.square().sum(), (x, m.weight))
+    p = nn.Linear(64, 64).cuda()
+    p.load_state_dict(m.state_dict())
+    z = p(x)
+    px, pw = torch.autograd.grad(z.square().sum(), (x, p.weight), create_graph=True)
+    rx, rw = torch.autograd.grad(px.square().sum() + pw.square().sum(), (x, p.weight))
+    close(hx, rx, 3e-2, "second order x")  # (a chain of four bf16 products)
+    close(hw, rw, 3e-2, "second order w")
+
+
+@pytest.mark.parametrize("which", ["tile", "rows", "tail"])
+def test_second_order_of_the_passes(which):
+    torch.manual_seed(1)
+    a = torch.randn(2, 16, 3, 5, device="cuda", dtype=F32, requires_grad=True)
+    w = torch.randn(16, device="cuda", requires_grad=True)
+    b = torch.randn(16, device="cuda", requires_grad=True)
+    nhwc = a.permute(0, 2, 3, 1).contiguous()
+    native, reference = {
+        "tile": (lambda: fused._TileNorm.apply(a, w, b, 1e-6, F32),
+                 lambda: F.layer_norm(a.permute(0, 2, 3, 1), (16,), w, b, 1e-6)),
+        "rows": (lambda: fused._RowNorm.apply(nhwc, w, b, 1e-6, True, F32),
+                 lambda: F.gelu(F.layer_norm(nhwc, (16,), w, b, 1e-6))),
+        "tail": (lambda: fused._BlockTail.apply(nhwc, w, a),
+                 lambda: a + (w * nhwc).permute(0, 3, 1, 2))}[which]
+    res = []
+    for f in (native, reference):
+        y = f()
+        g = torch.autograd.grad((y ** 3).sum(), (a, w), create_graph=True)
+        res.append(torch.autograd.grad(sum((t * t).sum() for t in g), (a, w)))
+    for got, ref in zip(*res):
+        close(got, ref.double(), 1e-4, which)  # (fp32 on both sides)
+
+
+def test_hooks_and_replaced_forwards_keep_the_module_path():
+    from oriented1d_amd.convnext1d import Block
+    torch.manual_seed(0)
+    blk = Block(32, (31,), False, layer_scale_init_value=0.5).cuda()
+    x = torch.randn(2, 32, 12, 12, device="cuda")
+    plain = blk(x)
+    assert type(plain.grad_fn).__name__ == "_BlockTailBackward"
+    seen = []
+    handle = blk.norm.register_forward_hook(lambda m, i, o: seen.append(tuple(i[0].shape)))
+    hooked = blk(x)
+    handle.remove()
+    assert seen == [(2, 12, 12, 32)]
+    close(hooked, plain.double(), 1e-5, "hooked")
+    blk.norm.forward = lambda t: torch.zeros_like(t)
+    zeroed = blk(x)
+    del blk.norm.forward
+    assert not torch.allclose(zeroed, plain)
+
+
+@pytest.mark.parametrize("variant", ["1d", "1dpp"])
+@pytest.mark.parametrize("mode", ["autocast", "bf16", "f32"])
+def test_network_gradients_against_the_composition(variant, mode, monkeypatch):
+    """A training pass on these kernels and on the PyTorch composition of the same network."""
+    from oriented1d_amd.convnext1d import ConvNeXt1D
+    torch.manual_seed(3)
+    net = ConvNeXt1D(depths=(1, 2, 1, 1), dims=(16, 32, 64, 128), variant=variant, num_classes=16,
+                     layer_scale_init_value=0.5, arbitrary_size=True).cuda()
+    net = net.to(BF16) if mode == "bf16" else net
+    img = torch.randn(3, 3, 72, 56, device="cuda").to(BF16 if mode == "bf16" else F32)
+    grads = []
+    for native in (True, False):
+        if not native:
+            monkeypatch.setattr(fused, "_recording", lambda *t: False)
+        net.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=BF16, enabled=mode == "autocast"):
+            y = net(img)
+        y.float().square().sum().backward()
+        grads.append([y.detach()] + [p.grad for p in net.parameters() if p.grad is not None])
+    assert len(grads[0]) == len(grads[1])
+    tol = 2e-5 if mode == "f32" else 4e-2  # (16-bit: two sets of roundings through the whole network)
+    for a, b in zip(*grads):
+        assert a.dtype == b.dtype and a.shape == b.shape
+        e = (a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-20)
+        assert e <= tol, (tuple(a.shape), float(e))
