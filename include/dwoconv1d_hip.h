@@ -266,6 +266,20 @@ size_t dwo_linear_wgrad_scratch_bytes(size_t rows, int N, int K);
 int dwo_linear_wgrad(const void *dy, const void *x, void *dw, void *db, void *scratch, size_t scratch_bytes,
                      size_t rows, int N, int K, int dtype, int grad_dtype, void *stream);
 
+/*
+ * A pointwise layer K -> N at inference with what follows it in a block (models/convnext.py:306-318), for 16-bit
+ * types (DWO_BF16, DWO_F16): y[m,n] = bias[n] + sum_k x[m,k] * w[n,k], summed in fp32; w [N,K] and bias [N] (may be
+ * null) have the activations' type.  N and K are multiples of 8 up to 65536, rows below 2^31; tensors are 16-byte aligned.
+ *
+ * dwo_linear_rows:   out [rows,N] = act(y), act = exact GELU when gelu != 0.
+ * dwo_linear_planes: x [images,HW,K] -> out [images,N,HW] = res + scale[n] * y; scale [N] and res (like out) may be
+ *                    null and have the activations' type.
+ */
+int dwo_linear_rows(const void *x, const void *w, const void *bias, void *out, size_t rows, int N, int K, int gelu,
+                    int dtype, void *stream);
+int dwo_linear_planes(const void *x, const void *w, const void *bias, const void *scale, const void *res, void *out,
+                      int images, int HW, int N, int K, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

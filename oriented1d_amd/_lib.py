@@ -42,6 +42,8 @@ SIGNATURES = {
     "dwo_block_tail": (_i, [_vp] * 4 + [_i] * 6 + [_vp]),
     "dwo_block_tail_backward": (_i, [_vp] * 6 + [_sz] + [_i] * 7 + [_vp]),
     "dwo_linear_wgrad_scratch_bytes": (_sz, [_sz, _i, _i]),
+    "dwo_linear_rows": (_i, [_vp] * 4 + [_sz] + [_i] * 4 + [_vp]),
+    "dwo_linear_planes": (_i, [_vp] * 6 + [_i] * 5 + [_vp]),
     "dwo_linear_wgrad": (_i, [_vp] * 5 + [_sz, _sz] + [_i] * 4 + [_vp]),
 }
 

@@ -185,12 +185,12 @@ class Block(nn.Module):
         else:  # (recorded by autograd: one pass each way as well)
             z = fused.tile_norm(y, self.norm, self.pwconv1) if fused.plain(self.norm, nn.LayerNorm) else None
             y = self.norm(y.permute(0, 2, 3, 1).contiguous()) if z is None else z
-        y = F.gelu(self.pwconv1(y))
+        y = fused.linear_gelu(y, self.pwconv1)
         if self.plus_plus:
             y = self.dwconv2(y)
+        if fuse:  # layer scale + permute + residual behind the layer (no stochastic depth in eval)
+            return fused.linear_tail(y, self.pwconv2, self.gamma, x)
         y = self.pwconv2(y)
-        if fuse:  # layer scale + permute + residual as one pass (no stochastic depth in eval)
-            return fused.nhwc_scale_add_nchw(y, self.gamma, x)
         if self.gamma is not None:
             if self._keeps_all():
                 out = fused.block_tail(y, self.gamma, x)

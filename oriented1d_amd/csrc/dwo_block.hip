@@ -42,7 +42,7 @@ int by_types(int in, int out, F &&f) {
 int esize(int dtype) { return dtype == DWO_F32 ? 4 : 2; }
 
 int column_sums(const float *part, void *out0, void *out1, int L, int split, int groups, int dtype, hipStream_t st) {
-    const dim3 grid((L + 31) / 32), block(kBlkThreads);
+    const dim3 grid((L + 31) / 32), block(kColThreads);
     switch (dtype) {
         case DWO_F32:
             column_sums_kernel<float><<<grid, block, 0, st>>>(part, (float *)out0, (float *)out1, L, split, groups);

@@ -44,6 +44,8 @@ struct Library {
     decltype(&::dwo_block_tail_backward) block_tail_backward;
     decltype(&::dwo_linear_wgrad_scratch_bytes) linear_wgrad_scratch_bytes;
     decltype(&::dwo_linear_wgrad) linear_wgrad;
+    decltype(&::dwo_linear_rows) linear_rows;
+    decltype(&::dwo_linear_planes) linear_planes;
 } lib;
 
 [[noreturn]] void fail(const std::string &msg) { throw std::runtime_error(msg); }
@@ -75,6 +77,8 @@ void bind_library(const std::string &path) {
     find(lib.block_tail_backward, "dwo_block_tail_backward");
     find(lib.linear_wgrad_scratch_bytes, "dwo_linear_wgrad_scratch_bytes");
     find(lib.linear_wgrad, "dwo_linear_wgrad");
+    find(lib.linear_rows, "dwo_linear_rows");
+    find(lib.linear_planes, "dwo_linear_planes");
 }
 
 void check(int status, const char *what) {
@@ -456,6 +460,56 @@ std::tuple<Tensor, Tensor> block_tail_backward(const Tensor &dout_, const Tensor
     return {dy, ds};
 }
 
+const void *optr(const OptTensor &t) { return t.has_value() ? t->const_data_ptr() : nullptr; }
+void check_layer(const Tensor &x, const Tensor &w, const OptTensor &b) {
+    check_glue(x, "x");
+    check_pair(x, w);
+    if (w.dim() != 2 || w.size(1) != x.size(-1) || w.scalar_type() != x.scalar_type())
+        fail("w must be [N, K] of the same type as x");
+    if (b.has_value() && (b->numel() != w.size(0) || b->scalar_type() != x.scalar_type() || !b->is_contiguous()))
+        fail("bias must be [N] of the same type as x");
+}
+
+// act(x w^T + b) over the last dimension
+Tensor linear_rows(const Tensor &x_, const Tensor &w_, const OptTensor &b, bool gelu) {
+    check_layer(x_, w_, b);
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const Tensor x = dense(x_), w = dense(w_);
+    const int64_t N = w.size(0), K = w.size(1);
+    auto shape = x.sizes().vec();
+    shape.back() = N;
+    Tensor out = at::empty(shape, x.options());
+    check(lib.linear_rows(ptr(x), ptr(w), optr(b), out.data_ptr(), (size_t)(x.numel() / std::max<int64_t>(K, 1)),
+                          as_int(N), as_int(K), gelu, dtype_code(x), at.stream),
+          "dwo_linear_rows");
+    return out;
+}
+
+// x [N,H,W,K] -> [N,C,H,W]: res + scale * (x w^T + b)
+Tensor linear_planes(const Tensor &x_, const Tensor &w_, const OptTensor &b, const OptTensor &scale,
+                     const OptTensor &res_) {
+    check_layer(x_, w_, b);
+    if (x_.dim() != 4) throw py::value_error("x must be a 4-d tensor");
+    const int64_t C = w_.size(0), K = w_.size(1);
+    if (scale.has_value() && (scale->numel() != C || scale->scalar_type() != x_.scalar_type() || !scale->is_contiguous()))
+        fail("scale must be [C] of the same type as x");
+    const Dims d(x_, true);
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const Tensor x = dense(x_), w = dense(w_);
+    Tensor out = at::empty({d.n, C, d.h, d.w}, x.options()), res;
+    if (res_.has_value()) {
+        if (res_->sizes() != out.sizes() || res_->scalar_type() != x.scalar_type())
+            fail("residual must be [N,C,H,W] of the same type as x");
+        res = dense(*res_);
+    }
+    check(lib.linear_planes(ptr(x), ptr(w), optr(b), optr(scale), res.defined() ? ptr(res) : nullptr, out.data_ptr(),
+                            as_int(d.n), as_int(d.h * d.w), as_int(C), as_int(K), dtype_code(x), at.stream),
+          "dwo_linear_planes");
+    return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -468,6 +522,8 @@ PYBIND11_MODULE(_host, m) {
     m.def("nchw_layernorm_nhwc", &nchw_layernorm_nhwc);
     m.def("nhwc_scale_add_nchw", &nhwc_scale_add_nchw);
     m.def("linear_wgrad", &linear_wgrad);
+    m.def("linear_rows", &linear_rows);
+    m.def("linear_planes", &linear_planes);
     m.def("ln_rows", &ln_rows);
     m.def("ln_rows_backward", &ln_rows_backward);
     m.def("ln_tile", &ln_tile);

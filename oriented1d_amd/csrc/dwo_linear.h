@@ -220,4 +220,370 @@ int launch_linear_reduce(const float *part, void *dw, void *db, int N, int K, in
     return e == hipSuccess ? 0 : (int)e;
 }
 
+// ------------------------------------------------------------------------------------------------- inference
+// y[m][n] = b[n] + sum_k x[m][k] * w[n][k] with what follows it in a block at inference (models/convnext.py:306-318):
+//   rows     exact GELU on the way out, [M][N]: the first layer
+//   planes   res + scale[n] * y as [image][N][HW]: the second layer, layer scale, permute and residual
+// so that neither the 4 C-channel tensor before GELU nor the product of the second layer goes through memory by itself.
+//
+// A product D = P * Q^T puts four neighbouring rows of P into a lane's registers: P is the operand whose index is the
+// fast one in the output (channels for rows, pixels for planes), and its rows are dealt to the fragments of a wave
+// so that a lane ends up with twice eight neighbours, and four lanes with 64 bytes of output per store (8-byte
+// stores left the L2 with four times as many writes: 401408 x 384 x 96 208 us, now 172).  Where planes are no multiple of four pixels
+// lanes run along the pixels instead (single values, 32 bytes per store).
+
+// GELU with erf from Abramowitz and Stegun, Handbook of Mathematical Functions, 7.1.26 (error of erf below 1.5e-7, next
+// to a rounding of 2^-9 or 2^-12 of the result on the way out): u > 0: u (1 - q), else -|u| q, q = erfc(|u| / sqrt 2) / 2.
+// erff takes twice the issue slots of the matrix products of a stage-1 block.
+__device__ __forceinline__ float lin_gelu(float u) {
+    const float z = __builtin_fabsf(u);
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(z, 0.3275911f * 0.70710678118654752f, 1.f));
+    float p = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
+    p = __builtin_fmaf(t, p, 0.5f * 1.421413741f);
+    p = __builtin_fmaf(t, p, 0.5f * -0.284496736f);
+    p = __builtin_fmaf(t, p, 0.5f * 0.254829592f);
+    p *= t;
+    const float e = __builtin_amdgcn_exp2f(u * u * -0.72134752044448170f);  // exp(-u^2 / 2)
+    return __builtin_fmaf(-p, z * e, __builtin_fmaxf(u, 0.f));
+}
+
+template <typename T>
+struct LinearArgs {
+    const T *x, *w, *bias, *scale, *res;
+    T *out;
+    long M;
+    int N, K, HW, gelu;
+};
+
+typedef unsigned mma_u2 __attribute__((ext_vector_type(2)));
+template <typename T>
+__device__ __forceinline__ unsigned lin_pack(float a, float b) {
+    return (unsigned)__builtin_bit_cast(uint16_t, from_float<T>(a)) |
+           (unsigned)__builtin_bit_cast(uint16_t, from_float<T>(b)) << 16;
+}
+template <typename T>
+__device__ __forceinline__ float lin_value(unsigned v, int e) {
+    return to_float(__builtin_bit_cast(T, (uint16_t)(v >> (16 * e))));
+}
+
+// Q neighbouring channels n .. n + Q - 1 of row m (Q 4 or 8, n a multiple of it; N is a multiple of eight)
+template <int Q, typename T>
+__device__ __forceinline__ void lin_emit_rows(const LinearArgs<T> &a, long m, int n, float (&v)[Q], const float (&b)[Q]) {
+    if (m >= a.M || n >= a.N) return;
+#pragma unroll
+    for (int r = 0; r < Q; r++) {
+        v[r] += b[r];
+        if (a.gelu) v[r] = lin_gelu(v[r]);
+    }
+    T *at = a.out + m * a.N + n;
+    if constexpr (Q == 8)
+        *reinterpret_cast<mma_u4 *>(at) = mma_u4{lin_pack<T>(v[0], v[1]), lin_pack<T>(v[2], v[3]),
+                                                 lin_pack<T>(v[4], v[5]), lin_pack<T>(v[6], v[7])};
+    else *reinterpret_cast<mma_u2 *>(at) = mma_u2{lin_pack<T>(v[0], v[1]), lin_pack<T>(v[2], v[3])};
+}
+template <int Q, typename T>
+__device__ __forceinline__ void lin_bias(const LinearArgs<T> &a, int n, float (&b)[Q]) {
+#pragma unroll
+    for (int r = 0; r < Q; r++) b[r] = a.bias != nullptr && n < a.N ? to_float(a.bias[n + r]) : 0.f;
+}
+// bias and scale of channel n
+template <typename T>
+__device__ __forceinline__ void lin_affine(const LinearArgs<T> &a, int n, float &b, float &s) {
+    b = a.bias != nullptr && n < a.N ? to_float(a.bias[n]) : 0.f;
+    s = a.scale != nullptr && n < a.N ? to_float(a.scale[n]) : 1.f;
+}
+// place of pixel m in channel 0 of its image
+template <typename T>
+__device__ __forceinline__ size_t lin_pixel(const LinearArgs<T> &a, long m) {
+    const long img = (unsigned)m / (unsigned)a.HW;
+    return (size_t)img * a.N * a.HW + (m - img * a.HW);
+}
+template <typename T>
+__device__ __forceinline__ void lin_emit_pixel(const LinearArgs<T> &a, size_t at, float v, float b, float s) {
+    a.out[at] = from_float<T>(__builtin_fmaf(v + b, s, a.res != nullptr ? to_float(a.res[at]) : 0.f));
+}
+// four neighbouring pixels m .. m + 3 of channel n (m a multiple of four)
+template <typename T>
+__device__ __forceinline__ void lin_emit_pixels4(const LinearArgs<T> &a, long m, int n, mma_f4 v, float b, float s) {
+    if (m >= a.M || n >= a.N) return;
+    if (a.HW % 4 == 0) {  // the four lie in one image, M is a multiple of four
+        const size_t at = lin_pixel(a, m) + (size_t)n * a.HW;
+        mma_u2 r = mma_u2{0u, 0u};
+        if (a.res != nullptr) r = *reinterpret_cast<const mma_u2 *>(a.res + at);
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = __builtin_fmaf(v[e] + b, s, a.res != nullptr ? lin_value<T>(r[e / 2], e % 2) : 0.f);
+        *reinterpret_cast<mma_u2 *>(a.out + at) = mma_u2{lin_pack<T>(o[0], o[1]), lin_pack<T>(o[2], o[3])};
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (m + e < a.M) lin_emit_pixel(a, lin_pixel(a, m + e) + (size_t)n * a.HW, v[e], b, s);
+}
+// eight neighbouring pixels m .. m + 7 of channel n (m a multiple of eight)
+template <typename T>
+__device__ __forceinline__ void lin_emit_pixels8(const LinearArgs<T> &a, long m, int n, mma_f4 v, mma_f4 w, float b, float s) {
+    if (a.HW % 8 != 0) {
+        lin_emit_pixels4(a, m, n, v, b, s);
+        lin_emit_pixels4(a, m + 4, n, w, b, s);
+        return;
+    }
+    if (m >= a.M || n >= a.N) return;
+    const size_t at = lin_pixel(a, m) + (size_t)n * a.HW;
+    mma_u4 r = mma_u4{0u, 0u, 0u, 0u};
+    if (a.res != nullptr) r = *reinterpret_cast<const mma_u4 *>(a.res + at);
+    float o[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        o[e] = __builtin_fmaf((e < 4 ? v[e] : w[e - 4]) + b, s, a.res != nullptr ? lin_value<T>(r[e / 2], e % 2) : 0.f);
+    *reinterpret_cast<mma_u4 *>(a.out + at) = mma_u4{lin_pack<T>(o[0], o[1]), lin_pack<T>(o[2], o[3]),
+                                                     lin_pack<T>(o[4], o[5]), lin_pack<T>(o[6], o[7])};
+}
+
+// Tiles of 64 columns lie in LDS as rows of 128 bytes whose 16-byte pieces are permuted by the row, so that eight lanes of
+// a fragment read meet on all banks.
+constexpr int kLinK = 64;
+
+// R rows x BK columns of a row-major operand from memory straight to LDS, zeros beyond its last row or column: a lane
+// brings sixteen bytes per load, a wave 1 KB (the permutation is in the addresses it reads).
+// DEAL: slot 32 h + 16 i + 4 g + r holds row 32 h + 8 g + 4 i + r.
+template <int R, int BK, bool DEAL>
+struct LinAsync {
+    static constexpr int PIECES = BK / 8, U = R * PIECES / kLinThreads;  // pieces per row, loads
+    unsigned off[U];
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ void init(const void *p, long rows, long r0, int K) {
+        r = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(p) + r0 * K * 2), 0,
+                                              (unsigned)min(max(rows - r0, 0L) * K * 2, 0x7fffffffL), 0x00020000);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int f = (int)threadIdx.x + u * kLinThreads, s = f / PIECES;
+            const int row = DEAL ? (s & ~31) + (s >> 2 & 3) * 8 + (s >> 4 & 1) * 4 + (s & 3) : s;
+            off[u] = (unsigned)row * (unsigned)K * 2 + piece() * 16;
+        }
+    }
+    // (the piece a lane reads is the same one in all its rows: they are a multiple of PIECES apart)
+    static __device__ __forceinline__ int piece() {
+        return (threadIdx.x % PIECES) ^ (threadIdx.x / PIECES % PIECES);
+    }
+    __device__ __forceinline__ void load(uint16_t *lds, int k0, int K) const {
+        typedef __attribute__((address_space(3))) void lds_void;
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        // beyond the last column a lane reads nowhere, which writes zeros
+        const unsigned kill = piece() * 8 < K - k0 ? 0u : kLinNowhere;
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(lds + (wave + 4 * u) * 512), 16, off[u] | kill,
+                                                     k0 * 2, 0, 0);
+#endif
+    }
+};
+// 16 rows x 32 columns for a product, columns 32 kk .. of the tile
+template <int BK>
+__device__ __forceinline__ mma_s8 lin_fragment(const uint16_t *lds, int slot0, int kk) {
+    const int lane = threadIdx.x & 63, s = slot0 + (lane & 15);
+    return *reinterpret_cast<const mma_s8 *>(lds + s * BK + ((kk * 4 + (lane >> 4)) ^ (s & (BK / 8 - 1))) * 8);
+}
+
+// Outputs of a wave's fragments: P rows p0 + 32 h + 8 g + 4 i + r of fragments (2 h + i, j) against Q row q0 + 16 j + c.
+enum { LIN_ROWS, LIN_PLANES, LIN_PIXELS };  // rows, planes, planes with lanes along the pixels (P rows not dealt)
+template <int OUT, typename T, int H, int QF>
+__device__ __forceinline__ void lin_emit(const LinearArgs<T> &a, long p0, long q0, const mma_f4 (&acc)[2 * H][QF]) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    if constexpr (OUT == LIN_PLANES) {
+#pragma unroll
+        for (int j = 0; j < QF; j++) {
+            const int n = (int)q0 + 16 * j + c;
+            float b, s;
+            lin_affine(a, n, b, s);
+#pragma unroll
+            for (int h = 0; h < H; h++) lin_emit_pixels8(a, p0 + 32 * h + 8 * g, n, acc[2 * h][j], acc[2 * h + 1][j], b, s);
+        }
+    } else if constexpr (OUT == LIN_PIXELS) {
+        size_t at[QF];
+#pragma unroll
+        for (int j = 0; j < QF; j++) at[j] = lin_pixel(a, q0 + 16 * j + c);
+#pragma unroll
+        for (int i = 0; i < 2 * H; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int n = (int)p0 + 16 * i + 4 * g + r;
+                float b, s;
+                lin_affine(a, n, b, s);
+#pragma unroll
+                for (int j = 0; j < QF; j++)
+                    if (n < a.N && q0 + 16 * j + c < a.M) lin_emit_pixel(a, at[j] + (size_t)n * a.HW, acc[i][j][r], b, s);
+            }
+    } else {
+#pragma unroll
+        for (int h = 0; h < H; h++) {
+            const int n = (int)p0 + 32 * h + 8 * g;
+            float b[8];
+            lin_bias(a, n, b);
+#pragma unroll
+            for (int j = 0; j < QF; j++) {
+                float v[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] = acc[2 * h + e / 4][j][e % 4];
+                lin_emit_rows(a, q0 + 16 * j + c, n, v, b);
+            }
+        }
+    }
+}
+
+// Large tiles: 128 rows of P, 32 * QF of Q, four waves of 64 x 16 QF products, two buffers: the next 64 columns travel
+// to LDS while these are multiplied, one barrier per step, two workgroups per CU.  bf16, us: 25088 x 1536 x 384 with GELU 60 (MFMA
+// 12, the GELU's vector instructions 30; library product and GELU kernel 92), 401408 x 384 x 96 172 (290); planes
+// 25088 x 384 x 1536 58 (library and scale kernel 57), 401408 x 96 x 384 109 (193).  Tried: staging through registers
+// (the same; -20 % where few workgroups run), three buffers with one workgroup per CU (+30 %).
+template <typename T, int QF>
+__device__ __forceinline__ void lin_products(const uint16_t *lp, const uint16_t *lq, int wp, int wq, mma_f4 (&acc)[4][QF]) {
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++) {
+        mma_s8 fp[4], fq[QF];
+#pragma unroll
+        for (int i = 0; i < 4; i++) fp[i] = lin_fragment<kLinK>(lp, wp + 16 * i, kk);
+#pragma unroll
+        for (int j = 0; j < QF; j++) fq[j] = lin_fragment<kLinK>(lq, wq + 16 * j, kk);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < QF; j++) acc[i][j] = Mma<T>::run(fp[i], fq[j], acc[i][j]);
+    }
+    // the second half's fragments are read between the products of the first
+    __builtin_amdgcn_sched_group_barrier(0x100, 4 + QF, 0);
+#pragma unroll
+    for (int i = 0; i < 4 + QF; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 8 * QF - 2 * (4 + QF), 0);
+}
+template <typename T, int OUT, int QF>
+__global__ __launch_bounds__(kLinThreads, 2) void linear_kernel(LinearArgs<T> a, int mtiles, int ntiles) {
+    constexpr bool PLANES = OUT == LIN_PLANES;  // P is x
+    constexpr int RP = 128, RQ = 32 * QF;
+    __shared__ __attribute__((aligned(16))) uint16_t lp0[RP * kLinK];
+    __shared__ __attribute__((aligned(16))) uint16_t lq0[RQ * kLinK];
+    __shared__ __attribute__((aligned(16))) uint16_t lp1[RP * kLinK];
+    __shared__ __attribute__((aligned(16))) uint16_t lq1[RQ * kLinK];
+    const int k = blockIdx.x / 8, mt = k / ntiles * 8 + blockIdx.x % 8, nt = k % ntiles;
+    if (mt >= mtiles) return;
+    const long m0 = (long)mt * (PLANES ? RP : RQ);
+    const int n0 = nt * (PLANES ? RQ : RP);
+    LinAsync<RP, kLinK, OUT != LIN_PIXELS> tp;
+    LinAsync<RQ, kLinK, false> tq;
+    if (PLANES) tp.init(a.x, a.M, m0, a.K), tq.init(a.w, a.N, n0, a.K);
+    else tp.init(a.w, a.N, n0, a.K), tq.init(a.x, a.M, m0, a.K);
+    const int wave = threadIdx.x >> 6, wp = wave / 2 * 64, wq = wave % 2 * 16 * QF;
+    mma_f4 acc[4][QF];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < QF; j++) acc[i][j] = mma_f4{0.f, 0.f, 0.f, 0.f};
+    tp.load(lp0, 0, a.K), tq.load(lq0, 0, a.K);
+    for (int k0 = 0; k0 < a.K; k0 += 2 * kLinK) {
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's pieces are there ..
+        __syncthreads();                     // .. and the other waves'; nobody reads the other buffer any more
+        if (k0 + kLinK < a.K) tp.load(lp1, k0 + kLinK, a.K), tq.load(lq1, k0 + kLinK, a.K);
+        lin_products<T, QF>(lp0, lq0, wp, wq, acc);
+        if (k0 + kLinK >= a.K) break;
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        __syncthreads();
+        if (k0 + 2 * kLinK < a.K) tp.load(lp0, k0 + 2 * kLinK, a.K), tq.load(lq0, k0 + 2 * kLinK, a.K);
+        lin_products<T, QF>(lp1, lq1, wp, wq, acc);
+    }
+    lin_emit<OUT, T, 2, QF>(a, (PLANES ? m0 : n0) + wp, (PLANES ? n0 : m0) + wq, acc);
+}
+
+// Fewer tiles than CUs: 64 x 64, and the four waves share the columns, a quarter of every 128 each (a chain half as long per
+// column, four times as many workgroups); their sums meet in LDS.  us, large tiles / these: 784 x 1536 x 384 9.7 / 6.8,
+// 196 x 768 x 3072 49 / 15.6, 3136 x 384 x 96 7.6 / 6.2; 3136 x 1536 x 384 (300 large tiles) 13.3 / 17.2.
+template <typename T, int OUT>
+__global__ __launch_bounds__(kLinThreads, 2) void linear_split_kernel(LinearArgs<T> a, int mtiles) {
+    constexpr bool PLANES = OUT == LIN_PLANES;
+    constexpr int BK = 128, R = 64;
+    __shared__ __attribute__((aligned(16))) uint16_t lp0[R * BK];
+    __shared__ __attribute__((aligned(16))) uint16_t lq0[R * BK];
+    __shared__ __attribute__((aligned(16))) uint16_t lp1[R * BK];
+    __shared__ __attribute__((aligned(16))) uint16_t lq1[R * BK];
+    const long m0 = (long)(blockIdx.x % mtiles) * R;
+    const int n0 = blockIdx.x / mtiles * R;
+    LinAsync<R, BK, OUT != LIN_PIXELS> tp;
+    LinAsync<R, BK, false> tq;
+    if (PLANES) tp.init(a.x, a.M, m0, a.K), tq.init(a.w, a.N, n0, a.K);
+    else tp.init(a.w, a.N, n0, a.K), tq.init(a.x, a.M, m0, a.K);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    mma_f4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i / 4][i % 4] = mma_f4{0.f, 0.f, 0.f, 0.f};
+    auto products = [&](const uint16_t *lp, const uint16_t *lq) {
+        mma_s8 fp[4], fq[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) fp[i] = lin_fragment<BK>(lp, 16 * i, wave), fq[i] = lin_fragment<BK>(lq, 16 * i, wave);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = Mma<T>::run(fp[i], fq[j], acc[i][j]);
+    };
+    tp.load(lp0, 0, a.K), tq.load(lq0, 0, a.K);
+    for (int k0 = 0; k0 < a.K; k0 += 2 * BK) {
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        __syncthreads();
+        if (k0 + BK < a.K) tp.load(lp1, k0 + BK, a.K), tq.load(lq1, k0 + BK, a.K);
+        products(lp0, lq0);
+        if (k0 + BK >= a.K) break;
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        __syncthreads();
+        if (k0 + 2 * BK < a.K) tp.load(lp0, k0 + 2 * BK, a.K), tq.load(lq0, k0 + 2 * BK, a.K);
+        products(lp1, lq1);
+    }
+    // four arrays of 16 KB: fragments (i, ..) of all waves in array i; wave 2 h + x ends up with fragments (2 h + .., 2 x + ..)
+    __syncthreads();
+    auto give = [&](uint16_t *to, int i) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) reinterpret_cast<mma_f4 *>(to)[(j * 4 + wave) * 64 + lane] = acc[i][j];
+    };
+    give(lp0, 0), give(lq0, 1), give(lp1, 2), give(lq1, 3);
+    __syncthreads();
+    const int h = wave / 2, x = wave % 2;
+    mma_f4 sum[2][2];
+    auto take = [&](const uint16_t *from, int i) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const mma_f4 *r = reinterpret_cast<const mma_f4 *>(from) + (2 * x + j) * 256 + lane;
+            sum[i][j] = (r[0] + r[64]) + (r[128] + r[192]);
+        }
+    };
+    if (h == 0) take(lp0, 0), take(lq0, 1);
+    else take(lp1, 0), take(lq1, 1);
+    lin_emit<OUT, T, 1, 2>(a, (PLANES ? m0 : n0) + 32 * h, (PLANES ? n0 : m0) + 32 * x, sum);
+}
+
+constexpr long kLinLargeTiles = 160;
+template <typename T, bool PLANES>
+int launch_linear(const LinearArgs<T> &a, hipStream_t st) {
+    // channels per large tile: 96 where that leaves no partial tile and 128 does (planes only)
+    const bool three = PLANES && a.HW % 4 == 0 && a.N % 128 != 0 && a.N % 96 == 0;
+    const int nt = three ? 96 : 128;
+    const long mtiles = (a.M + 127) / 128;
+    const int ntiles = (a.N + nt - 1) / nt;
+    if (mtiles * ntiles >= kLinLargeTiles) {  // (both kernels take the same time at 150 to 170 tiles)
+        const dim3 grid((unsigned)((mtiles + 7) / 8 * 8 * ntiles)), block(kLinThreads);
+        if constexpr (!PLANES) linear_kernel<T, LIN_ROWS, 4><<<grid, block, 0, st>>>(a, (int)mtiles, ntiles);
+        else if (a.HW % 4 != 0) linear_kernel<T, LIN_PIXELS, 4><<<grid, block, 0, st>>>(a, (int)mtiles, ntiles);
+        else if (three) linear_kernel<T, LIN_PLANES, 3><<<grid, block, 0, st>>>(a, (int)mtiles, ntiles);
+        else linear_kernel<T, LIN_PLANES, 4><<<grid, block, 0, st>>>(a, (int)mtiles, ntiles);
+    } else {
+        const int mt = (int)((a.M + 63) / 64);
+        const dim3 grid((unsigned)((long)mt * ((a.N + 63) / 64))), block(kLinThreads);
+        if constexpr (!PLANES) linear_split_kernel<T, LIN_ROWS><<<grid, block, 0, st>>>(a, mt);
+        else if (a.HW % 4 != 0) linear_split_kernel<T, LIN_PIXELS><<<grid, block, 0, st>>>(a, mt);
+        else linear_split_kernel<T, LIN_PLANES><<<grid, block, 0, st>>>(a, mt);
+    }
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : (int)e;
+}
+
 }  // namespace dwo

@@ -36,4 +36,49 @@ int dwo_linear_wgrad(const void *dy, const void *x, void *dw, void *db, void *sc
     }
 }
 
+// y = x w^T + b over 16-bit activations; x, w and out 16-byte aligned, N and K multiples of eight, offsets inside 31 bits
+static bool linear_ok(size_t rows, int N, int K, const void *x, const void *w, const void *out) {
+    return rows >= 1 && rows < (size_t)1 << 31 && N >= 8 && K >= 8 && N % 8 == 0 && K % 8 == 0 && N <= 65536 &&
+           K <= 65536 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0;
+}
+
+int dwo_linear_rows(const void *x, const void *w, const void *bias, void *out, size_t rows, int N, int K, int gelu,
+                    int dtype, void *stream) {
+    if (!x || !w || !out) return DWO_ERR_NULL_POINTER;
+    if (!linear_ok(rows, N, K, x, w, out)) return DWO_ERR_BAD_SHAPE;
+    (void)hipGetLastError();
+    hipStream_t st = (hipStream_t)stream;
+    switch (dtype) {
+        case DWO_BF16:
+            return launch_linear<bf16_t, false>({(const bf16_t *)x, (const bf16_t *)w, (const bf16_t *)bias, nullptr,
+                                                 nullptr, (bf16_t *)out, (long)rows, N, K, 1, gelu}, st);
+        case DWO_F16:
+            return launch_linear<f16_t, false>({(const f16_t *)x, (const f16_t *)w, (const f16_t *)bias, nullptr,
+                                                nullptr, (f16_t *)out, (long)rows, N, K, 1, gelu}, st);
+        default: return DWO_ERR_BAD_DTYPE;
+    }
+}
+
+int dwo_linear_planes(const void *x, const void *w, const void *bias, const void *scale, const void *res, void *out,
+                      int images, int HW, int N, int K, int dtype, void *stream) {
+    if (!x || !w || !out) return DWO_ERR_NULL_POINTER;
+    if (images < 1 || HW < 1 || (double)images * HW >= 2147483648.0 ||
+        !linear_ok((size_t)images * HW, N, K, x, w, out) || (uintptr_t)res % 16 != 0)
+        return DWO_ERR_BAD_SHAPE;
+    (void)hipGetLastError();
+    hipStream_t st = (hipStream_t)stream;
+    const long M = (long)images * HW;
+    switch (dtype) {
+        case DWO_BF16:
+            return launch_linear<bf16_t, true>({(const bf16_t *)x, (const bf16_t *)w, (const bf16_t *)bias,
+                                                (const bf16_t *)scale, (const bf16_t *)res, (bf16_t *)out, M, N, K, HW,
+                                                0}, st);
+        case DWO_F16:
+            return launch_linear<f16_t, true>({(const f16_t *)x, (const f16_t *)w, (const f16_t *)bias,
+                                               (const f16_t *)scale, (const f16_t *)res, (f16_t *)out, M, N, K, HW, 0},
+                                              st);
+        default: return DWO_ERR_BAD_DTYPE;
+    }
+}
+
 }  // extern "C"

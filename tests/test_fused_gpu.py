@@ -307,3 +307,38 @@ def test_pointwise_linear_inside_transforms(use):
 
     for a, b in zip(results(lin), results(plain)):
         _close(a, b, torch.float32, use)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape,N", [((1, 1, 1, 8), 8), ((1, 3, 5, 72), 96), ((2, 8, 8, 64), 64), ((1, 13, 5, 136), 328),
+                                     ((2, 33, 32, 96), 384), ((3, 7, 7, 1536), 200), ((40, 20, 28, 96), 128),
+                                     ((64, 14, 14, 200), 264), ((128, 7, 7, 384), 768)])
+def test_linear_rows_and_planes(shape, N, dtype):
+    """Both tile sizes of the product kernels, rows and columns that fill no tile, planes of 8 k, 4 k and odd pixels;
+    the GELU against the exact one."""
+    torch.manual_seed(N)
+    B, H, W, K = shape
+    x = torch.randn(*shape, device="cuda").to(dtype)
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).to(dtype)
+    b, s = torch.randn(N, device="cuda").to(dtype), torch.randn(N, device="cuda").to(dtype)
+    res = torch.randn(B, N, H, W, device="cuda").to(dtype)
+    host = fused._lib.host(0)
+    y = F.linear(x.double(), w.double(), b.double())
+    _close(host.linear_rows(x, w, b, True), F.gelu(y), dtype, "rows, gelu")
+    _close(host.linear_rows(x, w, None, False), y - b.double(), dtype, "rows")
+    _close(host.linear_planes(x, w, b, s, res), res.double() + (s.double() * y).permute(0, 3, 1, 2), dtype, "planes")
+    _close(host.linear_planes(x, w, b, None, None), y.permute(0, 3, 1, 2), dtype, "planes alone")
+
+
+def test_product_kernels_keep_refusals():
+    host = fused._lib.host(0)
+    x = torch.zeros(1, 2, 2, 16, device="cuda", dtype=torch.bfloat16)
+    w = torch.zeros(8, 16, device="cuda", dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError):
+        host.linear_rows(x, w.half(), None, True)
+    with pytest.raises(RuntimeError):
+        host.linear_rows(x, w[:, :8], None, True)
+    with pytest.raises(RuntimeError):
+        host.linear_rows(x.float(), w.float(), None, True)
+    with pytest.raises(RuntimeError):
+        host.linear_planes(x, w, None, None, torch.zeros(1, 8, 2, 3, device="cuda", dtype=torch.bfloat16))
