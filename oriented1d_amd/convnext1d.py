@@ -145,7 +145,7 @@ class Stem1D(nn.Module):
         x = self.pw2(x)
         y = fused.row_norm(x, self.norm3)
         y = self.norm3(x) if y is None else y
-        return y.permute(0, 3, 1, 2).contiguous()
+        return fused.planes(y)
 
     @staticmethod
     def _norm_gelu(x, norm, consumer=None):
@@ -259,10 +259,19 @@ class ConvNeXt1D(nn.Module):
             if m.bias is not None:
                 nn.init.zeros_(m.bias)
 
+    def _downsample(self, i, x):
+        layer = self.downsample_layers[i]
+        if (i > 0 and fused.plain(layer, nn.Sequential) and len(layer) == 2
+                and fused.plain(layer[0], ChannelsFirstLayerNorm)):
+            y = fused.downsample(x, layer[0], layer[1])
+            if y is not None:
+                return y
+        return layer(x)
+
     def forward(self, x):
         outs = []
         for i in range(4):
-            x = self.stages[i](self.downsample_layers[i](x))
+            x = self.stages[i](self._downsample(i, x))
             if self.out_stages:
                 outs.append(getattr(self, "norm%d" % i)(x))
         if self.out_stages:

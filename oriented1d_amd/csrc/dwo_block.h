@@ -3,6 +3,7 @@
 //
 //   ln_tile     y [N,C,HW] -> LayerNorm over C -> [N,HW,C]        permute + LayerNorm of a block
 //   ln_rows     rows of C  -> LayerNorm -> (GELU)                 the stem's
+//   ln_patch    y [N,C,H,W] -> LayerNorm over C -> 2 x 2 patches  in front of a downsampling layer
 //   tail        res + scale[c] * y, y [N,HW,C] -> [N,C,HW]        layer scale + permute + residual
 //
 // All of them are bound by memory: PyTorch's compositions move each tensor three to six times (permuted
@@ -129,7 +130,7 @@ __device__ __forceinline__ void write_param_partials(float (&dg)[NV][8], float (
 }
 
 // part [groups][L] -> out0 [split], out1 [L - split], fixed order.  Few columns and up to a thousand groups: latency binds,
-// so 32 threads share a column, each with four loads in flight (eight threads one load at a time: 23 us, now XX).
+// so 32 threads share a column, each with four loads in flight (eight threads one load at a time: 23 us for 1024 groups of 1024 columns, now 8).
 constexpr int kColThreads = 1024;
 template <typename TO>
 __global__ __launch_bounds__(kColThreads) void column_sums_kernel(const float *__restrict__ part, TO *out0, TO *out1,
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(kBlkThreads) void ln_rows_kernel(const TI *__restri
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     o[i] = __builtin_fmaf(v[k][i] * rstd, gm[k][i], bt[k][i]);
-                    if (gelu) o[i] = blk_gelu(o[i]);
+                    if (gelu) o[i] = sizeof(TO) == 2 ? gelu_rounded(o[i]) : blk_gelu(o[i]);
                 }
                 store8(out + r * C + ln.chan(k), o);
             }
@@ -261,31 +262,34 @@ __global__ __launch_bounds__(kBlkThreads) void ln_rows_backward_kernel(
 // ------------------------------------------------------------------------------------------------- tiles
 // P pixels x C channels of an image in LDS as [C][P + 1] values of the tensor's type: four workgroups per CU, but 16
 // pixels (whole 64-byte pieces of fp32 rows) while they fit the 64 KB that need no attribute
-inline int blk_tile_pixels(int C, int esize) {
+// Fewer pixels where the tiles would not fill the chip (a single image: the chain of one tile is what counts).
+inline int blk_tile_pixels(int C, int esize, long pixels) {
     int p = 64;
     while (p > 16 && (long)C * (p + 1) * esize > 36 * 1024) p >>= 1;
+    while (p > 8 && pixels / p < 256) p >>= 1;
     return (long)C * (p + 1) * esize > 64 * 1024 ? 8 : p;
 }
 inline size_t blk_tile_bytes(int C, int P, int esize) { return ((size_t)C * (P + 1) * esize + 15) / 16 * 16; }
 
 struct BlkTiles {
-    int C, HW, P, per, tiles;  // tiles per image, in all
+    int C, HW, P, log2P, per, tiles;  // tiles per image, in all
+    int H, W, W2;                     // patches: image extents, patches per row
 };
 
 template <typename T, int VEC>
 __device__ __forceinline__ void tile_in(const T *xn, T *tile, const BlkTiles &t, int np) {
-    const int per_row = t.P / VEC, total = t.C * per_row;
-    constexpr int U = 4;  // loads in flight
+    const int sh = t.log2P - (VEC == 4 ? 2 : 0), total = t.C << sh;
+    constexpr int U = 8;  // loads in flight
     for (int f0 = threadIdx.x; f0 < total; f0 += U * kBlkThreads) {
         float v[U][VEC];
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int f = f0 + u * kBlkThreads, c = f / per_row, p = f % per_row * VEC;  // (P is a power of two)
+            const int f = f0 + u * kBlkThreads, c = f >> sh, p = (f - (c << sh)) * VEC;
             if (f < total && p < np) load_run<T, VEC>(xn + (size_t)c * t.HW + p, v[u]);
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
-            const int f = f0 + u * kBlkThreads, c = f / per_row, p = f % per_row * VEC;
+            const int f = f0 + u * kBlkThreads, c = f >> sh, p = (f - (c << sh)) * VEC;
             if (f < total && p < np)
 #pragma unroll
                 for (int e = 0; e < VEC; e++) tile[c * (t.P + 1) + p + e] = from_float<T>(v[u][e]);
@@ -294,9 +298,9 @@ __device__ __forceinline__ void tile_in(const T *xn, T *tile, const BlkTiles &t,
 }
 template <typename T, int VEC>
 __device__ __forceinline__ void tile_out(T *xn, const T *tile, const BlkTiles &t, int np) {
-    const int per_row = t.P / VEC, total = t.C * per_row;
+    const int sh = t.log2P - (VEC == 4 ? 2 : 0), total = t.C << sh;
     for (int f = threadIdx.x; f < total; f += kBlkThreads) {
-        const int c = f / per_row, p = f % per_row * VEC;
+        const int c = f >> sh, p = (f - (c << sh)) * VEC;
         if (p >= np) continue;
         float v[VEC];
 #pragma unroll
@@ -417,6 +421,180 @@ __global__ __launch_bounds__(kBlkThreads) void ln_tile_backward_kernel(
     write_param_partials<LPR, NV>(dg, db, t.C, lds_block, part);
 }
 
+// ------------------------------------------------------------------------------------------------- patches
+// x [N,C,H,W] -> LayerNorm over C -> patches [N,H/2,W/2][C][2][2], the operand of the downsampling 2 x 2 convolution of stride
+// 2 as a product with its weights as they lie (models/convnext.py:548-553).  A tile is a run of
+// P / 4 patches of one row; a lane holds eight channels of the four pixels of a patch, 32 neighbouring values of the output.
+struct PatchTile {
+    int n, h, p0, np;  // image, row of patches, first patch, patches
+    __device__ __forceinline__ PatchTile(const BlkTiles &t, int u) {
+        const int P = t.P / 4, h2 = t.H / 2, row = u / t.per;
+        n = row / h2, h = row - n * h2;
+        p0 = u % t.per * P, np = min(P, t.W2 - p0);
+    }
+};
+template <typename T, int VEC, bool IN>
+__device__ __forceinline__ void patch_move(T *x, T *tile, const BlkTiles &t, const PatchTile &at) {
+    const int sh = t.log2P - (VEC == 4 ? 2 : 0), half = t.P / 2 / VEC, total = t.C << sh;
+    T *xn = x + (size_t)at.n * t.C * t.HW + (size_t)2 * at.h * t.W + 2 * at.p0;
+    constexpr int U = IN ? 8 : 1;
+    for (int f0 = threadIdx.x; f0 < total; f0 += U * kBlkThreads) {
+        float v[U][VEC];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int f = f0 + u * kBlkThreads, c = f >> sh, k = f - (c << sh), r = k >= half, q = (k - r * half) * VEC;
+            if (f >= total || q >= 2 * at.np) continue;
+            T *m = xn + (size_t)c * t.HW + r * t.W + q;
+            const T *l = tile + c * (t.P + 1) + r * (t.P / 2) + q;
+            if constexpr (IN) load_run<T, VEC>(m, v[u]);
+            else {
+#pragma unroll
+                for (int e = 0; e < VEC; e++) v[u][e] = to_float(l[e]);
+                store_run<T, VEC>(m, v[u]);
+            }
+        }
+        if constexpr (IN) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int f = f0 + u * kBlkThreads, c = f >> sh, k = f - (c << sh), r = k >= half, q = (k - r * half) * VEC;
+                if (f >= total || q >= 2 * at.np) continue;
+#pragma unroll
+                for (int e = 0; e < VEC; e++) tile[c * (t.P + 1) + r * (t.P / 2) + q + e] = from_float<T>(v[u][e]);
+            }
+        }
+    }
+}
+
+template <typename TI, typename TO, int LPR, int NV, int VEC>
+__global__ __launch_bounds__(kBlkThreads) void ln_patch_kernel(const TI *__restrict__ x, const float *__restrict__ gamma,
+                                                               const float *__restrict__ beta, TO *__restrict__ out,
+                                                               float2 *__restrict__ stats, BlkTiles t, float eps) {
+    extern __shared__ float lds_block[];
+    TI *tile = reinterpret_cast<TI *>(lds_block);
+    const Lanes<LPR, NV> ln;
+    const PatchTile at(t, blockIdx.x);
+    patch_move<TI, VEC, true>(const_cast<TI *>(x), tile, t, at);
+    float gm[NV][8], bt[NV][8];
+#pragma unroll
+    for (int k = 0; k < NV; k++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int c = ln.chan(k) + i;
+            gm[k][i] = c < t.C ? gamma[c] : 0.f, bt[k][i] = c < t.C ? beta[c] : 0.f;
+        }
+    __syncthreads();
+    const size_t first = ((size_t)at.n * (t.H / 2) + at.h) * t.W2 + at.p0;
+    for (int q0 = 0; q0 < at.np; q0 += ln.ROWS) {
+        const int p = q0 + ln.slot;
+        const bool row = p < at.np;
+        float v[NV][8][4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const TI *px = tile + q / 2 * (t.P / 2) + 2 * p + q % 2;
+            float s = 0.f;
+#pragma unroll
+            for (int k = 0; k < NV; k++)
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    v[k][i][q] = row && ln.chan(k) < t.C ? to_float(px[(ln.chan(k) + i) * (t.P + 1)]) : 0.f;
+                    s += v[k][i][q];
+                }
+            const float mean = group_total<LPR>(s) / (float)t.C;
+            float d = 0.f;
+#pragma unroll
+            for (int k = 0; k < NV; k++)
+                if (ln.chan(k) < t.C)
+#pragma unroll
+                    for (int i = 0; i < 8; i++) v[k][i][q] -= mean, d = __builtin_fmaf(v[k][i][q], v[k][i][q], d);
+            const float rstd = rsqrtf(group_total<LPR>(d) / (float)t.C + eps);
+#pragma unroll
+            for (int k = 0; k < NV; k++)
+#pragma unroll
+                for (int i = 0; i < 8; i++) v[k][i][q] = __builtin_fmaf(v[k][i][q] * rstd, gm[k][i], bt[k][i]);
+            if (stats != nullptr && row && ln.l == 0) stats[(first + p) * 4 + q] = make_float2(mean, rstd);
+        }
+        if (!row) continue;
+#pragma unroll
+        for (int k = 0; k < NV; k++)
+            if (ln.chan(k) < t.C)
+#pragma unroll
+                for (int i = 0; i < 8; i += 2) {
+                    float o[8];
+#pragma unroll
+                    for (int e = 0; e < 8; e++) o[e] = v[k][i + e / 4][e % 4];
+                    store8(out + ((first + p) * t.C + ln.chan(k) + i) * 4, o);
+                }
+    }
+}
+
+template <typename TI, typename TO, int LPR, int NV, int VEC>
+__global__ __launch_bounds__(kBlkThreads) void ln_patch_backward_kernel(
+    const TO *__restrict__ dout, const TI *__restrict__ x, const float2 *__restrict__ stats,
+    const float *__restrict__ gamma, TI *__restrict__ dx, float *__restrict__ part, BlkTiles t) {
+    extern __shared__ float lds_block[];
+    TI *tile = reinterpret_cast<TI *>(lds_block);
+    const Lanes<LPR, NV> ln;
+    float gm[NV][8], dg[NV][8], db[NV][8];
+#pragma unroll
+    for (int k = 0; k < NV; k++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int c = ln.chan(k) + i;
+            gm[k][i] = c < t.C ? gamma[c] : 0.f;
+            dg[k][i] = db[k][i] = 0.f;
+        }
+    for (int u = blockIdx.x; u < t.tiles; u += gridDim.x) {
+        const PatchTile at(t, u);
+        __syncthreads();
+        patch_move<TI, VEC, true>(const_cast<TI *>(x), tile, t, at);
+        __syncthreads();
+        const size_t first = ((size_t)at.n * (t.H / 2) + at.h) * t.W2 + at.p0;
+        for (int q0 = 0; q0 < at.np; q0 += ln.ROWS) {
+            const int p = q0 + ln.slot;
+            const bool row = p < at.np;
+            float g[NV][8][4];
+#pragma unroll
+            for (int k = 0; k < NV; k++)
+#pragma unroll
+                for (int i = 0; i < 8; i += 2) {
+                    float o[8];
+                    if (row && ln.chan(k) < t.C) load8(dout + ((first + p) * t.C + ln.chan(k) + i) * 4, o);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) g[k][i + e / 4][e % 4] = row && ln.chan(k) < t.C ? o[e] : 0.f;
+                }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                TI *px = tile + q / 2 * (t.P / 2) + 2 * p + q % 2;
+                const float2 st = row ? stats[(first + p) * 4 + q] : make_float2(0.f, 0.f);
+                float h[NV][8], s1 = 0.f, s2 = 0.f;
+#pragma unroll
+                for (int k = 0; k < NV; k++)
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const bool ok = row && ln.chan(k) < t.C;
+                        h[k][i] = ok ? (to_float(px[(ln.chan(k) + i) * (t.P + 1)]) - st.x) * st.y : 0.f;
+                        dg[k][i] = __builtin_fmaf(g[k][i][q], h[k][i], dg[k][i]);
+                        db[k][i] += g[k][i][q];
+                        g[k][i][q] *= gm[k][i];
+                        s1 += g[k][i][q];
+                        s2 = __builtin_fmaf(g[k][i][q], h[k][i], s2);
+                    }
+                s1 = group_total<LPR>(s1) / (float)t.C;
+                s2 = group_total<LPR>(s2) / (float)t.C;
+#pragma unroll
+                for (int k = 0; k < NV; k++)
+                    if (row && ln.chan(k) < t.C)
+#pragma unroll
+                        for (int i = 0; i < 8; i++)
+                            px[(ln.chan(k) + i) * (t.P + 1)] = from_float<TI>(st.y * (g[k][i][q] - s1 - h[k][i] * s2));
+            }
+        }
+        __syncthreads();
+        patch_move<TI, VEC, false>(dx, tile, t, at);
+    }
+    write_param_partials<LPR, NV>(dg, db, t.C, lds_block, part);
+}
+
 // ------------------------------------------------------------------------------------------------- tail
 // 64 pixels x 64 channels through LDS; thread = (piece of eight channels, pixel), piece threadIdx % 8
 constexpr int kTailP = 64, kTailC = 64, kTailPitch = kTailP + 1;
@@ -425,9 +603,10 @@ struct TailTiles {
     int C, HW, per, ctiles, units;  // pixel tiles per image, channel tiles, (image, pixel tile) pairs
 };
 
-template <typename TY, typename TR, int VEC>
+// (TS: the type of res; without res out is y in planes)
+template <typename TY, typename TS, typename TR, int VEC>
 __global__ __launch_bounds__(kBlkThreads) void tail_kernel(const TY *__restrict__ y, const float *__restrict__ scale,
-                                                           const TR *__restrict__ res, TR *__restrict__ out,
+                                                           const TS *__restrict__ res, TR *__restrict__ out,
                                                            TailTiles t) {
     __shared__ float tile[kTailC * kTailPitch];
     const int u = blockIdx.x / t.ctiles, c0 = blockIdx.x % t.ctiles * kTailC;
@@ -435,21 +614,29 @@ __global__ __launch_bounds__(kBlkThreads) void tail_kernel(const TY *__restrict_
     const size_t base = ((size_t)n * t.C + c0) * t.HW + p0;
     constexpr int PER = kTailP / VEC, R = kTailC * PER / kBlkThreads;  // residual runs per thread
     float rs[R][VEC];
-#pragma unroll
-    for (int k = 0; k < R; k++) {
-        const int f = threadIdx.x + k * kBlkThreads, c = f / PER, p = f % PER * VEC;
-        if (c < nc && p < np) load_run<TR, VEC>(res + base + (size_t)c * t.HW + p, rs[k]);
-    }
     const int c = threadIdx.x % 8 * 8;
+    float v[2][8];
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         const int p = threadIdx.x / 8 + 32 * k;
-        if (c < nc && p < np) {
-            float v[8];
-            load8(y + ((size_t)n * t.HW + p0 + p) * t.C + c0 + c, v);
+        if (c < nc && p < np) load8(y + ((size_t)n * t.HW + p0 + p) * t.C + c0 + c, v[k]);
+    }
 #pragma unroll
-            for (int i = 0; i < 8; i++) tile[(c + i) * kTailPitch + p] = v[i] * (scale != nullptr ? scale[c0 + c + i] : 1.f);
-        }
+    for (int k = 0; k < R; k++) {
+        const int f = threadIdx.x + k * kBlkThreads, cc = f / PER, p = f % PER * VEC;
+#pragma unroll
+        for (int e = 0; e < VEC; e++) rs[k][e] = 0.f;
+        if (res != nullptr && cc < nc && p < np) load_run<TS, VEC>(res + base + (size_t)cc * t.HW + p, rs[k]);
+    }
+    float sc[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) sc[i] = scale != nullptr && c < nc ? scale[c0 + c + i] : 1.f;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int p = threadIdx.x / 8 + 32 * k;
+        if (c < nc && p < np)
+#pragma unroll
+            for (int i = 0; i < 8; i++) tile[(c + i) * kTailPitch + p] = v[k][i] * sc[i];
     }
     __syncthreads();
 #pragma unroll
@@ -463,7 +650,8 @@ __global__ __launch_bounds__(kBlkThreads) void tail_kernel(const TY *__restrict_
     }
 }
 
-// dy [N,HW,C] = scale * dout, part [groups][C] = sums of dout * y; a workgroup keeps its channel tile
+// dy [N,HW,C] = scale * dout, part [groups][C] = sums of dout * y; a workgroup keeps its channel tile (y may be null: no
+// sums)
 template <typename TY, typename TR, int VEC>
 __global__ __launch_bounds__(kBlkThreads) void tail_backward_kernel(const TR *__restrict__ dout,
                                                                     const TY *__restrict__ y,
@@ -476,7 +664,7 @@ __global__ __launch_bounds__(kBlkThreads) void tail_backward_kernel(const TR *__
     const int c = threadIdx.x % 8 * 8;
     float sc[8], ds[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) sc[i] = c < nc ? scale[c0 + c + i] : 0.f, ds[i] = 0.f;
+    for (int i = 0; i < 8; i++) sc[i] = scale != nullptr && c < nc ? scale[c0 + c + i] : 1.f, ds[i] = 0.f;
     constexpr int PER = kTailP / VEC, R = kTailC * PER / kBlkThreads;
     for (int u = group; u < t.units; u += groups) {
         const int n = u / t.per, p0 = u % t.per * kTailP, np = min(kTailP, t.HW - p0);
@@ -491,7 +679,10 @@ __global__ __launch_bounds__(kBlkThreads) void tail_backward_kernel(const TR *__
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             const int p = threadIdx.x / 8 + 32 * k;
-            if (c < nc && p < np) load8(y + row + (size_t)p * t.C, yv[k]);
+            if (y != nullptr && c < nc && p < np) load8(y + row + (size_t)p * t.C, yv[k]);
+            else
+#pragma unroll
+                for (int i = 0; i < 8; i++) yv[k][i] = 0.f;
         }
         __syncthreads();  // the tile's last readers are done
 #pragma unroll
@@ -517,6 +708,7 @@ __global__ __launch_bounds__(kBlkThreads) void tail_backward_kernel(const TR *__
             }
         }
     }
+    if (y == nullptr) return;
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 8; i++) tile[i * kBlkThreads + threadIdx.x] = ds[i];

@@ -62,9 +62,19 @@ bool tile_ok(int N, int C, int H, int W) {
     return N >= 1 && H >= 1 && W >= 1 && channels_ok(C) && (double)N * C * H * W < 2147483648.0;
 }
 BlkTiles tiles_of(int N, int C, int HW, int bytes) {
-    BlkTiles t;
-    t.C = C, t.HW = HW, t.P = blk_tile_pixels(C, bytes);
+    BlkTiles t{};
+    t.C = C, t.HW = HW, t.P = blk_tile_pixels(C, bytes, (long)N * HW);
+    t.log2P = __builtin_ctz(t.P);
     t.per = (HW + t.P - 1) / t.P, t.tiles = N * t.per;
+    return t;
+}
+BlkTiles patches_of(int N, int C, int H, int W, int bytes) {
+    BlkTiles t{};
+    t.C = C, t.HW = H * W, t.H = H, t.W = W, t.W2 = W / 2;
+    t.P = blk_tile_pixels(C, bytes, (long)N * H * W);
+    while (t.P > 8 && t.P / 4 >= 2 * t.W2) t.P >>= 1;  // (no wider than a row)
+    t.log2P = __builtin_ctz(t.P);
+    t.per = (t.W2 + t.P / 4 - 1) / (t.P / 4), t.tiles = N * (H / 2) * t.per;
     return t;
 }
 TailTiles tail_of(int N, int C, int HW) {
@@ -182,43 +192,107 @@ int dwo_ln_tile_backward(const void *dout, const void *x, const float *stats, co
     return column_sums((const float *)scratch, dgamma, dbeta, 2 * C, C, groups, grad_dtype, st);
 }
 
+int dwo_ln_patch(const void *x, const float *gamma, const float *beta, void *out, float *stats, int N, int C, int H,
+                 int W, float eps, int in_dtype, int out_dtype, void *stream) {
+    if (!x || !gamma || !beta || !out) return DWO_ERR_NULL_POINTER;
+    if (!tile_ok(N, C, H, W) || H < 2 || W < 2 || !aligned16(x) || !aligned16(out)) return DWO_ERR_BAD_SHAPE;
+    (void)hipGetLastError();
+    const BlkTiles t = patches_of(N, C, H, W, esize(in_dtype));
+    return by_types(in_dtype, out_dtype, [&](auto ti, auto to) {
+        using TI = typename decltype(ti)::type;
+        using TO = typename decltype(to)::type;
+        return by_channels(C, [&](auto lpr, auto nv) {
+            constexpr int LPR = decltype(lpr)::value, NV = decltype(nv)::value;
+            const dim3 grid(t.tiles), block(kBlkThreads);
+            const size_t lds = blk_tile_bytes(C, t.P, sizeof(TI));
+            if (W % 4 == 0)
+                ln_patch_kernel<TI, TO, LPR, NV, 4><<<grid, block, lds, (hipStream_t)stream>>>(
+                    (const TI *)x, gamma, beta, (TO *)out, (float2 *)stats, t, eps);
+            else
+                ln_patch_kernel<TI, TO, LPR, NV, 1><<<grid, block, lds, (hipStream_t)stream>>>(
+                    (const TI *)x, gamma, beta, (TO *)out, (float2 *)stats, t, eps);
+            return status();
+        });
+    });
+}
+
+int dwo_ln_patch_backward(const void *dout, const void *x, const float *stats, const float *gamma, void *dx,
+                          void *dgamma, void *dbeta, void *scratch, size_t scratch_bytes, int N, int C, int H, int W,
+                          int in_dtype, int out_dtype, int grad_dtype, void *stream) {
+    if (!dout || !x || !stats || !gamma || !dx || !scratch) return DWO_ERR_NULL_POINTER;
+    if (!tile_ok(N, C, H, W) || H < 2 || W < 2 || !aligned16(x) || !aligned16(dout) || !aligned16(dx))
+        return DWO_ERR_BAD_SHAPE;
+    if (scratch_bytes < dwo_block_scratch_bytes(C)) return DWO_ERR_SCRATCH_TOO_SMALL;
+    (void)hipGetLastError();
+    hipStream_t st = (hipStream_t)stream;
+    const BlkTiles t = patches_of(N, C, H, W, esize(in_dtype));
+    const int groups = groups_of(t.tiles);
+    const int e = by_types(in_dtype, out_dtype, [&](auto ti, auto to) {
+        using TI = typename decltype(ti)::type;
+        using TO = typename decltype(to)::type;
+        return by_channels(C, [&](auto lpr, auto nv) {
+            constexpr int LPR = decltype(lpr)::value, NV = decltype(nv)::value;
+            const dim3 grid(groups), block(kBlkThreads);
+            size_t lds = blk_tile_bytes(C, t.P, sizeof(TI));
+            if (lds < 8 * kBlkThreads * sizeof(float)) lds = 8 * kBlkThreads * sizeof(float);  // the parameter sums
+            if (W % 4 == 0)
+                ln_patch_backward_kernel<TI, TO, LPR, NV, 4><<<grid, block, lds, st>>>(
+                    (const TO *)dout, (const TI *)x, (const float2 *)stats, gamma, (TI *)dx, (float *)scratch, t);
+            else
+                ln_patch_backward_kernel<TI, TO, LPR, NV, 1><<<grid, block, lds, st>>>(
+                    (const TO *)dout, (const TI *)x, (const float2 *)stats, gamma, (TI *)dx, (float *)scratch, t);
+            return status();
+        });
+    });
+    if (e != DWO_OK) return e;
+    return column_sums((const float *)scratch, dgamma, dbeta, 2 * C, C, groups, grad_dtype, st);
+}
+
 int dwo_block_tail(const void *y, const float *scale, const void *res, void *out, int N, int C, int H, int W,
-                   int y_dtype, int dtype, void *stream) {
-    if (!y || !scale || !res || !out) return DWO_ERR_NULL_POINTER;
+                   int y_dtype, int res_dtype, int dtype, void *stream) {
+    if (!y || !out) return DWO_ERR_NULL_POINTER;
     if (N < 1 || H < 1 || W < 1 || C < 8 || C % 8 != 0 || (double)N * C * H * W >= 2147483648.0 || !aligned16(y) ||
         !aligned16(res) || !aligned16(out))
         return DWO_ERR_BAD_SHAPE;
     (void)hipGetLastError();
     const TailTiles t = tail_of(N, C, H * W);
+    const dim3 grid((unsigned)t.units * t.ctiles), block(kBlkThreads);
+    // out is y's type or fp32, res has out's type or y's
     return by_types(dtype, y_dtype, [&](auto tr, auto ty) {
         using TR = typename decltype(tr)::type;
         using TY = typename decltype(ty)::type;
-        const dim3 grid((unsigned)t.units * t.ctiles), block(kBlkThreads);
-        if (t.HW % 4 == 0)
-            tail_kernel<TY, TR, 4><<<grid, block, 0, (hipStream_t)stream>>>((const TY *)y, scale, (const TR *)res,
-                                                                            (TR *)out, t);
-        else
-            tail_kernel<TY, TR, 1><<<grid, block, 0, (hipStream_t)stream>>>((const TY *)y, scale, (const TR *)res,
-                                                                            (TR *)out, t);
-        return status();
+        auto launch = [&](auto ts) {
+            using TS = typename decltype(ts)::type;
+            if (t.HW % 4 == 0)
+                tail_kernel<TY, TS, TR, 4><<<grid, block, 0, (hipStream_t)stream>>>((const TY *)y, scale, (const TS *)res,
+                                                                                    (TR *)out, t);
+            else
+                tail_kernel<TY, TS, TR, 1><<<grid, block, 0, (hipStream_t)stream>>>((const TY *)y, scale, (const TS *)res,
+                                                                                    (TR *)out, t);
+            return status();
+        };
+        if (res == nullptr || res_dtype == dtype) return launch(Type<TR>{});
+        if (res_dtype == y_dtype) return launch(Type<TY>{});
+        return (int)DWO_ERR_BAD_DTYPE;
     });
 }
 
 int dwo_block_tail_backward(const void *dout, const void *y, const float *scale, void *dy, void *dscale, void *scratch,
                             size_t scratch_bytes, int N, int C, int H, int W, int y_dtype, int dtype, int grad_dtype,
                             void *stream) {
-    if (!dout || !y || !scale || !dy || !scratch) return DWO_ERR_NULL_POINTER;
+    if (!dout || !dy || (y && !scratch)) return DWO_ERR_NULL_POINTER;
     if (N < 1 || H < 1 || W < 1 || C < 8 || C % 8 != 0 || (double)N * C * H * W >= 2147483648.0 || !aligned16(y) ||
         !aligned16(dout) || !aligned16(dy))
         return DWO_ERR_BAD_SHAPE;
-    if (scratch_bytes < dwo_block_scratch_bytes(C)) return DWO_ERR_SCRATCH_TOO_SMALL;
+    if (y && scratch_bytes < dwo_block_scratch_bytes(C)) return DWO_ERR_SCRATCH_TOO_SMALL;
     (void)hipGetLastError();
     hipStream_t st = (hipStream_t)stream;
     const TailTiles t = tail_of(N, C, H * W);
-    long g = 2048 / t.ctiles;
+    // without sums a workgroup per tile, else workgroups that keep them over several tiles
+    long g = y ? 2048 / t.ctiles : t.units;
     if (g < 1) g = 1;
     if (g > t.units) g = t.units;
-    const int groups = groups_of(g);
+    const int groups = y ? groups_of(g) : (int)g;
     const int e = by_types(dtype, y_dtype, [&](auto tr, auto ty) {
         using TR = typename decltype(tr)::type;
         using TY = typename decltype(ty)::type;
@@ -231,7 +305,7 @@ int dwo_block_tail_backward(const void *dout, const void *y, const float *scale,
                                                                     (float *)scratch, t);
         return status();
     });
-    if (e != DWO_OK) return e;
+    if (e != DWO_OK || !y) return e;
     return column_sums((const float *)scratch, dscale, nullptr, C, C, groups, grad_dtype, st);
 }
 

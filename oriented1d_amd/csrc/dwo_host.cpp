@@ -44,6 +44,8 @@ struct Library {
     decltype(&::dwo_block_tail_backward) block_tail_backward;
     decltype(&::dwo_linear_wgrad_scratch_bytes) linear_wgrad_scratch_bytes;
     decltype(&::dwo_linear_wgrad) linear_wgrad;
+    decltype(&::dwo_ln_patch) ln_patch;
+    decltype(&::dwo_ln_patch_backward) ln_patch_backward;
     decltype(&::dwo_linear_rows) linear_rows;
     decltype(&::dwo_linear_planes) linear_planes;
 } lib;
@@ -77,6 +79,8 @@ void bind_library(const std::string &path) {
     find(lib.block_tail_backward, "dwo_block_tail_backward");
     find(lib.linear_wgrad_scratch_bytes, "dwo_linear_wgrad_scratch_bytes");
     find(lib.linear_wgrad, "dwo_linear_wgrad");
+    find(lib.ln_patch, "dwo_ln_patch");
+    find(lib.ln_patch_backward, "dwo_ln_patch_backward");
     find(lib.linear_rows, "dwo_linear_rows");
     find(lib.linear_planes, "dwo_linear_planes");
 }
@@ -340,17 +344,18 @@ std::tuple<Tensor, OptTensor> linear_wgrad(const Tensor &dy_, const Tensor &x_, 
 }
 
 // LayerNorm (+ GELU) over the last dimension; (out, stats)
-std::tuple<Tensor, Tensor> ln_rows(const Tensor &x_, const Tensor &g, const Tensor &b, double eps, bool gelu,
-                                   at::ScalarType out_dtype) {
+std::tuple<Tensor, OptTensor> ln_rows(const Tensor &x_, const Tensor &g, const Tensor &b, double eps, bool gelu,
+                                      at::ScalarType out_dtype, bool with_stats) {
     check_glue(x_, "x");
     py::gil_scoped_release nogil;
     const Place at(x_);
     const Tensor x = dense(x_);
     const int64_t C = x.size(-1), rows = x.numel() / std::max<int64_t>(C, 1);
     Tensor out = at::empty(x.sizes(), x.options().dtype(out_dtype));
-    Tensor stats = at::empty({rows, 2}, x.options().dtype(at::kFloat));
-    check(lib.ln_rows(ptr(x), (const float *)ptr(g), (const float *)ptr(b), out.data_ptr(), (float *)stats.data_ptr(),
-                      (size_t)rows, as_int(C), (float)eps, gelu, dtype_code(x), dtype_code(out_dtype), at.stream),
+    OptTensor stats;
+    if (with_stats) stats = at::empty({rows, 2}, x.options().dtype(at::kFloat));
+    check(lib.ln_rows(ptr(x), (const float *)ptr(g), (const float *)ptr(b), out.data_ptr(),
+                      stats.has_value() ? (float *)stats->data_ptr() : nullptr, (size_t)rows, as_int(C), (float)eps, gelu, dtype_code(x), dtype_code(out_dtype), at.stream),
           "dwo_ln_rows");
     return {out, stats};
 }
@@ -378,84 +383,105 @@ std::tuple<Tensor, Tensor, Tensor> ln_rows_backward(const Tensor &dout_, const T
     return {dx, dg, db};
 }
 
-// [N,C,H,W] -> LayerNorm over C -> [N,H,W,C]; (out, stats)
-std::tuple<Tensor, Tensor> ln_tile(const Tensor &x_, const Tensor &g, const Tensor &b, double eps,
-                                   at::ScalarType out_dtype) {
+// [N,C,H,W] -> LayerNorm over C -> [N,H,W,C], or with `patches` [N,H/2,W/2,4C]; (out, stats)
+std::tuple<Tensor, OptTensor> ln_tile(const Tensor &x_, const Tensor &g, const Tensor &b, double eps, bool patches,
+                                      at::ScalarType out_dtype, bool with_stats) {
     check_glue(x_, "x");
     if (x_.dim() != 4) throw py::value_error("x must be a 4-d tensor");
     py::gil_scoped_release nogil;
     const Place at(x_);
     const Tensor x = dense(x_);
     const Dims d(x, false);
-    Tensor out = at::empty({d.n, d.h, d.w, d.c}, x.options().dtype(out_dtype));
-    Tensor stats = at::empty({d.n * d.h * d.w, 2}, x.options().dtype(at::kFloat));
-    check(lib.ln_tile(ptr(x), (const float *)ptr(g), (const float *)ptr(b), out.data_ptr(), (float *)stats.data_ptr(),
-                      as_int(d.n), as_int(d.c), as_int(d.h), as_int(d.w), (float)eps, dtype_code(x),
-                      dtype_code(out_dtype), at.stream),
-          "dwo_ln_tile");
+    const std::array<int64_t, 4> shape = patches ? std::array<int64_t, 4>{d.n, d.h / 2, d.w / 2, 4 * d.c}
+                                                 : std::array<int64_t, 4>{d.n, d.h, d.w, d.c};
+    Tensor out = at::empty(shape, x.options().dtype(out_dtype));
+    OptTensor stats;
+    if (with_stats) stats = at::empty({out.numel() / std::max<int64_t>(d.c, 1), 2}, x.options().dtype(at::kFloat));
+    check((patches ? lib.ln_patch : lib.ln_tile)(ptr(x), (const float *)ptr(g), (const float *)ptr(b), out.data_ptr(),
+                                                 stats.has_value() ? (float *)stats->data_ptr() : nullptr, as_int(d.n),
+                                                 as_int(d.c), as_int(d.h), as_int(d.w), (float)eps, dtype_code(x),
+                                                 dtype_code(out_dtype), at.stream),
+          patches ? "dwo_ln_patch" : "dwo_ln_tile");
     return {out, stats};
 }
 
 std::tuple<Tensor, Tensor, Tensor> ln_tile_backward(const Tensor &dout_, const Tensor &x_, const Tensor &stats,
-                                                    const Tensor &g, at::ScalarType grad_dtype) {
+                                                    const Tensor &g, bool patches, at::ScalarType grad_dtype) {
     check_glue(dout_, "dout");
     check_glue(x_, "x");
     check_pair(dout_, x_);
     const Dims d(x_, false);
-    const std::array<int64_t, 4> want = {d.n, d.h, d.w, d.c};
-    if (dout_.sizes() != at::IntArrayRef(want)) fail("dout must be [N,H,W,C]");
+    const std::array<int64_t, 4> want = patches ? std::array<int64_t, 4>{d.n, d.h / 2, d.w / 2, 4 * d.c}
+                                                : std::array<int64_t, 4>{d.n, d.h, d.w, d.c};
+    if (dout_.sizes() != at::IntArrayRef(want)) fail("dout does not match x");
     py::gil_scoped_release nogil;
     const Place at(x_);
     const Tensor x = dense(x_), dout = dense(dout_);
     const size_t nbytes = lib.block_scratch_bytes(as_int(d.c));
     const Tensor scratch = bytes(x, nbytes);
-    Tensor dx = at::empty(x.sizes(), x.options());
+    // (an odd last row or column is in no patch)
+    Tensor dx = patches && (d.h % 2 != 0 || d.w % 2 != 0) ? at::zeros(x.sizes(), x.options()) : at::empty(x.sizes(), x.options());
     Tensor dg = at::empty({d.c}, x.options().dtype(grad_dtype)), db = at::empty({d.c}, dg.options());
-    check(lib.ln_tile_backward(ptr(dout), ptr(x), (const float *)ptr(stats), (const float *)ptr(g), dx.data_ptr(),
-                               dg.data_ptr(), db.data_ptr(), scratch.data_ptr(), nbytes, as_int(d.n), as_int(d.c),
-                               as_int(d.h), as_int(d.w), dtype_code(x), dtype_code(dout), dtype_code(grad_dtype),
-                               at.stream),
-          "dwo_ln_tile_backward");
+    check((patches ? lib.ln_patch_backward : lib.ln_tile_backward)(
+              ptr(dout), ptr(x), (const float *)ptr(stats), (const float *)ptr(g), dx.data_ptr(), dg.data_ptr(),
+              db.data_ptr(), scratch.data_ptr(), nbytes, as_int(d.n), as_int(d.c), as_int(d.h), as_int(d.w),
+              dtype_code(x), dtype_code(dout), dtype_code(grad_dtype), at.stream),
+          patches ? "dwo_ln_patch_backward" : "dwo_ln_tile_backward");
     return {dx, dg, db};
 }
 
-// res + scale * y: y [N,H,W,C], res [N,C,H,W]
-Tensor block_tail(const Tensor &y_, const Tensor &scale, const Tensor &res_) {
+// res + scale * y as planes of out_dtype: y [N,H,W,C], res [N,C,H,W]
+Tensor block_tail(const Tensor &y_, const OptTensor &scale, const OptTensor &res_, at::ScalarType out_dtype) {
     check_glue(y_, "y");
-    check_glue(res_, "res");
-    check_pair(y_, res_);
     if (y_.dim() != 4) throw py::value_error("y must be a 4-d tensor");
     const Dims d(y_, true);
-    const std::array<int64_t, 4> want = {d.n, d.c, d.h, d.w};
-    if (res_.sizes() != at::IntArrayRef(want)) fail("res must be [N,C,H,W]");
+    const std::array<int64_t, 4> shape = {d.n, d.c, d.h, d.w};
+    if (res_.has_value()) {
+        check_glue(*res_, "res");
+        check_pair(y_, *res_);
+        if (res_->sizes() != at::IntArrayRef(shape)) fail("res must be [N,C,H,W]");
+    }
     py::gil_scoped_release nogil;
     const Place at(y_);
-    const Tensor y = dense(y_), res = dense(res_);
-    Tensor out = at::empty(res.sizes(), res.options());
-    check(lib.block_tail(ptr(y), (const float *)ptr(scale), ptr(res), out.data_ptr(), as_int(d.n), as_int(d.c),
-                         as_int(d.h), as_int(d.w), dtype_code(y), dtype_code(res), at.stream),
+    const Tensor y = dense(y_);
+    Tensor res, out = at::empty(shape, y.options().dtype(out_dtype));
+    if (res_.has_value()) res = dense(*res_);
+    check(lib.block_tail(ptr(y), fptr(scale), res.defined() ? ptr(res) : nullptr, out.data_ptr(), as_int(d.n),
+                         as_int(d.c), as_int(d.h), as_int(d.w), dtype_code(y),
+                         res.defined() ? dtype_code(res) : dtype_code(out_dtype), dtype_code(out_dtype), at.stream),
           "dwo_block_tail");
     return out;
 }
 
-std::tuple<Tensor, Tensor> block_tail_backward(const Tensor &dout_, const Tensor &y_, const Tensor &scale,
-                                               at::ScalarType grad_dtype) {
+// dout [N,C,H,W] -> (dy [N,H,W,C] of y_dtype, dscale); without y only dy
+std::tuple<Tensor, OptTensor> block_tail_backward(const Tensor &dout_, const OptTensor &y_, const OptTensor &scale,
+                                                  at::ScalarType y_dtype, at::ScalarType grad_dtype) {
     check_glue(dout_, "dout");
-    check_glue(y_, "y");
-    check_pair(dout_, y_);
-    const Dims d(y_, true);
-    const std::array<int64_t, 4> want = {d.n, d.c, d.h, d.w};
-    if (dout_.sizes() != at::IntArrayRef(want)) fail("dout must be [N,C,H,W]");
+    if (dout_.dim() != 4) throw py::value_error("dout must be a 4-d tensor");
+    const Dims d(dout_, false);
+    const std::array<int64_t, 4> shape = {d.n, d.h, d.w, d.c};
+    if (y_.has_value()) {
+        check_glue(*y_, "y");
+        check_pair(dout_, *y_);
+        if (y_->sizes() != at::IntArrayRef(shape) || y_->scalar_type() != y_dtype) fail("y does not match dout");
+    }
     py::gil_scoped_release nogil;
-    const Place at(y_);
-    const Tensor y = dense(y_), dout = dense(dout_);
-    const size_t nbytes = lib.block_scratch_bytes(as_int(d.c));
-    const Tensor scratch = bytes(y, nbytes);
-    Tensor dy = at::empty(y.sizes(), y.options());
-    Tensor ds = at::empty({d.c}, y.options().dtype(grad_dtype));
-    check(lib.block_tail_backward(ptr(dout), ptr(y), (const float *)ptr(scale), dy.data_ptr(), ds.data_ptr(),
-                                  scratch.data_ptr(), nbytes, as_int(d.n), as_int(d.c), as_int(d.h), as_int(d.w),
-                                  dtype_code(y), dtype_code(dout), dtype_code(grad_dtype), at.stream),
+    const Place at(dout_);
+    const Tensor dout = dense(dout_);
+    Tensor y, scratch, dy = at::empty(shape, dout.options().dtype(y_dtype));
+    OptTensor ds;
+    size_t nbytes = 0;
+    if (y_.has_value()) {
+        y = dense(*y_);
+        nbytes = lib.block_scratch_bytes(as_int(d.c));
+        scratch = bytes(y, nbytes);
+        ds = at::empty({d.c}, y.options().dtype(grad_dtype));
+    }
+    check(lib.block_tail_backward(ptr(dout), y.defined() ? ptr(y) : nullptr, fptr(scale), dy.data_ptr(),
+                                  ds.has_value() ? ds->data_ptr() : nullptr,
+                                  scratch.defined() ? scratch.data_ptr() : nullptr, nbytes, as_int(d.n), as_int(d.c),
+                                  as_int(d.h), as_int(d.w), dtype_code(y_dtype), dtype_code(dout),
+                                  dtype_code(grad_dtype), at.stream),
           "dwo_block_tail_backward");
     return {dy, ds};
 }

@@ -232,21 +232,6 @@ int launch_linear_reduce(const float *part, void *dw, void *db, int N, int K, in
 // stores left the L2 with four times as many writes: 401408 x 384 x 96 208 us, now 172).  Where planes are no multiple of four pixels
 // lanes run along the pixels instead (single values, 32 bytes per store).
 
-// GELU with erf from Abramowitz and Stegun, Handbook of Mathematical Functions, 7.1.26 (error of erf below 1.5e-7, next
-// to a rounding of 2^-9 or 2^-12 of the result on the way out): u > 0: u (1 - q), else -|u| q, q = erfc(|u| / sqrt 2) / 2.
-// erff takes twice the issue slots of the matrix products of a stage-1 block.
-__device__ __forceinline__ float lin_gelu(float u) {
-    const float z = __builtin_fabsf(u);
-    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(z, 0.3275911f * 0.70710678118654752f, 1.f));
-    float p = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
-    p = __builtin_fmaf(t, p, 0.5f * 1.421413741f);
-    p = __builtin_fmaf(t, p, 0.5f * -0.284496736f);
-    p = __builtin_fmaf(t, p, 0.5f * 0.254829592f);
-    p *= t;
-    const float e = __builtin_amdgcn_exp2f(u * u * -0.72134752044448170f);  // exp(-u^2 / 2)
-    return __builtin_fmaf(-p, z * e, __builtin_fmaxf(u, 0.f));
-}
-
 template <typename T>
 struct LinearArgs {
     const T *x, *w, *bias, *scale, *res;
@@ -273,7 +258,7 @@ __device__ __forceinline__ void lin_emit_rows(const LinearArgs<T> &a, long m, in
 #pragma unroll
     for (int r = 0; r < Q; r++) {
         v[r] += b[r];
-        if (a.gelu) v[r] = lin_gelu(v[r]);
+        if (a.gelu) v[r] = gelu_rounded(v[r]);
     }
     T *at = a.out + m * a.N + n;
     if constexpr (Q == 8)

@@ -39,14 +39,25 @@ def usable(x, C, tiled):
             and C <= (MAX_C_TILE if tiled else MAX_C_ROWS) and not torch.is_grad_enabled())
 
 
+def _pieces(x, C):
+    """True where the kernels that take eight channels per lane cover LayerNorm over C channels of x."""
+    return x.is_cuda and x.dtype in _DTYPES and C % 8 == 0 and 8 <= C <= MAX_C_TRAIN and 0 < x.numel() < 1 << 31
+
+
 def layernorm_nhwc(x, weight, bias, eps, gelu=False):
     """LayerNorm over the last dimension of a contiguous tensor (+ exact GELU)."""
-    return _lib.host(x.get_device()).layernorm_nhwc(x, _f32(weight), _f32(bias), eps, gelu)
+    host, C = _lib.host(x.get_device()), x.shape[-1]
+    if _pieces(x, C):
+        return host.ln_rows(x, _f32(weight), _f32(bias), eps, gelu, x.dtype, False)[0]
+    return host.layernorm_nhwc(x, _f32(weight), _f32(bias), eps, gelu)
 
 
 def nchw_layernorm_nhwc(x, weight, bias, eps):
     """[N,C,H,W] -> [N,H,W,C], LayerNorm over C: ``norm(x.permute(0, 2, 3, 1))`` in one pass."""
-    return _lib.host(x.get_device()).nchw_layernorm_nhwc(x, _f32(weight), _f32(bias), eps)
+    host = _lib.host(x.get_device())
+    if x.dim() == 4 and _pieces(x, x.shape[1]):
+        return host.ln_tile(x, _f32(weight), _f32(bias), eps, False, x.dtype, False)[0]
+    return host.nchw_layernorm_nhwc(x, _f32(weight), _f32(bias), eps)
 
 
 def nhwc_scale_add_nchw(y, scale=None, residual=None):
@@ -206,30 +217,37 @@ def _second_order(value, inputs, dout):
     return [next(got) if t.requires_grad else None for t in inputs]
 
 
+def _patches(x):
+    """[N,H,W,C] -> [N,H/2,W/2,4C]: the 2 x 2 patches, channel first (an odd last row or column is in none)."""
+    N, H, W, C = x.shape
+    x = x[:, :H // 2 * 2, :W // 2 * 2].reshape(N, H // 2, 2, W // 2, 2, C)
+    return x.permute(0, 1, 3, 5, 2, 4).reshape(N, H // 2, W // 2, 4 * C)
+
+
 class _TileNorm(torch.autograd.Function):
-    """LayerNorm over dim 1 of an NCHW tensor, as [N,H,W,C]."""
+    """LayerNorm over dim 1 of an NCHW tensor, as [N,H,W,C] or as 2 x 2 patches."""
 
     @staticmethod
-    def forward(ctx, x, w, b, eps, dtype):
+    def forward(ctx, x, w, b, eps, dtype, patches=False):
         ctx.set_materialize_grads(False)
         x = x.contiguous()
-        out, stats = _lib.host(x.get_device()).ln_tile(x, _f32(w), _f32(b), eps, dtype)
+        out, stats = _lib.host(x.get_device()).ln_tile(x, _f32(w), _f32(b), eps, patches, dtype, True)
         ctx.save_for_backward(x, w, b, stats)
-        ctx.eps, ctx.dtype = eps, dtype
+        ctx.eps, ctx.dtype, ctx.patches = eps, dtype, patches
         return out
 
     @staticmethod
     def backward(ctx, dout):
         if dout is None:
-            return None, None, None, None, None
+            return None, None, None, None, None, None
         x, w, b, stats = ctx.saved_tensors
         if torch.is_grad_enabled():
             def value(x, w, b):
                 y = F.layer_norm(x.permute(0, 2, 3, 1).float(), w.shape, w.float(), b.float(), ctx.eps)
-                return y.to(ctx.dtype)
-            return (*_second_order(value, (x, w, b), dout), None, None)
-        dx, dw, db = _lib.host(x.get_device()).ln_tile_backward(dout, x, stats, _f32(w), w.dtype)
-        return dx, dw, db.to(b.dtype), None, None
+                return (_patches(y) if ctx.patches else y).to(ctx.dtype)
+            return (*_second_order(value, (x, w, b), dout), None, None, None)
+        dx, dw, db = _lib.host(x.get_device()).ln_tile_backward(dout, x, stats, _f32(w), ctx.patches, w.dtype)
+        return dx, dw, db.to(b.dtype), None, None, None
 
 
 class _RowNorm(torch.autograd.Function):
@@ -239,7 +257,7 @@ class _RowNorm(torch.autograd.Function):
     def forward(ctx, x, w, b, eps, gelu, dtype):
         ctx.set_materialize_grads(False)
         x = x.contiguous()
-        out, stats = _lib.host(x.get_device()).ln_rows(x, _f32(w), _f32(b), eps, gelu, dtype)
+        out, stats = _lib.host(x.get_device()).ln_rows(x, _f32(w), _f32(b), eps, gelu, dtype, True)
         ctx.save_for_backward(x, w, b, stats)
         ctx.eps, ctx.gelu, ctx.dtype = eps, gelu, dtype
         return out
@@ -259,30 +277,37 @@ class _RowNorm(torch.autograd.Function):
 
 
 class _BlockTail(torch.autograd.Function):
-    """``x + (gamma * y).permute(0, 3, 1, 2)`` for y [N,H,W,C] and x [N,C,H,W]."""
+    """``x + (gamma * y).permute(0, 3, 1, 2)`` in ``dtype`` for y [N,H,W,C] and x [N,C,H,W]; without gamma and x the
+    permutation alone."""
 
     @staticmethod
-    def forward(ctx, y, gamma, x):
+    def forward(ctx, y, gamma, x, dtype):
         ctx.set_materialize_grads(False)
         y = y.contiguous()
-        out = _lib.host(y.get_device()).block_tail(y, _f32(gamma), x)
-        ctx.save_for_backward(y, gamma)
+        out = _lib.host(y.get_device()).block_tail(y, None if gamma is None else _f32(gamma), x, dtype)
+        ctx.save_for_backward(*(() if gamma is None else (y, gamma)))
+        ctx.types = y.dtype, None if x is None else x.dtype
         return out
 
     @staticmethod
     def backward(ctx, dout):
         if dout is None:
-            return None, None, None
-        y, gamma = ctx.saved_tensors
-        dx = dout if ctx.needs_input_grad[2] else None
+            return None, None, None, None
+        dtype, x_dtype = ctx.types
+        dx = dout.to(x_dtype) if ctx.needs_input_grad[2] else None
         if not (ctx.needs_input_grad[0] or ctx.needs_input_grad[1]):
-            return None, None, dx
+            return None, None, dx, None
+        y, gamma = ctx.saved_tensors if ctx.saved_tensors else (None, None)
         if torch.is_grad_enabled():
+            if gamma is None:
+                return dout.permute(0, 2, 3, 1).to(dtype), None, dx, None
+
             def value(y, gamma):
                 return (gamma * y).permute(0, 3, 1, 2).to(dout.dtype)
-            return (*_second_order(value, (y, gamma), dout), dx)
-        dy, dg = _lib.host(y.get_device()).block_tail_backward(dout, y, _f32(gamma), gamma.dtype)
-        return dy, dg, dx
+            return (*_second_order(value, (y, gamma), dout), dx, None)
+        scale, grad = (None, torch.float32) if gamma is None else (_f32(gamma), gamma.dtype)
+        dy, dg = _lib.host(dout.get_device()).block_tail_backward(dout, y, scale, dtype, grad)
+        return dy, dg, dx, None
 
 
 class _Linear(torch.autograd.Function):
@@ -365,15 +390,56 @@ def row_norm(x, norm, gelu=False, consumer=None):
     return None if dtype is None else _RowNorm.apply(x, norm.weight, norm.bias, norm.eps, gelu, dtype)
 
 
+def _tail_covers(y):
+    return y.dim() == 4 and y.shape[-1] % 8 == 0 and y.shape[-1] <= MAX_C_TRAIN and y.numel() < 1 << 31
+
+
 def block_tail(y, gamma, x):
     """``x + (gamma * y).permute(0, 3, 1, 2)`` recorded by autograd; None where the kernels do not cover the call."""
-    if not (_recording(y, gamma, x) and y.dim() == 4 and gamma.shape == y.shape[-1:] and y.shape[-1] % 8 == 0
-            and y.shape[-1] <= MAX_C_TRAIN and y.numel() < 1 << 31
-            and x.shape == (y.shape[0], y.shape[3], y.shape[1], y.shape[2])
-            and torch.promote_types(torch.promote_types(gamma.dtype, y.dtype), x.dtype) == x.dtype
-            and x.dtype in (y.dtype, torch.float32)):
+    if not (_recording(y, gamma, x) and _tail_covers(y) and gamma.shape == y.shape[-1:]
+            and x.shape == (y.shape[0], y.shape[3], y.shape[1], y.shape[2])):
         return None
-    return _BlockTail.apply(y, gamma, x)
+    dtype = torch.promote_types(torch.promote_types(gamma.dtype, y.dtype), x.dtype)
+    if dtype not in (y.dtype, torch.float32) or x.dtype not in (y.dtype, dtype):
+        return None
+    return _BlockTail.apply(y, gamma, x, dtype)
+
+
+def planes(y):
+    """``y.permute(0, 3, 1, 2).contiguous()``, recorded by autograd where the kernels cover it."""
+    if _recording(y) and _tail_covers(y):
+        return _BlockTail.apply(y, None, None, y.dtype)
+    return y.permute(0, 3, 1, 2).contiguous()
+
+
+def downsample(x, norm, conv):
+    """``conv(norm(x))`` of a LayerNorm over the channels of an NCHW tensor and a 2 x 2 convolution of stride 2: a pointwise layer
+    over normalised patches, with the weights as they lie in memory.  None where the kernels do not cover the call."""
+    w, b = conv.weight, conv.bias
+    if not (plain(conv, torch.nn.Conv2d) and conv.kernel_size == (2, 2) == conv.stride and conv.padding == (0, 0)
+            and conv.dilation == (1, 1) and conv.groups == 1 and conv.padding_mode == "zeros"
+            and x.dim() == 4 and x.is_cuda and min(x.shape[2:]) >= 2 and 0 < x.numel() < 1 << 31
+            and w.shape[1] == x.shape[1] and w.shape[0] % 8 == 0 and x.shape[1] % 8 == 0 and x.shape[1] <= MAX_C_TRAIN
+            and w.shape[0] <= MAX_C_TRAIN and w.is_contiguous()):
+        return None
+    rows = w.view(w.shape[0], -1)
+    if torch.is_grad_enabled():
+        if not (_recording(x, norm.weight, norm.bias, w, b) and w.requires_grad):
+            return None
+        ac = _autocast(x)
+        dtype = ac or x.dtype
+        if dtype not in (torch.bfloat16, torch.float16) or x.dtype not in (dtype, torch.float32):
+            return None
+        if ac is None and not (x.dtype == norm.weight.dtype == norm.bias.dtype == w.dtype
+                               and (b is None or b.dtype == w.dtype)):
+            return None
+        p = _TileNorm.apply(x, norm.weight, norm.bias, norm.eps, dtype, True)
+        return planes(_Linear.apply(p, rows, b))
+    if norm.weight.device != x.device or not _layer16(x.permute(0, 2, 3, 1), w[:, :, 0, 0], b) or not _eager(w):
+        return None
+    host = _lib.host(x.get_device())
+    p = host.ln_tile(x, _f32(norm.weight), _f32(norm.bias), norm.eps, True, x.dtype, False)[0]
+    return host.linear_planes(p, rows, b, None, None)
 
 
 def pointwise_dwconv_nhwc(x, linear, conv):

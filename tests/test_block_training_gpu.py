@@ -80,7 +80,7 @@ def test_block_tail(N, C, H, W, ty, tr):
     g = (torch.randn(C, device="cuda") * 0.5).requires_grad_(True)
     x = torch.randn(N, C, H, W, device="cuda").to(tr).requires_grad_(True)
     dout = torch.randn(N, C, H, W, device="cuda").to(tr)
-    out = fused._BlockTail.apply(y, g, x)
+    out = fused._BlockTail.apply(y, g, x, tr)
     got = torch.autograd.grad(out, (y, g, x), dout)
     leaves = [t.detach().double().requires_grad_(True) for t in (y, g, x)]
     ref = leaves[2] + (leaves[1] * leaves[0]).permute(0, 3, 1, 2)
@@ -89,6 +89,75 @@ def test_block_tail(N, C, H, W, ty, tr):
     close(got[0], want[0], TOL[ty], "dy")
     close(got[1], want[1], 1e-5, "dgamma")
     assert torch.equal(got[2], dout)
+
+
+def test_block_tail_of_a_16_bit_stream_and_planes_alone():
+    torch.manual_seed(5)
+    y = torch.randn(2, 5, 9, 72, device="cuda").to(BF16).requires_grad_(True)
+    g = torch.randn(72, device="cuda", requires_grad=True)
+    x = torch.randn(2, 72, 5, 9, device="cuda").to(BF16).requires_grad_(True)
+    out = fused.block_tail(y, g, x)  # (16-bit stream, fp32 layer scale: the sum is fp32)
+    assert out.dtype == F32 and (x + (g * y).permute(0, 3, 1, 2)).dtype == F32
+    dout = torch.randn_like(out)
+    got = torch.autograd.grad(out, (y, g, x), dout)
+    leaves = [t.detach().double().requires_grad_(True) for t in (y, g, x)]
+    ref = leaves[2] + (leaves[1] * leaves[0]).permute(0, 3, 1, 2)
+    want = torch.autograd.grad(ref, leaves, dout.double())
+    close(out, ref, 1e-5, "out")
+    for a, b, tol in zip(got, want, (TOL[BF16], 1e-5, TOL[BF16])):
+        close(a, b, tol, "gradient")
+    z = fused.planes(y)
+    assert type(z.grad_fn).__name__ == "_BlockTailBackward" and torch.equal(z, y.permute(0, 3, 1, 2))
+    d = torch.randn_like(z)
+    assert torch.equal(torch.autograd.grad(z, y, d)[0], d.permute(0, 2, 3, 1))
+
+
+@pytest.mark.parametrize("types", [(F32, F32), (F32, BF16), (BF16, BF16), (F16, F16)], ids=str)
+@pytest.mark.parametrize("N,C,H,W", [(1, 8, 2, 2), (2, 96, 8, 12), (3, 64, 5, 13), (2, 72, 17, 6), (1, 256, 33, 64),
+                                     (2, 520, 6, 4), (1, 1024, 3, 9), (30, 96, 56, 56)])
+def test_patch_norm(N, C, H, W, types):
+    tin, tout = types
+    torch.manual_seed(C + H)
+    x = (torch.randn(N, C, H, W, device="cuda") * 2 + 0.5).to(tin)
+    w, b = torch.randn(C, device="cuda") * 0.5 + 1, torch.randn(C, device="cuda") * 0.1
+    dout = torch.randn(N, H // 2, W // 2, 4 * C, device="cuda").to(tout)
+    run_norm(x, w, b, dout, lambda x, w, b: fused._TileNorm.apply(x, w, b, 1e-6, tout, True),
+             lambda x, w, b: fused._patches(F.layer_norm(x.permute(0, 2, 3, 1), (C,), w, b, 1e-6)), TOL[tout], TOL[tin])
+
+
+@pytest.mark.parametrize("mode", ["autocast", "bf16", "infer"])
+@pytest.mark.parametrize("N,C,D,H,W", [(2, 64, 128, 12, 12), (1, 96, 192, 7, 9), (3, 32, 40, 14, 6), (1, 768, 1024, 4, 4)])
+def test_downsample_against_the_convolution(N, C, D, H, W, mode):
+    from oriented1d_amd.convnext1d import ChannelsFirstLayerNorm
+    torch.manual_seed(C)
+    norm, conv = ChannelsFirstLayerNorm(C).cuda(), nn.Conv2d(C, D, 2, 2).cuda()
+    with torch.no_grad():
+        norm.weight.add_(torch.randn_like(norm.weight) * 0.3)
+        norm.bias.add_(torch.randn_like(norm.bias) * 0.3)
+    x = torch.randn(N, C, H, W, device="cuda")
+    if mode != "autocast":
+        norm, conv, x = norm.to(BF16), conv.to(BF16), x.to(BF16)
+    params = [norm.weight, norm.bias, conv.weight, conv.bias]
+    ref_leaves = [t.detach().double().requires_grad_(True) for t in [x] + params]
+    rx, rw, rb, rc, rd = ref_leaves
+    ref = F.conv2d(F.layer_norm(rx.permute(0, 2, 3, 1), (C,), rw, rb, 1e-6).permute(0, 3, 1, 2), rc, rd, stride=2)
+    if mode == "infer":
+        with torch.no_grad():
+            y = fused.downsample(x, norm, conv)
+        close(y, ref, TOL[BF16], "y")
+        return
+    x.requires_grad_(True)
+    with torch.autocast("cuda", dtype=BF16, enabled=mode == "autocast"):
+        y = fused.downsample(x, norm, conv)
+    assert y.dtype == BF16 and y.is_contiguous()
+    dy = torch.randn_like(y)
+    got = torch.autograd.grad(y, [x] + params, dy)
+    want = torch.autograd.grad(ref, ref_leaves, dy.double())
+    close(y, ref, TOL[BF16], "y")
+    # (through a 16-bit product of K = 4 C terms and its 16-bit gradient)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape
+        close(a, b, 2 * TOL[BF16], "gradient")
 
 
 @pytest.mark.parametrize("dtype", [BF16, F16], ids=str)
@@ -148,7 +217,7 @@ def test_second_order_of_the_passes(which):
                  lambda: F.layer_norm(a.permute(0, 2, 3, 1), (16,), w, b, 1e-6)),
         "rows": (lambda: fused._RowNorm.apply(nhwc, w, b, 1e-6, True, F32),
                  lambda: F.gelu(F.layer_norm(nhwc, (16,), w, b, 1e-6))),
-        "tail": (lambda: fused._BlockTail.apply(nhwc, w, a),
+        "tail": (lambda: fused._BlockTail.apply(nhwc, w, a, F32),
                  lambda: a + (w * nhwc).permute(0, 3, 1, 2))}[which]
     res = []
     for f in (native, reference):
