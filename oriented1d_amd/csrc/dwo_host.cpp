@@ -4,8 +4,10 @@
 // What bounds a call on small tensors is this path (the stage convolutions of ConvNeXt-T at batch
 // 64 take 216 us of GPU time in 12 kernels).  Kept in Python, with one ctypes call, one device query,
 // one stream object and up to four tensor constructions per kernel, forward and backward of one
-// layer took 90 to 170 us of host time, hence native code, without the GIL.  The autograd function
-// itself stays a Python one (its hooks, modes and refusals are PyTorch's own).
+// layer took 90 to 170 us of host time, hence native code, without the GIL.  For ordinary tensors the
+// autograd function is native as well (Convolution below): as a Python one its backward pass took the GIL on the
+// engine's device thread while the caller waited for it, and the stage convolutions of ConvNeXt-T, forward and backward,
+// took 190 or 380 us of wall time from process to process for the same 186 us of kernels.
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
@@ -107,8 +109,11 @@ void check_activation(const Tensor &t, const char *name) {
     if (!t.is_cuda()) fail(std::string(name) + " must be a CUDA tensor");
     if (!t.is_contiguous()) fail(std::string(name) + " must be contiguous");
     if (dtype_code(t) < 0)
-        fail(std::string(name) + " has unsupported dtype " +
-             py::cast<std::string>(py::str(py::cast(t).attr("dtype"))));
+        {
+            py::gil_scoped_acquire gil;
+            fail(std::string(name) + " has unsupported dtype " +
+                 py::cast<std::string>(py::str(py::cast(t).attr("dtype"))));
+        }
     if (t.dim() != 4) fail(std::string(name) + " must be a 4-d tensor");
 }
 
@@ -167,7 +172,6 @@ Tensor fprop(const Tensor &x, const Tensor &w, const Tensor &taps, int64_t strid
     const Tensor w2 = rows_f32(w, d.c);
     const int64_t K = w2.numel() / std::max<int64_t>(d.c, 1);
     check_taps(taps, d.c, K);
-    py::gil_scoped_release nogil;
     const Place at(x);
     Tensor y = at::empty(shape_of(d.n, d.c, up(d.h, stride), up(d.w, stride), nhwc), x.options());
     check(lib.fprop(ptr(x), (const float *)ptr(w2), fptr(bias), ptr(taps), y.data_ptr(), as_int(d.n),
@@ -187,7 +191,6 @@ Tensor dgrad(const Tensor &dy, const Tensor &w, const Tensor &taps, int64_t H, i
     const Tensor w2 = rows_f32(w, d.c);
     const int64_t K = w2.numel() / std::max<int64_t>(d.c, 1);
     check_taps(taps, d.c, K);
-    py::gil_scoped_release nogil;
     const Place at(dy);
     Tensor dx = at::empty(shape_of(d.n, d.c, H, W, nhwc), dy.options());
     check(lib.dgrad(ptr(dy), (const float *)ptr(w2), ptr(taps), dx.data_ptr(), as_int(d.n), as_int(d.c),
@@ -207,7 +210,6 @@ std::tuple<Tensor, OptTensor> wgrad(const Tensor &dy, const Tensor &x, const Ten
     const auto want = shape_of(d.n, d.c, up(d.h, stride), up(d.w, stride), nhwc);
     if (dy.sizes() != at::IntArrayRef(want)) fail("dy extent does not match the input extent and stride");
     check_taps(taps, d.c, K);
-    py::gil_scoped_release nogil;
     const Place at(x);
     const int n = as_int(d.n), c = as_int(d.c), h = as_int(d.h), wd = as_int(d.w), k = as_int(K),
               s = as_int(stride), dt = dtype_code(x);
@@ -221,6 +223,74 @@ std::tuple<Tensor, OptTensor> wgrad(const Tensor &dy, const Tensor &x, const Ten
                     scratch.data_ptr(), nbytes, n, c, h, wd, k, s, dt, (int)layout, at.stream),
           "dwo_wgrad");
     return {dw, db};
+}
+
+// the same for callers that hold the GIL
+Tensor fprop_entry(const Tensor &x, const Tensor &w, const Tensor &taps, int64_t stride, const OptTensor &bias,
+                   int64_t layout) {
+    py::gil_scoped_release nogil;
+    return fprop(x, w, taps, stride, bias, layout);
+}
+Tensor dgrad_entry(const Tensor &dy, const Tensor &w, const Tensor &taps, int64_t H, int64_t W, int64_t stride,
+                   int64_t layout) {
+    py::gil_scoped_release nogil;
+    return dgrad(dy, w, taps, H, W, stride, layout);
+}
+std::tuple<Tensor, OptTensor> wgrad_entry(const Tensor &dy, const Tensor &x, const Tensor &taps, int64_t K,
+                                          int64_t stride, int64_t layout, bool with_bias) {
+    py::gil_scoped_release nogil;
+    return wgrad(dy, x, taps, K, stride, layout, with_bias);
+}
+
+// The operator as a node of autograd (the contract of models/dwoconv1d/dwoconv1d.py:18-69): gradients of x, w and bias, none
+// of theta.  w32 and bias32 are fp32 copies where the parameters are not dense fp32 themselves; resid is added to the weights.
+struct Convolution : torch::autograd::Function<Convolution> {
+    using Context = torch::autograd::AutogradContext;
+    using List = torch::autograd::variable_list;
+
+    static Tensor forward(Context *ctx, const Tensor &x_, const Tensor &w, const OptTensor &bias, const OptTensor &w32,
+                          const OptTensor &bias32, const OptTensor &resid, const Tensor &taps, int64_t stride,
+                          int64_t layout) {
+        ctx->set_materialize_grads(false);
+        const Tensor x = x_.contiguous();
+        Tensor weights = w32.has_value() ? *w32 : w;
+        if (resid.has_value()) weights = weights + resid->to(weights.options());
+        ctx->save_for_backward({x, weights, taps});
+        const bool has_bias = bias.has_value();
+        ctx->saved_data["p"] = std::vector<int64_t>{
+            stride, layout, w.size(-1), (int64_t)w.scalar_type(), has_bias ? (int64_t)bias->scalar_type() : -1};
+        return fprop(x, weights, taps, stride, bias32.has_value() ? bias32 : bias, layout);
+    }
+
+    static List backward(Context *ctx, const List &grads) {
+        List out(9);
+        if (!grads[0].defined()) return out;
+        const List saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &weights = saved[1], &taps = saved[2];
+        const std::vector<int64_t> p = ctx->saved_data["p"].toIntVector();
+        const int64_t stride = p[0], layout = p[1], K = p[2];
+        const auto w_type = (at::ScalarType)p[3];
+        const bool nhwc = layout & DWO_NHWC, has_bias = p[4] >= 0, need_db = has_bias && ctx->needs_input_grad(2);
+        Tensor dy = grads[0].contiguous();
+        if (dy.scalar_type() != x.scalar_type()) dy = dy.to(x.scalar_type());
+        if (ctx->needs_input_grad(0))
+            out[0] = dgrad(dy, weights, taps, x.size(nhwc ? 1 : 2), x.size(nhwc ? 2 : 3), stride, layout);
+        if (ctx->needs_input_grad(1)) {
+            auto [dw, db] = wgrad(dy, x, taps, K, stride, layout, need_db);
+            out[1] = dw.scalar_type() == w_type ? dw : dw.to(w_type);
+            if (need_db) out[2] = db->to((at::ScalarType)p[4]);
+        } else if (need_db) {
+            out[2] = dy.sum(nhwc ? at::IntArrayRef{0, 1, 2} : at::IntArrayRef{0, 2, 3}, false, at::kFloat)
+                         .to((at::ScalarType)p[4]);
+        }
+        return out;
+    }
+};
+
+Tensor convolution(const Tensor &x, const Tensor &w, const OptTensor &bias, const OptTensor &w32,
+                   const OptTensor &bias32, const OptTensor &resid, const Tensor &taps, int64_t stride, int64_t layout) {
+    py::gil_scoped_release nogil;
+    return Convolution::apply(x, w, bias, w32, bias32, resid, taps, stride, layout);
 }
 
 void check_glue(const Tensor &t, const char *name) {
@@ -540,9 +610,10 @@ Tensor linear_planes(const Tensor &x_, const Tensor &w_, const OptTensor &b, con
 
 PYBIND11_MODULE(_host, m) {
     m.def("bind", &bind_library);
-    m.def("fprop", &fprop);
-    m.def("dgrad", &dgrad);
-    m.def("wgrad", &wgrad);
+    m.def("convolution", &convolution);
+    m.def("fprop", &fprop_entry);
+    m.def("dgrad", &dgrad_entry);
+    m.def("wgrad", &wgrad_entry);
     m.def("pointwise_wgrad", &pointwise_wgrad);
     m.def("layernorm_nhwc", &layernorm_nhwc);
     m.def("nchw_layernorm_nhwc", &nchw_layernorm_nhwc);

@@ -22,6 +22,7 @@ import weakref
 
 import numpy as np
 import torch
+import torch.autograd.forward_ad as fwd
 import torch.nn as nn
 
 from . import _lib
@@ -29,6 +30,23 @@ from . import _lib
 __all__ = ["DepthwiseOrientedConv1d"]
 
 _DTYPES = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
+
+
+def ordinary(*tensors):
+    """True for ordinary tensors (None for an absent one) in ordinary execution: no compilation, tracing, torch.func
+    transform, dispatch mode, forward-mode derivative or tensor subclass, all of which an autograd function around native
+    code would hide a layer from."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack()):
+        return False
+    dual = fwd._current_level >= 0
+    for t in tensors:
+        if t is not None and (type(t) not in _PLAIN or (dual and fwd.unpack_dual(t).tangent is not None)):
+            return False
+    return True
+
+
+_PLAIN = (torch.Tensor, nn.Parameter)
 
 
 def _ptr(t):
@@ -315,6 +333,25 @@ def oriented_dwconv1d_get_module_from_params(ftype, kernel_size, stride, pad, Sb
     return kt
 
 
+def _is_f32(p):
+    return p.dtype == torch.float32 and p.is_contiguous()
+
+
+def _native_covers(x, w, theta, bias, resid, module, nhwc):
+    """True for the calls that the native autograd node takes: ordinary tensors on one GPU whose sizes and types pass every check
+    of the Python function (which reports the others)."""
+    if not (x.is_cuda and x.dtype in _DTYPES and x.dim() == 4 and type(module) is KernelTuple
+            and w.shape[-1] == module.kernel_size and x.device == w.device and w.is_floating_point()
+            and (bias is None or bias.device == x.device) and (resid is None or resid.device == x.device)
+            and ordinary(x, w, theta, bias, resid)):
+        return False
+    if theta.requires_grad and torch.is_grad_enabled() and not (
+            x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)):
+        return False  # (a graph for theta alone, which never receives a gradient)
+    _, C, H, W = _dims(x, nhwc)
+    return C == w.shape[0] and (module.arbitrary_size or (H % module.stride == 0 and W % module.stride == 0))
+
+
 class DepthwiseOrientedConv1d(nn.Conv2d):
     """Drop-in for models/dwoconv1d/dwoconv1d.py:92-198.
 
@@ -395,13 +432,22 @@ class DepthwiseOrientedConv1d(nn.Conv2d):
         """Arbitrary H, W (reference: dwoconv1d.py:154-187): no padding to a power of two, no
         crop and no permuted copies; the kernels produce ceil(H/stride) x ceil(W/stride)
         outputs in the tensor's own layout, the values that path returns."""
-        return _DepthwiseOrientedConv1d.apply(
-            x, self.weight, self.theta, self.bias, self.module_fp32_large, self.nhwc, self.resid
-        )
+        return self._apply_operator(x, self.module_fp32_large)
 
     def forward(self, x):
         if self.arbitrary_size:  # the reference rebinds forward to forward_safe (:148-149)
             return self.forward_safe(x)
-        return _DepthwiseOrientedConv1d.apply(
-            x, self.weight, self.theta, self.bias, self.module_fp32, self.nhwc, self.resid
-        )
+        return self._apply_operator(x, self.module_fp32)
+
+    def _apply_operator(self, x, module):
+        w, theta, bias, resid = self.weight, self.theta, self.bias, self.resid
+        nhwc = bool(self.nhwc)
+        if _native_covers(x, w, theta, bias, resid, module, nhwc):
+            # the native node: the same checks, kernels and gradients without Python in the backward pass
+            C, K = w.shape[0], w.shape[-1]
+            taps, layouts = module.taps.lookup(theta, C, K, x.device)
+            return _lib.host(x.get_device()).convolution(
+                x, w, bias, None if _is_f32(w) else f32_copy(w),
+                None if bias is None or _is_f32(bias) else f32_copy(bias), resid, taps, module.stride,
+                layouts[x.element_size()] if nhwc else _lib.NCHW)
+        return _DepthwiseOrientedConv1d.apply(x, w, theta, bias, module, self.nhwc, resid)

@@ -7,11 +7,11 @@ transforms, tracing, subclasses or hooks: those compose the same values from PyT
 import ctypes
 
 import torch
-import torch.autograd.forward_ad as fwd
 import torch.nn.functional as F
 import torch.nn.modules.module as _mod
 
 from . import _lib
+from .dwoconv1d import ordinary
 
 _DTYPES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 MAX_C_ROWS, MAX_C_TILE = 2048, 1536
@@ -73,7 +73,7 @@ def _layer16(x, w, b):
     return (not torch.is_grad_enabled() and x.is_cuda and x.numel() > 0 and x.dtype in (torch.bfloat16, torch.float16)
             and w.dtype == x.dtype and w.device == x.device and w.shape[1] == x.shape[-1]
             and (b is None or (b.dtype == x.dtype and b.device == x.device))
-            and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and max(w.shape) <= 65536 and _eager(x, w, b)
+            and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and max(w.shape) <= 65536 and ordinary(x, w, b)
             and not torch.is_autocast_enabled(x.device.type) and x.numel() // w.shape[1] < 1 << 31)
 
 
@@ -145,17 +145,6 @@ class _PointwiseLinear(torch.autograd.Function):
         return dx, dw, db
 
 
-def _eager(*tensors):
-    """True for ordinary tensors in ordinary execution: no compilation, tracing, torch.func transform,
-    dispatch mode, forward-mode derivative or tensor subclass, all of which an autograd function around native
-    code would hide the layer from."""
-    if (torch.compiler.is_compiling() or torch.jit.is_tracing()
-            or torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack()):
-        return False
-    return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter)
-                             and fwd.unpack_dual(t).tangent is None) for t in tensors)
-
-
 def pointwise_linear(x, linear):
     """``linear(x)`` of an ``nn.Linear`` with at most four inputs; where its parameters are being
     trained on a GPU, with the parameter gradients of ``dwo_pointwise_wgrad``."""
@@ -163,7 +152,7 @@ def pointwise_linear(x, linear):
     dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else x.dtype
     # (what autocast converts is saved converted, without its history: an input that is differentiated
     # itself stays with PyTorch then, whose gradients of gradients reach it and the weights)
-    if (torch.is_grad_enabled() and _eager(x, w, b)
+    if (torch.is_grad_enabled() and ordinary(x, w, b)
             and w.requires_grad and x.is_cuda and w.device == x.device and x.numel() > 0
             and (x.dtype == w.dtype == dtype or not x.requires_grad) and dtype in _DTYPES
             and all(t is None or t.dtype in _DTYPES for t in (x, w, b))
@@ -186,7 +175,7 @@ def _recording(*tensors):
     """True where the training kernels may stand for a composition of PyTorch ops on these tensors (None for
     an absent one): gradients are being recorded, on one GPU, for ordinary non-empty tensors of a known type."""
     x = tensors[0]
-    return (torch.is_grad_enabled() and x.is_cuda and x.numel() > 0 and _eager(*tensors)
+    return (torch.is_grad_enabled() and x.is_cuda and x.numel() > 0 and ordinary(*tensors)
             and all(t is None or (t.device == x.device and t.dtype in _DTYPES) for t in tensors))
 
 
@@ -435,7 +424,7 @@ def downsample(x, norm, conv):
             return None
         p = _TileNorm.apply(x, norm.weight, norm.bias, norm.eps, dtype, True)
         return planes(_Linear.apply(p, rows, b))
-    if norm.weight.device != x.device or not _layer16(x.permute(0, 2, 3, 1), w[:, :, 0, 0], b) or not _eager(w):
+    if norm.weight.device != x.device or not _layer16(x.permute(0, 2, 3, 1), w[:, :, 0, 0], b) or not ordinary(w):
         return None
     host = _lib.host(x.get_device())
     p = host.ln_tile(x, _f32(norm.weight), _f32(norm.bias), norm.eps, True, x.dtype, False)[0]

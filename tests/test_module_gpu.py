@@ -10,6 +10,7 @@ from parity_util import assert_close, grouped_theta, host
 pytestmark = pytest.mark.gpu
 
 from oriented1d_amd import DepthwiseOrientedConv1d  # noqa: E402
+from oriented1d_amd import dwoconv1d as dwm  # noqa: E402
 
 
 def _mk(C, K, stride=1, nhwc=False, resid=False, bias=True, offset=0.0, arbitrary=False):
@@ -223,3 +224,66 @@ def test_tap_table_of_another_size_is_rejected():
     w = torch.randn(16, 1, 1, 31, device="cuda")
     with pytest.raises(RuntimeError, match="tap table does not match"):
         op.fprop(x, w, taps)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("nhwc,resid,stride,bias", [(False, False, 1, True), (True, True, 2, True), (True, False, 1, False)])
+def test_native_node_equals_the_python_function(nhwc, resid, stride, bias, dtype):
+    """The module's native autograd node against ``_DepthwiseOrientedConv1d.apply`` on the same tensors: outputs and gradients are
+    the same bits, for fp32 and 16-bit parameters, a gradient of another type and layout, and each subset of inputs."""
+    torch.manual_seed(2)
+    m = DepthwiseOrientedConv1d(24, 24, 15, groups=24, stride=stride, padding=7, bias=bias, nhwc=nhwc, resid=resid,
+                                angle=[i * math.pi / 24 for i in range(24)], arbitrary_size=True).cuda()
+    m = m.to(dtype)
+    shape = (3, 13, 18, 24) if nhwc else (3, 24, 13, 18)
+    x = torch.randn(*shape, device="cuda").to(dtype)
+    for needs in ((1, 1, 1), (1, 0, 0), (0, 1, 0), (0, 0, 1)):
+        if needs == (0, 0, 1) and not bias:
+            continue
+        outs = []
+        for native in (True, False):
+            xi = x.clone().requires_grad_(bool(needs[0]))
+            m.weight.requires_grad_(bool(needs[1]))
+            if bias:
+                m.bias.requires_grad_(bool(needs[2]))
+            y = m(xi) if native else dwm._DepthwiseOrientedConv1d.apply(
+                xi, m.weight, m.theta, m.bias, m.module_fp32_large, nhwc, m.resid)
+            assert ("Convolution" in type(y.grad_fn).__name__ or "CppNode" in type(y.grad_fn).__name__
+                    or "CppFunction" in type(y.grad_fn).__name__) == native
+            leaves = [t for t, n in zip((xi, m.weight, m.bias), needs) if n and t is not None]
+            torch.manual_seed(4)
+            g = torch.randn(tuple(reversed(y.shape)), device="cuda").to(y.dtype).permute(3, 2, 1, 0)
+            outs.append([y.detach()] + list(torch.autograd.grad(y, leaves, g)))
+        assert len(outs[0]) == len(outs[1])
+        for a, b in zip(*outs):
+            assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+def test_native_node_keeps_autograd_rules():
+    torch.manual_seed(3)
+    m = DepthwiseOrientedConv1d(16, 16, 7, groups=16, padding=3, angle=0.3, arbitrary_size=True).cuda()
+    x = torch.randn(2, 16, 9, 11, device="cuda", requires_grad=True)
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t.shape) or t.cpu(), lambda t: t.cuda()):
+        y = m(x)
+    y.sum().backward()
+    assert x.shape in seen and x.grad is not None  # (saved tensors pass through the hooks)
+    y = m(x)
+    y.sum().backward()
+    with pytest.raises(RuntimeError, match="second time"):
+        y.sum().backward()
+    y = m(x)
+    with torch.no_grad():
+        m.weight.mul_(2.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.sum().backward()
+    for p in (m.weight, m.bias):
+        p.requires_grad_(False)
+    y = m(x.detach())
+    assert y.requires_grad  # (theta alone: a graph without a gradient, as before)
+    y.sum().backward()
+    assert m.theta.grad is None
+    with torch.inference_mode():
+        assert torch.equal(m(x), y)
+    with pytest.raises(RuntimeError, match="channels"):
+        m(torch.randn(2, 8, 9, 11, device="cuda"))
