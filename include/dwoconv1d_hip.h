@@ -232,13 +232,15 @@ int dwo_pointwise_wgrad(const void *dy, const void *x, float *dw, float *db, voi
  * backward pass takes (forward only: may be null); dgamma, dbeta and dscale are written as grad_dtype and may be null;
  * scratch holds at least dwo_block_scratch_bytes(C) bytes.
  *
- * dwo_ln_rows:     out[r,:] = act(LN(x[r,:])) for rows of C channels (act = exact GELU when gelu != 0);
+ * dwo_ln_rows:     out[r,:] = act(LN(x[r,:])) for rows of C channels (act = exact GELU where gelu & 1; where gelu & 2 what it
+ *                  takes, and its gradient in the backward pass, are rounded to out_dtype as separate passes round them);
  *                  _backward also takes dout [rows,C] (out_dtype) and writes dx (in_dtype).
  * dwo_ln_tile:     x [N,C,H,W] -> out [N,H,W,C] = LN over C; _backward: dout [N,H,W,C] -> dx [N,C,H,W].
  * dwo_ln_patch:    x [N,C,H,W] -> LN over C -> out [N,H/2,W/2,4C], patches [C][2][2] (H, W at least 2; an odd last row or
  *                  column is in no patch); stats [N,H/2,W/2,2,2]; _backward writes dx of the pixels in patches.
  * dwo_block_tail:  out [N,C,H,W] = res + scale[c] * y for y [N,H,W,C] of y_dtype, out of dtype (y's type or DWO_F32) and
- *                  res of res_dtype (either); scale and res may be null.  _backward: dout [N,C,H,W] (dtype) ->
+ *                  res of res_dtype (either); scale and res may be null; where rounded != 0 scale[c] * y is rounded to y_dtype
+ *                  before the sum.  _backward: dout [N,C,H,W] (dtype) ->
  *                  dy [N,H,W,C] (y_dtype) and, where y is not null, dscale.  (The gradient of res is dout.)
  */
 size_t dwo_block_scratch_bytes(int C);
@@ -258,7 +260,7 @@ int dwo_ln_patch_backward(const void *dout, const void *x, const float *stats, c
                           void *dgamma, void *dbeta, void *scratch, size_t scratch_bytes, int N, int C, int H, int W,
                           int in_dtype, int out_dtype, int grad_dtype, void *stream);
 int dwo_block_tail(const void *y, const float *scale, const void *res, void *out, int N, int C, int H, int W,
-                   int y_dtype, int res_dtype, int dtype, void *stream);
+                   int rounded, int y_dtype, int res_dtype, int dtype, void *stream);
 int dwo_block_tail_backward(const void *dout, const void *y, const float *scale, void *dy, void *dscale, void *scratch,
                             size_t scratch_bytes, int N, int C, int H, int W, int y_dtype, int dtype, int grad_dtype,
                             void *stream);

@@ -41,7 +41,7 @@ SIGNATURES = {
     "dwo_ln_tile_backward": (_i, [_vp] * 8 + [_sz] + [_i] * 7 + [_vp]),
     "dwo_ln_patch": (_i, [_vp] * 5 + [_i] * 4 + [ctypes.c_float] + [_i] * 2 + [_vp]),
     "dwo_ln_patch_backward": (_i, [_vp] * 8 + [_sz] + [_i] * 7 + [_vp]),
-    "dwo_block_tail": (_i, [_vp] * 4 + [_i] * 7 + [_vp]),
+    "dwo_block_tail": (_i, [_vp] * 4 + [_i] * 8 + [_vp]),
     "dwo_block_tail_backward": (_i, [_vp] * 6 + [_sz] + [_i] * 7 + [_vp]),
     "dwo_linear_wgrad_scratch_bytes": (_sz, [_sz, _i, _i]),
     "dwo_linear_rows": (_i, [_vp] * 4 + [_sz] + [_i] * 4 + [_vp]),

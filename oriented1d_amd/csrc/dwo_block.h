@@ -89,6 +89,11 @@ __device__ __forceinline__ float group_total(float v) {
     return v;
 }
 
+// flags of the row kernels
+enum { ROWS_GELU = 1, ROWS_ROUNDED = 2 };  // GELU; what it takes (and its gradient) rounded to the output's type
+template <typename T>
+__device__ __forceinline__ float rounded(float v) { return to_float(from_float<T>(v)); }
+
 __device__ __forceinline__ float blk_gelu(float u) { return 0.5f * u * (1.f + erff(u * 0.70710678118654752f)); }
 __device__ __forceinline__ float blk_gelu_slope(float u) {
     return 0.5f * (1.f + erff(u * 0.70710678118654752f)) + u * 0.39894228040143268f * expf(-0.5f * u * u);
@@ -199,7 +204,8 @@ __global__ __launch_bounds__(kBlkThreads) void ln_rows_kernel(const TI *__restri
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     o[i] = __builtin_fmaf(v[k][i] * rstd, gm[k][i], bt[k][i]);
-                    if (gelu) o[i] = sizeof(TO) == 2 ? gelu_rounded(o[i]) : blk_gelu(o[i]);
+                    if (gelu & ROWS_ROUNDED) o[i] = rounded<TO>(o[i]);
+                    if (gelu & ROWS_GELU) o[i] = sizeof(TO) == 2 ? gelu_rounded(o[i]) : blk_gelu(o[i]);
                 }
                 store8(out + r * C + ln.chan(k), o);
             }
@@ -237,7 +243,12 @@ __global__ __launch_bounds__(kBlkThreads) void ln_rows_backward_kernel(
             for (int i = 0; i < 8; i++) {
                 if (!ok) h[k][i] = st.x, g[k][i] = 0.f;
                 h[k][i] = (h[k][i] - st.x) * st.y;
-                if (gelu && ok) g[k][i] *= blk_gelu_slope(__builtin_fmaf(h[k][i], gm[k][i], bt[k][i]));
+                if ((gelu & ROWS_GELU) && ok) {
+                    float u = __builtin_fmaf(h[k][i], gm[k][i], bt[k][i]);
+                    if (gelu & ROWS_ROUNDED) u = rounded<TO>(u);
+                    g[k][i] *= blk_gelu_slope(u);
+                    if (gelu & ROWS_ROUNDED) g[k][i] = rounded<TO>(g[k][i]);
+                }
                 dg[k][i] = __builtin_fmaf(g[k][i], h[k][i], dg[k][i]);
                 db[k][i] += g[k][i];
                 g[k][i] *= gm[k][i];
@@ -603,11 +614,11 @@ struct TailTiles {
     int C, HW, per, ctiles, units;  // pixel tiles per image, channel tiles, (image, pixel tile) pairs
 };
 
-// (TS: the type of res; without res out is y in planes)
+// (TS: the type of res; without res out is y in planes; round: scale * y is rounded to y's type, as a product by itself is)
 template <typename TY, typename TS, typename TR, int VEC>
 __global__ __launch_bounds__(kBlkThreads) void tail_kernel(const TY *__restrict__ y, const float *__restrict__ scale,
                                                            const TS *__restrict__ res, TR *__restrict__ out,
-                                                           TailTiles t) {
+                                                           TailTiles t, int round) {
     __shared__ float tile[kTailC * kTailPitch];
     const int u = blockIdx.x / t.ctiles, c0 = blockIdx.x % t.ctiles * kTailC;
     const int n = u / t.per, p0 = u % t.per * kTailP, np = min(kTailP, t.HW - p0), nc = min(kTailC, t.C - c0);
@@ -636,7 +647,8 @@ __global__ __launch_bounds__(kBlkThreads) void tail_kernel(const TY *__restrict_
         const int p = threadIdx.x / 8 + 32 * k;
         if (c < nc && p < np)
 #pragma unroll
-            for (int i = 0; i < 8; i++) tile[(c + i) * kTailPitch + p] = v[k][i] * sc[i];
+            for (int i = 0; i < 8; i++)
+                tile[(c + i) * kTailPitch + p] = round ? rounded<TY>(v[k][i] * sc[i]) : v[k][i] * sc[i];
     }
     __syncthreads();
 #pragma unroll

@@ -249,7 +249,7 @@ int dwo_ln_patch_backward(const void *dout, const void *x, const float *stats, c
 }
 
 int dwo_block_tail(const void *y, const float *scale, const void *res, void *out, int N, int C, int H, int W,
-                   int y_dtype, int res_dtype, int dtype, void *stream) {
+                   int rounded, int y_dtype, int res_dtype, int dtype, void *stream) {
     if (!y || !out) return DWO_ERR_NULL_POINTER;
     if (N < 1 || H < 1 || W < 1 || C < 8 || C % 8 != 0 || (double)N * C * H * W >= 2147483648.0 || !aligned16(y) ||
         !aligned16(res) || !aligned16(out))
@@ -265,10 +265,10 @@ int dwo_block_tail(const void *y, const float *scale, const void *res, void *out
             using TS = typename decltype(ts)::type;
             if (t.HW % 4 == 0)
                 tail_kernel<TY, TS, TR, 4><<<grid, block, 0, (hipStream_t)stream>>>((const TY *)y, scale, (const TS *)res,
-                                                                                    (TR *)out, t);
+                                                                                    (TR *)out, t, rounded);
             else
                 tail_kernel<TY, TS, TR, 1><<<grid, block, 0, (hipStream_t)stream>>>((const TY *)y, scale, (const TS *)res,
-                                                                                    (TR *)out, t);
+                                                                                    (TR *)out, t, rounded);
             return status();
         };
         if (res == nullptr || res_dtype == dtype) return launch(Type<TR>{});

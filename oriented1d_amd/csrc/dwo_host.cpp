@@ -414,7 +414,7 @@ std::tuple<Tensor, OptTensor> linear_wgrad(const Tensor &dy_, const Tensor &x_, 
 }
 
 // LayerNorm (+ GELU) over the last dimension; (out, stats)
-std::tuple<Tensor, OptTensor> ln_rows(const Tensor &x_, const Tensor &g, const Tensor &b, double eps, bool gelu,
+std::tuple<Tensor, OptTensor> ln_rows(const Tensor &x_, const Tensor &g, const Tensor &b, double eps, int64_t gelu,
                                       at::ScalarType out_dtype, bool with_stats) {
     check_glue(x_, "x");
     py::gil_scoped_release nogil;
@@ -425,13 +425,13 @@ std::tuple<Tensor, OptTensor> ln_rows(const Tensor &x_, const Tensor &g, const T
     OptTensor stats;
     if (with_stats) stats = at::empty({rows, 2}, x.options().dtype(at::kFloat));
     check(lib.ln_rows(ptr(x), (const float *)ptr(g), (const float *)ptr(b), out.data_ptr(),
-                      stats.has_value() ? (float *)stats->data_ptr() : nullptr, (size_t)rows, as_int(C), (float)eps, gelu, dtype_code(x), dtype_code(out_dtype), at.stream),
+                      stats.has_value() ? (float *)stats->data_ptr() : nullptr, (size_t)rows, as_int(C), (float)eps, (int)gelu, dtype_code(x), dtype_code(out_dtype), at.stream),
           "dwo_ln_rows");
     return {out, stats};
 }
 
 std::tuple<Tensor, Tensor, Tensor> ln_rows_backward(const Tensor &dout_, const Tensor &x_, const Tensor &stats,
-                                                    const Tensor &g, const Tensor &b, bool gelu,
+                                                    const Tensor &g, const Tensor &b, int64_t gelu,
                                                     at::ScalarType grad_dtype) {
     check_glue(dout_, "dout");
     check_glue(x_, "x");
@@ -447,7 +447,7 @@ std::tuple<Tensor, Tensor, Tensor> ln_rows_backward(const Tensor &dout_, const T
     Tensor dg = at::empty({C}, x.options().dtype(grad_dtype)), db = at::empty({C}, dg.options());
     check(lib.ln_rows_backward(ptr(dout), ptr(x), (const float *)ptr(stats), (const float *)ptr(g),
                                (const float *)ptr(b), dx.data_ptr(), dg.data_ptr(), db.data_ptr(), scratch.data_ptr(),
-                               nbytes, (size_t)rows, as_int(C), gelu, dtype_code(x), dtype_code(dout),
+                               nbytes, (size_t)rows, as_int(C), (int)gelu, dtype_code(x), dtype_code(dout),
                                dtype_code(grad_dtype), at.stream),
           "dwo_ln_rows_backward");
     return {dx, dg, db};
@@ -501,7 +501,8 @@ std::tuple<Tensor, Tensor, Tensor> ln_tile_backward(const Tensor &dout_, const T
 }
 
 // res + scale * y as planes of out_dtype: y [N,H,W,C], res [N,C,H,W]
-Tensor block_tail(const Tensor &y_, const OptTensor &scale, const OptTensor &res_, at::ScalarType out_dtype) {
+Tensor block_tail(const Tensor &y_, const OptTensor &scale, const OptTensor &res_, at::ScalarType out_dtype,
+                  bool rounded) {
     check_glue(y_, "y");
     if (y_.dim() != 4) throw py::value_error("y must be a 4-d tensor");
     const Dims d(y_, true);
@@ -517,7 +518,7 @@ Tensor block_tail(const Tensor &y_, const OptTensor &scale, const OptTensor &res
     Tensor res, out = at::empty(shape, y.options().dtype(out_dtype));
     if (res_.has_value()) res = dense(*res_);
     check(lib.block_tail(ptr(y), fptr(scale), res.defined() ? ptr(res) : nullptr, out.data_ptr(), as_int(d.n),
-                         as_int(d.c), as_int(d.h), as_int(d.w), dtype_code(y),
+                         as_int(d.c), as_int(d.h), as_int(d.w), rounded, dtype_code(y),
                          res.defined() ? dtype_code(res) : dtype_code(out_dtype), dtype_code(out_dtype), at.stream),
           "dwo_block_tail");
     return out;

@@ -240,7 +240,7 @@ class _TileNorm(torch.autograd.Function):
 
 
 class _RowNorm(torch.autograd.Function):
-    """LayerNorm over the last dimension (+ exact GELU)."""
+    """LayerNorm over the last dimension (gelu & 1: + exact GELU, gelu & 2: of the value rounded to the output's type)."""
 
     @staticmethod
     def forward(ctx, x, w, b, eps, gelu, dtype):
@@ -259,6 +259,8 @@ class _RowNorm(torch.autograd.Function):
         if torch.is_grad_enabled():
             def value(x, w, b):
                 y = F.layer_norm(x.float(), w.shape, w.float(), b.float(), ctx.eps)
+                if ctx.gelu & 2:
+                    y = y.to(ctx.dtype).float()
                 return (F.gelu(y) if ctx.gelu else y).to(ctx.dtype)
             return (*_second_order(value, (x, w, b), dout), None, None, None)
         dx, dw, db = _lib.host(x.get_device()).ln_rows_backward(dout, x, stats, _f32(w), _f32(b), ctx.gelu, w.dtype)
@@ -266,14 +268,14 @@ class _RowNorm(torch.autograd.Function):
 
 
 class _BlockTail(torch.autograd.Function):
-    """``x + (gamma * y).permute(0, 3, 1, 2)`` in ``dtype`` for y [N,H,W,C] and x [N,C,H,W]; without gamma and x the
-    permutation alone."""
+    """``x + (gamma * y).permute(0, 3, 1, 2)`` in ``dtype`` for y [N,H,W,C] and x [N,C,H,W] (``rounded``: the product is a
+    tensor of y's type by itself); without gamma and x the permutation alone."""
 
     @staticmethod
-    def forward(ctx, y, gamma, x, dtype):
+    def forward(ctx, y, gamma, x, dtype, rounded):
         ctx.set_materialize_grads(False)
         y = y.contiguous()
-        out = _lib.host(y.get_device()).block_tail(y, None if gamma is None else _f32(gamma), x, dtype)
+        out = _lib.host(y.get_device()).block_tail(y, None if gamma is None else _f32(gamma), x, dtype, rounded)
         ctx.save_for_backward(*(() if gamma is None else (y, gamma)))
         ctx.types = y.dtype, None if x is None else x.dtype
         return out
@@ -281,22 +283,22 @@ class _BlockTail(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         if dout is None:
-            return None, None, None, None
+            return None, None, None, None, None
         dtype, x_dtype = ctx.types
         dx = dout.to(x_dtype) if ctx.needs_input_grad[2] else None
         if not (ctx.needs_input_grad[0] or ctx.needs_input_grad[1]):
-            return None, None, dx, None
+            return None, None, dx, None, None
         y, gamma = ctx.saved_tensors if ctx.saved_tensors else (None, None)
         if torch.is_grad_enabled():
             if gamma is None:
-                return dout.permute(0, 2, 3, 1).to(dtype), None, dx, None
+                return dout.permute(0, 2, 3, 1).to(dtype), None, dx, None, None
 
             def value(y, gamma):
                 return (gamma * y).permute(0, 3, 1, 2).to(dout.dtype)
-            return (*_second_order(value, (y, gamma), dout), dx, None)
+            return (*_second_order(value, (y, gamma), dout), dx, None, None)
         scale, grad = (None, torch.float32) if gamma is None else (_f32(gamma), gamma.dtype)
         dy, dg = _lib.host(dout.get_device()).block_tail_backward(dout, y, scale, dtype, grad)
-        return dy, dg, dx, None
+        return dy, dg, dx, None, None
 
 
 class _Linear(torch.autograd.Function):
@@ -376,7 +378,9 @@ def row_norm(x, norm, gelu=False, consumer=None):
             and x.numel() // max(x.shape[-1], 1) < 1 << 31):
         return None
     dtype = _norm_type(x, x.shape[-1], norm, consumer)
-    return None if dtype is None else _RowNorm.apply(x, norm.weight, norm.bias, norm.eps, gelu, dtype)
+    # (without autocast a 16-bit LayerNorm's output is a 16-bit tensor by itself)
+    mode = 0 if not gelu else 1 if _autocast(x) is not None or dtype == torch.float32 else 3
+    return None if dtype is None else _RowNorm.apply(x, norm.weight, norm.bias, norm.eps, mode, dtype)
 
 
 def _tail_covers(y):
@@ -391,13 +395,14 @@ def block_tail(y, gamma, x):
     dtype = torch.promote_types(torch.promote_types(gamma.dtype, y.dtype), x.dtype)
     if dtype not in (y.dtype, torch.float32) or x.dtype not in (y.dtype, dtype):
         return None
-    return _BlockTail.apply(y, gamma, x, dtype)
+    product = torch.promote_types(gamma.dtype, y.dtype)
+    return _BlockTail.apply(y, gamma, x, dtype, product == y.dtype != torch.float32)
 
 
 def planes(y):
     """``y.permute(0, 3, 1, 2).contiguous()``, recorded by autograd where the kernels cover it."""
     if _recording(y) and _tail_covers(y):
-        return _BlockTail.apply(y, None, None, y.dtype)
+        return _BlockTail.apply(y, None, None, y.dtype, False)
     return y.permute(0, 3, 1, 2).contiguous()
 
 

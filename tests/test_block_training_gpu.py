@@ -67,7 +67,7 @@ def test_row_norm(shape, gelu, types):
     def reference(x, w, b):
         y = F.layer_norm(x, (C,), w, b, 1e-6)
         return F.gelu(y) if gelu else y
-    run_norm(x, w, b, dout, lambda x, w, b: fused._RowNorm.apply(x, w, b, 1e-6, gelu, tout), reference,
+    run_norm(x, w, b, dout, lambda x, w, b: fused._RowNorm.apply(x, w, b, 1e-6, int(gelu), tout), reference,
              TOL[tout], TOL[tin])
 
 
@@ -80,7 +80,7 @@ def test_block_tail(N, C, H, W, ty, tr):
     g = (torch.randn(C, device="cuda") * 0.5).requires_grad_(True)
     x = torch.randn(N, C, H, W, device="cuda").to(tr).requires_grad_(True)
     dout = torch.randn(N, C, H, W, device="cuda").to(tr)
-    out = fused._BlockTail.apply(y, g, x, tr)
+    out = fused._BlockTail.apply(y, g, x, tr, False)
     got = torch.autograd.grad(out, (y, g, x), dout)
     leaves = [t.detach().double().requires_grad_(True) for t in (y, g, x)]
     ref = leaves[2] + (leaves[1] * leaves[0]).permute(0, 3, 1, 2)
@@ -205,6 +205,25 @@ def test_linear_covers_batches_views_and_second_order():
     close(hw, rw, 3e-2, "second order w")
 
 
+def test_16_bit_passes_round_where_separate_passes_do():
+    """Without autocast every pass of the composition returns a 16-bit tensor: the fused passes round at the same places, so
+    that they differ from it only where a sum's last bit decides a rounding."""
+    torch.manual_seed(8)
+    norm = nn.LayerNorm(64, eps=1e-6).cuda().to(BF16)
+    with torch.no_grad():
+        norm.weight.add_(torch.randn_like(norm.weight) * 0.3)
+    x = torch.randn(4, 20, 20, 64, device="cuda").to(BF16).requires_grad_(True)
+    gamma = torch.randn(64, device="cuda").to(BF16)
+    planes = torch.randn(4, 64, 20, 20, device="cuda").to(BF16)
+    for native, composed in ((lambda: fused.row_norm(x, norm, gelu=True), lambda: F.gelu(norm(x))),
+                             (lambda: fused.block_tail(x, gamma, planes),
+                              lambda: planes + (gamma * x).permute(0, 3, 1, 2).contiguous())):
+        y, z = native(), composed()
+        d = torch.randn_like(y)
+        for a, b in zip((y, *torch.autograd.grad(y, x, d)), (z, *torch.autograd.grad(z, x, d))):
+            assert (a != b).float().mean() < 5e-3
+
+
 @pytest.mark.parametrize("which", ["tile", "rows", "tail"])
 def test_second_order_of_the_passes(which):
     torch.manual_seed(1)
@@ -215,9 +234,9 @@ def test_second_order_of_the_passes(which):
     native, reference = {
         "tile": (lambda: fused._TileNorm.apply(a, w, b, 1e-6, F32),
                  lambda: F.layer_norm(a.permute(0, 2, 3, 1), (16,), w, b, 1e-6)),
-        "rows": (lambda: fused._RowNorm.apply(nhwc, w, b, 1e-6, True, F32),
+        "rows": (lambda: fused._RowNorm.apply(nhwc, w, b, 1e-6, 1, F32),
                  lambda: F.gelu(F.layer_norm(nhwc, (16,), w, b, 1e-6))),
-        "tail": (lambda: fused._BlockTail.apply(nhwc, w, a, F32),
+        "tail": (lambda: fused._BlockTail.apply(nhwc, w, a, F32, False),
                  lambda: a + (w * nhwc).permute(0, 3, 1, 2))}[which]
     res = []
     for f in (native, reference):
