@@ -221,6 +221,10 @@ int dwo_nhwc_scale_add_nchw(const void *y, const float *scale, const void *res, 
  * dwo_pointwise_wgrad_scratch_bytes(Cin, C) bytes.
  */
 size_t dwo_pointwise_wgrad_scratch_bytes(int Cin, int C);
+/* The layer itself: y[p,c] = b[c] + sum_k x[p,k] * w[c,k] (b may be null), all of one 16-bit type, summed in fp32; y is
+ * 16-byte aligned, C a multiple of 64. */
+int dwo_pointwise_forward(const void *x, const void *w, const void *b, void *y, size_t rows, int Cin, int C, int dtype,
+                          void *stream);
 int dwo_pointwise_wgrad(const void *dy, const void *x, float *dw, float *db, void *scratch, size_t scratch_bytes,
                         size_t rows, int Cin, int C, int dtype, void *stream);
 

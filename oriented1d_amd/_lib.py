@@ -34,6 +34,7 @@ SIGNATURES = {
     "dwo_nhwc_scale_add_nchw": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "dwo_pointwise_wgrad_scratch_bytes": (_sz, [_i, _i]),
     "dwo_pointwise_wgrad": (_i, [_vp] * 5 + [_sz, _sz] + [_i] * 3 + [_vp]),
+    "dwo_pointwise_forward": (_i, [_vp] * 4 + [_sz] + [_i] * 3 + [_vp]),
     "dwo_block_scratch_bytes": (_sz, [_i]),
     "dwo_ln_rows": (_i, [_vp] * 5 + [_sz, _i, ctypes.c_float] + [_i] * 3 + [_vp]),
     "dwo_ln_rows_backward": (_i, [_vp] * 9 + [_sz, _sz] + [_i] * 5 + [_vp]),

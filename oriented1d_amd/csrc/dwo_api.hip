@@ -218,9 +218,10 @@ int try_grouped_conv(const void *src, const float *w, const float *bias, const v
     return -100;
 }
 bool grouped_wgrad_covers(const ConvDims &d, int layout, size_t esize) {
-    // (with fewer planes than half the slots the fixed cost of a workgroup's sums shows: 4 x 64 x 20 x 20 in
-    // bf16 takes 14.6 us, on the tile kernels 11.7; 16 x 256 x 16 x 16 22.9 against 25.7)
-    if ((long)d.N * d.C < (long)kGrpSlots / 2 * grp_channels(esize)) return false;
+    // (with fewer planes than half the slots the plane kernels stay: 1 x 768 x 28 x 28 in bf16 takes 13.8 us, there 9.9; the tile
+    // kernels, which fit their windows to any plane, do not: 8 x 64 x 512 x 512 in bf16 at stride 2 250 us against 480, 2 x 384 x 32 x
+    // 32 14.3 against 22.7; of 75 random shapes three were slower, 1 x 256 x 62 x 62 fp32 at K = 7 the most, 16.2 against 13.6)
+    if ((long)d.N * d.C < (long)kGrpSlots / 2 * grp_channels(esize) && nhwc_plane_batch(d, layout) != 0) return false;
     return grouped_shape(d, layout, esize) && !(nhwc_plane_batch(d, layout) != 0 && reg_plane_shape_rt(d.H, d.W));
 }
 template <typename T>

@@ -48,6 +48,7 @@ struct Library {
     decltype(&::dwo_linear_wgrad) linear_wgrad;
     decltype(&::dwo_ln_patch) ln_patch;
     decltype(&::dwo_ln_patch_backward) ln_patch_backward;
+    decltype(&::dwo_pointwise_forward) pointwise_forward;
     decltype(&::dwo_linear_rows) linear_rows;
     decltype(&::dwo_linear_planes) linear_planes;
 } lib;
@@ -83,6 +84,7 @@ void bind_library(const std::string &path) {
     find(lib.linear_wgrad, "dwo_linear_wgrad");
     find(lib.ln_patch, "dwo_ln_patch");
     find(lib.ln_patch_backward, "dwo_ln_patch_backward");
+    find(lib.pointwise_forward, "dwo_pointwise_forward");
     find(lib.linear_rows, "dwo_linear_rows");
     find(lib.linear_planes, "dwo_linear_planes");
 }
@@ -413,6 +415,31 @@ std::tuple<Tensor, OptTensor> linear_wgrad(const Tensor &dy_, const Tensor &x_, 
     return {dw, db};
 }
 
+const void *optr(const OptTensor &t) { return t.has_value() ? t->const_data_ptr() : nullptr; }
+void check_layer(const Tensor &x, const Tensor &w, const OptTensor &b) {
+    check_glue(x, "x");
+    check_pair(x, w);
+    if (w.dim() != 2 || w.size(1) != x.size(-1) || w.scalar_type() != x.scalar_type())
+        fail("w must be [N, K] of the same type as x");
+    if (b.has_value() && (b->numel() != w.size(0) || b->scalar_type() != x.scalar_type() || !b->is_contiguous()))
+        fail("bias must be [N] of the same type as x");
+}
+
+// x [.., Cin] -> [.., C]: x w^T + b, all of one type
+Tensor pointwise_forward(const Tensor &x_, const Tensor &w_, const OptTensor &b) {
+    check_layer(x_, w_, b);
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const Tensor x = x_.contiguous(), w = w_.contiguous();
+    auto shape = x.sizes().vec();
+    shape.back() = w.size(0);
+    Tensor y = at::empty(shape, x.options());
+    check(lib.pointwise_forward(ptr(x), ptr(w), optr(b), y.data_ptr(), (size_t)(x.numel() / std::max<int64_t>(w.size(1), 1)),
+                                as_int(w.size(1)), as_int(w.size(0)), dtype_code(x), at.stream),
+          "dwo_pointwise_forward");
+    return y;
+}
+
 // LayerNorm (+ GELU) over the last dimension; (out, stats)
 std::tuple<Tensor, OptTensor> ln_rows(const Tensor &x_, const Tensor &g, const Tensor &b, double eps, int64_t gelu,
                                       at::ScalarType out_dtype, bool with_stats) {
@@ -557,16 +584,6 @@ std::tuple<Tensor, OptTensor> block_tail_backward(const Tensor &dout_, const Opt
     return {dy, ds};
 }
 
-const void *optr(const OptTensor &t) { return t.has_value() ? t->const_data_ptr() : nullptr; }
-void check_layer(const Tensor &x, const Tensor &w, const OptTensor &b) {
-    check_glue(x, "x");
-    check_pair(x, w);
-    if (w.dim() != 2 || w.size(1) != x.size(-1) || w.scalar_type() != x.scalar_type())
-        fail("w must be [N, K] of the same type as x");
-    if (b.has_value() && (b->numel() != w.size(0) || b->scalar_type() != x.scalar_type() || !b->is_contiguous()))
-        fail("bias must be [N] of the same type as x");
-}
-
 // act(x w^T + b) over the last dimension
 Tensor linear_rows(const Tensor &x_, const Tensor &w_, const OptTensor &b, bool gelu) {
     check_layer(x_, w_, b);
@@ -620,6 +637,7 @@ PYBIND11_MODULE(_host, m) {
     m.def("nchw_layernorm_nhwc", &nchw_layernorm_nhwc);
     m.def("nhwc_scale_add_nchw", &nhwc_scale_add_nchw);
     m.def("linear_wgrad", &linear_wgrad);
+    m.def("pointwise_forward", &pointwise_forward);
     m.def("linear_rows", &linear_rows);
     m.def("linear_planes", &linear_planes);
     m.def("ln_rows", &ln_rows);

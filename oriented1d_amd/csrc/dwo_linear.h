@@ -571,4 +571,76 @@ int launch_linear(const LinearArgs<T> &a, hipStream_t st) {
     return e == hipSuccess ? 0 : (int)e;
 }
 
+// ------------------------------------------------------------------------------------------------- few inputs
+// y[m][n] = b[n] + sum_k x[m][k] * w[n][k] for K <= 4 (the stem's first layer, models/convnext.py:143,177) and N a multiple of
+// 64.  Writing y bounds it (64 x 224 x 224 pixels of 64 channels in bf16: 411 MB; as a library product 312 us, here 92).
+// One matrix instruction per 16 pixels x 16 channels, 28 of its 32 columns zero: the same sums, bit for
+// bit, as a library product's.
+constexpr int kFewThreads = 256;
+template <typename T, int K>
+__global__ __launch_bounds__(kFewThreads) void few_inputs_kernel(const T *__restrict__ x, const T *__restrict__ w,
+                                                                 const T *__restrict__ b, T *__restrict__ y, long M,
+                                                                 int N) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    const int n0 = blockIdx.y * 64;
+    // fragment 2 h + i: channels 32 h + 8 g' + 4 i + r for its rows 4 g' + r
+    mma_s8 fw[4];
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+        fw[f] = mma_s8{0, 0, 0, 0, 0, 0, 0, 0};
+        const int n = n0 + 32 * (f / 2) + 8 * (c / 4) + 4 * (f % 2) + c % 4;
+        if (g == 0)
+#pragma unroll
+            for (int k = 0; k < K; k++) fw[f][k] = __builtin_bit_cast(short, w[(size_t)n * K + k]);
+    }
+    float bias[4][4];
+#pragma unroll
+    for (int f = 0; f < 4; f++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            bias[f][r] = b != nullptr ? to_float(b[n0 + 32 * (f / 2) + 8 * g + 4 * (f % 2) + r]) : 0.f;
+    constexpr int U = 4;  // groups of 16 pixels per step
+    const long step = (long)gridDim.x * (kFewThreads / 64) * 16 * U;
+    for (long m0 = ((long)blockIdx.x * (kFewThreads / 64) + (threadIdx.x >> 6)) * 16 * U; m0 < M; m0 += step) {
+        mma_s8 fx[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            fx[u] = mma_s8{0, 0, 0, 0, 0, 0, 0, 0};
+            const long m = m0 + 16 * u + c;
+            if (g == 0 && m < M)
+#pragma unroll
+                for (int k = 0; k < K; k++) fx[u][k] = __builtin_bit_cast(short, x[m * K + k]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const long m = m0 + 16 * u + c;
+            mma_f4 v[4];
+#pragma unroll
+            for (int f = 0; f < 4; f++) {
+                v[f] = Mma<T>::run(fw[f], fx[u], mma_f4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[f][r] += bias[f][r];
+            }
+            if (m < M)
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    *reinterpret_cast<mma_u4 *>(y + m * N + n0 + 32 * h + 8 * g) =
+                        mma_u4{lin_pack<T>(v[2 * h][0], v[2 * h][1]), lin_pack<T>(v[2 * h][2], v[2 * h][3]),
+                               lin_pack<T>(v[2 * h + 1][0], v[2 * h + 1][1]), lin_pack<T>(v[2 * h + 1][2], v[2 * h + 1][3])};
+        }
+    }
+}
+
+template <typename T>
+int launch_few_inputs(const void *x, const void *w, const void *b, void *y, long M, int N, int K, hipStream_t st) {
+    const long want = (M + 255) / 256, most = 8192 / (N / 64) > 0 ? 8192 / (N / 64) : 1;
+    const dim3 grid((unsigned)(want < most ? want : most), N / 64), block(kFewThreads);
+#define DWO_FEW(K_) \
+    case K_: few_inputs_kernel<T, K_><<<grid, block, 0, st>>>((const T *)x, (const T *)w, (const T *)b, (T *)y, M, N); break;
+    switch (K) { DWO_FEW(1) DWO_FEW(2) DWO_FEW(3) DWO_FEW(4) }
+#undef DWO_FEW
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : (int)e;
+}
+
 }  // namespace dwo

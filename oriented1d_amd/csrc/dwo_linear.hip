@@ -81,4 +81,18 @@ int dwo_linear_planes(const void *x, const void *w, const void *bias, const void
     }
 }
 
+int dwo_pointwise_forward(const void *x, const void *w, const void *b, void *y, size_t rows, int Cin, int C, int dtype,
+                          void *stream) {
+    if (!x || !w || !y) return DWO_ERR_NULL_POINTER;
+    if (rows < 1 || rows > (size_t)1 << 40 || Cin < 1 || Cin > 4 || C < 64 || C % 64 != 0 || C > 65536 ||
+        (uintptr_t)y % 16 != 0)
+        return DWO_ERR_BAD_SHAPE;
+    (void)hipGetLastError();
+    switch (dtype) {
+        case DWO_BF16: return launch_few_inputs<bf16_t>(x, w, b, y, (long)rows, C, Cin, (hipStream_t)stream);
+        case DWO_F16: return launch_few_inputs<f16_t>(x, w, b, y, (long)rows, C, Cin, (hipStream_t)stream);
+        default: return DWO_ERR_BAD_DTYPE;
+    }
+}
+
 }  // extern "C"

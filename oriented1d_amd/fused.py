@@ -102,8 +102,8 @@ def linear_tail(x, linear, gamma, residual):
 
 
 class _PointwiseLinear(torch.autograd.Function):
-    """``F.linear`` whose parameter gradients come from the library: with a few input channels
-    and every pixel of a batch as rows they are a reduction, not a matrix product."""
+    """``F.linear`` in the library: with a few input channels and every pixel of a batch as rows it is a pass over its output,
+    and its parameter gradients are a reduction, not matrix products."""
 
     @staticmethod
     def forward(ctx, x, w, b):
@@ -114,8 +114,11 @@ class _PointwiseLinear(torch.autograd.Function):
             # it keeps for the rest of the region would be cut off from the parameters
             dtype = torch.get_autocast_dtype(x.device.type)
             xc, wc, bc = (t if t is None else t.to(dtype) for t in (x, w, b))
-        with torch.autocast(x.device.type, enabled=False):
-            y = F.linear(xc, wc, bc)
+        if xc.dtype != torch.float32 and wc.shape[0] % 64 == 0:
+            y = _lib.host(xc.get_device()).pointwise_forward(xc, wc, bc)
+        else:
+            with torch.autocast(x.device.type, enabled=False):
+                y = F.linear(xc, wc, bc)
         # (only what backward reads: parameters may be updated between the passes where the input takes
         # no gradient)
         ctx.save_for_backward(xc, w if ctx.needs_input_grad[0] else None)

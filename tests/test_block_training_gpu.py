@@ -291,3 +291,33 @@ def test_network_gradients_against_the_composition(variant, mode, monkeypatch):
         assert a.dtype == b.dtype and a.shape == b.shape
         e = (a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-20)
         assert e <= tol, (tuple(a.shape), float(e))
+
+
+def test_row_norm_gelu_of_infinities():
+    """The cheaper erf of 16-bit outputs gives what u * (1 + erf) gives where LayerNorm's parameters overflow."""
+    x = torch.randn(4, 64, device="cuda").to(F16).requires_grad_(True)
+    w, b = torch.ones(64, device="cuda"), torch.zeros(64, device="cuda")
+    b[:3] = torch.tensor([float("inf"), float("-inf"), float("nan")])
+    y = fused._RowNorm.apply(x, w, b, 1e-6, 1, F16)
+    z = F.gelu(F.layer_norm(x.float(), (64,), w, b, 1e-6)).to(F16)
+    assert torch.equal(torch.isnan(y), torch.isnan(z)) and torch.equal(torch.isinf(y), torch.isinf(z))
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16], ids=str)
+@pytest.mark.parametrize("N,C,H,W,K,stride", [(1, 64, 17, 17, 31, 1), (1, 64, 58, 58, 31, 1), (2, 64, 20, 33, 7, 2),
+                                              (3, 128, 21, 45, 15, 2), (1, 256, 62, 62, 7, 1), (2, 64, 130, 70, 27, 2)])
+def test_grouped_wgrad_of_few_planes(N, C, H, W, K, stride, dtype):
+    """Channels grouped by orientation, fewer planes than workgroup slots: the grouped kernels against the tile kernels (the
+    same call without the claim); both sum fp32 products of the same values in fp32."""
+    from oriented1d_amd import _lib
+    from oriented1d_amd.convnext1d import channel_angles
+    from oriented1d_amd.dwoconv1d import build_taps
+    torch.manual_seed(H)
+    taps = build_taps(torch.tensor(channel_angles(C)), C, K).cuda()
+    x = torch.randn(N, H, W, C, device="cuda").to(dtype)
+    dy = torch.randn(N, -(-H // stride), -(-W // stride), C, device="cuda").to(dtype)
+    host = _lib.host(0)
+    got = host.wgrad(dy, x, taps, K, stride, _lib.NHWC + _lib.GROUPED, True)
+    ref = host.wgrad(dy, x, taps, K, stride, _lib.NHWC, True)
+    for a, b in zip(got, ref):
+        close(a, b.double(), 1e-5, "wgrad")
