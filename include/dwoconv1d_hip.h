@@ -294,6 +294,14 @@ int dwo_linear_rows(const void *x, const void *w, const void *bias, void *out, s
 int dwo_linear_planes(const void *x, const void *w, const void *bias, const void *scale, const void *res, void *out,
                       int images, int HW, int N, int K, int dtype, void *stream);
 
+/*
+ * Both pointwise layers of a block at inference in one kernel (models/convnext.py:306-318), for 16-bit types and C = 96, 128,
+ * 192 or 384: out [images,C,HW] = res + scale[c] * (b2 + w2 gelu(b1 + w1 x)) for x [images,HW,C], w1 [4C,C], w2 [C,4C], all
+ * of the activations' type, 16-byte aligned, images * HW below 2^31; scale [C] may be null.
+ */
+int dwo_block_mlp(const void *x, const void *w1, const void *b1, const void *w2, const void *b2, const void *scale,
+                  const void *res, void *out, int images, int HW, int C, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -47,6 +47,7 @@ SIGNATURES = {
     "dwo_linear_wgrad_scratch_bytes": (_sz, [_sz, _i, _i]),
     "dwo_linear_rows": (_i, [_vp] * 4 + [_sz] + [_i] * 4 + [_vp]),
     "dwo_linear_planes": (_i, [_vp] * 6 + [_i] * 5 + [_vp]),
+    "dwo_block_mlp": (_i, [_vp] * 8 + [_i] * 4 + [_vp]),
     "dwo_linear_wgrad": (_i, [_vp] * 5 + [_sz, _sz] + [_i] * 4 + [_vp]),
 }
 

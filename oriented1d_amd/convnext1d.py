@@ -185,6 +185,10 @@ class Block(nn.Module):
         else:  # (recorded by autograd: one pass each way as well)
             z = fused.tile_norm(y, self.norm, self.pwconv1) if fused.plain(self.norm, nn.LayerNorm) else None
             y = self.norm(y.permute(0, 2, 3, 1).contiguous()) if z is None else z
+        if fuse and not self.plus_plus:
+            out = fused.block_mlp(y, self.pwconv1, self.pwconv2, self.gamma, x)
+            if out is not None:
+                return out
         y = fused.linear_gelu(y, self.pwconv1)
         if self.plus_plus:
             y = self.dwconv2(y)

@@ -117,27 +117,27 @@ __device__ __forceinline__ f16_t from_float<f16_t>(float v) {
 }
 
 // GELU with erf from Abramowitz and Stegun, Handbook of Mathematical Functions, 7.1.26 (error of erf below 1.5e-7), for results
-// that are rounded to 2^-9 or 2^-12 on the way out: u * Phi(u) with Phi = 1 - q for u > 0, else q, and
-// q = erfc(|u| / sqrt 2) / 2.  Half the issue slots of erff, which took more of them than the matrix products of a
-// stage-1 block.  Infinities and NaN give what u * (1 + erf) gives.
-__device__ __forceinline__ float normal_cdf_rounded(float u, float &density) {
+// that are rounded to 2^-9 or 2^-12 on the way out: u Phi(u) = |u| (1/2 - q) + u / 2 with q = erfc(|u| / sqrt 2) / 2.  Half
+// the issue slots of erff, which took more of them than the matrix products of a stage-1 block.  Infinities and NaN
+// give what u * (1 + erf) gives.
+__device__ __forceinline__ float half_erfc_rounded(float u, float &density) {
     const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_fabsf(u), 0.3275911f * 0.70710678118654752f, 1.f));
     float p = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
     p = __builtin_fmaf(t, p, 0.5f * 1.421413741f);
     p = __builtin_fmaf(t, p, 0.5f * -0.284496736f);
     p = __builtin_fmaf(t, p, 0.5f * 0.254829592f);
     density = __builtin_amdgcn_exp2f(u * u * -0.72134752044448170f);  // exp(-u^2 / 2)
-    const float q = p * t * density;
-    return u > 0.f ? 1.f - q : q;
+    return p * t * density;
 }
 __device__ __forceinline__ float gelu_rounded(float u) {
     float e;
-    return u * normal_cdf_rounded(u, e);
+    const float q = half_erfc_rounded(u, e);
+    return __builtin_fmaf(__builtin_fabsf(u), 0.5f - q, 0.5f * u);
 }
 __device__ __forceinline__ float gelu_slope_rounded(float u) {
     float e;
-    const float cdf = normal_cdf_rounded(u, e);
-    return __builtin_fmaf(u * 0.39894228040143268f, e, cdf);
+    const float q = half_erfc_rounded(u, e);
+    return __builtin_fmaf(u * 0.39894228040143268f, e, u > 0.f ? 1.f - q : q);
 }
 
 // Wave64 sum via cross-lane shuffles; every lane ends with the total of lanes >= itself folded

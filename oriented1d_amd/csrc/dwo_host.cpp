@@ -49,6 +49,7 @@ struct Library {
     decltype(&::dwo_ln_patch) ln_patch;
     decltype(&::dwo_ln_patch_backward) ln_patch_backward;
     decltype(&::dwo_pointwise_forward) pointwise_forward;
+    decltype(&::dwo_block_mlp) block_mlp;
     decltype(&::dwo_linear_rows) linear_rows;
     decltype(&::dwo_linear_planes) linear_planes;
 } lib;
@@ -85,6 +86,7 @@ void bind_library(const std::string &path) {
     find(lib.ln_patch, "dwo_ln_patch");
     find(lib.ln_patch_backward, "dwo_ln_patch_backward");
     find(lib.pointwise_forward, "dwo_pointwise_forward");
+    find(lib.block_mlp, "dwo_block_mlp");
     find(lib.linear_rows, "dwo_linear_rows");
     find(lib.linear_planes, "dwo_linear_planes");
 }
@@ -624,6 +626,34 @@ Tensor linear_planes(const Tensor &x_, const Tensor &w_, const OptTensor &b, con
     return out;
 }
 
+// x [N,H,W,C], res [N,C,H,W] -> res + scale * (w2 gelu(w1 x + b1) + b2), planes
+Tensor block_mlp(const Tensor &x_, const Tensor &w1_, const Tensor &b1, const Tensor &w2_, const Tensor &b2,
+                 const OptTensor &scale, const Tensor &res_) {
+    check_layer(x_, w1_, b1);
+    check_layer(x_, w1_, std::nullopt);
+    if (x_.dim() != 4) throw py::value_error("x must be a 4-d tensor");
+    const int64_t C = x_.size(3);
+    if (w1_.size(0) != 4 * C || w2_.dim() != 2 || w2_.size(0) != C || w2_.size(1) != 4 * C ||
+        w2_.scalar_type() != x_.scalar_type() || b2.numel() != C || b2.scalar_type() != x_.scalar_type() ||
+        !b2.is_contiguous())
+        fail("w1 must be [4C, C], w2 [C, 4C] and b2 [C], of the same type as x");
+    if (scale.has_value() && (scale->numel() != C || scale->scalar_type() != x_.scalar_type() || !scale->is_contiguous()))
+        fail("scale must be [C] of the same type as x");
+    const Dims d(x_, true);
+    const std::array<int64_t, 4> shape = {d.n, d.c, d.h, d.w};
+    if (res_.sizes() != at::IntArrayRef(shape) || res_.scalar_type() != x_.scalar_type())
+        fail("residual must be [N,C,H,W] of the same type as x");
+    check_pair(x_, w2_), check_pair(x_, b2), check_pair(x_, res_);
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const Tensor x = dense(x_), w1 = dense(w1_), w2 = dense(w2_), c1 = dense(b1), res = dense(res_);
+    Tensor out = at::empty(shape, x.options());
+    check(lib.block_mlp(ptr(x), ptr(w1), ptr(c1), ptr(w2), ptr(b2), optr(scale), ptr(res), out.data_ptr(), as_int(d.n),
+                        as_int(d.h * d.w), as_int(C), dtype_code(x), at.stream),
+          "dwo_block_mlp");
+    return out;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -638,6 +668,7 @@ PYBIND11_MODULE(_host, m) {
     m.def("nhwc_scale_add_nchw", &nhwc_scale_add_nchw);
     m.def("linear_wgrad", &linear_wgrad);
     m.def("pointwise_forward", &pointwise_forward);
+    m.def("block_mlp", &block_mlp);
     m.def("linear_rows", &linear_rows);
     m.def("linear_planes", &linear_planes);
     m.def("ln_rows", &ln_rows);

@@ -101,6 +101,25 @@ def linear_tail(x, linear, gamma, residual):
     return nhwc_scale_add_nchw(linear(x), gamma, residual)
 
 
+# Rows from which both layers run as one kernel: enough workgroups of 128 pixels that its long chain is paid for (bf16, us, two
+# kernels / one: 12544 x 96 25 / 18, 6272 x 96 14 / 18; 100352 x 192 160 / 124, 25088 x 192 46 / 46; 25088 x 384 120 / 105,
+# 12544 x 384 65 / 100)
+_MLP_ROWS = {96: 12288, 128: 16384, 192: 28672, 384: 24576}
+
+
+def block_mlp(y, first, second, gamma, residual):
+    """``linear_tail(linear_gelu(y, first), second, gamma, residual)`` as one kernel where that is faster, else None."""
+    C = y.shape[-1]
+    w1, b1, w2, b2 = first.weight, first.bias, second.weight, second.bias
+    if not (y.dim() == 4 and C in _MLP_ROWS and y.numel() // C >= _MLP_ROWS[C] and plain(first, Linear)
+            and plain(second, Linear) and b1 is not None and b2 is not None and w1.shape == (4 * C, C)
+            and w2.shape == (C, 4 * C) and _layer16(y, w1, b1) and residual.dtype == y.dtype
+            and all(t is None or (t.dtype == y.dtype and t.device == y.device) for t in (w2, b2, gamma))
+            and ordinary(w2, b2, gamma, residual)):
+        return None
+    return _lib.host(y.get_device()).block_mlp(y, w1, b1, w2, b2, gamma, residual)
+
+
 class _PointwiseLinear(torch.autograd.Function):
     """``F.linear`` in the library: with a few input channels and every pixel of a batch as rows it is a pass over its output,
     and its parameter gradients are a reduction, not matrix products."""

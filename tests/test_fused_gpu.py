@@ -342,3 +342,25 @@ def test_product_kernels_keep_refusals():
         host.linear_rows(x.float(), w.float(), None, True)
     with pytest.raises(RuntimeError):
         host.linear_planes(x, w, None, None, torch.zeros(1, 8, 2, 3, device="cuda", dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("C", [96, 128, 192, 384])
+@pytest.mark.parametrize("N,H,W,scaled", [(1, 1, 1, True), (3, 13, 7, True), (2, 8, 24, False), (5, 14, 14, True), (9, 4, 32, True)])
+def test_block_mlp(N, H, W, scaled, C, dtype):
+    """Both layers in one kernel: rows that fill no workgroup, waves without pixels, planes of 8 k, 4 k and odd pixels (a wave's run
+    then crosses images)."""
+    torch.manual_seed(C + H)
+    x = torch.randn(N, H, W, C, device="cuda").to(dtype)
+    w1, b1 = (torch.randn(4 * C, C, device="cuda") * C ** -0.5).to(dtype), torch.randn(4 * C, device="cuda").to(dtype)
+    w2, b2 = (torch.randn(C, 4 * C, device="cuda") * C ** -0.5).to(dtype), torch.randn(C, device="cuda").to(dtype)
+    s = torch.randn(C, device="cuda").to(dtype) if scaled else None
+    res = torch.randn(N, C, H, W, device="cuda").to(dtype)
+    got = fused._lib.host(0).block_mlp(x, w1, b1, w2, b2, s, res)
+    y = F.linear(F.gelu(F.linear(x.double(), w1.double(), b1.double())), w2.double(), b2.double())
+    y = y if s is None else y * s.double()
+    _close(got, res.double() + y.permute(0, 3, 1, 2), dtype, "block_mlp")
+    with pytest.raises(RuntimeError):
+        fused._lib.host(0).block_mlp(x, w1[:, :8], b1, w2, b2, s, res)
+    with pytest.raises(RuntimeError):
+        fused._lib.host(0).block_mlp(x, w1, b1, w2, b2, s, res.float())
