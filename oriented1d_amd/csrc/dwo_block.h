@@ -9,7 +9,7 @@
 // All of them are bound by memory: PyTorch's compositions move each tensor three to six times (permuted
 // copies, conversions, separate parameter gradients) at 0.4 to 2 TB/s.  Input and output have types of their
 // own, so the conversions of autocast happen on the way out (fp32 stream, 16-bit pointwise layers).  Channels
-// are handled in pieces of eight by groups of 8 to 64 lanes, sums over channels stay inside a group, and
+// are handled in pieces of eight, rows by groups of 8 to 64 lanes, and
 // parameter gradients are kept in registers over all the tiles of a workgroup, written as
 // partial sums and added in a fixed order by a second kernel.  Statistics and sums are fp32.
 #pragma once
@@ -23,6 +23,7 @@ constexpr int kBlkThreads = 256, kBlkMaxC = 1024, kBlkGroups = 1024;
 typedef unsigned blk_u4 __attribute__((ext_vector_type(4)));
 typedef unsigned blk_u2 __attribute__((ext_vector_type(2)));
 typedef float blk_f4 __attribute__((ext_vector_type(4)));
+typedef float blk_f2 __attribute__((ext_vector_type(2)));
 
 // eight neighbouring values as floats
 template <typename T>
@@ -135,20 +136,24 @@ __device__ __forceinline__ void write_param_partials(float (&dg)[NV][8], float (
 }
 
 // part [groups][L] -> out0 [split], out1 [L - split], fixed order.  Few columns and up to a thousand groups: latency binds,
-// so 32 threads share a column, each with four loads in flight (eight threads one load at a time: 23 us for 1024 groups of 1024 columns, now 8).
+// so 32 threads share a column, each with eight loads in flight (eight threads, one load at a
+// time: 23 us for 1024 groups of 1024 columns, now 8).
 constexpr int kColThreads = 1024;
 template <typename TO>
 __global__ __launch_bounds__(kColThreads) void column_sums_kernel(const float *__restrict__ part, TO *out0, TO *out1,
                                                                   int L, int split, int groups) {
     __shared__ float red[kColThreads];
     const int c = blockIdx.x * 32 + threadIdx.x % 32;
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (c < L)
-        for (int g = threadIdx.x / 32; g < groups; g += 128)
+        for (int g = threadIdx.x / 32; g < groups; g += 256) {
+            float v[8];
 #pragma unroll
-            for (int u = 0; u < 4; u++)
-                if (g + 32 * u < groups) s[u] += part[(size_t)(g + 32 * u) * L + c];
-    red[threadIdx.x] = (s[0] + s[1]) + (s[2] + s[3]);
+            for (int u = 0; u < 8; u++) v[u] = g + 32 * u < groups ? part[(size_t)(g + 32 * u) * L + c] : 0.f;
+#pragma unroll
+            for (int u = 0; u < 8; u++) s[u] += v[u];
+        }
+    red[threadIdx.x] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
     __syncthreads();
     if (threadIdx.x >= 32 || c >= L) return;
     float t = red[threadIdx.x];
@@ -270,340 +275,342 @@ __global__ __launch_bounds__(kBlkThreads) void ln_rows_backward_kernel(
     write_param_partials<LPR, NV>(dg, db, C, red, part);
 }
 
-// ------------------------------------------------------------------------------------------------- tiles
-// P pixels x C channels of an image in LDS as [C][P + 1] values of the tensor's type: four workgroups per CU, but 16
-// pixels (whole 64-byte pieces of fp32 rows) while they fit the 64 KB that need no attribute
-// Fewer pixels where the tiles would not fill the chip (a single image: the chain of one tile is what counts).
-inline int blk_tile_pixels(int C, int esize, long pixels) {
-    int p = 64;
-    while (p > 16 && (long)C * (p + 1) * esize > 36 * 1024) p >>= 1;
-    while (p > 8 && pixels / p < 256) p >>= 1;
-    return (long)C * (p + 1) * esize > 64 * 1024 ? 8 : p;
-}
-inline size_t blk_tile_bytes(int C, int P, int esize) { return ((size_t)C * (P + 1) * esize + 15) / 16 * 16; }
+// ------------------------------------------------------------------------------------------------- quads
+// LayerNorm over the channels of planes.  A lane holds eight channels of four pixels: eight runs of the planes on one
+// side, four runs of eight channels (16 bytes and more) on the other, so the transposition is the order of the registers
+// and LDS only carries the sums over channels from wave to wave.  A wave covers 64 channels x 32 pixels: 64-byte pieces and longer
+// both ways.  Neighbouring tiles stay on one XCD (they share the lines at their edges).
+//
+// The four pixels are neighbours (their index m runs over the images' pixels), or a 2 x 2 patch of a
+// downsampling layer (m = 4 * patch + pixel; out is [patch][C][2][2], the operand of that 2 x 2 convolution of stride 2
+// as a product with its weights as they lie, models/convnext.py:548-553).
+//
+// Memory bounds it from a few thousand pixels on, latency below.  Through LDS tiles of [C][pixels], value by value (before) / so,
+// us: forward bf16 128 x 96 x 56 x 56 57 / 28 (5.6 TB/s), 128 x 384 x 14 x 14 25 / 12, 128 x 768 x 7 x 7 36 / 13, fp32 to bf16
+// 64 x 512 x 14 x 14 24 / 9.5; patches of 128 x 96 x 56 x 56 72 / 37.  Backward with the parameter sums, fp32 stream: 64 x 512 x
+// 14 x 14 42 / 22, 64 x 128 x 56 x 56 64 / 49; above 512 channels the 1024 threads have 128 registers each, which spills: 64
+// x 1024 x 7 x 7 40 / 43.
+enum { QUAD_RUN, QUAD_SINGLE, QUAD_PATCH, QUAD_PATCH_SINGLE };  // four pixels by one load, by four; patches by two, by four
 
-struct BlkTiles {
-    int C, HW, P, log2P, per, tiles;  // tiles per image, in all
-    int H, W, W2;                     // patches: image extents, patches per row
+struct BlkQuads {
+    int C, HW, H, W;
+    int wc, pt;        // waves across the channels, tiles of 32 pixels per workgroup
+    int per;           // workgroup tiles per XCD
+    unsigned M;        // pixels (in patches)
 };
 
-template <typename T, int VEC>
-__device__ __forceinline__ void tile_in(const T *xn, T *tile, const BlkTiles &t, int np) {
-    const int sh = t.log2P - (VEC == 4 ? 2 : 0), total = t.C << sh;
-    constexpr int U = 8;  // loads in flight
-    for (int f0 = threadIdx.x; f0 < total; f0 += U * kBlkThreads) {
-        float v[U][VEC];
+// places of the four pixels m .. m + 3 in channel `chan` of their image (a tensor has fewer than 2^31 values)
+template <int MODE>
+struct QuadAt {
+    static constexpr int RUNS = MODE == QUAD_RUN ? 1 : MODE == QUAD_PATCH ? 2 : 4;
+    unsigned at[RUNS];
+    __device__ __forceinline__ QuadAt(const BlkQuads &t, unsigned m, int chan) {
+        if constexpr (MODE == QUAD_RUN || MODE == QUAD_SINGLE) {
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int f = f0 + u * kBlkThreads, c = f >> sh, p = (f - (c << sh)) * VEC;
-            if (f < total && p < np) load_run<T, VEC>(xn + (size_t)c * t.HW + p, v[u]);
+            for (int e = 0; e < RUNS; e++) {
+                const unsigned img = (m + e) / (unsigned)t.HW;
+                at[e] = (img * t.C + chan) * t.HW + (m + e - img * t.HW);
+            }
+        } else {
+            const unsigned w2 = (unsigned)t.W / 2, h2 = (unsigned)t.H / 2, k = m / 4;
+            const unsigned row = k / w2, img = row / h2;
+            const unsigned o = (img * t.C + chan) * t.HW + (row - img * h2) * 2 * t.W + (k - row * w2) * 2;
+            if constexpr (MODE == QUAD_PATCH) at[0] = o, at[1] = o + t.W;
+            else at[0] = o, at[1] = o + 1, at[2] = o + t.W, at[3] = o + t.W + 1;
         }
+    }
+    // the addresses made from these are made again where they are used next, instead of being kept in registers
+    __device__ __forceinline__ void forget() {
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int f = f0 + u * kBlkThreads, c = f >> sh, p = (f - (c << sh)) * VEC;
-            if (f < total && p < np)
+        for (int e = 0; e < RUNS; e++) asm volatile("" : "+v"(at[e]));
+    }
+};
+// two neighbouring values
+template <typename T>
+__device__ __forceinline__ void store_pair(T *p, float a, float b) {
+    if constexpr (sizeof(T) == 4) *reinterpret_cast<blk_f2 *>(p) = blk_f2{a, b};
+    else *reinterpret_cast<unsigned *>(p) = pack2<T>(a, b);
+}
+// N neighbouring values as they lie in memory
+template <typename T, int N>
+struct RawRun {
+    static constexpr int WORDS = N * (int)sizeof(T) / 4;
+    typedef unsigned vec __attribute__((ext_vector_type(WORDS < 4 ? WORDS : 4)));
+    unsigned w[WORDS];
+    __device__ __forceinline__ void clear() {
 #pragma unroll
-                for (int e = 0; e < VEC; e++) tile[c * (t.P + 1) + p + e] = from_float<T>(v[u][e]);
+        for (int k = 0; k < WORDS; k++) w[k] = 0u;
+    }
+    // L of them, from value `at` on
+    template <int L>
+    __device__ __forceinline__ void load(const T *p, int at) {
+        constexpr int n = L * (int)sizeof(T) / 4;
+        if constexpr (n == 0) w[at / 2] |= (unsigned)__builtin_bit_cast(uint16_t, *p) << (16 * (at % 2));
+        else if constexpr (n == 1) w[at * (int)sizeof(T) / 4] = *reinterpret_cast<const unsigned *>(p);
+        else if constexpr (n == 2) {
+            const blk_u2 v = *reinterpret_cast<const blk_u2 *>(p);
+            w[at * (int)sizeof(T) / 4] = v[0], w[at * (int)sizeof(T) / 4 + 1] = v[1];
+        } else {
+#pragma unroll
+            for (int k = 0; k < n / 4; k++) {
+                const blk_u4 v = reinterpret_cast<const blk_u4 *>(p)[k];
+#pragma unroll
+                for (int j = 0; j < 4; j++) w[4 * k + j] = v[j];
+            }
+        }
+    }
+    __device__ __forceinline__ float get(int i) const {
+        if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, w[i]);
+        else return to_float(__builtin_bit_cast(T, (uint16_t)(w[i / 2] >> (16 * (i % 2)))));
+    }
+    // what was made of these values is made again, instead of being kept in registers beside them
+    __device__ __forceinline__ void forget() {
+#pragma unroll
+        for (int k = 0; k < WORDS; k++) asm volatile("" : "+v"(w[k]));
+    }
+};
+// eight channels (planes HW apart) of four pixels, of which `live` exist (all or none but for QUAD_SINGLE)
+template <int MODE, typename T>
+struct QuadPlanes {
+    RawRun<T, 4> run[8];
+    __device__ __forceinline__ void load(const T *x, const QuadAt<MODE> &q, int HW, int live) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) run[i].clear();
+        if (live == 0) return;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const T *xi = x + (size_t)i * HW;  // (uniform)
+            if constexpr (MODE == QUAD_RUN) {
+                run[i].template load<4>(xi + q.at[0], 0);
+            } else if constexpr (MODE == QUAD_PATCH) {
+                run[i].template load<2>(xi + q.at[0], 0), run[i].template load<2>(xi + q.at[1], 2);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (MODE == QUAD_PATCH_SINGLE || e < live) run[i].template load<1>(xi + q.at[e], e);
+            }
+        }
+    }
+    __device__ __forceinline__ float get(int i, int e) const { return run[i].get(e); }
+    __device__ __forceinline__ void forget() {
+#pragma unroll
+        for (int i = 0; i < 8; i++) run[i].forget();
+    }
+};
+// the same values as rows: [m][C], or [patch][C][4]
+template <int MODE, typename T>
+struct QuadRows {
+    static constexpr bool PATCHES = MODE == QUAD_PATCH || MODE == QUAD_PATCH_SINGLE;
+    RawRun<T, 8> piece[4];  // a pixel's eight channels; two channels' four pixels
+    __device__ __forceinline__ void load(const T *rows, unsigned m, int chan, int C, int live) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) piece[k].clear();
+        if (live == 0) return;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (MODE != QUAD_SINGLE || k < live)
+                piece[k].template load<8>(PATCHES ? rows + ((size_t)(m / 4) * C + chan + 2 * k) * 4
+                                                  : rows + (size_t)(m + k) * C + chan, 0);
+        }
+    }
+    __device__ __forceinline__ float get(int i, int e) const {
+        return PATCHES ? piece[i / 2].get(i % 2 * 4 + e) : piece[e].get(i);
+    }
+    __device__ __forceinline__ void forget() {
+#pragma unroll
+        for (int k = 0; k < 4; k++) piece[k].forget();
+    }
+};
+template <int MODE, typename T>
+__device__ __forceinline__ void quad_store(T *x, const QuadAt<MODE> &q, int HW, int live, const float (&v)[8][4]) {
+    if (live == 0) return;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        T *xi = x + (size_t)i * HW;
+        if constexpr (MODE == QUAD_RUN) {
+            store_run<T, 4>(xi + q.at[0], v[i]);
+        } else if constexpr (MODE == QUAD_PATCH) {
+            store_pair(xi + q.at[0], v[i][0], v[i][1]), store_pair(xi + q.at[1], v[i][2], v[i][3]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (MODE == QUAD_PATCH_SINGLE || e < live) xi[q.at[e]] = from_float<T>(v[i][e]);
         }
     }
 }
-template <typename T, int VEC>
-__device__ __forceinline__ void tile_out(T *xn, const T *tile, const BlkTiles &t, int np) {
-    const int sh = t.log2P - (VEC == 4 ? 2 : 0), total = t.C << sh;
-    for (int f = threadIdx.x; f < total; f += kBlkThreads) {
-        const int c = f >> sh, p = (f - (c << sh)) * VEC;
-        if (p >= np) continue;
-        float v[VEC];
+template <int MODE, typename T>
+__device__ __forceinline__ void quad_store_rows(T *rows, unsigned m, int chan, int C, int live, const float (&v)[8][4]) {
+    if (live == 0) return;
+    if constexpr (MODE == QUAD_RUN || MODE == QUAD_SINGLE) {
 #pragma unroll
-        for (int e = 0; e < VEC; e++) v[e] = to_float(tile[c * (t.P + 1) + p + e]);
-        store_run<T, VEC>(xn + (size_t)c * t.HW + p, v);
+        for (int e = 0; e < 4; e++) {
+            float o[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) o[i] = v[i][e];
+            if (MODE == QUAD_RUN || e < live) store8(rows + (size_t)(m + e) * C + chan, o);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) {
+            float o[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[e] = v[i + e / 4][e % 4];
+            store8(rows + (size_t)(m / 4) * C * 4 + (chan + i) * 4, o);
+        }
     }
 }
 
-template <typename TI, typename TO, int LPR, int NV, int VEC>
-__global__ __launch_bounds__(kBlkThreads) void ln_tile_kernel(const TI *__restrict__ x, const float *__restrict__ gamma,
-                                                              const float *__restrict__ beta, TO *__restrict__ out,
-                                                              float2 *__restrict__ stats, BlkTiles t, float eps) {
-    extern __shared__ float lds_block[];
-    TI *tile = reinterpret_cast<TI *>(lds_block);
-    const Lanes<LPR, NV> ln;
-    const int n = blockIdx.x / t.per, p0 = blockIdx.x % t.per * t.P, np = min(t.P, t.HW - p0);
-    tile_in<TI, VEC>(x + (size_t)n * t.C * t.HW + p0, tile, t, np);
-    float gm[NV][8], bt[NV][8];
+// Lane: pixels 4 * (lane % 8) .. of the wave's 32, channels 8 * (lane / 8) .. of its 64
+struct QuadLane {
+    int wave, wch, wp, pq, chan, step;  // step: pixels per workgroup tile
+    __device__ __forceinline__ QuadLane(const BlkQuads &t)
+        : wave(threadIdx.x >> 6), wch(wave % t.wc), wp(wave / t.wc), pq(threadIdx.x % 8),
+          chan(wch * 64 + (int)(threadIdx.x >> 3 & 7) * 8), step(32 * t.pt) {}
+    // pixel of tile `tile`
+    __device__ __forceinline__ unsigned pixel(int tile) const { return (unsigned)tile * step + wp * 32 + pq * 4; }
+    // pixels that exist, 0 beyond the channels
+    __device__ __forceinline__ int live(const BlkQuads &t, unsigned m) const {
+        return chan < t.C && m < t.M ? (int)min(4u, t.M - m) : 0;
+    }
+    // this wave's sums over its channels go to red, [wave][32]
+    __device__ __forceinline__ void give(float *red, float (&s)[4]) const {
 #pragma unroll
-    for (int k = 0; k < NV; k++)
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int c = ln.chan(k) + i;
-            gm[k][i] = c < t.C ? gamma[c] : 0.f, bt[k][i] = c < t.C ? beta[c] : 0.f;
+        for (int e = 0; e < 4; e++) {
+            s[e] = dpp_add<0x128>(s[e]);  // row_ror:8
+            s[e] += __shfl_xor(s[e], 16, 64);
+            s[e] += __shfl_xor(s[e], 32, 64);
         }
-    __syncthreads();
-    const long row0 = (long)n * t.HW + p0;
-    for (int q0 = 0; q0 < np; q0 += ln.ROWS) {
-        const int p = q0 + ln.slot;
-        const bool row = p < np;
-        float v[NV][8], s = 0.f;
+        if ((threadIdx.x & 63) < 8) *reinterpret_cast<blk_f4 *>(red + wave * 32 + pq * 4) = blk_f4{s[0], s[1], s[2], s[3]};
+    }
+    __device__ __forceinline__ void take(const float *red, const BlkQuads &t, float (&s)[4]) const {
+        blk_f4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+        for (int w = 0; w < t.wc; w++) v += *reinterpret_cast<const blk_f4 *>(red + (wp * t.wc + w) * 32 + pq * 4);
 #pragma unroll
-        for (int k = 0; k < NV; k++) {
-            const bool ok = row && ln.chan(k) < t.C;
+        for (int e = 0; e < 4; e++) s[e] = v[e];
+    }
+};
+
+template <typename TI, typename TO, int MODE, int THREADS>
+__global__ __launch_bounds__(THREADS) void ln_quad_kernel(const TI *__restrict__ x, const float *__restrict__ gamma,
+                                                          const float *__restrict__ beta, TO *__restrict__ out,
+                                                          float2 *__restrict__ stats, BlkQuads t, float eps) {
+    __shared__ __attribute__((aligned(16))) float red[2][THREADS / 64 * 32];
+    const QuadLane ln(t);
+    const int tile = blockIdx.x % 8 * t.per + blockIdx.x / 8;
+    const unsigned m = ln.pixel(tile);
+    if (m - ln.pq * 4 - ln.wp * 32 >= t.M) return;  // (the whole workgroup)
+    const int live = ln.live(t, m);
+    float v[8][4], mean[4], rstd[4];
+    QuadPlanes<MODE, TI> in;
+    in.load(x, QuadAt<MODE>(t, m, ln.chan), t.HW, live);
+    float gm[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, bt[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (ln.chan < t.C)
+#pragma unroll
+        for (int i = 0; i < 8; i++) gm[i] = gamma[ln.chan + i], bt[i] = beta[ln.chan + i];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        mean[e] = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i][e] = in.get(i, e), mean[e] += v[i][e];
+    }
+    ln.give(red[0], mean);
+    __syncthreads();
+    ln.take(red[0], t, mean);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        mean[e] /= (float)t.C;
+        rstd[e] = 0.f;
+        if (e < live)
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i][e] -= mean[e], rstd[e] = __builtin_fmaf(v[i][e], v[i][e], rstd[e]);
+    }
+    ln.give(red[1], rstd);
+    __syncthreads();
+    ln.take(red[1], t, rstd);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        rstd[e] = rsqrtf(rstd[e] / (float)t.C + eps);
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i][e] = __builtin_fmaf(v[i][e] * rstd[e], gm[i], bt[i]);
+        if (stats != nullptr && ln.chan == 0 && e < live) stats[m + e] = make_float2(mean[e], rstd[e]);
+    }
+    quad_store_rows<MODE>(out, m, ln.chan, t.C, live, v);
+}
+
+// part: [workgroups][2][C].  The tensors' own values stay in registers over the barrier, not the floats made of them.
+template <typename TI, typename TO, int MODE, int THREADS>
+__global__ __launch_bounds__(THREADS) void ln_quad_backward_kernel(
+    const TO *__restrict__ dout, const TI *__restrict__ x, const float2 *__restrict__ stats,
+    const float *__restrict__ gamma, TI *__restrict__ dx, float *__restrict__ part, BlkQuads t) {
+    __shared__ __attribute__((aligned(16))) float red[2][2][THREADS / 64 * 32];
+    const QuadLane ln(t);
+    float gm[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, dg[8], db[8];
+    if (ln.chan < t.C)
+#pragma unroll
+        for (int i = 0; i < 8; i++) gm[i] = gamma[ln.chan + i];
+#pragma unroll
+    for (int i = 0; i < 8; i++) dg[i] = db[i] = 0.f;
+    int turn = 0;
+    // (the sums of a turn are read before the barrier of the next one, and written again after it)
+    for (int k = blockIdx.x / 8; k < t.per; k += gridDim.x / 8, turn ^= 1) {
+        const unsigned m = ln.pixel(blockIdx.x % 8 * t.per + k);
+        if (m - ln.pq * 4 - ln.wp * 32 >= t.M) break;  // (the whole workgroup)
+        const int live = ln.live(t, m);
+        QuadAt<MODE> at(t, m, ln.chan);
+        QuadPlanes<MODE, TI> xs;
+        QuadRows<MODE, TO> gs;
+        xs.load(x, at, t.HW, live), gs.load(dout, m, ln.chan, t.C, live);
+        float s1[4], s2[4];
+        float2 st[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            st[e] = e < live ? stats[m + e] : make_float2(0.f, 0.f), s1[e] = s2[e] = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                v[k][i] = ok ? to_float(tile[(ln.chan(k) + i) * (t.P + 1) + p]) : 0.f;
-                s += v[k][i];
+                const float g = gs.get(i, e), h = (xs.get(i, e) - st[e].x) * st[e].y, v = g * gm[i];
+                dg[i] = __builtin_fmaf(g, h, dg[i]);
+                db[i] += g;
+                s1[e] += v;
+                s2[e] = __builtin_fmaf(v, h, s2[e]);
             }
+            __builtin_amdgcn_sched_barrier(0);  // (a pixel's floats are gone before the next one's are made)
         }
-        const float mean = group_total<LPR>(s) / (float)t.C;
-        float q = 0.f;
+        ln.give(red[turn][0], s1), ln.give(red[turn][1], s2);
+        __syncthreads();
+        at.forget(), xs.forget(), gs.forget();
+        ln.take(red[turn][0], t, s1), ln.take(red[turn][1], t, s2);
+        float o[8][4];
 #pragma unroll
-        for (int k = 0; k < NV; k++)
-            if (ln.chan(k) < t.C)
+        for (int e = 0; e < 4; e++) {
+            s1[e] /= (float)t.C, s2[e] /= (float)t.C;
 #pragma unroll
-                for (int i = 0; i < 8; i++) v[k][i] -= mean, q = __builtin_fmaf(v[k][i], v[k][i], q);
-        const float rstd = rsqrtf(group_total<LPR>(q) / (float)t.C + eps);
-        if (!row) continue;
+            for (int i = 0; i < 8; i++)
+                o[i][e] = st[e].y * (gs.get(i, e) * gm[i] - s1[e] - (xs.get(i, e) - st[e].x) * st[e].y * s2[e]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        quad_store<MODE>(dx, at, t.HW, live, o);
+    }
+    // the waves of equal channels meet in LDS
 #pragma unroll
-        for (int k = 0; k < NV; k++)
-            if (ln.chan(k) < t.C) {
-                float o[8];
+    for (int i = 0; i < 8; i++) dg[i] = group_total<8>(dg[i]), db[i] = group_total<8>(db[i]);
+    __shared__ __attribute__((aligned(16))) float sums[4][2][64];
+    if (t.pt > 1) {
+        const int l = ln.chan - ln.wch * 64;
+        if (ln.pq == 0) store8(&sums[ln.wave][0][l], dg), store8(&sums[ln.wave][1][l], db);
+        __syncthreads();
+        if (ln.wp == 0 && ln.pq == 0)
+            for (int p = 1; p < t.pt; p++) {
+                float a[8], b[8];
+                load8(&sums[p * t.wc + ln.wch][0][l], a), load8(&sums[p * t.wc + ln.wch][1][l], b);
 #pragma unroll
-                for (int i = 0; i < 8; i++) o[i] = __builtin_fmaf(v[k][i] * rstd, gm[k][i], bt[k][i]);
-                store8(out + (row0 + p) * t.C + ln.chan(k), o);
+                for (int i = 0; i < 8; i++) dg[i] += a[i], db[i] += b[i];
             }
-        if (stats != nullptr && ln.l == 0) stats[row0 + p] = make_float2(mean, rstd);
     }
-}
-
-template <typename TI, typename TO, int LPR, int NV, int VEC>
-__global__ __launch_bounds__(kBlkThreads) void ln_tile_backward_kernel(
-    const TO *__restrict__ dout, const TI *__restrict__ x, const float2 *__restrict__ stats,
-    const float *__restrict__ gamma, TI *__restrict__ dx, float *__restrict__ part, BlkTiles t) {
-    extern __shared__ float lds_block[];
-    TI *tile = reinterpret_cast<TI *>(lds_block);
-    const Lanes<LPR, NV> ln;
-    float gm[NV][8], dg[NV][8], db[NV][8];
-#pragma unroll
-    for (int k = 0; k < NV; k++)
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int c = ln.chan(k) + i;
-            gm[k][i] = c < t.C ? gamma[c] : 0.f;
-            dg[k][i] = db[k][i] = 0.f;
-        }
-    for (int u = blockIdx.x; u < t.tiles; u += gridDim.x) {
-        const int n = u / t.per, p0 = u % t.per * t.P, np = min(t.P, t.HW - p0);
-        const size_t base = (size_t)n * t.C * t.HW + p0;
-        const long row0 = (long)n * t.HW + p0;
-        __syncthreads();
-        tile_in<TI, VEC>(x + base, tile, t, np);
-        __syncthreads();
-        for (int q0 = 0; q0 < np; q0 += ln.ROWS) {
-            const int p = q0 + ln.slot;
-            const bool row = p < np;
-            const float2 st = row ? stats[row0 + p] : make_float2(0.f, 0.f);
-            float h[NV][8], g[NV][8], s1 = 0.f, s2 = 0.f;
-#pragma unroll
-            for (int k = 0; k < NV; k++) {
-                const bool ok = row && ln.chan(k) < t.C;
-                if (ok) load8(dout + (row0 + p) * t.C + ln.chan(k), g[k]);
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    h[k][i] = ok ? (to_float(tile[(ln.chan(k) + i) * (t.P + 1) + p]) - st.x) * st.y : 0.f;
-                    if (!ok) g[k][i] = 0.f;
-                    dg[k][i] = __builtin_fmaf(g[k][i], h[k][i], dg[k][i]);
-                    db[k][i] += g[k][i];
-                    g[k][i] *= gm[k][i];
-                    s1 += g[k][i];
-                    s2 = __builtin_fmaf(g[k][i], h[k][i], s2);
-                }
-            }
-            s1 = group_total<LPR>(s1) / (float)t.C;
-            s2 = group_total<LPR>(s2) / (float)t.C;
-#pragma unroll
-            for (int k = 0; k < NV; k++)
-                if (row && ln.chan(k) < t.C)
-#pragma unroll
-                    for (int i = 0; i < 8; i++)
-                        tile[(ln.chan(k) + i) * (t.P + 1) + p] =
-                            from_float<TI>(st.y * (g[k][i] - s1 - h[k][i] * s2));
-        }
-        __syncthreads();
-        tile_out<TI, VEC>(dx + base, tile, t, np);
+    if (ln.wp == 0 && ln.pq == 0 && ln.chan < t.C) {
+        float *to = part + (size_t)blockIdx.x * 2 * t.C + ln.chan;
+        store8(to, dg), store8(to + t.C, db);
     }
-    write_param_partials<LPR, NV>(dg, db, t.C, lds_block, part);
-}
-
-// ------------------------------------------------------------------------------------------------- patches
-// x [N,C,H,W] -> LayerNorm over C -> patches [N,H/2,W/2][C][2][2], the operand of the downsampling 2 x 2 convolution of stride
-// 2 as a product with its weights as they lie (models/convnext.py:548-553).  A tile is a run of
-// P / 4 patches of one row; a lane holds eight channels of the four pixels of a patch, 32 neighbouring values of the output.
-struct PatchTile {
-    int n, h, p0, np;  // image, row of patches, first patch, patches
-    __device__ __forceinline__ PatchTile(const BlkTiles &t, int u) {
-        const int P = t.P / 4, h2 = t.H / 2, row = u / t.per;
-        n = row / h2, h = row - n * h2;
-        p0 = u % t.per * P, np = min(P, t.W2 - p0);
-    }
-};
-template <typename T, int VEC, bool IN>
-__device__ __forceinline__ void patch_move(T *x, T *tile, const BlkTiles &t, const PatchTile &at) {
-    const int sh = t.log2P - (VEC == 4 ? 2 : 0), half = t.P / 2 / VEC, total = t.C << sh;
-    T *xn = x + (size_t)at.n * t.C * t.HW + (size_t)2 * at.h * t.W + 2 * at.p0;
-    constexpr int U = IN ? 8 : 1;
-    for (int f0 = threadIdx.x; f0 < total; f0 += U * kBlkThreads) {
-        float v[U][VEC];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int f = f0 + u * kBlkThreads, c = f >> sh, k = f - (c << sh), r = k >= half, q = (k - r * half) * VEC;
-            if (f >= total || q >= 2 * at.np) continue;
-            T *m = xn + (size_t)c * t.HW + r * t.W + q;
-            const T *l = tile + c * (t.P + 1) + r * (t.P / 2) + q;
-            if constexpr (IN) load_run<T, VEC>(m, v[u]);
-            else {
-#pragma unroll
-                for (int e = 0; e < VEC; e++) v[u][e] = to_float(l[e]);
-                store_run<T, VEC>(m, v[u]);
-            }
-        }
-        if constexpr (IN) {
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const int f = f0 + u * kBlkThreads, c = f >> sh, k = f - (c << sh), r = k >= half, q = (k - r * half) * VEC;
-                if (f >= total || q >= 2 * at.np) continue;
-#pragma unroll
-                for (int e = 0; e < VEC; e++) tile[c * (t.P + 1) + r * (t.P / 2) + q + e] = from_float<T>(v[u][e]);
-            }
-        }
-    }
-}
-
-template <typename TI, typename TO, int LPR, int NV, int VEC>
-__global__ __launch_bounds__(kBlkThreads) void ln_patch_kernel(const TI *__restrict__ x, const float *__restrict__ gamma,
-                                                               const float *__restrict__ beta, TO *__restrict__ out,
-                                                               float2 *__restrict__ stats, BlkTiles t, float eps) {
-    extern __shared__ float lds_block[];
-    TI *tile = reinterpret_cast<TI *>(lds_block);
-    const Lanes<LPR, NV> ln;
-    const PatchTile at(t, blockIdx.x);
-    patch_move<TI, VEC, true>(const_cast<TI *>(x), tile, t, at);
-    float gm[NV][8], bt[NV][8];
-#pragma unroll
-    for (int k = 0; k < NV; k++)
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int c = ln.chan(k) + i;
-            gm[k][i] = c < t.C ? gamma[c] : 0.f, bt[k][i] = c < t.C ? beta[c] : 0.f;
-        }
-    __syncthreads();
-    const size_t first = ((size_t)at.n * (t.H / 2) + at.h) * t.W2 + at.p0;
-    for (int q0 = 0; q0 < at.np; q0 += ln.ROWS) {
-        const int p = q0 + ln.slot;
-        const bool row = p < at.np;
-        float v[NV][8][4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const TI *px = tile + q / 2 * (t.P / 2) + 2 * p + q % 2;
-            float s = 0.f;
-#pragma unroll
-            for (int k = 0; k < NV; k++)
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    v[k][i][q] = row && ln.chan(k) < t.C ? to_float(px[(ln.chan(k) + i) * (t.P + 1)]) : 0.f;
-                    s += v[k][i][q];
-                }
-            const float mean = group_total<LPR>(s) / (float)t.C;
-            float d = 0.f;
-#pragma unroll
-            for (int k = 0; k < NV; k++)
-                if (ln.chan(k) < t.C)
-#pragma unroll
-                    for (int i = 0; i < 8; i++) v[k][i][q] -= mean, d = __builtin_fmaf(v[k][i][q], v[k][i][q], d);
-            const float rstd = rsqrtf(group_total<LPR>(d) / (float)t.C + eps);
-#pragma unroll
-            for (int k = 0; k < NV; k++)
-#pragma unroll
-                for (int i = 0; i < 8; i++) v[k][i][q] = __builtin_fmaf(v[k][i][q] * rstd, gm[k][i], bt[k][i]);
-            if (stats != nullptr && row && ln.l == 0) stats[(first + p) * 4 + q] = make_float2(mean, rstd);
-        }
-        if (!row) continue;
-#pragma unroll
-        for (int k = 0; k < NV; k++)
-            if (ln.chan(k) < t.C)
-#pragma unroll
-                for (int i = 0; i < 8; i += 2) {
-                    float o[8];
-#pragma unroll
-                    for (int e = 0; e < 8; e++) o[e] = v[k][i + e / 4][e % 4];
-                    store8(out + ((first + p) * t.C + ln.chan(k) + i) * 4, o);
-                }
-    }
-}
-
-template <typename TI, typename TO, int LPR, int NV, int VEC>
-__global__ __launch_bounds__(kBlkThreads) void ln_patch_backward_kernel(
-    const TO *__restrict__ dout, const TI *__restrict__ x, const float2 *__restrict__ stats,
-    const float *__restrict__ gamma, TI *__restrict__ dx, float *__restrict__ part, BlkTiles t) {
-    extern __shared__ float lds_block[];
-    TI *tile = reinterpret_cast<TI *>(lds_block);
-    const Lanes<LPR, NV> ln;
-    float gm[NV][8], dg[NV][8], db[NV][8];
-#pragma unroll
-    for (int k = 0; k < NV; k++)
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int c = ln.chan(k) + i;
-            gm[k][i] = c < t.C ? gamma[c] : 0.f;
-            dg[k][i] = db[k][i] = 0.f;
-        }
-    for (int u = blockIdx.x; u < t.tiles; u += gridDim.x) {
-        const PatchTile at(t, u);
-        __syncthreads();
-        patch_move<TI, VEC, true>(const_cast<TI *>(x), tile, t, at);
-        __syncthreads();
-        const size_t first = ((size_t)at.n * (t.H / 2) + at.h) * t.W2 + at.p0;
-        for (int q0 = 0; q0 < at.np; q0 += ln.ROWS) {
-            const int p = q0 + ln.slot;
-            const bool row = p < at.np;
-            float g[NV][8][4];
-#pragma unroll
-            for (int k = 0; k < NV; k++)
-#pragma unroll
-                for (int i = 0; i < 8; i += 2) {
-                    float o[8];
-                    if (row && ln.chan(k) < t.C) load8(dout + ((first + p) * t.C + ln.chan(k) + i) * 4, o);
-#pragma unroll
-                    for (int e = 0; e < 8; e++) g[k][i + e / 4][e % 4] = row && ln.chan(k) < t.C ? o[e] : 0.f;
-                }
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                TI *px = tile + q / 2 * (t.P / 2) + 2 * p + q % 2;
-                const float2 st = row ? stats[(first + p) * 4 + q] : make_float2(0.f, 0.f);
-                float h[NV][8], s1 = 0.f, s2 = 0.f;
-#pragma unroll
-                for (int k = 0; k < NV; k++)
-#pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        const bool ok = row && ln.chan(k) < t.C;
-                        h[k][i] = ok ? (to_float(px[(ln.chan(k) + i) * (t.P + 1)]) - st.x) * st.y : 0.f;
-                        dg[k][i] = __builtin_fmaf(g[k][i][q], h[k][i], dg[k][i]);
-                        db[k][i] += g[k][i][q];
-                        g[k][i][q] *= gm[k][i];
-                        s1 += g[k][i][q];
-                        s2 = __builtin_fmaf(g[k][i][q], h[k][i], s2);
-                    }
-                s1 = group_total<LPR>(s1) / (float)t.C;
-                s2 = group_total<LPR>(s2) / (float)t.C;
-#pragma unroll
-                for (int k = 0; k < NV; k++)
-                    if (row && ln.chan(k) < t.C)
-#pragma unroll
-                        for (int i = 0; i < 8; i++)
-                            px[(ln.chan(k) + i) * (t.P + 1)] = from_float<TI>(st.y * (g[k][i][q] - s1 - h[k][i] * s2));
-            }
-        }
-        __syncthreads();
-        patch_move<TI, VEC, false>(dx, tile, t, at);
-    }
-    write_param_partials<LPR, NV>(dg, db, t.C, lds_block, part);
 }
 
 // ------------------------------------------------------------------------------------------------- tail

@@ -39,7 +39,6 @@ int by_types(int in, int out, F &&f) {
     if (in == DWO_F16 && out == DWO_F32) return f(Type<f16_t>{}, Type<float>{});
     return DWO_ERR_BAD_DTYPE;
 }
-int esize(int dtype) { return dtype == DWO_F32 ? 4 : 2; }
 
 int column_sums(const float *part, void *out0, void *out1, int L, int split, int groups, int dtype, hipStream_t st) {
     const dim3 grid((L + 31) / 32), block(kColThreads);
@@ -61,21 +60,57 @@ int column_sums(const float *part, void *out0, void *out1, int L, int split, int
 bool tile_ok(int N, int C, int H, int W) {
     return N >= 1 && H >= 1 && W >= 1 && channels_ok(C) && (double)N * C * H * W < 2147483648.0;
 }
-BlkTiles tiles_of(int N, int C, int HW, int bytes) {
-    BlkTiles t{};
-    t.C = C, t.HW = HW, t.P = blk_tile_pixels(C, bytes, (long)N * HW);
-    t.log2P = __builtin_ctz(t.P);
-    t.per = (HW + t.P - 1) / t.P, t.tiles = N * t.per;
+// m runs over `pixels` pixels (in patches: four per patch)
+BlkQuads quads_of(int C, int H, int W, long pixels) {
+    BlkQuads t{};
+    t.C = C, t.HW = H * W, t.H = H, t.W = W, t.M = (unsigned)pixels;
+    t.wc = (C + 63) / 64;
+    t.pt = t.wc >= 3 ? 1 : 4 / t.wc;  // four waves where that many fit
+    t.per = (int)(((pixels + 32 * t.pt - 1) / (32 * t.pt) + 7) / 8);
     return t;
 }
-BlkTiles patches_of(int N, int C, int H, int W, int bytes) {
-    BlkTiles t{};
-    t.C = C, t.HW = H * W, t.H = H, t.W = W, t.W2 = W / 2;
-    t.P = blk_tile_pixels(C, bytes, (long)N * H * W);
-    while (t.P > 8 && t.P / 4 >= 2 * t.W2) t.P >>= 1;  // (no wider than a row)
-    t.log2P = __builtin_ctz(t.P);
-    t.per = (t.W2 + t.P / 4 - 1) / (t.P / 4), t.tiles = N * (H / 2) * t.per;
-    return t;
+// f(MODE, THREADS)
+template <class F>
+int by_quads(const BlkQuads &t, bool patches, F &&f) {
+    using std::integral_constant;
+    auto threads = [&](auto mode) {
+        if (t.C <= 256) return f(mode, integral_constant<int, 256>{});
+        if (t.C <= 512) return f(mode, integral_constant<int, 512>{});
+        return f(mode, integral_constant<int, 1024>{});
+    };
+    if (patches)
+        return t.W % 2 == 0 ? threads(integral_constant<int, QUAD_PATCH>{}) : threads(integral_constant<int, QUAD_PATCH_SINGLE>{});
+    return t.HW % 4 == 0 ? threads(integral_constant<int, QUAD_RUN>{}) : threads(integral_constant<int, QUAD_SINGLE>{});
+}
+int ln_quads(const void *x, const float *gamma, const float *beta, void *out, float *stats, const BlkQuads &t, bool patches,
+             float eps, int in_dtype, int out_dtype, hipStream_t st) {
+    return by_types(in_dtype, out_dtype, [&](auto ti, auto to) {
+        using TI = typename decltype(ti)::type;
+        using TO = typename decltype(to)::type;
+        return by_quads(t, patches, [&](auto mode, auto threads) {
+            ln_quad_kernel<TI, TO, decltype(mode)::value, decltype(threads)::value>
+                <<<dim3((unsigned)t.per * 8), dim3(64 * t.wc * t.pt), 0, st>>>((const TI *)x, gamma, beta, (TO *)out,
+                                                                               (float2 *)stats, t, eps);
+            return status();
+        });
+    });
+}
+int ln_quads_backward(const void *dout, const void *x, const float *stats, const float *gamma, void *dx, void *dgamma,
+                      void *dbeta, float *part, const BlkQuads &t, bool patches, int in_dtype, int out_dtype, int grad_dtype,
+                      hipStream_t st) {
+    const int grid = 8 * (t.per < kBlkGroups / 8 ? t.per : kBlkGroups / 8);
+    const int e = by_types(in_dtype, out_dtype, [&](auto ti, auto to) {
+        using TI = typename decltype(ti)::type;
+        using TO = typename decltype(to)::type;
+        return by_quads(t, patches, [&](auto mode, auto threads) {
+            ln_quad_backward_kernel<TI, TO, decltype(mode)::value, decltype(threads)::value>
+                <<<dim3(grid), dim3(64 * t.wc * t.pt), 0, st>>>((const TO *)dout, (const TI *)x, (const float2 *)stats, gamma,
+                                                                (TI *)dx, part, t);
+            return status();
+        });
+    });
+    if (e != DWO_OK) return e;
+    return column_sums(part, dgamma, dbeta, 2 * t.C, t.C, grid, grad_dtype, st);
 }
 TailTiles tail_of(int N, int C, int HW) {
     TailTiles t;
@@ -142,23 +177,8 @@ int dwo_ln_tile(const void *x, const float *gamma, const float *beta, void *out,
     if (!x || !gamma || !beta || !out) return DWO_ERR_NULL_POINTER;
     if (!tile_ok(N, C, H, W) || !aligned16(x) || !aligned16(out)) return DWO_ERR_BAD_SHAPE;
     (void)hipGetLastError();
-    const BlkTiles t = tiles_of(N, C, H * W, esize(in_dtype));
-    return by_types(in_dtype, out_dtype, [&](auto ti, auto to) {
-        using TI = typename decltype(ti)::type;
-        using TO = typename decltype(to)::type;
-        return by_channels(C, [&](auto lpr, auto nv) {
-            constexpr int LPR = decltype(lpr)::value, NV = decltype(nv)::value;
-            const dim3 grid(t.tiles), block(kBlkThreads);
-            const size_t lds = blk_tile_bytes(C, t.P, sizeof(TI));
-            if (t.HW % 4 == 0)
-                ln_tile_kernel<TI, TO, LPR, NV, 4><<<grid, block, lds, (hipStream_t)stream>>>(
-                    (const TI *)x, gamma, beta, (TO *)out, (float2 *)stats, t, eps);
-            else
-                ln_tile_kernel<TI, TO, LPR, NV, 1><<<grid, block, lds, (hipStream_t)stream>>>(
-                    (const TI *)x, gamma, beta, (TO *)out, (float2 *)stats, t, eps);
-            return status();
-        });
-    });
+    return ln_quads(x, gamma, beta, out, stats, quads_of(C, H, W, (long)N * H * W), false, eps, in_dtype, out_dtype,
+                    (hipStream_t)stream);
 }
 
 int dwo_ln_tile_backward(const void *dout, const void *x, const float *stats, const float *gamma, void *dx,
@@ -168,28 +188,9 @@ int dwo_ln_tile_backward(const void *dout, const void *x, const float *stats, co
     if (!tile_ok(N, C, H, W) || !aligned16(x) || !aligned16(dout) || !aligned16(dx)) return DWO_ERR_BAD_SHAPE;
     if (scratch_bytes < dwo_block_scratch_bytes(C)) return DWO_ERR_SCRATCH_TOO_SMALL;
     (void)hipGetLastError();
-    hipStream_t st = (hipStream_t)stream;
-    const BlkTiles t = tiles_of(N, C, H * W, esize(in_dtype));
-    const int groups = groups_of(t.tiles);
-    const int e = by_types(in_dtype, out_dtype, [&](auto ti, auto to) {
-        using TI = typename decltype(ti)::type;
-        using TO = typename decltype(to)::type;
-        return by_channels(C, [&](auto lpr, auto nv) {
-            constexpr int LPR = decltype(lpr)::value, NV = decltype(nv)::value;
-            const dim3 grid(groups), block(kBlkThreads);
-            size_t lds = blk_tile_bytes(C, t.P, sizeof(TI));
-            if (lds < 8 * kBlkThreads * sizeof(float)) lds = 8 * kBlkThreads * sizeof(float);  // the parameter sums
-            if (t.HW % 4 == 0)
-                ln_tile_backward_kernel<TI, TO, LPR, NV, 4><<<grid, block, lds, st>>>(
-                    (const TO *)dout, (const TI *)x, (const float2 *)stats, gamma, (TI *)dx, (float *)scratch, t);
-            else
-                ln_tile_backward_kernel<TI, TO, LPR, NV, 1><<<grid, block, lds, st>>>(
-                    (const TO *)dout, (const TI *)x, (const float2 *)stats, gamma, (TI *)dx, (float *)scratch, t);
-            return status();
-        });
-    });
-    if (e != DWO_OK) return e;
-    return column_sums((const float *)scratch, dgamma, dbeta, 2 * C, C, groups, grad_dtype, st);
+    return ln_quads_backward(dout, x, stats, gamma, dx, dgamma, dbeta, (float *)scratch,
+                             quads_of(C, H, W, (long)N * H * W), false, in_dtype, out_dtype, grad_dtype,
+                             (hipStream_t)stream);
 }
 
 int dwo_ln_patch(const void *x, const float *gamma, const float *beta, void *out, float *stats, int N, int C, int H,
@@ -197,23 +198,8 @@ int dwo_ln_patch(const void *x, const float *gamma, const float *beta, void *out
     if (!x || !gamma || !beta || !out) return DWO_ERR_NULL_POINTER;
     if (!tile_ok(N, C, H, W) || H < 2 || W < 2 || !aligned16(x) || !aligned16(out)) return DWO_ERR_BAD_SHAPE;
     (void)hipGetLastError();
-    const BlkTiles t = patches_of(N, C, H, W, esize(in_dtype));
-    return by_types(in_dtype, out_dtype, [&](auto ti, auto to) {
-        using TI = typename decltype(ti)::type;
-        using TO = typename decltype(to)::type;
-        return by_channels(C, [&](auto lpr, auto nv) {
-            constexpr int LPR = decltype(lpr)::value, NV = decltype(nv)::value;
-            const dim3 grid(t.tiles), block(kBlkThreads);
-            const size_t lds = blk_tile_bytes(C, t.P, sizeof(TI));
-            if (W % 4 == 0)
-                ln_patch_kernel<TI, TO, LPR, NV, 4><<<grid, block, lds, (hipStream_t)stream>>>(
-                    (const TI *)x, gamma, beta, (TO *)out, (float2 *)stats, t, eps);
-            else
-                ln_patch_kernel<TI, TO, LPR, NV, 1><<<grid, block, lds, (hipStream_t)stream>>>(
-                    (const TI *)x, gamma, beta, (TO *)out, (float2 *)stats, t, eps);
-            return status();
-        });
-    });
+    return ln_quads(x, gamma, beta, out, stats, quads_of(C, H, W, (long)N * (H / 2) * (W / 2) * 4), true, eps, in_dtype,
+                    out_dtype, (hipStream_t)stream);
 }
 
 int dwo_ln_patch_backward(const void *dout, const void *x, const float *stats, const float *gamma, void *dx,
@@ -224,28 +210,9 @@ int dwo_ln_patch_backward(const void *dout, const void *x, const float *stats, c
         return DWO_ERR_BAD_SHAPE;
     if (scratch_bytes < dwo_block_scratch_bytes(C)) return DWO_ERR_SCRATCH_TOO_SMALL;
     (void)hipGetLastError();
-    hipStream_t st = (hipStream_t)stream;
-    const BlkTiles t = patches_of(N, C, H, W, esize(in_dtype));
-    const int groups = groups_of(t.tiles);
-    const int e = by_types(in_dtype, out_dtype, [&](auto ti, auto to) {
-        using TI = typename decltype(ti)::type;
-        using TO = typename decltype(to)::type;
-        return by_channels(C, [&](auto lpr, auto nv) {
-            constexpr int LPR = decltype(lpr)::value, NV = decltype(nv)::value;
-            const dim3 grid(groups), block(kBlkThreads);
-            size_t lds = blk_tile_bytes(C, t.P, sizeof(TI));
-            if (lds < 8 * kBlkThreads * sizeof(float)) lds = 8 * kBlkThreads * sizeof(float);  // the parameter sums
-            if (W % 4 == 0)
-                ln_patch_backward_kernel<TI, TO, LPR, NV, 4><<<grid, block, lds, st>>>(
-                    (const TO *)dout, (const TI *)x, (const float2 *)stats, gamma, (TI *)dx, (float *)scratch, t);
-            else
-                ln_patch_backward_kernel<TI, TO, LPR, NV, 1><<<grid, block, lds, st>>>(
-                    (const TO *)dout, (const TI *)x, (const float2 *)stats, gamma, (TI *)dx, (float *)scratch, t);
-            return status();
-        });
-    });
-    if (e != DWO_OK) return e;
-    return column_sums((const float *)scratch, dgamma, dbeta, 2 * C, C, groups, grad_dtype, st);
+    return ln_quads_backward(dout, x, stats, gamma, dx, dgamma, dbeta, (float *)scratch,
+                             quads_of(C, H, W, (long)N * (H / 2) * (W / 2) * 4), true, in_dtype, out_dtype, grad_dtype,
+                             (hipStream_t)stream);
 }
 
 int dwo_block_tail(const void *y, const float *scale, const void *res, void *out, int N, int C, int H, int W,

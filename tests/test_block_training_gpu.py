@@ -39,7 +39,8 @@ def run_norm(x, w, b, dout, native, reference, tol_out, tol_dx):
 
 @pytest.mark.parametrize("types", TYPES, ids=str)
 @pytest.mark.parametrize("N,C,H,W", [(2, 96, 9, 8), (1, 8, 1, 1), (3, 64, 5, 13), (2, 72, 16, 16), (1, 128, 33, 2),
-                                     (2, 256, 7, 7), (2, 520, 3, 4), (1, 1024, 7, 7), (40, 96, 56, 56)])
+                                     (2, 256, 7, 7), (2, 520, 3, 4), (1, 1024, 7, 7), (40, 96, 56, 56),
+                                     (33, 64, 1, 3), (7, 264, 3, 5), (9, 512, 2, 2), (260, 128, 7, 12)])
 def test_tile_norm(N, C, H, W, types):
     if N == 40 and types != (F32, BF16):
         pytest.skip("one type at the size where workgroups take several tiles")
