@@ -69,7 +69,7 @@ def host_command(out):
 
 
 def build(verbose=False, jobs=None, only=None):
-    """Compile csrc/dwo_host.cpp (the extension module _host.so), csrc/dwo_api.hip, csrc/dwo_block.hip, csrc/dwo_linear.hip, csrc/dwo_mlp.hip and one csrc/dwo_inst.hip object per (element type, plane
+    """Compile csrc/dwo_host.cpp (the extension module _host.so), csrc/dwo_api.hip, csrc/dwo_block.hip, csrc/dwo_linear.hip, csrc/dwo_mlp.hip, csrc/dwo_stem.hip and one csrc/dwo_inst.hip object per (element type, plane
     extent) in parallel, then link libdwoconv1d_hip.so into the package directory.  ``only``
     (substrings of object names, e.g. ``["dwo_api", "float_k31_56"]``) recompiles just those
     units and links them with the objects a previous full build left in place."""
@@ -80,7 +80,7 @@ def build(verbose=False, jobs=None, only=None):
     common = [hipcc()] + [f for f in HIPCC_FLAGS if f != "-shared"] + [
         "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-c"]
     units = [(os.path.join(CSRC, name + ".hip"), os.path.join(objdir, name + ".o"), [])
-             for name in ("dwo_block", "dwo_api", "dwo_linear", "dwo_mlp")]
+             for name in ("dwo_block", "dwo_api", "dwo_linear", "dwo_mlp", "dwo_stem")]
     for K in sorted(WINDOW_KS, reverse=True):
         for t in PLANE_TYPES:
             for family in ("window", "grouped"):

@@ -21,6 +21,11 @@
 
 using namespace dwo;
 
+namespace dwo {
+int launch_stem(const bf16_t *x, const float *pw_w, const float *pw_b, const float *w, const float *bias, const void *taps,
+                bf16_t *y, const ConvDims &d, hipStream_t st);  // dwo_stem.hip
+}
+
 namespace {
 
 int log2_stride(int stride) { return stride == 1 ? 0 : (stride == 2 ? 1 : (stride == 4 ? 2 : -1)); }
@@ -499,6 +504,13 @@ int pointwise_fprop_t(const void *x, const float *pw_w, const float *pw_b, const
                       const float *bias, const void *taps, void *y, int Cin, const ConvDims &d,
                       hipStream_t st) {
     // (the input is read element by element: only the output's alignment matters)
+    if constexpr (std::is_same<T, bf16_t>::value)
+        // matrix products from 32768 output pixels on (K = 31, us, projecting / this: 128 x 224 x 224 520 / 123, 8 x 225 x 131
+        // 31 / 23); below, a workgroup's weights take longer than its share of the pixels (1 x 224 x 224 12.9 / 15.7)
+        if (Cin == 3 && (long)d.N * d.P * d.Q >= 32768 && d.stride == 2 && grouped_shape(d, DWO_NHWC, sizeof(T)) && aligned16(y)) {
+            const int rc = launch_stem((const bf16_t *)x, pw_w, pw_b, w, bias, taps, (bf16_t *)y, d, st);
+            if (rc != -100) return rc;
+        }
     if (Cin == kGrpProjected && d.stride == 2 && grouped_shape(d, DWO_NHWC, sizeof(T)) && aligned16(y)) {
         int rc = -100;
 #define DWO_MATCH(K_) \
@@ -600,6 +612,12 @@ int init_type() {
         DWO_GROUPED_KS(DWO_PREP)
 #undef DWO_PREP
     }
+    if constexpr (std::is_same<T, bf16_t>::value)
+        for (int K : {7, 15, 31}) {  // a kernel for each eight taps up to 8, 16 and 32
+            ConvDims g = d;
+            g.stride = 2, g.K = K;
+            rc |= launch_stem(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, g, nullptr);
+        }
     rc |= launch_nchw_tile_fprop<T>(nullptr, nullptr, nullptr, nullptr, nullptr, d, 0, nullptr);
     rc |= launch_nhwc_tile_fprop<T>(nullptr, nullptr, nullptr, nullptr, nullptr, d, 0, nullptr);
     rc |= launch_tile_dgrad_strided<T>(nullptr, nullptr, nullptr, nullptr, d, true, nullptr);

@@ -223,6 +223,42 @@ def test_projected_stem_tile_edges(C, H, W, K, dtype):
             _close(got, conv(mid), dtype, "projected")
 
 
+@pytest.mark.parametrize("N,C,H,W,K", [(40, 64, 66, 131, 31), (30, 64, 97, 70, 15), (1700, 64, 5, 13, 7), (1200, 64, 2, 59, 27),
+                                       (3, 128, 260, 201, 31), (40000, 64, 1, 1, 13)])
+def test_projected_stem_as_products(N, C, H, W, K):
+    """The stem's matrix products at the edges of their tiles against the two layers in 64 and 32 bits: nothing but the
+    result is rounded to bf16 (2^-9 of a value, 1e-2 is the operator's bound)."""
+    from oriented1d_amd.convnext1d import channel_angles
+    from oriented1d_amd.dwoconv1d import DepthwiseOrientedConv1d
+
+    torch.manual_seed(H)
+    lin = torch.nn.Linear(3, C).cuda()
+    x = torch.randn(N, H, W, 3, device="cuda").to(torch.bfloat16)
+    conv = DepthwiseOrientedConv1d(C, C, K, groups=C, stride=2, padding=K // 2, bias=True, angle=channel_angles(C),
+                                   nhwc=True, arbitrary_size=True).cuda()
+    torch.nn.init.normal_(conv.bias, std=0.3)
+    with torch.no_grad():
+        def layers(rounded):
+            mid = torch.nn.functional.linear(x.double(), lin.weight.double(), lin.bias.double())
+            return conv(mid.to(torch.bfloat16 if rounded else torch.float32))
+        _close(fused.pointwise_dwconv_nhwc(x, lin, conv), layers(False), torch.bfloat16, "products")
+        # a claim of common orientations that does not hold, infinities and NaN: tap by tap
+        look = conv._taps.lookup
+        mixed = DepthwiseOrientedConv1d(C, C, K, groups=C, stride=2, padding=K // 2, bias=True, nhwc=True,
+                                        angle=[c % 8 * 0.39 for c in range(C)], arbitrary_size=True).cuda()
+        conv._taps.lookup = lambda *a: (mixed._taps.lookup(mixed.theta, *a[1:])[0], {2: 3, 4: 3})
+        got = fused.pointwise_dwconv_nhwc(x, lin, conv)
+        conv._taps.lookup = look
+        mixed.weight.copy_(conv.weight), mixed.bias.copy_(conv.bias)
+        mid = torch.nn.functional.linear(x.double(), lin.weight.double(), lin.bias.double()).to(torch.bfloat16)
+        _close(got, mixed(mid), torch.bfloat16, "mixed orientations")
+        x[0, 0, 0, 0], x[-1, -1, -1, 2] = float("inf"), float("nan")
+        got, ref = fused.pointwise_dwconv_nhwc(x, lin, conv), layers(True)
+        # (the grouped kernels add up the weights of taps that meet on a pixel, inf (w1 + w2) for inf w1 + inf w2: an
+        # infinity there may be NaN here)
+        assert torch.equal(got.isfinite(), ref.isfinite())
+
+
 @pytest.mark.parametrize("dtype", DTYPES[1:], ids=["bf16", "f16"])
 def test_pointwise_linear_leaves_the_autocast_cache_alone(dtype):
     """Two passes of one autocast region, the second on an input that is differentiated itself (it stays
