@@ -219,13 +219,14 @@ def _norm_type(x, C, norm, consumer):
     return out if x.dtype == out or torch.float32 in (x.dtype, out) else None
 
 
-def _second_order(value, inputs, dout):
-    """Gradients of ``value(*inputs)`` with their own history (a backward pass that is being recorded)."""
-    needed = [t for t in inputs if t.requires_grad]
+def _second_order(value, inputs, needed, dout):
+    """Gradients of ``value(*inputs)`` with their own history (a backward pass that is being recorded), for the inputs that
+    ``needed`` marks: what was saved has to be what ``apply`` was given, a copy made inside ``forward`` has no history."""
+    leaves = [t for t, n in zip(inputs, needed) if n]
     with torch.autocast(dout.device.type, enabled=False):
         y = value(*inputs)
-        got = iter(torch.autograd.grad(y, needed, dout, create_graph=True, allow_unused=True))
-    return [next(got) if t.requires_grad else None for t in inputs]
+        got = iter(torch.autograd.grad(y, leaves, dout, create_graph=True, allow_unused=True))
+    return [next(got) if n else None for n in needed]
 
 
 def _patches(x):
@@ -241,7 +242,6 @@ class _TileNorm(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, b, eps, dtype, patches=False):
         ctx.set_materialize_grads(False)
-        x = x.contiguous()
         out, stats = _lib.host(x.get_device()).ln_tile(x, _f32(w), _f32(b), eps, patches, dtype, True)
         ctx.save_for_backward(x, w, b, stats)
         ctx.eps, ctx.dtype, ctx.patches = eps, dtype, patches
@@ -256,7 +256,7 @@ class _TileNorm(torch.autograd.Function):
             def value(x, w, b):
                 y = F.layer_norm(x.permute(0, 2, 3, 1).float(), w.shape, w.float(), b.float(), ctx.eps)
                 return (_patches(y) if ctx.patches else y).to(ctx.dtype)
-            return (*_second_order(value, (x, w, b), dout), None, None, None)
+            return (*_second_order(value, (x, w, b), ctx.needs_input_grad[:3], dout), None, None, None)
         dx, dw, db = _lib.host(x.get_device()).ln_tile_backward(dout, x, stats, _f32(w), ctx.patches, w.dtype)
         return dx, dw, db.to(b.dtype), None, None, None
 
@@ -267,7 +267,6 @@ class _RowNorm(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, b, eps, gelu, dtype):
         ctx.set_materialize_grads(False)
-        x = x.contiguous()
         out, stats = _lib.host(x.get_device()).ln_rows(x, _f32(w), _f32(b), eps, gelu, dtype, True)
         ctx.save_for_backward(x, w, b, stats)
         ctx.eps, ctx.gelu, ctx.dtype = eps, gelu, dtype
@@ -284,7 +283,7 @@ class _RowNorm(torch.autograd.Function):
                 if ctx.gelu & 2:
                     y = y.to(ctx.dtype).float()
                 return (F.gelu(y) if ctx.gelu else y).to(ctx.dtype)
-            return (*_second_order(value, (x, w, b), dout), None, None, None)
+            return (*_second_order(value, (x, w, b), ctx.needs_input_grad[:3], dout), None, None, None)
         dx, dw, db = _lib.host(x.get_device()).ln_rows_backward(dout, x, stats, _f32(w), _f32(b), ctx.gelu, w.dtype)
         return dx, dw, db.to(b.dtype), None, None, None
 
@@ -296,7 +295,6 @@ class _BlockTail(torch.autograd.Function):
     @staticmethod
     def forward(ctx, y, gamma, x, dtype, rounded):
         ctx.set_materialize_grads(False)
-        y = y.contiguous()
         out = _lib.host(y.get_device()).block_tail(y, None if gamma is None else _f32(gamma), x, dtype, rounded)
         ctx.save_for_backward(*(() if gamma is None else (y, gamma)))
         ctx.types = y.dtype, None if x is None else x.dtype
@@ -317,7 +315,7 @@ class _BlockTail(torch.autograd.Function):
 
             def value(y, gamma):
                 return (gamma * y).permute(0, 3, 1, 2).to(dout.dtype)
-            return (*_second_order(value, (y, gamma), dout), dx, None, None)
+            return (*_second_order(value, (y, gamma), ctx.needs_input_grad[:2], dout), dx, None, None)
         scale, grad = (None, torch.float32) if gamma is None else (_f32(gamma), gamma.dtype)
         dy, dg = _lib.host(dout.get_device()).block_tail_backward(dout, y, scale, dtype, grad)
         return dy, dg, dx, None, None
@@ -391,7 +389,7 @@ def tile_norm(x, norm, consumer=None):
     if not (_recording(x, norm.weight, norm.bias) and x.dim() == 4 and x.numel() < 1 << 31):
         return None
     dtype = _norm_type(x, x.shape[1], norm, consumer)
-    return None if dtype is None else _TileNorm.apply(x, norm.weight, norm.bias, norm.eps, dtype)
+    return None if dtype is None else _TileNorm.apply(x.contiguous(), norm.weight, norm.bias, norm.eps, dtype)
 
 
 def row_norm(x, norm, gelu=False, consumer=None):
@@ -402,7 +400,7 @@ def row_norm(x, norm, gelu=False, consumer=None):
     dtype = _norm_type(x, x.shape[-1], norm, consumer)
     # (without autocast a 16-bit LayerNorm's output is a 16-bit tensor by itself)
     mode = 0 if not gelu else 1 if _autocast(x) is not None or dtype == torch.float32 else 3
-    return None if dtype is None else _RowNorm.apply(x, norm.weight, norm.bias, norm.eps, mode, dtype)
+    return None if dtype is None else _RowNorm.apply(x.contiguous(), norm.weight, norm.bias, norm.eps, mode, dtype)
 
 
 def _tail_covers(y):
@@ -418,13 +416,13 @@ def block_tail(y, gamma, x):
     if dtype not in (y.dtype, torch.float32) or x.dtype not in (y.dtype, dtype):
         return None
     product = torch.promote_types(gamma.dtype, y.dtype)
-    return _BlockTail.apply(y, gamma, x, dtype, product == y.dtype != torch.float32)
+    return _BlockTail.apply(y.contiguous(), gamma, x, dtype, product == y.dtype != torch.float32)
 
 
 def planes(y):
     """``y.permute(0, 3, 1, 2).contiguous()``, recorded by autograd where the kernels cover it."""
     if _recording(y) and _tail_covers(y):
-        return _BlockTail.apply(y, None, None, y.dtype, False)
+        return _BlockTail.apply(y.contiguous(), None, None, y.dtype, False)
     return y.permute(0, 3, 1, 2).contiguous()
 
 
@@ -449,7 +447,7 @@ def downsample(x, norm, conv):
         if ac is None and not (x.dtype == norm.weight.dtype == norm.bias.dtype == w.dtype
                                and (b is None or b.dtype == w.dtype)):
             return None
-        p = _TileNorm.apply(x, norm.weight, norm.bias, norm.eps, dtype, True)
+        p = _TileNorm.apply(x.contiguous(), norm.weight, norm.bias, norm.eps, dtype, True)
         return planes(_Linear.apply(p, rows, b))
     if norm.weight.device != x.device or not _layer16(x.permute(0, 2, 3, 1), w[:, :, 0, 0], b) or not ordinary(w):
         return None

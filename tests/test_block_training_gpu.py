@@ -248,6 +248,54 @@ def test_second_order_of_the_passes(which):
         close(got, ref.double(), 1e-4, which)  # (fp32 on both sides)
 
 
+@pytest.mark.parametrize("which", ["tile", "patch", "rows", "tail", "planes"])
+def test_recorded_backward_of_inputs_that_are_not_dense(which):
+    """Gradients and gradients of gradients of views in another order, through the functions that the modules call, against the
+    composition (fp32 on both sides, the patches' layer in bf16)."""
+    from oriented1d_amd.convnext1d import ChannelsFirstLayerNorm
+    torch.manual_seed(2)
+    a = torch.randn(2, 6, 4, 16, device="cuda", requires_grad=True)
+    w = torch.randn(16, device="cuda", requires_grad=True)
+    norm = (nn.LayerNorm(16, eps=1e-6) if which == "rows" else ChannelsFirstLayerNorm(16)).cuda()
+    conv = nn.Conv2d(16, 24, 2, 2).cuda()
+    planes = a.permute(0, 3, 1, 2)                  # [N,C,H,W], channels last in memory
+    rows = a.permute(0, 2, 1, 3)                    # [N,W,H,C]
+    assert not planes.is_contiguous() and not rows.is_contiguous()
+
+    def normed(x):
+        return F.layer_norm(x, (16,), norm.weight, norm.bias, 1e-6)
+
+    def native():
+        if which == "tile":
+            return norm(planes)
+        if which == "patch":
+            with torch.autocast("cuda", dtype=BF16):
+                return fused.downsample(planes, norm, conv).float()
+        if which == "rows":
+            return fused.row_norm(rows, norm, gelu=True)
+        return fused.block_tail(rows, w, planes.transpose(2, 3)) if which == "tail" else fused.planes(rows)
+
+    def reference():
+        if which == "tile":
+            return normed(planes.permute(0, 2, 3, 1)).permute(0, 3, 1, 2)
+        if which == "patch":
+            return conv(normed(planes.permute(0, 2, 3, 1)).permute(0, 3, 1, 2))
+        if which == "rows":
+            return F.gelu(normed(rows))
+        return planes.transpose(2, 3) + (w * rows).permute(0, 3, 1, 2) if which == "tail" else rows.permute(0, 3, 1, 2)
+
+    params = {"tail": [w], "planes": []}.get(which, [norm.weight, norm.bias])
+    res = []
+    for f in (native, reference):
+        y = f()
+        assert y.grad_fn is not None
+        first = torch.autograd.grad((y ** 3).sum(), [a] + params, create_graph=True)
+        res.append(list(first) + list(torch.autograd.grad(sum((t * t).sum() for t in first), [a] + params)))
+    # (fp32 sums in another order; a chain of four 16-bit products behind the patches)
+    for got, ref in zip(*res):
+        close(got, ref.double(), 5e-2 if which == "patch" else 1e-4, which)
+
+
 def test_hooks_and_replaced_forwards_keep_the_module_path():
     from oriented1d_amd.convnext1d import Block
     torch.manual_seed(0)
