@@ -323,46 +323,47 @@ class _BlockTail(torch.autograd.Function):
 
 class _Linear(torch.autograd.Function):
     """``F.linear`` over 16-bit activations whose parameter gradients come from ``dwo_linear_wgrad``, in the parameters'
-    own type."""
+    own type.  ``wc`` is w in x's type where w has another one: an input of its own, so that the copy of the forward pass is
+    what the backward pass reads, with its history where that pass is recorded; w takes the whole gradient otherwise."""
 
     @staticmethod
-    def forward(ctx, x, w, b):
+    def forward(ctx, x, w, wc, b):
         ctx.set_materialize_grads(False)
-        # (conversions as autocast makes them, but not kept for the rest of its region: gradients are off here, and
-        # such copies would be cut off from the parameters)
-        wc, bc = w.to(x.dtype), b if b is None else b.to(x.dtype)
-        y = F.linear(x, wc, bc)
-        # (only what backward reads: the parameters themselves may be updated between the passes where the input
-        # takes no gradient, and always where they were converted)
-        need = ctx.needs_input_grad[0]
-        ctx.save_for_backward(x, wc if need else None)
-        ctx.weight = w if need and wc is not w else None
+        wc = w if wc is None else wc
+        y = F.linear(x, wc, b if b is None else b.to(x.dtype))
+        # (only what backward reads: parameters may be updated between the passes where the input takes no gradient, and
+        # always where they were converted)
+        ctx.save_for_backward(x, wc if ctx.needs_input_grad[0] else None)
         ctx.w_dtype, ctx.b_dtype = w.dtype, b.dtype if b is not None else None
         return y
 
     @staticmethod
     def backward(ctx, dy):
         if dy is None:
-            return None, None, None
+            return None, None, None, None
         x, wc = ctx.saved_tensors
         dx = dw = db = None
-        need_db = ctx.b_dtype is not None and ctx.needs_input_grad[2]
-        if torch.is_grad_enabled():  # gradients of gradients: with the history of x and of the weights themselves
-            if ctx.needs_input_grad[0]:
-                dx = torch.matmul(dy, wc if ctx.weight is None else ctx.weight.to(dy.dtype))
+        need_db = ctx.b_dtype is not None and ctx.needs_input_grad[3]
+        if ctx.needs_input_grad[0]:
+            dx = torch.matmul(dy, wc)
+        if torch.is_grad_enabled():  # gradients of gradients: with the history of x and of the weights
             rows = dy.reshape(-1, dy.shape[-1])
             if ctx.needs_input_grad[1]:
                 dw = torch.matmul(rows.t(), x.reshape(-1, x.shape[-1])).to(ctx.w_dtype)
             if need_db:
                 db = rows.sum(0).to(ctx.b_dtype)
-            return dx, dw, db
-        if ctx.needs_input_grad[0]:
-            dx = torch.matmul(dy, wc)
+            return dx, dw, None, db
         if ctx.needs_input_grad[1] or need_db:
             dw, db = _lib.host(x.get_device()).linear_wgrad(dy, x, need_db, ctx.w_dtype)
             if need_db and ctx.b_dtype != ctx.w_dtype:
                 db = db.to(ctx.b_dtype)
-        return dx, dw if ctx.needs_input_grad[1] else None, db
+        return dx, dw if ctx.needs_input_grad[1] else None, None, db
+
+
+def _linear16(x, w, b):
+    """``F.linear(x, w, b)`` for a 16-bit x and parameters of any type.  (Conversions as autocast makes them, recorded, but
+    not kept for the rest of its region.)"""
+    return _Linear.apply(x, w, None if w.dtype == x.dtype else w.to(x.dtype), b)
 
 
 class Linear(torch.nn.Linear):
@@ -378,7 +379,7 @@ class Linear(torch.nn.Linear):
             dtype = ac or x.dtype
             if dtype in (torch.bfloat16, torch.float16) and (
                     ac is not None or (x.dtype == w.dtype and (b is None or b.dtype == w.dtype))):
-                return _Linear.apply(x.to(dtype), w, b)
+                return _linear16(x.to(dtype), w, b)
         return F.linear(x, w, b)
 
 
@@ -448,7 +449,7 @@ def downsample(x, norm, conv):
                                and (b is None or b.dtype == w.dtype)):
             return None
         p = _TileNorm.apply(x.contiguous(), norm.weight, norm.bias, norm.eps, dtype, True)
-        return planes(_Linear.apply(p, rows, b))
+        return planes(_linear16(p, rows, b))
     if norm.weight.device != x.device or not _layer16(x.permute(0, 2, 3, 1), w[:, :, 0, 0], b) or not ordinary(w):
         return None
     host = _lib.host(x.get_device())

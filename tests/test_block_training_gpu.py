@@ -296,6 +296,31 @@ def test_recorded_backward_of_inputs_that_are_not_dense(which):
         close(got, ref.double(), 5e-2 if which == "patch" else 1e-4, which)
 
 
+def test_recorded_backward_takes_the_weights_of_the_forward_pass():
+    """Parameters that autocast converts may be updated between the passes, as with PyTorch's own layers: their 16-bit copies of the
+    forward pass are what every backward pass differentiates."""
+    from oriented1d_amd.convnext1d import ChannelsFirstLayerNorm
+    torch.manual_seed(6)
+    lin, norm, conv = fused.Linear(16, 8).cuda(), ChannelsFirstLayerNorm(16).cuda(), nn.Conv2d(16, 8, 2, 2).cuda()
+    for layer, weight, shape in ((lin, lin.weight, (4, 16)), (lambda x: fused.downsample(x, norm, conv), conv.weight, (1, 16, 4, 4))):
+        x = torch.randn(*shape, device="cuda", requires_grad=True)
+
+        def run(recorded, factor):
+            with torch.autocast("cuda", dtype=BF16):
+                y = layer(x)
+            with torch.no_grad():
+                weight.mul_(factor)
+            g, = torch.autograd.grad(y.float().square().sum(), x, create_graph=recorded)
+            h = torch.autograd.grad(g.square().sum(), (x, weight)) if recorded else ()
+            with torch.no_grad():
+                weight.mul_(1.0 / factor)
+            return [g, *h]
+        (plain,), kept, doubled = run(False, 2.0), run(True, 1.0), run(True, 2.0)
+        close(kept[0], plain.double(), 2 * TOL[BF16], "dx")  # (products in 16 bits on both sides)
+        for got, ref in zip(doubled, kept):
+            assert torch.equal(got, ref)
+
+
 def test_hooks_and_replaced_forwards_keep_the_module_path():
     from oriented1d_amd.convnext1d import Block
     torch.manual_seed(0)
