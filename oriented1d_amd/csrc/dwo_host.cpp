@@ -247,14 +247,15 @@ std::tuple<Tensor, OptTensor> wgrad_entry(const Tensor &dy, const Tensor &x, con
 }
 
 // The operator as a node of autograd (the contract of models/dwoconv1d/dwoconv1d.py:18-69): gradients of x, w and bias, none
-// of theta.  w32 and bias32 are fp32 copies where the parameters are not dense fp32 themselves; resid is added to the weights.
+// of theta, which is an input all the same: data-parallel wrappers wait for every parameter that takes gradients and
+// is not part of the graph.  w32 and bias32 are fp32 copies where the parameters are not dense fp32 themselves; resid is added to the weights.
 struct Convolution : torch::autograd::Function<Convolution> {
     using Context = torch::autograd::AutogradContext;
     using List = torch::autograd::variable_list;
 
     static Tensor forward(Context *ctx, const Tensor &x_, const Tensor &w, const OptTensor &bias, const OptTensor &w32,
-                          const OptTensor &bias32, const OptTensor &resid, const Tensor &taps, int64_t stride,
-                          int64_t layout) {
+                          const OptTensor &bias32, const OptTensor &resid, const Tensor &taps, const Tensor & /*theta*/,
+                          int64_t stride, int64_t layout) {
         ctx->set_materialize_grads(false);
         const Tensor x = x_.contiguous();
         Tensor weights = w32.has_value() ? *w32 : w;
@@ -267,7 +268,7 @@ struct Convolution : torch::autograd::Function<Convolution> {
     }
 
     static List backward(Context *ctx, const List &grads) {
-        List out(9);
+        List out(10);
         if (!grads[0].defined()) return out;
         const List saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &weights = saved[1], &taps = saved[2];
@@ -292,9 +293,10 @@ struct Convolution : torch::autograd::Function<Convolution> {
 };
 
 Tensor convolution(const Tensor &x, const Tensor &w, const OptTensor &bias, const OptTensor &w32,
-                   const OptTensor &bias32, const OptTensor &resid, const Tensor &taps, int64_t stride, int64_t layout) {
+                   const OptTensor &bias32, const OptTensor &resid, const Tensor &taps, const Tensor &theta,
+                   int64_t stride, int64_t layout) {
     py::gil_scoped_release nogil;
-    return Convolution::apply(x, w, bias, w32, bias32, resid, taps, stride, layout);
+    return Convolution::apply(x, w, bias, w32, bias32, resid, taps, theta, stride, layout);
 }
 
 void check_glue(const Tensor &t, const char *name) {

@@ -345,9 +345,6 @@ def _native_covers(x, w, theta, bias, resid, module, nhwc):
             and (bias is None or bias.device == x.device) and (resid is None or resid.device == x.device)
             and ordinary(x, w, theta, bias, resid)):
         return False
-    if theta.requires_grad and torch.is_grad_enabled() and not (
-            x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)):
-        return False  # (a graph for theta alone, which never receives a gradient)
     _, C, H, W = _dims(x, nhwc)
     return C == w.shape[0] and (module.arbitrary_size or (H % module.stride == 0 and W % module.stride == 0))
 
@@ -448,6 +445,6 @@ class DepthwiseOrientedConv1d(nn.Conv2d):
             taps, layouts = module.taps.lookup(theta, C, K, x.device)
             return _lib.host(x.get_device()).convolution(
                 x, w, bias, None if _is_f32(w) else f32_copy(w),
-                None if bias is None or _is_f32(bias) else f32_copy(bias), resid, taps, module.stride,
+                None if bias is None or _is_f32(bias) else f32_copy(bias), resid, taps, theta, module.stride,
                 layouts[x.element_size()] if nhwc else _lib.NCHW)
         return _DepthwiseOrientedConv1d.apply(x, w, theta, bias, module, self.nhwc, resid)

@@ -287,3 +287,22 @@ def test_native_node_keeps_autograd_rules():
         assert torch.equal(m(x), y)
     with pytest.raises(RuntimeError, match="channels"):
         m(torch.randn(2, 8, 9, 11, device="cuda"))
+
+
+@pytest.mark.parametrize("nhwc", [False, True])
+def test_angles_are_part_of_the_graph(nhwc):
+    """theta gets no gradient, but the node reaches it (as the Python function's does): a data-parallel wrapper that looks for
+    unused parameters only where it is asked to waits for every parameter that takes gradients."""
+    m = DepthwiseOrientedConv1d(16, 16, 7, groups=16, padding=3, angle=0.3, nhwc=nhwc, resid=nhwc, arbitrary_size=True).cuda()
+    x = torch.randn(2, 16, 16, 16, device="cuda")
+    y = m(x)
+    assert "_DepthwiseOrientedConv1d" not in type(y.grad_fn).__name__
+    reached = [n for n, _ in y.grad_fn.next_functions if hasattr(n, "variable")]
+    assert {id(n.variable) for n in reached} == {id(p) for p in (m.weight, m.bias, m.theta)}
+    called = []
+    handles = [n.register_hook(lambda *a, n=n: called.append(id(n.variable))) for n in reached]
+    y.sum().backward()
+    for h in handles:
+        h.remove()
+    assert sorted(called) == sorted(id(p) for p in (m.weight, m.bias, m.theta))
+    assert m.theta.grad is None and m.weight.grad is not None and m.bias.grad is not None
