@@ -304,8 +304,20 @@ void check_glue(const Tensor &t, const char *name) {
         fail(std::string(name) + " must be a CUDA tensor of type float32, bfloat16 or float16");
 }
 
+// gamma, beta or a layer scale, which the kernels read as C dense floats
+void check_channels(const Tensor &x, const Tensor &p, int64_t C, const char *name) {
+    if (p.device() != x.device() || p.scalar_type() != at::kFloat || !p.is_contiguous() || p.numel() != C)
+        fail(std::string(name) + " must be " + std::to_string(C) + " contiguous float32 values on x's device");
+}
+void check_norm(const Tensor &x, const Tensor &g, const Tensor &b, int64_t C) {
+    check_channels(x, g, C, "weight");
+    check_channels(x, b, C, "bias");
+}
+
 Tensor layernorm_nhwc(const Tensor &x_, const Tensor &g, const Tensor &b, double eps, bool gelu) {
     check_glue(x_, "x");
+    if (x_.dim() < 1) fail("x must have a dimension of channels");
+    check_norm(x_, g, b, x_.size(-1));
     py::gil_scoped_release nogil;
     const Place at(x_);
     const Tensor x = x_.contiguous();
@@ -321,6 +333,7 @@ Tensor layernorm_nhwc(const Tensor &x_, const Tensor &g, const Tensor &b, double
 Tensor nchw_layernorm_nhwc(const Tensor &x_, const Tensor &g, const Tensor &b, double eps) {
     check_glue(x_, "x");
     if (x_.dim() != 4) throw py::value_error("x must be a 4-d tensor");
+    check_norm(x_, g, b, x_.size(1));
     py::gil_scoped_release nogil;
     const Place at(x_);
     const Tensor x = x_.contiguous();
@@ -336,6 +349,7 @@ Tensor nchw_layernorm_nhwc(const Tensor &x_, const Tensor &g, const Tensor &b, d
 Tensor nhwc_scale_add_nchw(const Tensor &y_, const OptTensor &scale, const OptTensor &residual) {
     check_glue(y_, "y");
     if (y_.dim() != 4) throw py::value_error("y must be a 4-d tensor");
+    if (scale.has_value()) check_channels(y_, *scale, y_.size(3), "scale");
     py::gil_scoped_release nogil;
     const Place at(y_);
     const Tensor y = y_.contiguous();
@@ -448,6 +462,8 @@ Tensor pointwise_forward(const Tensor &x_, const Tensor &w_, const OptTensor &b)
 std::tuple<Tensor, OptTensor> ln_rows(const Tensor &x_, const Tensor &g, const Tensor &b, double eps, int64_t gelu,
                                       at::ScalarType out_dtype, bool with_stats) {
     check_glue(x_, "x");
+    if (x_.dim() < 1) fail("x must have a dimension of channels");
+    check_norm(x_, g, b, x_.size(-1));
     py::gil_scoped_release nogil;
     const Place at(x_);
     const Tensor x = dense(x_);
@@ -468,6 +484,7 @@ std::tuple<Tensor, Tensor, Tensor> ln_rows_backward(const Tensor &dout_, const T
     check_glue(x_, "x");
     check_pair(dout_, x_);
     if (dout_.sizes() != x_.sizes()) fail("dout and x must have the same shape");
+    check_norm(x_, g, b, x_.size(-1));
     py::gil_scoped_release nogil;
     const Place at(x_);
     const Tensor x = dense(x_), dout = dense(dout_);
@@ -489,6 +506,7 @@ std::tuple<Tensor, OptTensor> ln_tile(const Tensor &x_, const Tensor &g, const T
                                       at::ScalarType out_dtype, bool with_stats) {
     check_glue(x_, "x");
     if (x_.dim() != 4) throw py::value_error("x must be a 4-d tensor");
+    check_norm(x_, g, b, x_.size(1));
     py::gil_scoped_release nogil;
     const Place at(x_);
     const Tensor x = dense(x_);
@@ -512,6 +530,7 @@ std::tuple<Tensor, Tensor, Tensor> ln_tile_backward(const Tensor &dout_, const T
     check_glue(x_, "x");
     check_pair(dout_, x_);
     const Dims d(x_, false);
+    check_channels(x_, g, d.c, "weight");
     const std::array<int64_t, 4> want = patches ? std::array<int64_t, 4>{d.n, d.h / 2, d.w / 2, 4 * d.c}
                                                 : std::array<int64_t, 4>{d.n, d.h, d.w, d.c};
     if (dout_.sizes() != at::IntArrayRef(want)) fail("dout does not match x");
@@ -537,6 +556,7 @@ Tensor block_tail(const Tensor &y_, const OptTensor &scale, const OptTensor &res
     check_glue(y_, "y");
     if (y_.dim() != 4) throw py::value_error("y must be a 4-d tensor");
     const Dims d(y_, true);
+    if (scale.has_value()) check_channels(y_, *scale, d.c, "scale");
     const std::array<int64_t, 4> shape = {d.n, d.c, d.h, d.w};
     if (res_.has_value()) {
         check_glue(*res_, "res");
@@ -561,6 +581,7 @@ std::tuple<Tensor, OptTensor> block_tail_backward(const Tensor &dout_, const Opt
     check_glue(dout_, "dout");
     if (dout_.dim() != 4) throw py::value_error("dout must be a 4-d tensor");
     const Dims d(dout_, false);
+    if (scale.has_value()) check_channels(dout_, *scale, d.c, "scale");
     const std::array<int64_t, 4> shape = {d.n, d.h, d.w, d.c};
     if (y_.has_value()) {
         check_glue(*y_, "y");

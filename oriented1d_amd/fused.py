@@ -435,7 +435,8 @@ def downsample(x, norm, conv):
             and conv.dilation == (1, 1) and conv.groups == 1 and conv.padding_mode == "zeros"
             and x.dim() == 4 and x.is_cuda and min(x.shape[2:]) >= 2 and 0 < x.numel() < 1 << 31
             and w.shape[1] == x.shape[1] and w.shape[0] % 8 == 0 and x.shape[1] % 8 == 0 and x.shape[1] <= MAX_C_TRAIN
-            and w.shape[0] <= MAX_C_TRAIN and w.is_contiguous()):
+            and w.shape[0] <= MAX_C_TRAIN and w.is_contiguous()
+            and norm.weight.shape == norm.bias.shape == x.shape[1:2]):
         return None
     rows = w.view(w.shape[0], -1)
     if torch.is_grad_enabled():

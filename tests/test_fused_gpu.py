@@ -400,3 +400,37 @@ def test_block_mlp(N, H, W, scaled, C, dtype):
         fused._lib.host(0).block_mlp(x, w1[:, :8], b1, w2, b2, s, res)
     with pytest.raises(RuntimeError):
         fused._lib.host(0).block_mlp(x, w1, b1, w2, b2, s, res.float())
+
+
+def test_parameters_of_another_length_are_refused():
+    """The kernels read as many values as x has channels: what is shorter, on the host or not fp32 is refused before a launch."""
+    from oriented1d_amd import _lib
+    from oriented1d_amd.convnext1d import ChannelsFirstLayerNorm
+    host, dt = _lib.host(0), torch.bfloat16
+    x, rows = torch.randn(2, 16, 4, 4, device="cuda").to(dt), torch.randn(5, 16, device="cuda").to(dt)
+    good, stats = torch.ones(16, device="cuda"), torch.zeros(32, 2, device="cuda")
+    nhwc, patches = x.permute(0, 2, 3, 1).contiguous(), torch.randn(2, 2, 2, 64, device="cuda").to(dt)
+    for bad in (torch.ones(8, device="cuda"), torch.ones(16), torch.ones(16, device="cuda", dtype=dt),
+                torch.ones(16, 2, device="cuda")[:, 0]):
+        for call in (lambda: host.layernorm_nhwc(rows, bad, good, 1e-6, False),
+                     lambda: host.layernorm_nhwc(rows, good, bad, 1e-6, True),
+                     lambda: host.nchw_layernorm_nhwc(x, bad, good, 1e-6),
+                     lambda: host.nhwc_scale_add_nchw(nhwc, bad, None),
+                     lambda: host.ln_rows(rows, good, bad, 1e-6, 0, dt, True),
+                     lambda: host.ln_rows_backward(rows, rows, stats, bad, good, 0, torch.float32),
+                     lambda: host.ln_tile(x, bad, good, 1e-6, False, dt, True),
+                     lambda: host.ln_tile_backward(nhwc, x, stats, bad, False, torch.float32),
+                     lambda: host.ln_tile_backward(patches, x, stats, bad, True, torch.float32),
+                     lambda: host.block_tail(nhwc, bad, x, dt, False),
+                     lambda: host.block_tail_backward(x, nhwc, bad, dt, torch.float32)):
+            with pytest.raises(RuntimeError, match="contiguous float32 values"):
+                call()
+    # a norm of half the channels in front of a downsampling layer: as F.layer_norm refuses it
+    norm, conv = ChannelsFirstLayerNorm(8).cuda().to(dt), torch.nn.Conv2d(16, 24, 2, 2).cuda().to(dt)
+    assert fused.downsample(x, norm, conv) is None
+    with pytest.raises(RuntimeError):
+        norm(x)
+    with torch.no_grad():
+        assert fused.downsample(x, norm, conv) is None
+        with pytest.raises(RuntimeError):
+            norm(x)
