@@ -434,20 +434,27 @@ std::tuple<Tensor, OptTensor> linear_wgrad(const Tensor &dy_, const Tensor &x_, 
 }
 
 const void *optr(const OptTensor &t) { return t.has_value() ? t->const_data_ptr() : nullptr; }
-void check_layer(const Tensor &x, const Tensor &w, const OptTensor &b) {
+void check_layer(const Tensor &x, const Tensor &w) {
     check_glue(x, "x");
     check_pair(x, w);
     if (w.dim() != 2 || w.size(1) != x.size(-1) || w.scalar_type() != x.scalar_type())
         fail("w must be [N, K] of the same type as x");
-    if (b.has_value() && (b->numel() != w.size(0) || b->scalar_type() != x.scalar_type() || !b->is_contiguous()))
-        fail("bias must be [N] of the same type as x");
+}
+// a bias or layer scale of n values of x's type, dense (a parameter may be a view with a stride)
+OptTensor dense_values(const Tensor &x, const OptTensor &t, int64_t n, const char *name) {
+    if (!t.has_value()) return t;
+    check_pair(x, *t);
+    if (t->numel() != n || t->scalar_type() != x.scalar_type())
+        fail(std::string(name) + " must be " + std::to_string(n) + " values of the same type as x");
+    return t->contiguous();
 }
 
 // x [.., Cin] -> [.., C]: x w^T + b, all of one type
-Tensor pointwise_forward(const Tensor &x_, const Tensor &w_, const OptTensor &b) {
-    check_layer(x_, w_, b);
+Tensor pointwise_forward(const Tensor &x_, const Tensor &w_, const OptTensor &b_) {
+    check_layer(x_, w_);
     py::gil_scoped_release nogil;
     const Place at(x_);
+    const OptTensor b = dense_values(x_, b_, w_.size(0), "bias");
     const Tensor x = x_.contiguous(), w = w_.contiguous();
     auto shape = x.sizes().vec();
     shape.back() = w.size(0);
@@ -610,10 +617,11 @@ std::tuple<Tensor, OptTensor> block_tail_backward(const Tensor &dout_, const Opt
 }
 
 // act(x w^T + b) over the last dimension
-Tensor linear_rows(const Tensor &x_, const Tensor &w_, const OptTensor &b, bool gelu) {
-    check_layer(x_, w_, b);
+Tensor linear_rows(const Tensor &x_, const Tensor &w_, const OptTensor &b_, bool gelu) {
+    check_layer(x_, w_);
     py::gil_scoped_release nogil;
     const Place at(x_);
+    const OptTensor b = dense_values(x_, b_, w_.size(0), "bias");
     const Tensor x = dense(x_), w = dense(w_);
     const int64_t N = w.size(0), K = w.size(1);
     auto shape = x.sizes().vec();
@@ -626,19 +634,19 @@ Tensor linear_rows(const Tensor &x_, const Tensor &w_, const OptTensor &b, bool 
 }
 
 // x [N,H,W,K] -> [N,C,H,W]: res + scale * (x w^T + b)
-Tensor linear_planes(const Tensor &x_, const Tensor &w_, const OptTensor &b, const OptTensor &scale,
+Tensor linear_planes(const Tensor &x_, const Tensor &w_, const OptTensor &b_, const OptTensor &scale_,
                      const OptTensor &res_) {
-    check_layer(x_, w_, b);
+    check_layer(x_, w_);
     if (x_.dim() != 4) throw py::value_error("x must be a 4-d tensor");
     const int64_t C = w_.size(0), K = w_.size(1);
-    if (scale.has_value() && (scale->numel() != C || scale->scalar_type() != x_.scalar_type() || !scale->is_contiguous()))
-        fail("scale must be [C] of the same type as x");
     const Dims d(x_, true);
     py::gil_scoped_release nogil;
     const Place at(x_);
+    const OptTensor b = dense_values(x_, b_, C, "bias"), scale = dense_values(x_, scale_, C, "scale");
     const Tensor x = dense(x_), w = dense(w_);
     Tensor out = at::empty({d.n, C, d.h, d.w}, x.options()), res;
     if (res_.has_value()) {
+        check_pair(x_, *res_);
         if (res_->sizes() != out.sizes() || res_->scalar_type() != x.scalar_type())
             fail("residual must be [N,C,H,W] of the same type as x");
         res = dense(*res_);
@@ -650,28 +658,26 @@ Tensor linear_planes(const Tensor &x_, const Tensor &w_, const OptTensor &b, con
 }
 
 // x [N,H,W,C], res [N,C,H,W] -> res + scale * (w2 gelu(w1 x + b1) + b2), planes
-Tensor block_mlp(const Tensor &x_, const Tensor &w1_, const Tensor &b1, const Tensor &w2_, const Tensor &b2,
-                 const OptTensor &scale, const Tensor &res_) {
-    check_layer(x_, w1_, b1);
-    check_layer(x_, w1_, std::nullopt);
+Tensor block_mlp(const Tensor &x_, const Tensor &w1_, const Tensor &b1_, const Tensor &w2_, const Tensor &b2_,
+                 const OptTensor &scale_, const Tensor &res_) {
+    check_layer(x_, w1_);
     if (x_.dim() != 4) throw py::value_error("x must be a 4-d tensor");
     const int64_t C = x_.size(3);
     if (w1_.size(0) != 4 * C || w2_.dim() != 2 || w2_.size(0) != C || w2_.size(1) != 4 * C ||
-        w2_.scalar_type() != x_.scalar_type() || b2.numel() != C || b2.scalar_type() != x_.scalar_type() ||
-        !b2.is_contiguous())
-        fail("w1 must be [4C, C], w2 [C, 4C] and b2 [C], of the same type as x");
-    if (scale.has_value() && (scale->numel() != C || scale->scalar_type() != x_.scalar_type() || !scale->is_contiguous()))
-        fail("scale must be [C] of the same type as x");
+        w2_.scalar_type() != x_.scalar_type())
+        fail("w1 must be [4C, C] and w2 [C, 4C], of the same type as x");
     const Dims d(x_, true);
     const std::array<int64_t, 4> shape = {d.n, d.c, d.h, d.w};
     if (res_.sizes() != at::IntArrayRef(shape) || res_.scalar_type() != x_.scalar_type())
         fail("residual must be [N,C,H,W] of the same type as x");
-    check_pair(x_, w2_), check_pair(x_, b2), check_pair(x_, res_);
+    check_pair(x_, w2_), check_pair(x_, res_);
     py::gil_scoped_release nogil;
     const Place at(x_);
-    const Tensor x = dense(x_), w1 = dense(w1_), w2 = dense(w2_), c1 = dense(b1), res = dense(res_);
+    const OptTensor b1 = dense_values(x_, b1_, 4 * C, "first bias"), b2 = dense_values(x_, b2_, C, "second bias"),
+                    scale = dense_values(x_, scale_, C, "scale");
+    const Tensor x = dense(x_), w1 = dense(w1_), w2 = dense(w2_), c1 = dense(*b1), res = dense(res_);
     Tensor out = at::empty(shape, x.options());
-    check(lib.block_mlp(ptr(x), ptr(w1), ptr(c1), ptr(w2), ptr(b2), optr(scale), ptr(res), out.data_ptr(), as_int(d.n),
+    check(lib.block_mlp(ptr(x), ptr(w1), ptr(c1), ptr(w2), optr(b2), optr(scale), ptr(res), out.data_ptr(), as_int(d.n),
                         as_int(d.h * d.w), as_int(C), dtype_code(x), at.stream),
           "dwo_block_mlp");
     return out;

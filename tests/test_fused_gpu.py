@@ -434,3 +434,32 @@ def test_parameters_of_another_length_are_refused():
         assert fused.downsample(x, norm, conv) is None
         with pytest.raises(RuntimeError):
             norm(x)
+
+
+@pytest.mark.parametrize("which", ["first bias", "second bias", "layer scale", "stem bias"])
+@pytest.mark.parametrize("rows", [4, 112])
+def test_parameters_that_are_not_dense(which, rows):
+    """Biases and layer scales that are views with a stride, in a block at inference (two kernels, one kernel) and in the stem's
+    first layer in training: the values of dense ones."""
+    from oriented1d_amd.convnext1d import Block
+    torch.manual_seed(rows)
+    dt = torch.bfloat16
+    block = Block(96, (7,), False, layer_scale_init_value=1.0, arbitrary_size=True).cuda().to(dt).eval()
+    stem = torch.nn.Linear(3, 64).cuda().to(dt)
+    owner, name = {"first bias": (block.pwconv1, "bias"), "second bias": (block.pwconv2, "bias"),
+                   "layer scale": (block, "gamma"), "stem bias": (stem, "bias")}[which]
+    n = getattr(owner, name).numel()
+    x = torch.randn(1, 96, rows, 112, device="cuda").to(dt)
+    px = torch.randn(1, rows, 112, 3, device="cuda").to(dt)
+
+    def outputs():
+        with torch.no_grad():
+            y = block(x)
+        return y, fused.pointwise_linear(px, stem).detach()
+    wide = torch.randn(n, 3, device="cuda").to(dt)
+    setattr(owner, name, torch.nn.Parameter(wide[:, 1]))
+    assert not getattr(owner, name).is_contiguous()
+    got = outputs()
+    setattr(owner, name, torch.nn.Parameter(wide[:, 1].contiguous()))
+    for a, b in zip(got, outputs()):
+        assert torch.equal(a, b)
