@@ -251,7 +251,8 @@ __global__ __launch_bounds__(kBlkThreads) void ln_rows_backward_kernel(
                 if ((gelu & ROWS_GELU) && ok) {
                     float u = __builtin_fmaf(h[k][i], gm[k][i], bt[k][i]);
                     if (gelu & ROWS_ROUNDED) u = rounded<TO>(u);
-                    g[k][i] *= sizeof(TI) == 2 ? gelu_slope_rounded(u) : blk_gelu_slope(u);
+                    // (a gradient that stays in 32 bits takes erff's slope)
+                    g[k][i] *= sizeof(TO) == 2 && (gelu & ROWS_ROUNDED) ? gelu_slope_rounded(u) : blk_gelu_slope(u);
                     if (gelu & ROWS_ROUNDED) g[k][i] = rounded<TO>(g[k][i]);
                 }
                 dg[k][i] = __builtin_fmaf(g[k][i], h[k][i], dg[k][i]);

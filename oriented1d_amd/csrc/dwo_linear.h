@@ -245,6 +245,21 @@ struct LinearArgs {
     int N, K, HW, gelu;
 };
 
+// GELU of a sum that nothing has rounded, with erf from Abramowitz and Stegun, Handbook of Mathematical Functions, 7.1.26 (error
+// of erf below 1.5e-7): |u| (1/2 - q) + u / 2 with q = erfc(|u| / sqrt 2) / 2.  Two issue slots less than gelu_rounded, whose
+// tail is exact to the result's rounding; here a separate layer's rounding of u, which the tail magnifies by u^2, is gone, and is
+// worth ten times the difference (mean relative error on [-4, -3], separate layers / this, bf16 1.3e-2 / 1.4e-3, fp16 1.7e-3 / 2.5e-4).  gelu_rounded
+// here: 401408 x 384 x 96 in 178 us instead of 174, a block of 100352 x 192 in 132 instead of 127.  Infinities and NaN give what u * (1 + erf) gives.
+__device__ __forceinline__ float lin_gelu(float u) {
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_fabsf(u), 0.3275911f * 0.70710678118654752f, 1.f));
+    float p = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
+    p = __builtin_fmaf(t, p, 0.5f * 1.421413741f);
+    p = __builtin_fmaf(t, p, 0.5f * -0.284496736f);
+    p = __builtin_fmaf(t, p, 0.5f * 0.254829592f);
+    const float q = p * t * __builtin_amdgcn_exp2f(u * u * -0.72134752044448170f);  // exp(-u^2 / 2)
+    return __builtin_fmaf(__builtin_fabsf(u), 0.5f - q, 0.5f * u);
+}
+
 typedef unsigned mma_u2 __attribute__((ext_vector_type(2)));
 template <typename T>
 __device__ __forceinline__ unsigned lin_pack(float a, float b) {
@@ -263,7 +278,7 @@ __device__ __forceinline__ void lin_emit_rows(const LinearArgs<T> &a, long m, in
 #pragma unroll
     for (int r = 0; r < Q; r++) {
         v[r] += b[r];
-        if (a.gelu) v[r] = gelu_rounded(v[r]);
+        if (a.gelu) v[r] = lin_gelu(v[r]);
     }
     T *at = a.out + m * a.N + n;
     if constexpr (Q == 8)

@@ -146,7 +146,7 @@ __global__ __launch_bounds__(Mlp<C>::THREADS, 2) void mlp_kernel(MlpArgs<T> a) {
             mma_u4 v;
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                v[e] = lin_pack<T>(gelu_rounded(h[e / 2][p][2 * e % 4]), gelu_rounded(h[e / 2][p][2 * e % 4 + 1]));
+                v[e] = lin_pack<T>(lin_gelu(h[e / 2][p][2 * e % 4]), lin_gelu(h[e / 2][p][2 * e % 4 + 1]));
             hb[p] = __builtin_bit_cast(mma_s8, v);
         }
         __builtin_amdgcn_sched_barrier(0);

@@ -463,3 +463,26 @@ def test_parameters_that_are_not_dense(which, rows):
     setattr(owner, name, torch.nn.Parameter(wide[:, 1].contiguous()))
     for a, b in zip(got, outputs()):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype,unit", [(torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11)], ids=["bf16", "f16"])
+def test_gelu_of_the_negative_tail(dtype, unit):
+    """GELU value by value, as far as results are normal numbers.  Behind LayerNorm: the rounding of the result (``unit`` of it)
+    and 2 % for what GELU takes, whose fp32 rounding the tail magnifies (relative slope about u^2 <= 16).  In a product
+    kernel no more than separate layers, whose u is rounded first: units of the result, and u^2 of them."""
+    from oriented1d_amd import _lib
+    torch.manual_seed(0)
+    x = torch.randn(20000, 64, device="cuda").to(dtype)
+    w, b = torch.full((64,), 2.0, device="cuda"), torch.full((64,), -1.0, device="cuda")
+    host = _lib.host(0)
+    u1 = (-4 + 8 * torch.rand(4096, 8, device="cuda")).to(dtype)  # a product of one term: u is what the kernel holds
+    for u, y, bound in (
+            (F.layer_norm(x.double(), (64,), w.double(), b.double(), 1e-6), host.ln_rows(x, w, b, 1e-6, 1, dtype, False)[0],
+             lambda u: 1.02 * unit),
+            (u1.double(), host.linear_rows(u1, torch.eye(8, device="cuda").to(dtype), None, True),
+             lambda u: (1 + u * u) * unit)):
+        ref = u * torch.special.erfc(-u * 0.5 ** 0.5) / 2
+        # (normal results; around zero the sum of LayerNorm's scale and shift cancels)
+        some = (u.abs() >= 0.25) & (u.abs() <= 4) & (ref.abs() >= 2.0 ** -14)
+        assert (u[some] < -3).sum() > 100
+        assert (((y.double() - ref).abs() / ref.abs()) <= bound(u))[some].all()
