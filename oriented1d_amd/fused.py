@@ -102,16 +102,27 @@ def linear_tail(x, linear, gamma, residual):
 
 
 # Rows from which both layers run as one kernel: enough workgroups of 128 pixels that its long chain is paid for (bf16, us, two
-# kernels / one: 12544 x 96 25 / 18, 6272 x 96 14 / 18; 100352 x 192 160 / 124, 25088 x 192 46 / 46; 25088 x 384 120 / 105,
-# 12544 x 384 65 / 100)
-_MLP_ROWS = {96: 12288, 128: 16384, 192: 28672, 384: 24576}
+# kernels / one: 12544 x 96 25 / 17, 8192 x 96 15.9 / 16.8; 16384 x 128 21 / 25, 17408 x 128, where the first product has more
+# tiles than the chip holds, 30 / 25; 29008 x 192 47 / 43, 25088 x 192 43 / 42 and in odd planes 67 / 70).  There is no instance for
+# 256 channels.
+_MLP_ROWS = {96: 12288, 128: 16385, 192: 28672}
+# At 384 channels a workgroup has a CU to itself (101 KB of LDS): its time goes in rounds of 256 workgroups, about 95 us each, and
+# the last round pays from two thirds on (20384 rows 85 / 98, 22540 115 / 97, 32732 151 / 109, 32928 155 / 191, 39984 186 / 192, 42924
+# 192 / 193, 43904 217 / 192, 66052 314 / 309)
+_MLP_ROUND = 32768
+
+
+def _mlp_pays(rows, C):
+    if C == 384:
+        return 3 * rows >= 2 * _MLP_ROUND * -(-rows // _MLP_ROUND)
+    return rows >= _MLP_ROWS.get(C, rows + 1)
 
 
 def block_mlp(y, first, second, gamma, residual):
     """``linear_tail(linear_gelu(y, first), second, gamma, residual)`` as one kernel where that is faster, else None."""
     C = y.shape[-1]
     w1, b1, w2, b2 = first.weight, first.bias, second.weight, second.bias
-    if not (y.dim() == 4 and C in _MLP_ROWS and y.numel() // C >= _MLP_ROWS[C] and plain(first, Linear)
+    if not (y.dim() == 4 and C > 0 and _mlp_pays(y.numel() // C, C) and plain(first, Linear)
             and plain(second, Linear) and b1 is not None and b2 is not None and w1.shape == (4 * C, C)
             and w2.shape == (C, 4 * C) and _layer16(y, w1, b1) and residual.dtype == y.dtype
             and all(t is None or (t.dtype == y.dtype and t.device == y.device) for t in (w2, b2, gamma))

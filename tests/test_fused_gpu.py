@@ -486,3 +486,50 @@ def test_gelu_of_the_negative_tail(dtype, unit):
         some = (u.abs() >= 0.25) & (u.abs() <= 4) & (ref.abs() >= 2.0 ** -14)
         assert (u[some] < -3).sum() > 100
         assert (((y.double() - ref).abs() / ref.abs()) <= bound(u))[some].all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("C,images,H,W,want", [
+    (96, 1, 128, 96, "one"), (96, 1, 128, 95, "two"), (128, 5, 29, 113, "one"), (128, 1, 128, 128, "two"),
+    (192, 7, 64, 64, "one"), (192, 1, 169, 169, "two"), (384, 6, 11, 331, "one"), (384, 5, 17, 257, "two"),
+    (384, 1, 256, 128, "one"), (384, 1, 331, 99, "two"), (384, 10, 17, 257, "two"), (384, 23, 38, 50, "one"),
+    (512, 2, 32, 32, "two"), (512, 1, 32, 64, "two"), (520, 1, 32, 64, "two"), (520, 1, 32, 65, "rows"), (64, 1, 9, 7, "two")])
+@pytest.mark.parametrize("scaled", [True, False])
+def test_block_dispatch_at_inference(C, images, H, W, want, scaled, dtype, monkeypatch):
+    """A block at inference on both sides of each line between its routes (one kernel for both layers, two product kernels,
+    the first one and the library's product), against the composition in fp64 behind the block's own convolution; the entry points
+    that were called are those that the rule names."""
+    from oriented1d_amd import _lib
+    from oriented1d_amd.convnext1d import Block
+    if dtype == torch.float16 and not scaled:
+        pytest.skip("one type without a layer scale")
+    torch.manual_seed(C + W)
+    block = Block(C, (7,), False, layer_scale_init_value=1.0 if scaled else 0.0, arbitrary_size=True).cuda().to(dtype).eval()
+    with torch.no_grad():
+        for p in block.parameters():
+            if p.dim() == 1:
+                p.add_((torch.randn_like(p) * 0.3))
+        block.dwconv.theta.zero_()
+    x = torch.randn(images, C, H, W, device="cuda").to(dtype)
+    called, real = [], _lib.host(0)
+
+    class Host:
+        def __getattr__(self, name):
+            called.append(name)
+            return getattr(real, name)
+    monkeypatch.setattr(_lib, "host", lambda device: Host())
+    with torch.no_grad():
+        got = block(x)
+    monkeypatch.undo()
+    assert (block.gamma is not None) == scaled
+    assert [n for n in called if n in ("block_mlp", "linear_rows", "linear_planes", "nhwc_scale_add_nchw")] == {
+        "one": ["block_mlp"], "two": ["linear_rows", "linear_planes"], "rows": ["linear_rows", "nhwc_scale_add_nchw"]}[want]
+    with torch.no_grad():
+        y = block.dwconv(x).permute(0, 2, 3, 1)
+        d = [t if t is None else t.double() for t in (block.norm.weight, block.norm.bias, block.pwconv1.weight, block.pwconv1.bias,
+                                                      block.pwconv2.weight, block.pwconv2.bias, block.gamma)]
+        for n in range(images):  # (an image at a time: the hidden tensor in fp64)
+            h = F.gelu(F.linear(F.layer_norm(y[n].double(), (C,), d[0], d[1], 1e-6), d[2], d[3]))
+            h = F.linear(h, d[4], d[5])
+            ref = x[n].double() + (h if d[6] is None else d[6] * h).permute(2, 0, 1)
+            _close(got[n], ref, dtype, "block")
