@@ -67,6 +67,12 @@ def nhwc_scale_add_nchw(y, scale=None, residual=None):
     return _lib.host(y.get_device()).nhwc_scale_add_nchw(y, sc, residual)
 
 
+def _product_fits(rows, N):
+    """True where the product kernels' launch, a workgroup of 256 threads per 128 rows and 96 or 128 outputs, has fewer than 2^32
+    threads (more only with billions of rows of few outputs)."""
+    return rows < 1 << 31 and rows * max(N, 128) <= 1 << 37
+
+
 def _layer16(x, w, b):
     """True where the product kernels of the library cover ``F.linear(x, w, b)`` without gradients: 16-bit tensors of one type on
     one GPU, sizes in multiples of eight."""
@@ -74,7 +80,7 @@ def _layer16(x, w, b):
             and w.dtype == x.dtype and w.device == x.device and w.shape[1] == x.shape[-1]
             and (b is None or (b.dtype == x.dtype and b.device == x.device))
             and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and max(w.shape) <= 65536 and ordinary(x, w, b)
-            and not torch.is_autocast_enabled(x.device.type) and x.numel() // w.shape[1] < 1 << 31)
+            and not torch.is_autocast_enabled(x.device.type) and _product_fits(x.numel() // w.shape[1], w.shape[0]))
 
 
 def linear_gelu(x, linear):
@@ -385,7 +391,7 @@ class Linear(torch.nn.Linear):
         w, b = self.weight, self.bias
         if (w.requires_grad and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and max(w.shape) <= 65536
                 and x.dim() >= 1 and x.shape[-1] == w.shape[1] and _recording(x, w, b)
-                and x.numel() // w.shape[1] <= 1 << 31):
+                and x.numel() // w.shape[1] <= 1 << 31 and w.numel() + w.shape[0] < 1 << 31):  # (two threads per gradient)
             ac = _autocast(x)
             dtype = ac or x.dtype
             if dtype in (torch.bfloat16, torch.float16) and (
@@ -416,7 +422,10 @@ def row_norm(x, norm, gelu=False, consumer=None):
 
 
 def _tail_covers(y):
-    return y.dim() == 4 and y.shape[-1] % 8 == 0 and y.shape[-1] <= MAX_C_TRAIN and y.numel() < 1 << 31
+    if y.dim() != 4 or y.shape[-1] % 8 != 0 or y.shape[-1] > MAX_C_TRAIN or y.numel() >= 1 << 31:
+        return False
+    N, H, W, C = y.shape  # (fewer than 2^32 threads: 256 per 64 pixels x 64 channels of an image)
+    return N * -(-H * W // 64) * -(-C // 64) < 1 << 24
 
 
 def block_tail(y, gamma, x):
