@@ -113,10 +113,18 @@ def test_argument_errors():
         assert fused.usable(w, 8, tiled=True)
 
 
+def _composed(m, x, monkeypatch):
+    """m(x) with PyTorch's passes around the operator: gradient recording switches the inference kernels off, and what is not
+    ordinary execution the training kernels."""
+    with monkeypatch.context() as patch:
+        patch.setattr(fused, "ordinary", lambda *tensors: False)
+        return m(x.detach().requires_grad_(True)).detach()
+
+
 @pytest.mark.parametrize("variant", ["1d", "1dpp"])
-def test_block_and_stem_fused_equal_unfused(variant):
+def test_block_and_stem_fused_equal_unfused(variant, monkeypatch):
     """Block-level parity: the harness in no-grad eval mode (fused glue) against the same
-    modules with autograd on (PyTorch composition)."""
+    modules as PyTorch composes them."""
     from oriented1d_amd.convnext1d import ConvNeXt1D
 
     torch.manual_seed(3)
@@ -128,11 +136,11 @@ def test_block_and_stem_fused_equal_unfused(variant):
     x = torch.randn(2, 3, 64, 64, device="cuda")
     with torch.no_grad():
         y_fused = m(x)
-    y_plain = m(x.requires_grad_(True))  # gradient recording switches the glue kernels off
-    _close(y_fused, y_plain.detach(), torch.float32, "network")
+    y_plain = _composed(m, x, monkeypatch)
+    _close(y_fused, y_plain, torch.float32, "network")
 
 
-def test_bf16_network_fused_equal_unfused_and_parameter_copies_refresh():
+def test_bf16_network_fused_equal_unfused_and_parameter_copies_refresh(monkeypatch):
     """The 16-bit network (parameters cast with .bfloat16(): the library works from cached fp32
     copies of them) with and without the glue kernels, and the copies follow in-place updates."""
     from oriented1d_amd.convnext1d import ConvNeXt1D
@@ -143,12 +151,12 @@ def test_bf16_network_fused_equal_unfused_and_parameter_copies_refresh():
     x = torch.randn(2, 3, 64, 64, device="cuda").bfloat16()
     with torch.no_grad():
         y_fused = m(x)
-    y_plain = m(x.requires_grad_(True)).detach()
+    y_plain = _composed(m, x, monkeypatch)
     _close(y_fused, y_plain, torch.bfloat16, "bf16 network")
     with torch.no_grad():
         m.stages[0][0].dwconv.weight.mul_(3.0)   # in-place update: the cached copy must refresh
-        y_fused2 = m(x.detach())
-    y_plain2 = m(x).detach()
+        y_fused2 = m(x)
+    y_plain2 = _composed(m, x, monkeypatch)
     _close(y_fused2, y_plain2, torch.bfloat16, "bf16 network after update")
     assert not torch.equal(y_fused, y_fused2)
 
