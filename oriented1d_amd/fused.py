@@ -67,10 +67,9 @@ def nhwc_scale_add_nchw(y, scale=None, residual=None):
     return _lib.host(y.get_device()).nhwc_scale_add_nchw(y, sc, residual)
 
 
-def _product_fits(rows, N):
-    """True where the product kernels' launch, a workgroup of 256 threads per 128 rows and 96 or 128 outputs, has fewer than 2^32
-    threads (more only with billions of rows of few outputs)."""
-    return rows < 1 << 31 and rows * max(N, 128) <= 1 << 37
+# A product kernel's launch, a workgroup of 256 threads per 128 rows and 96 or 128 outputs, has fewer than 2^32 threads below so many
+# inputs (eight per row at least; more than 2^37 outputs do not fit the card)
+_PRODUCT_MAX = 1 << 33
 
 
 def _layer16(x, w, b):
@@ -80,7 +79,7 @@ def _layer16(x, w, b):
             and w.dtype == x.dtype and w.device == x.device and w.shape[1] == x.shape[-1]
             and (b is None or (b.dtype == x.dtype and b.device == x.device))
             and w.shape[0] % 8 == 0 and w.shape[1] % 8 == 0 and max(w.shape) <= 65536 and ordinary(x, w, b)
-            and not torch.is_autocast_enabled(x.device.type) and _product_fits(x.numel() // w.shape[1], w.shape[0]))
+            and not torch.is_autocast_enabled(x.device.type) and x.numel() < _PRODUCT_MAX)
 
 
 def linear_gelu(x, linear):
@@ -111,24 +110,21 @@ def linear_tail(x, linear, gamma, residual):
 # kernels / one: 12544 x 96 25 / 17, 8192 x 96 15.9 / 16.8; 16384 x 128 21 / 25, 17408 x 128, where the first product has more
 # tiles than the chip holds, 30 / 25; 29008 x 192 47 / 43, 25088 x 192 43 / 42 and in odd planes 67 / 70).  There is no instance for
 # 256 channels.
-_MLP_ROWS = {96: 12288, 128: 16385, 192: 28672}
+_MLP_ROWS = {96: 12288, 128: 16385, 192: 28672, 384: 21846}
 # At 384 channels a workgroup has a CU to itself (101 KB of LDS): its time goes in rounds of 256 workgroups, about 95 us each, and
 # the last round pays from two thirds on (20384 rows 85 / 98, 22540 115 / 97, 32732 151 / 109, 32928 155 / 191, 39984 186 / 192, 42924
 # 192 / 193, 43904 217 / 192, 66052 314 / 309)
 _MLP_ROUND = 32768
 
 
-def _mlp_pays(rows, C):
-    if C == 384:
-        return 3 * rows >= 2 * _MLP_ROUND * -(-rows // _MLP_ROUND)
-    return rows >= _MLP_ROWS.get(C, rows + 1)
-
-
 def block_mlp(y, first, second, gamma, residual):
     """``linear_tail(linear_gelu(y, first), second, gamma, residual)`` as one kernel where that is faster, else None."""
     C = y.shape[-1]
+    rows = y.numel() // max(C, 1)
+    if rows < _MLP_ROWS.get(C, rows + 1) or (C == 384 and 3 * rows < 2 * _MLP_ROUND * -(-rows // _MLP_ROUND)):
+        return None
     w1, b1, w2, b2 = first.weight, first.bias, second.weight, second.bias
-    if not (y.dim() == 4 and C > 0 and _mlp_pays(y.numel() // C, C) and plain(first, Linear)
+    if not (y.dim() == 4 and plain(first, Linear)
             and plain(second, Linear) and b1 is not None and b2 is not None and w1.shape == (4 * C, C)
             and w2.shape == (C, 4 * C) and _layer16(y, w1, b1) and residual.dtype == y.dtype
             and all(t is None or (t.dtype == y.dtype and t.device == y.device) for t in (w2, b2, gamma))

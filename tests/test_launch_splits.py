@@ -28,17 +28,13 @@ def test_product_and_tail_launches_stay_below_two_to_the_32_threads():
 
     from oriented1d_amd import fused
     rng = random.Random(0)
-    edges = [(1 << 31) - 1, (1 << 31) - 1024, 1 << 30, (1 << 30) - 1, 1 << 24, 1]
-    taken = 0
     for _ in range(4000):
-        N = 8 * rng.choice([1, 2, 3, 8, 12, 15, 16, 17, 32, 33, 48, 512, 8192])
-        rows = rng.choice(edges + [(1 << 37) // max(N, 128), rng.randint(1, (1 << 31) - 1)])
-        if fused._product_fits(rows, N):
-            taken += 1
-            mtiles = -(-rows // 128)
-            for nt in {96, 128} if N % 96 == 0 else {128}:
-                assert -(-mtiles // 8) * 8 * -(-N // nt) * 256 < 1 << 32, (rows, N)
-    assert 1000 < taken < 4000 and fused._product_fits(401408, 3072) and not fused._product_fits((1 << 31) - 1, 8)
+        N, K = 8 * rng.choice([1, 2, 3, 8, 12, 15, 16, 17, 32, 33, 48, 512, 8192]), 8 * rng.choice([1, 2, 12, 128])
+        most = min((fused._PRODUCT_MAX - 1) // K, (1 << 37) // N)  # (2^37 outputs: 275 GB)
+        rows = rng.choice([most, rng.randint(1, most)])
+        mtiles = -(-rows // 128)
+        for nt in {96, 128} if N % 96 == 0 else {128}:
+            assert -(-mtiles // 8) * 8 * -(-N // nt) * 256 < 1 << 32, (rows, N)
     for shape in ((1 << 24, 1, 1, 8), ((1 << 24) - 1, 1, 1, 8), (1 << 20, 9, 9, 24), (1 << 22, 2, 2, 72), (64, 56, 56, 128), (0, 7, 7, 8)):
         y = torch.empty(shape, device="meta")
         if fused._tail_covers(y):
