@@ -6,12 +6,13 @@
 //   ln_patch    y [N,C,H,W] -> LayerNorm over C -> 2 x 2 patches  in front of a downsampling layer
 //   tail        res + scale[c] * y, y [N,HW,C] -> [N,C,HW]        layer scale + permute + residual
 //
-// All of them are bound by memory: PyTorch's compositions move each tensor three to six times (permuted
-// copies, conversions, separate parameter gradients) at 0.4 to 2 TB/s.  Input and output have types of their
-// own, so the conversions of autocast happen on the way out (fp32 stream, 16-bit pointwise layers).  Channels
-// are handled in pieces of eight, rows by groups of 8 to 64 lanes, and
-// parameter gradients are kept in registers over all the tiles of a workgroup, written as
-// partial sums and added in a fixed order by a second kernel.  Statistics and sums are fp32.
+// Memory bounds them (ln_tile 5.4 TB/s with the VALU busy for 85 %, tail 6.5, backward 5.7) but for ln_rows with GELU, where it
+// is the vector instructions (87 % of the time forward, 94 % backward with an fp32 gradient), and small tensors.  PyTorch's
+// compositions move each tensor three to six times (permuted copies, conversions, separate parameter gradients).  Input and output
+// have types of their own, so the conversions of autocast happen on the way out (fp32 stream, 16-bit pointwise layers).
+// Channels are handled in pieces of eight, rows by groups of 8 to 64 lanes, and parameter gradients are kept in registers
+// over all the tiles of a workgroup, written as partial sums and added in a fixed order by a second kernel.  Statistics and
+// sums are fp32.
 #pragma once
 
 #include "dwo_common.h"
@@ -100,10 +101,9 @@ __device__ __forceinline__ float blk_gelu_slope(float u) {
     return 0.5f * (1.f + erff(u * 0.70710678118654752f)) + u * 0.39894228040143268f * expf(-0.5f * u * u);
 }
 
-// Channels of a lane: pieces lane % LPR + k * LPR for k < NV, of which `live` exist.
+// Channels of a lane: pieces lane % LPR + k * LPR for k < NV.
 template <int LPR, int NV>
 struct Lanes {
-    static constexpr int PER = 64 / LPR;  // rows of channels per wave and step
     int l, slot;                          // place in the group, row within a step of the workgroup
     __device__ __forceinline__ Lanes() : l(threadIdx.x % LPR), slot(threadIdx.x / LPR) {}
     static constexpr int ROWS = kBlkThreads / LPR;  // rows per step of the workgroup
@@ -114,7 +114,6 @@ struct Lanes {
 template <int LPR, int NV>
 __device__ __forceinline__ void write_param_partials(float (&dg)[NV][8], float (&db)[NV][8], int C, float *red,
                                                      float *part) {
-    const Lanes<LPR, NV> ln;
     constexpr int ROWS = Lanes<LPR, NV>::ROWS;
 #pragma unroll
     for (int k = 0; k < NV; k++)

@@ -11,10 +11,11 @@
 // operands, hence free: a read takes rows 4 g .. 4 g + 3 for its lane group g.  The bias gradient is a product with
 // ones, in the workgroups of the first column of tiles.
 //
-// LDS bounds it: a step of 64 rows stores 32 KB and reads 64 KB, 768 cycles at 128 bytes each for 256 of the matrix cores.
-// 12544 x 512 x 2048 with its reduction 47.8 us, 131072 x 384 x 96 37.4.  Tried: two buffers with one barrier per step (47.9 and
-// 38.7: two workgroups per CU already cover the barriers).  Larger tiles would read less per product, but fewer
-// tiles mean more splits, whose partial sums (33 MB for the first size) go through memory.
+// 12544 x 512 x 2048 with its reduction 43.5 us, 131072 x 384 x 96 32.7.  No unit is busy for more than a quarter of that (by
+// counters at the first size: matrix cores and LDS 24 % each, VALU 10 %, no bank conflicts, 111 MB through memory at 2.6 TB/s;
+// at the second LDS 16 %, 151 MB at 4.6 TB/s): what is left is the chain of a step, loads to LDS, barrier, reads, products, with two
+// workgroups per CU to overlap it.  Tried: two buffers with one barrier per step (no faster).  Larger tiles would read less per
+// product, but fewer tiles mean more splits, whose partial sums (33 MB for the first size) go through memory.
 #pragma once
 
 #include "dwo_common.h"
@@ -191,8 +192,9 @@ __global__ __launch_bounds__(kLinThreads) void linear_reduce_kernel(const float 
     for (int e = 0; e < 4; e++) out[e] = from_float<TO>(s[e]);
 }
 
-// Splits of the rows: two workgroups per CU (512), each with at least 256 rows; a multiple of eight
-// where there are as many (whole splits per XCD).
+// Splits of the rows: two workgroups per CU (512), each with 256 rows where they were dealt evenly; a multiple of eight
+// where there are as many (whole splits per XCD).  A split holds whole steps of 64 rows, rounded up, so the last few may hold no
+// rows (10 of 168 for 131072 x 384 x 96): their sums are zeros.
 inline int linear_splits(size_t rows, int N, int K) {
     const long tiles = (long)((N + kLinTile - 1) / kLinTile) * ((K + kLinTile - 1) / kLinTile);
     const long steps = (long)((rows + kLinRows - 1) / kLinRows);
@@ -248,8 +250,9 @@ struct LinearArgs {
 // GELU of a sum that nothing has rounded, with erf from Abramowitz and Stegun, Handbook of Mathematical Functions, 7.1.26 (error
 // of erf below 1.5e-7): |u| (1/2 - q) + u / 2 with q = erfc(|u| / sqrt 2) / 2.  Two issue slots less than gelu_rounded, whose
 // tail is exact to the result's rounding; here a separate layer's rounding of u, which the tail magnifies by u^2, is gone, and is
-// worth ten times the difference (mean relative error on [-4, -3], separate layers / this, bf16 1.3e-2 / 1.4e-3, fp16 1.7e-3 / 2.5e-4).  gelu_rounded
-// here: 401408 x 384 x 96 in 178 us instead of 174, a block of 100352 x 192 in 132 instead of 127.  Infinities and NaN give what u * (1 + erf) gives.
+// worth five to nine times the difference (mean relative error on [-4, -3], separate layers / this, bf16 1.3e-2 / 1.4e-3, fp16
+// 1.7e-3 / 2.5e-4).  With gelu_rounded 401408 x 384 x 96 took 178 us instead of 174, a block of 100352 x 192 132 instead
+// of 127.  Infinities and NaN give what u * (1 + erf) gives.
 __device__ __forceinline__ float lin_gelu(float u) {
     const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_fabsf(u), 0.3275911f * 0.70710678118654752f, 1.f));
     float p = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
@@ -593,7 +596,8 @@ int launch_linear(const LinearArgs<T> &a, hipStream_t st) {
 
 // ------------------------------------------------------------------------------------------------- few inputs
 // y[m][n] = b[n] + sum_k x[m][k] * w[n][k] for K <= 4 (the stem's first layer, models/convnext.py:143,177) and N a multiple of
-// 64.  Writing y bounds it (64 x 224 x 224 pixels of 64 channels in bf16: 411 MB; as a library product 312 us, here 92).
+// 64.  Writing y bounds it (64 x 224 x 224 pixels of 64 channels in bf16: 411 MB; back to back 147 us, as a library product 330;
+// in a training pass 118).
 // One matrix instruction per 16 pixels x 16 channels, 28 of its 32 columns zero: the same sums, bit for
 // bit, as a library product's.
 constexpr int kFewThreads = 256;

@@ -7,10 +7,12 @@
 // round the 3 -> C result to bf16 (2^-9).
 //
 // A workgroup stages its window of x4 once for all channels (8 bytes per pixel, even and odd columns apart: 16 output
-// pixels read 128 neighbouring bytes); a wave takes 16 channels x 16 pixels at a time and keeps its weights for all tiles.  LDS bounds it: eight bytes per
-// lane and tap (60 us of 123 at 128 x 224 x 224 and K = 31), and staging, each input six times.  Against tap by tap with the
-// projection repeated for each group (us, K = 31 unless noted): 128 x 224 x 224 520 / 123, 4 x 512 x 512 92 / 33, 64 x 224 x 224
-// at K = 15 170 / 57.  Error against 64 bits 1.66e-3, which is the result's own rounding (tap by tap 2.39e-3).
+// pixels read 128 neighbouring bytes); a wave takes 16 channels x 16 pixels at a time and keeps its weights for all tiles.  Busiest are
+// the vector instructions (54 % of the time at 128 x 224 x 224 and K = 31 by counters: staging, each input six times, and
+// addresses), then LDS with eight bytes per lane and tap (36 %, bank conflicts included) and the matrix cores (18 %).  Against tap
+// by tap with the projection repeated for each group (us, K = 31 unless noted): 128 x 224 x 224 520 / 114, 4 x 512 x 512
+// 92 / 33, 64 x 224 x 224 at K = 15 170 / 57.  Error against 64 bits 1.64e-3 to 1.70e-3 over seven shapes with K = 7 to 31, which is the result's own
+// rounding (tap by tap 1.75e-3 to 2.34e-3).  bf16 only: in fp16 the low halves of weights below 1/4 leave the normal range.
 #pragma once
 
 #include "dwo_linear.h"
