@@ -321,7 +321,7 @@ class _BlockTail(torch.autograd.Function):
         dx = dout.to(x_dtype) if ctx.needs_input_grad[2] else None
         if not (ctx.needs_input_grad[0] or ctx.needs_input_grad[1]):
             return None, None, dx, None, None
-        y, gamma = ctx.saved_tensors if ctx.saved_tensors else (None, None)
+        y, gamma = ctx.saved_tensors or (None, None)  # (read once: hooks, as of checkpointing, may unpack a tensor only once)
         if torch.is_grad_enabled():
             if gamma is None:
                 return dout.permute(0, 2, 3, 1).to(dtype), None, dx, None, None

@@ -340,6 +340,40 @@ def test_hooks_and_replaced_forwards_keep_the_module_path():
     assert not torch.allclose(zeroed, plain)
 
 
+@pytest.mark.parametrize("mode", ["autocast", "f32"])
+@pytest.mark.parametrize("variant", ["1d", "1dpp"])
+@pytest.mark.parametrize("hooks", ["checkpoint", "cpu"])
+def test_passes_under_saved_tensor_hooks(hooks, variant, mode):
+    """Activation checkpointing and activations kept on the host, around a stem, a downsampling layer and a block: the gradients
+    without them (the same kernels on the same values; the library's convolution gradients sum in an order of their own)."""
+    from torch.autograd.graph import save_on_cpu
+    from torch.utils.checkpoint import checkpoint
+    from oriented1d_amd.convnext1d import ConvNeXt1D
+    torch.manual_seed(9)
+    net = ConvNeXt1D(depths=(1, 1, 1, 1), dims=(16, 32, 64, 128), variant=variant, stem_dim1=64, num_classes=8,
+                     layer_scale_init_value=0.5, arbitrary_size=True).cuda()
+    img = torch.randn(2, 3, 36, 44, device="cuda")
+
+    def part(x):
+        return net.stages[1](net._downsample(1, net.stages[0](net._downsample(0, x))))
+    grads = []
+    for hooked in (False, True):
+        net.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=BF16, enabled=mode == "autocast"):
+            if not hooked:
+                y = part(img)
+            elif hooks == "checkpoint":
+                y = checkpoint(part, img, use_reentrant=False)
+            else:
+                with save_on_cpu():
+                    y = part(img)
+        y.float().square().sum().backward()
+        grads.append([p.grad for p in net.parameters() if p.grad is not None])
+    assert len(grads[0]) == len(grads[1]) > 20
+    for a, b in zip(*grads):
+        close(a, b.double(), 1e-5, "gradient")
+
+
 @pytest.mark.parametrize("variant", ["1d", "1dpp"])
 @pytest.mark.parametrize("mode", ["autocast", "bf16", "f32"])
 def test_network_gradients_against_the_composition(variant, mode, monkeypatch):
