@@ -153,6 +153,11 @@ class Stem1D(nn.Module):
         return F.gelu(norm(x)) if y is None else y
 
 
+def _operator(conv):
+    """The operator in a block's slot: what a wrapper without hooks calls."""
+    return conv.conv if fused.plain(conv, ConvWrapper) else conv
+
+
 class Block(nn.Module):
     """ConvNeXt-1D block (one oriented conv, models/convnext.py:255-319) or 1D++ block (a second
     oriented conv with a residual tap on the 4*dim hidden tensor in NHWC, :322-399)."""
@@ -178,7 +183,12 @@ class Block(nn.Module):
         self.plus_plus = plus_plus
 
     def forward(self, x):
-        y = (self.dwconv1 if self.plus_plus else self.dwconv)(x)
+        conv = self.dwconv1 if self.plus_plus else self.dwconv
+        if not self.training:
+            out = fused.infer_block(x, self, _operator(conv), _operator(self.dwconv2) if self.plus_plus else None)
+            if out is not None:
+                return out
+        y = conv(x)
         fuse = fused.usable(y, y.shape[1], tiled=True) and not self.training
         if fuse:  # permute + LayerNorm as one pass
             y = fused.nchw_layernorm_nhwc(y, self.norm.weight, self.norm.bias, self.norm.eps)

@@ -683,6 +683,14 @@ Tensor block_mlp(const Tensor &x_, const Tensor &w1_, const Tensor &b1_, const T
     return out;
 }
 
+// [N,C,H,W] -> operator (NCHW, stride 1; fp32 weights and bias) -> LayerNorm over C -> [N,H,W,C], without gradients (`pieces`: by
+// ln_tile)
+Tensor conv_norm(const Tensor &x, const Tensor &w, const OptTensor &bias, const Tensor &taps, const Tensor &g,
+                 const Tensor &b, double eps, bool pieces) {
+    const Tensor y = fprop(x, w, taps, 1, bias, DWO_NCHW);
+    return pieces ? std::get<0>(ln_tile(y, g, b, eps, false, y.scalar_type(), false)) : nchw_layernorm_nhwc(y, g, b, eps);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -698,6 +706,7 @@ PYBIND11_MODULE(_host, m) {
     m.def("linear_wgrad", &linear_wgrad);
     m.def("pointwise_forward", &pointwise_forward);
     m.def("block_mlp", &block_mlp);
+    m.def("conv_norm", &conv_norm);
     m.def("linear_rows", &linear_rows);
     m.def("linear_planes", &linear_planes);
     m.def("ln_rows", &ln_rows);

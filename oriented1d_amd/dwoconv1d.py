@@ -143,7 +143,7 @@ def f32_copy(p):
     every call costs a kernel launch each)."""
     if p.dtype == torch.float32 and p.is_contiguous():
         return p.detach()
-    key = (p._version, p.data_ptr(), p.dtype, str(p.device))
+    key = (p._version, p.data_ptr(), p.dtype, p.device)
     hit = _F32_COPIES.get(id(p))
     if hit is None or hit[0]() is not p or hit[1] != key:
         pid = id(p)

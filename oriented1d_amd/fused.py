@@ -11,7 +11,7 @@ import torch.nn.functional as F
 import torch.nn.modules.module as _mod
 
 from . import _lib
-from .dwoconv1d import ordinary
+from .dwoconv1d import DepthwiseOrientedConv1d, KernelTuple, _native_covers, f32_copy as _f32, ordinary
 
 _DTYPES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 MAX_C_ROWS, MAX_C_TILE = 2048, 1536
@@ -24,11 +24,6 @@ def _ptr(t):
 
 def _stream(t):
     return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
-
-
-def _f32(p):
-    from .dwoconv1d import f32_copy
-    return f32_copy(p)
 
 
 def usable(x, C, tiled):
@@ -117,11 +112,15 @@ _MLP_ROWS = {96: 12288, 128: 16385, 192: 28672, 384: 21846}
 _MLP_ROUND = 32768
 
 
+def _mlp_pays(C, rows):
+    """True where ``block_mlp`` is the faster route for this many rows of C channels."""
+    return rows >= _MLP_ROWS.get(C, rows + 1) and (C != 384 or 3 * rows >= 2 * _MLP_ROUND * -(-rows // _MLP_ROUND))
+
+
 def block_mlp(y, first, second, gamma, residual):
     """``linear_tail(linear_gelu(y, first), second, gamma, residual)`` as one kernel where that is faster, else None."""
     C = y.shape[-1]
-    rows = y.numel() // max(C, 1)
-    if rows < _MLP_ROWS.get(C, rows + 1) or (C == 384 and 3 * rows < 2 * _MLP_ROUND * -(-rows // _MLP_ROUND)):
+    if not _mlp_pays(C, y.numel() // max(C, 1)):
         return None
     w1, b1, w2, b2 = first.weight, first.bias, second.weight, second.bias
     if not (y.dim() == 4 and plain(first, Linear)
@@ -131,6 +130,58 @@ def block_mlp(y, first, second, gamma, residual):
             and ordinary(w2, b2, gamma, residual)):
         return None
     return _lib.host(y.get_device()).block_mlp(y, w1, b1, w2, b2, gamma, residual)
+
+
+def infer_block(x, block, conv, inner):
+    """A ConvNeXt-1D block (operator ``conv``) or 1D++ block (and ``inner``, between the pointwise layers) without gradients: the
+    kernels of its layers one by one, with what they check checked once for all of them (layer by layer 45 to 50 us of host time
+    per block, four launches of which are 19); None where one of them would not take the path that is taken here."""
+    if (torch.compiler.is_compiling() or torch.is_grad_enabled() or not x.is_cuda or x.dim() != 4 or x.numel() == 0
+            or x.dtype not in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda")):
+        return None
+    layers = block._modules
+    first, last, norm = layers.get("pwconv1"), layers.get("pwconv2"), layers.get("norm")
+    if not (plain(conv, DepthwiseOrientedConv1d) and plain(first, Linear) and plain(last, Linear)
+            and type(norm) is torch.nn.LayerNorm and (inner is None or plain(inner, DepthwiseOrientedConv1d))):
+        return None
+    N, C, H, W = x.shape
+    rows, dtype, device = N * H * W, x.dtype, x.device
+    p, q, r, s = conv._parameters, first._parameters, last._parameters, norm._parameters
+    w, theta, g, b = p.get("weight"), p.get("theta"), s.get("weight"), s.get("bias")
+    w1, b1, w2, b2 = q.get("weight"), q.get("bias"), r.get("weight"), r.get("bias")
+    bias, gamma = conv.bias, block.gamma
+    module = conv.module_fp32_large if conv.arbitrary_size else conv.module_fp32
+    if (w is None or theta is None or g is None or b is None or w1 is None or b1 is None or w2 is None or b2 is None
+            or conv.nhwc or conv.resid is not None or module.stride != 1 or C % 8 != 0 or C > MAX_C_TILE
+            or 4 * rows * C >= _PRODUCT_MAX or w1.shape != (4 * C, C) or w2.shape != (C, 4 * C)
+            or not _native_covers(x, w, theta, bias, None, module, False) or not ordinary(g, b, w1, b1, w2, b2, gamma)):
+        return None
+    for t in (w1, b1, w2, b2) if gamma is None else (w1, b1, w2, b2, gamma):
+        if t.dtype != dtype or t.device != device:
+            return None
+    if g.device != device or b.device != device:
+        return None
+    if inner is not None:
+        v, angles, vb, resid = inner._parameters.get("weight"), inner._parameters.get("theta"), inner.bias, inner.resid
+        wide = inner.module_fp32_large if inner.arbitrary_size else inner.module_fp32
+        if not (v is not None and angles is not None and inner.nhwc and type(wide) is KernelTuple and wide.stride == 1
+                and v.shape[0] == 4 * C and v.shape[-1] == wide.kernel_size and v.is_floating_point()
+                and ordinary(v, angles, vb, resid) and all(t is None or t.device == device for t in (v, vb, resid))):
+            return None
+        taps, layouts = wide.taps.lookup(angles, 4 * C, v.shape[-1], device)
+    host, x = _lib.host(x.get_device()), x.contiguous()
+    y = host.conv_norm(x, _f32(w), None if bias is None else _f32(bias),
+                       module.taps.lookup(theta, C, w.shape[-1], device)[0], _f32(g), _f32(b), norm.eps, _pieces(x, C))
+    if inner is None and _mlp_pays(C, rows):
+        return host.block_mlp(y, w1, b1, w2, b2, gamma, x)
+    y = host.linear_rows(y, w1, b1, True)
+    if inner is not None:
+        v = _f32(v)
+        y = host.fprop(y, v if resid is None else v + resid.to(v), taps, 1, None if vb is None else _f32(vb),
+                       layouts[x.element_size()])
+    if 4 * C <= _PLANES_MAX_K or rows <= _PLANES_MAX_ROWS:
+        return host.linear_planes(y, w2, b2, gamma, x)
+    return host.nhwc_scale_add_nchw(F.linear(y, w2, b2), None if gamma is None else _f32(gamma), x)
 
 
 class _PointwiseLinear(torch.autograd.Function):

@@ -541,3 +541,37 @@ def test_block_dispatch_at_inference(C, images, H, W, want, scaled, dtype, monke
             h = F.linear(h, d[4], d[5])
             ref = x[n].double() + (h if d[6] is None else d[6] * h).permute(2, 0, 1)
             _close(got[n], ref, dtype, "block")
+
+
+@pytest.mark.parametrize("C,plus_plus,hw,N,dtype,gamma,wrapped", [
+    (96, False, 9, 3, torch.bfloat16, 0.1, False), (96, True, 12, 2, torch.float16, 0.1, True),
+    (384, False, 14, 128, torch.bfloat16, 0.0, False),  # (both layers as one kernel, no layer scale)
+    (768, True, 7, 50, torch.bfloat16, 0.1, False)])    # (second layer by the library)
+def test_inference_block_checked_once(C, plus_plus, hw, N, dtype, gamma, wrapped, monkeypatch):
+    """A block at inference whose layers are checked once gives the bits of its layers one by one, and leaves blocks with hooks,
+    in autocast or of another type to them."""
+    from oriented1d_amd import fused
+    from oriented1d_amd.convnext1d import Block
+    torch.manual_seed(C + hw)
+    block = Block(C, (15, 31) if plus_plus else (31,), plus_plus, layer_scale_init_value=gamma, arbitrary_size=True,
+                  wrapped=wrapped).cuda().to(dtype).eval()
+    x = torch.randn(N, C, hw, hw, device="cuda").to(dtype)
+    taken = []
+    whole = fused.infer_block
+    monkeypatch.setattr(fused, "infer_block", lambda *a: taken.append(whole(*a)) or taken[-1])
+    with torch.no_grad():
+        got = block(x.transpose(2, 3).contiguous().transpose(2, 3))  # (not dense)
+        assert taken[-1] is not None
+        monkeypatch.setattr(fused, "infer_block", lambda *a: None)
+        assert torch.equal(got, block(x))
+        monkeypatch.setattr(fused, "infer_block", lambda *a: taken.append(whole(*a)) or taken[-1])
+        seen = []
+        handle = block.pwconv2.register_forward_hook(lambda *_: seen.append(1))
+        block(x)
+        handle.remove()
+        assert taken[-1] is None and seen
+        with torch.autocast("cuda", dtype=dtype):
+            block(x)
+        assert taken[-1] is None
+        block.float()(x.float())
+        assert taken[-1] is None
