@@ -14,12 +14,12 @@
 //
 // What bounds them, from counters (K = 31): at stride 1 in bf16 the issue slots of the multiply-adds and those
 // unpacking instructions (64 x 512 x 56 x 56 fprop 151 of 233 us; L2 lookups 42 %, LDS 25 %); at stride 2 lines that cross
-// the fabric again, as the eight groups of a line come to it at different times (64 x 64 x 224 x 224: fprop reads x
-// 2.4 times, wgrad x and dy 5.4 times, at 6 TB/s; dgrad writes dx twice).  Two workgroups per CU (80 KB of LDS,
+// the fabric again, as the eight groups of a line come to it at different times, and the L1, which takes a line of 128 bytes in two
+// clocks whatever part of it is used (64 x 64 x 224 x 224).  Two workgroups per CU (80 KB of LDS,
 // 128 registers) overlap staging and evaluation.
 // Measured (us, fprop / wgrad, K = 31, angles of the networks): 64 x 512 x 56 x 56 bf16 233 / 264 (slice
 // kernels 335 / 428), 64 x 1024 x 28 x 28 bf16 114 / 121 (129 / 190), 64 x 384 x 56 x 56 fp32 298 / 355 (326 / 551);
-// stride 2, 64 x 64 x 224 x 224 bf16 310 / 451 (tile kernels 574 / 817).
+// stride 2, 64 x 64 x 224 x 224 bf16 307 / 367 (tile kernels 574 / 817).
 #pragma once
 
 #include "dwo_grouped_dispatch.h"
@@ -213,12 +213,27 @@ struct Word {
 struct GrpTile {
     int n, p, q, th, tw;  // image, corner, nominal extents
     int vh, vw;           // extents inside the image
+    // NEAR (stride 2, where a window is up to four times its tile's share of the image): neighbouring tiles on one XCD at about
+    // the same time, so that they find each other's lines in its L2.  grp_task deals units to the XCDs in turn; here XCD x
+    // gets the x-th eighth of them, in bands of two tile columns (a tile shares more with the rows below than with the columns
+    // beside).  Where the tile columns are a multiple of eight an XCD has whole columns as it is.  bf16, K = 31, us, in turn / like
+    // this: 64 x 64 x 224 x 224 fprop 318 / 307, dgrad 245 / 198, wgrad 451 / 367, at 112 x 112 81 / 73, 41 / 40, 117 / 98; without
+    // bands wgrad 381, and 8 x 512 x 512 fprop 190, in turn 176.  At stride 1 between 2 % more and 1 % less.
+    template <bool NEAR>
     __device__ __forceinline__ void set(const ConvDims &d, const GrpTiles &t, int unit) {
         const int per = t.nth * t.ntw;
-        n = unit / per;
-        const int k = unit - n * per, a = k / t.ntw;
         th = t.th, tw = t.tw;
-        p = a * th, q = (k - a * t.ntw) * tw;
+        if (NEAR && t.run > 0) {
+            if (unit < 8 * t.run) unit = unit % 8 * t.run + unit / 8;
+            n = unit / per;
+            const int k = unit - n * per, b = k / (2 * t.nth), j = k - b * (2 * t.nth), two = 2 * b + 1 < t.ntw ? 1 : 0;
+            const int a = j >> two;
+            p = a * th, q = (2 * b + (j & two)) * tw;
+        } else {
+            n = unit / per;
+            const int k = unit - n * per, a = k / t.ntw;
+            p = a * th, q = (k - a * t.ntw) * tw;
+        }
         vh = min(th, d.P - p), vw = min(tw, d.Q - q);
     }
 };
@@ -391,7 +406,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
     if (!grp_task(blockIdx.x, d.N * tiles.nth * tiles.ntw, d.C / CG, unit, group)) return;
     const int c0 = group * CG;
     GrpTile t;
-    t.set(d, tiles, unit);
+    t.set<S == 2>(d, tiles, unit);
     const T *xn = x + (size_t)t.n * d.H * d.W * d.C + c0;
     T *yn = y + (size_t)t.n * d.P * d.Q * d.C + c0;
     if (threadIdx.x < CG * K) {  // (dgrad: in reverse tap order)
@@ -519,7 +534,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
     if (!grp_task(blockIdx.x, d.N * tiles.nth * tiles.ntw, d.C / CG, unit, group)) return;
     const int c0 = group * CG;
     GrpTile t;
-    t.set(d, tiles, unit);
+    t.set<true>(d, tiles, unit);
     const T *img = x + (size_t)t.n * d.H * d.W * CIN;
     T *yn = y + (size_t)t.n * d.P * d.Q * d.C + c0;
     if (threadIdx.x < CG * K) lw[threadIdx.x] = wt[(size_t)c0 * K + threadIdx.x];
@@ -546,7 +561,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
 
 // ---------------------------------------------------------------------------------------------
 // dgrad at stride 2 (QuadPlan).  `d` describes dy as both the source and the plane of quads (H = P,
-// W = Q); dx is dxh x dxw.  64 x 64 x 224 x 224 bf16, K = 31: 247 us, bound by the writes in 16-byte
+// W = Q); dx is dxh x dxw.  64 x 64 x 224 x 224 bf16, K = 31: 198 us, bound by the writes in 16-byte
 // pieces, twice dx (the residue classes one after the other from a sorted tap table, dwo_nhwc_tile.h: 544).
 template <int O, typename T, int K>
 __device__ __forceinline__ void grp_dgrad2_body(grp_u4 *lds, float *lw, const T *dyn, T *dxn, const ConvDims &d,
@@ -651,7 +666,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
     if (!grp_task(blockIdx.x, d.N * tiles.nth * tiles.ntw, d.C / CG, unit, group)) return;
     const int c0 = group * CG;
     GrpTile t;
-    t.set(d, tiles, unit);
+    t.set<true>(d, tiles, unit);
     const T *dyn = dy + (size_t)t.n * d.H * d.W * d.C + c0;
     T *dxn = dx + (size_t)t.n * dxh * dxw * d.C + c0;
     if (threadIdx.x < CG * K) lw[threadIdx.x] = wt[(size_t)c0 * K + threadIdx.x];
@@ -677,7 +692,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
 // wgrad: the same windows and items; a lane keeps the running sums of its channels' taps (62 for
 // two channels) over all tiles of its workgroup and reads the item's dy words from memory.  Lanes
 // and waves are added up at the end, in a fixed order.
-template <int O, int S, typename T, int K>
+template <int O, int S, bool NEAR, typename T, int K>
 __device__ __forceinline__ void grp_wgrad_body(grp_u4 *lds, const T *x, const T *dy, float *part,
                                                const ConvDims &d, const GrpTiles &tiles, int c0, int g, int NG) {
     using G = GrpGeo<O, K, S>;
@@ -693,7 +708,7 @@ __device__ __forceinline__ void grp_wgrad_body(grp_u4 *lds, const T *x, const T 
     const int units = d.N * tiles.nth * tiles.ntw;
     for (int u = g; u < units; u += NG) {
         GrpTile t;
-        t.set(d, tiles, u);
+        t.set<NEAR>(d, tiles, u);
         const T *dyn = dy + (size_t)t.n * d.P * d.Q * d.C + c0;
         const __amdgpu_buffer_rsrc_t in = win_rsrc(dyn, dyn + (size_t)d.P * d.Q * d.C - c0);
         __syncthreads();  // the previous window is consumed
@@ -772,7 +787,7 @@ __device__ __forceinline__ void grp_wgrad_body(grp_u4 *lds, const T *x, const T 
 }
 
 // a group without a common canonical orientation: a thread per (channel, tap), straight from memory
-template <int S, typename T, int K>
+template <int S, bool NEAR, typename T, int K>
 __device__ void grp_wgrad_any(const T *x, const T *dy, const int8_t *dhdw, float *part, const ConvDims &d,
                               const GrpTiles &tiles, int c0, int g, int NG) {
     constexpr int CG = grp_channels(sizeof(T));
@@ -782,7 +797,7 @@ __device__ void grp_wgrad_any(const T *x, const T *dy, const int8_t *dhdw, float
     float total = 0.f;
     for (int u = g; u < d.N * tiles.nth * tiles.ntw; u += NG) {
         GrpTile t;
-        t.set(d, tiles, u);
+        t.set<NEAR>(d, tiles, u);
         for (int o = 0; o < t.vh * t.vw; o++) {
             const int p = t.p + o / t.vw, q = t.q + o % t.vw, h = p * S + dh, w = q * S + dw;
             const float gy = to_float(dy[(((size_t)t.n * d.P + p) * d.Q + q) * d.C + c]);
@@ -794,7 +809,7 @@ __device__ void grp_wgrad_any(const T *x, const T *dy, const int8_t *dhdw, float
     part[((size_t)c0 * (K + 1) + threadIdx.x) * NG + g] = total;
 }
 
-template <int S, typename T, int K>
+template <int S, bool NEAR, typename T, int K>
 __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void grouped_wgrad_kernel(
     const T *__restrict__ x, const T *__restrict__ dy, const void *__restrict__ blob, float *__restrict__ part,
     ConvDims d, GrpTiles tiles, int NG) {
@@ -806,7 +821,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
     const int c0 = group * CG;
 #define DWO_CASE(O)                                                               \
     case O:                                                                       \
-        grp_wgrad_body<O, S, T, K>(lds, x, dy, part, d, tiles, c0, g, NG);        \
+        grp_wgrad_body<O, S, NEAR, T, K>(lds, x, dy, part, d, tiles, c0, g, NG);  \
         break;
     switch (grp_class<CG>(taps_class(blob, d.C, K) + c0)) {
         DWO_CASE(0)
@@ -817,7 +832,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
         DWO_CASE(5)
         DWO_CASE(6)
         DWO_CASE(7)
-        default: grp_wgrad_any<S, T, K>(x, dy, taps_dhdw(blob), part, d, tiles, c0, g, NG);
+        default: grp_wgrad_any<S, NEAR, T, K>(x, dy, taps_dhdw(blob), part, d, tiles, c0, g, NG);
     }
 #undef DWO_CASE
 }
@@ -840,7 +855,15 @@ GrpTiles grp_tiles(int P, int Q, long planes) {
         t.th = cmax((t.th / 2 + 3) & ~3, kGrpLeastRows);
         t.nth = (P + t.th - 1) / t.th;
     }
+    t.run = 0;
     return t;
+}
+
+// Tiles of an XCD where they are dealt in runs (GrpTile::set): images cut into tiles, many more tasks than run at once (3 x 64 x
+// 200 x 300 with 840 of them: wgrad 47 us in turn, 49 in runs; 8 x 64 x 256 x 256 with 2048: 84 and 76).
+inline int grp_run(const GrpTiles &t, int N, int ngroups) {
+    const long units = (long)N * t.nth * t.ntw;
+    return t.nth * t.ntw > 1 && t.ntw % 8 != 0 && units * ngroups >= 4 * kGrpSlots ? (int)(units / 8) : 0;
 }
 
 template <typename T, int K, int S>
@@ -854,7 +877,8 @@ int launch_grouped_conv_s(const void *src, const float *w, const float *bias, co
     });
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
-    const GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, (long)d.N * ngroups);
+    GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, (long)d.N * ngroups);
+    if (S == 2) t.run = grp_run(t, d.N, ngroups);
     const int pixels = grp_pixels<ConvSet<K, S>>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (!grp_grid_fits(grid)) return -100;
@@ -878,7 +902,8 @@ int launch_grouped_dgrad2(const void *dy, const float *w, const void *taps, void
     ConvDims d = d_;
     d.H = d.P, d.W = d.Q;
     const int ngroups = d.C / CG;
-    const GrpTiles t = grp_tiles<Set>(d.P, d.Q, (long)d.N * ngroups);
+    GrpTiles t = grp_tiles<Set>(d.P, d.Q, (long)d.N * ngroups);
+    t.run = grp_run(t, d.N, ngroups);
     const int pixels = grp_pixels<Set>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (!grp_grid_fits(grid)) return -100;
@@ -904,15 +929,20 @@ int launch_grouped_wgrad_s(const void *x, const void *dy, const void *taps, floa
     static_assert(kRed <= kGrpPixels * 4, "the waves' sums fit where the window was");
     static int cache[kMaxDevices];
     per_device_once(cache, [&] {
-        allow_large_lds(grouped_wgrad_kernel<S, T, K>, kGrpPixels * 16);
+        allow_large_lds(grouped_wgrad_kernel<S, false, T, K>, kGrpPixels * 16);
+        if constexpr (S == 2) allow_large_lds(grouped_wgrad_kernel<S, true, T, K>, kGrpPixels * 16);
         return 1;
     });
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
-    const GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, kGrpSlots);  // (lower tiles would cost more partial sums)
-    const int floats = cmax(grp_pixels<ConvSet<K, S>>(t.th) * 4, kRed);
-    grouped_wgrad_kernel<S, T, K><<<dim3((unsigned)grp_grid(NG, ngroups)), dim3(kGrpThreads), floats * sizeof(float), st>>>(
-        (const T *)x, (const T *)dy, taps, part, d, t, NG);
+    GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, kGrpSlots);  // (lower tiles would cost more partial sums)
+    if (S == 2) t.run = grp_run(t, d.N, ngroups);
+    const size_t lds = cmax(grp_pixels<ConvSet<K, S>>(t.th) * 4, kRed) * sizeof(float);
+    const dim3 grid((unsigned)grp_grid(NG, ngroups)), block(kGrpThreads);
+    // (a kernel of its own where tiles are dealt in turn: finding a tile's place in its run costs scalar registers)
+    if (S == 2 && t.run > 0)
+        grouped_wgrad_kernel<S, S == 2, T, K><<<grid, block, lds, st>>>((const T *)x, (const T *)dy, taps, part, d, t, NG);
+    else grouped_wgrad_kernel<S, false, T, K><<<grid, block, lds, st>>>((const T *)x, (const T *)dy, taps, part, d, t, NG);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : (int)e;
 }
@@ -937,7 +967,8 @@ int launch_grouped_projected(const void *x, const float *pw_w, const float *pw_b
     });
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
-    const GrpTiles t = grp_tiles<ConvSet<K, 2>>(d.P, d.Q, (long)d.N * ngroups);
+    GrpTiles t = grp_tiles<ConvSet<K, 2>>(d.P, d.Q, (long)d.N * ngroups);
+    t.run = grp_run(t, d.N, ngroups);
     const int pixels = grp_pixels<ConvSet<K, 2>>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (!grp_grid_fits(grid)) return -100;

@@ -45,6 +45,7 @@ __host__ __device__ inline bool grp_task(unsigned block, int units, int ngroups,
 
 struct GrpTiles {
     int th, tw, nth, ntw;  // tile extents and counts
+    int run;               // tiles of an XCD where they are dealt in runs (GrpTile::set), else 0
 };
 
 // Partial sums per (channel, tap): about two rounds of the chip's slots at most, and no more than there are tiles of

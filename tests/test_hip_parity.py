@@ -255,6 +255,13 @@ def test_grouped_nhwc_kernels(oracle, N, C, H, W, K, stride, dtype):
         _case(oracle, N, C, H, W, K, stride, dtype, 3, theta, seed=H + W + K)
 
 
+# stride-2 tiles dealt in runs: more than two thousand tasks, tile counts that eight does not divide, one to five tile columns
+@pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("N,C,H,W,K", [(5, 256, 150, 150, 31), (11, 256, 290, 38, 15), (3, 256, 101, 301, 7), (7, 320, 97, 130, 13)])
+def test_grouped_nhwc_tiles_in_runs(oracle, N, C, H, W, K, dtype):
+    _case(oracle, N, C, H, W, K, 2, dtype, 3, grouped_theta(C, 0.5), seed=H + W)
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
 @pytest.mark.parametrize("stride", [1, 2])
 def test_grouped_claim_that_does_not_hold(oracle, stride, dtype):
