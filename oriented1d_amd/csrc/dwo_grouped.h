@@ -860,8 +860,11 @@ GrpTiles grp_tiles(int P, int Q, long planes) {
 }
 
 // Tiles of an XCD where they are dealt in runs (GrpTile::set): images cut into tiles, many more tasks than run at once (3 x 64 x
-// 200 x 300 with 840 of them: wgrad 47 us in turn, 49 in runs; 8 x 64 x 256 x 256 with 2048: 84 and 76).
-inline int grp_run(const GrpTiles &t, int N, int ngroups) {
+// 200 x 300 with 840 of them: wgrad 47 us in turn, 49 in runs; 8 x 64 x 256 x 256 with 2048: 84 and 76), and windows whose halo
+// weighs: at K = 15 a tile shares half as much with its neighbours, and in fp32, where an XCD has half as many tiles under way, the
+// runs only spread its accesses (34 x 64 x 320 x 288 wgrad 539 / 594; bf16 64 x 64 x 224 x 224 298 / 269; K = 31 fp32 457 / 405).
+inline int grp_run(const GrpTiles &t, int N, int ngroups, int K, size_t esize) {
+    if (K <= 15 && esize == 4) return 0;
     const long units = (long)N * t.nth * t.ntw;
     return t.nth * t.ntw > 1 && t.ntw % 8 != 0 && units * ngroups >= 4 * kGrpSlots ? (int)(units / 8) : 0;
 }
@@ -878,7 +881,7 @@ int launch_grouped_conv_s(const void *src, const float *w, const float *bias, co
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
     GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, (long)d.N * ngroups);
-    if (S == 2) t.run = grp_run(t, d.N, ngroups);
+    if (S == 2) t.run = grp_run(t, d.N, ngroups, K, sizeof(T));
     const int pixels = grp_pixels<ConvSet<K, S>>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (!grp_grid_fits(grid)) return -100;
@@ -903,7 +906,7 @@ int launch_grouped_dgrad2(const void *dy, const float *w, const void *taps, void
     d.H = d.P, d.W = d.Q;
     const int ngroups = d.C / CG;
     GrpTiles t = grp_tiles<Set>(d.P, d.Q, (long)d.N * ngroups);
-    t.run = grp_run(t, d.N, ngroups);
+    t.run = grp_run(t, d.N, ngroups, K, sizeof(T));
     const int pixels = grp_pixels<Set>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (!grp_grid_fits(grid)) return -100;
@@ -936,7 +939,7 @@ int launch_grouped_wgrad_s(const void *x, const void *dy, const void *taps, floa
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
     GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, kGrpSlots);  // (lower tiles would cost more partial sums)
-    if (S == 2) t.run = grp_run(t, d.N, ngroups);
+    if (S == 2) t.run = grp_run(t, d.N, ngroups, K, sizeof(T));
     const size_t lds = cmax(grp_pixels<ConvSet<K, S>>(t.th) * 4, kRed) * sizeof(float);
     const dim3 grid((unsigned)grp_grid(NG, ngroups)), block(kGrpThreads);
     // (a kernel of its own where tiles are dealt in turn: finding a tile's place in its run costs scalar registers)
@@ -968,7 +971,7 @@ int launch_grouped_projected(const void *x, const float *pw_w, const float *pw_b
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
     GrpTiles t = grp_tiles<ConvSet<K, 2>>(d.P, d.Q, (long)d.N * ngroups);
-    t.run = grp_run(t, d.N, ngroups);
+    t.run = grp_run(t, d.N, ngroups, K, sizeof(T));
     const int pixels = grp_pixels<ConvSet<K, 2>>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (!grp_grid_fits(grid)) return -100;
