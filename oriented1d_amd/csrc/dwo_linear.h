@@ -5,17 +5,18 @@
 // The sum runs over the pixels of a batch (3 136 to 802 816 rows) for outputs of 64 x 96 to 4096 x 1024, so
 // most shapes have far fewer output tiles than the chip has CUs: the rows are split over workgroups, each
 // writes fp32 partial sums and a second kernel adds them in a fixed order.  Both operands have the
-// summed index as their slow one: tiles of 64 rows go to LDS as they lie in memory (rows padded by
-// 32 bytes, so that the eight rows a half-wave reads lie on different banks) and come out
+// summed index as their slow one: stages of 32 rows go to LDS as they lie in memory (the 32-byte units of a row permuted by the row,
+// so that the eight rows a half-wave reads lie on different banks) and come out
 // transposed (ds_read_b64_tr_b16).  The order of the rows inside a product is the same for both
 // operands, hence free: a read takes rows 4 g .. 4 g + 3 for its lane group g.  The bias gradient is a product with
 // ones, in the workgroups of the first column of tiles.
 //
-// 12544 x 512 x 2048 with its reduction 43.5 us, 131072 x 384 x 96 32.7.  No unit is busy for more than a quarter of that (by
-// counters at the first size: matrix cores and LDS 24 % each, VALU 10 %, no bank conflicts, 111 MB through memory at 2.6 TB/s;
-// at the second LDS 16 %, 151 MB at 4.6 TB/s): what is left is the chain of a step, loads to LDS, barrier, reads, products, with two
-// workgroups per CU to overlap it.  Tried: two buffers with one barrier per step (no faster).  Larger tiles would read less per
-// product, but fewer tiles mean more splits, whose partial sums (33 MB for the first size) go through memory.
+// What binds it is the chain of a step, not a unit (by counters, with two barriers per 64 rows and staging through registers, at 12544 x
+// 512 x 2048 matrix cores and LDS 24 % each, no bank conflicts, 111 MB through memory at 2.6 TB/s): so the loads go straight to
+// LDS, three stages ahead, with one barrier per stage, and where the partial sums weigh more there are fewer of them (LinearSplits).
+// us with the reduction, before / so: 12544 x 512 x 2048 46.3 / 39.6, 3136 x 4096 x 1024 56 / 42.5, 8192 x 384 x 1536 30.4 / 25.0,
+// 131072 x 384 x 96 37.7 / 33.9, 200704 x 512 x 128 62 / 56.  Tried: three stages and three workgroups per CU (its partial sums
+// cost more than it gives, 200704 x 512 x 128 78).  Larger tiles would read less per product, but fewer tiles mean more splits.
 #pragma once
 
 #include "dwo_common.h"
@@ -51,23 +52,27 @@ struct Mma<f16_t> {
 };
 
 constexpr int kLinThreads = 256, kLinTile = 128, kLinRows = 64;
-constexpr int kLinPitch = kLinTile + 16;  // elements per LDS row
+constexpr int kLinStage = 32;  // rows that travel together
+constexpr long kLinFew = 4, kLinAlone = 224;  // tiles (LinearSplits)
 constexpr unsigned kLinNowhere = 0x80000000u;
 
+// Place of a fragment in a stage: columns [16 unit, 16 unit + 16) of rows 4 g + i / 4 and 16 rows on, as the transposing read
+// takes them (lane 16 g + i; rows of 256 bytes, their 32-byte units permuted by the row)
+__device__ __forceinline__ int lin_column_at(int unit) {
+    const int lane = threadIdx.x & 63, i = lane & 15, row = 4 * (lane >> 4) + (i >> 2);
+    return row * kLinTile + (unit ^ (row & 7)) * 16 + (i & 3) * 4;
+}
 // eight values of a column in rows [r, r + 4) and [r + 16, r + 20), r = 4 * (lane / 16)
-__device__ __forceinline__ mma_s8 lin_column(const uint16_t *tile, int row, int col) {
-    const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15;
-    const uint16_t *p = tile + (row + 4 * g + (i >> 2)) * kLinPitch + col + (i & 3) * 4;
+__device__ __forceinline__ mma_s8 lin_column(const uint16_t *stage, int at) {
     typedef __attribute__((address_space(3))) mma_s4 lds_s4;
-    const mma_s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)p);
-    const mma_s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(p + 16 * kLinPitch));
+    const mma_s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(stage + at));
+    const mma_s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(stage + at + 16 * kLinTile));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// rows [m, m + 64) of one operand's column tile, 16 bytes per load; zeros beyond its last row or column
+// 32 rows of one operand's column tile straight to LDS, 16 bytes per lane and load; zeros beyond its last row or column
 struct LinSource {
-    mma_u4 v[4];
-    unsigned off[4];
+    unsigned off[2];
     const char *at;
     long left;  // bytes from `at` to the end
     __device__ __forceinline__ void init(const void *p, long rows, long m0, int cols, int c0) {
@@ -75,35 +80,44 @@ struct LinSource {
         at = reinterpret_cast<const char *>(p) + m0 * pitch;
         left = max(rows - m0, 0L) * (long)pitch;
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int f = threadIdx.x + u * kLinThreads, c = c0 + f % 16 * 8;
-            off[u] = c < cols ? (unsigned)(f / 16) * pitch + (unsigned)c * 2 : kLinNowhere;
+        for (int u = 0; u < 2; u++) {
+            const int f = threadIdx.x + u * kLinThreads, row = f / 16, q = f % 16;
+            const int c = c0 + ((q >> 1 ^ (row & 7)) * 2 + (q & 1)) * 8;
+            off[u] = c < cols ? (unsigned)row * pitch + (unsigned)c * 2 : kLinNowhere;
         }
     }
-    __device__ __forceinline__ void load(int cols) {
-        const __amdgpu_buffer_rsrc_t r =
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(at), 0, (unsigned)min(left, 0x7fffffffL), 0x00020000);
+    __device__ __forceinline__ void load(uint16_t *stage, int cols) {
+        typedef __attribute__((address_space(3))) void lds_void;
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<char *>(at), 0, (unsigned)max(0L, min(left, 0x7fffffffL)), 0x00020000);
+#ifdef __HIP_DEVICE_COMPILE__
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-            v[u] = __builtin_bit_cast(mma_u4, __builtin_amdgcn_raw_buffer_load_b128(r, off[u], 0, 0));
-        at += (long)kLinRows * cols * 2, left -= (long)kLinRows * cols * 2;
-    }
-    __device__ __forceinline__ void store(uint16_t *tile) const {
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int f = threadIdx.x + u * kLinThreads;
-            *reinterpret_cast<mma_u4 *>(tile + f / 16 * kLinPitch + f % 16 * 8) = v[u];
-        }
+        for (int u = 0; u < 2; u++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(stage + (u * kLinThreads + wave * 64) * 8), 16, off[u], 0,
+                                                     0, 0);
+#endif
+        at += (long)kLinStage * cols * 2, left -= (long)kLinStage * cols * 2;
     }
 };
 
-// part [split][N * K + N]
-template <typename T>
+// dw [split][stride] and db [split][stride]: partial sums, or with one split the gradients themselves (db may be null).
+// HALVES: the sums of the first half of a split's rows wait in registers of their own, so that no chain is longer than where
+// twice as many splits share the rows (error against 64 bits at 200704 x 512 x 128 with 256 workgroups 3.5e-7, like this 2.5e-7, with
+// 512 2.5e-7).
+template <typename T, typename TO, bool HALVES>
 __global__ __launch_bounds__(kLinThreads, 2) void linear_wgrad_kernel(const T *__restrict__ dy,
-                                                                      const T *__restrict__ x,
-                                                                      float *__restrict__ part, long rows, int N,
-                                                                      int K, int splits, int steps, int with_bias) {
-    __shared__ __attribute__((aligned(16))) uint16_t lds[2][kLinRows * kLinPitch];
+                                                                      const T *__restrict__ x, TO *__restrict__ dw,
+                                                                      TO *__restrict__ db, size_t stride, long rows,
+                                                                      int N, int K, int splits, int steps) {
+    __shared__ __attribute__((aligned(16))) uint16_t sa0[kLinStage * kLinTile];
+    __shared__ __attribute__((aligned(16))) uint16_t sb0[kLinStage * kLinTile];
+    __shared__ __attribute__((aligned(16))) uint16_t sa1[kLinStage * kLinTile];
+    __shared__ __attribute__((aligned(16))) uint16_t sb1[kLinStage * kLinTile];
+    __shared__ __attribute__((aligned(16))) uint16_t sa2[kLinStage * kLinTile];
+    __shared__ __attribute__((aligned(16))) uint16_t sb2[kLinStage * kLinTile];
+    __shared__ __attribute__((aligned(16))) uint16_t sa3[kLinStage * kLinTile];
+    __shared__ __attribute__((aligned(16))) uint16_t sb3[kLinStage * kLinTile];
     const int tk = (K + kLinTile - 1) / kLinTile, tiles = (N + kLinTile - 1) / kLinTile * tk;
     // the tiles of a split read the same rows: one XCD (workgroup ids modulo eight) takes whole splits
     int split, tile;
@@ -117,11 +131,13 @@ __global__ __launch_bounds__(kLinThreads, 2) void linear_wgrad_kernel(const T *_
     const long m0 = (long)split * steps * kLinRows;
     const long last = min(rows, m0 + (long)steps * kLinRows);
     const int wave = threadIdx.x >> 6, wn = wave / 2 * 64, wk = wave % 2 * 64;
-    const bool bias = with_bias != 0 && k0 == 0 && wk == 0;
+    const bool bias = db != nullptr && k0 == 0 && wk == 0;
     mma_f4 acc[4][4], accb[4];
+    int ca[4], cb[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         accb[i] = mma_f4{0.f, 0.f, 0.f, 0.f};
+        ca[i] = lin_column_at(wn / 16 + i), cb[i] = lin_column_at(wk / 16 + i);
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[i][j] = mma_f4{0.f, 0.f, 0.f, 0.f};
     }
@@ -129,32 +145,61 @@ __global__ __launch_bounds__(kLinThreads, 2) void linear_wgrad_kernel(const T *_
 #pragma unroll
     for (int i = 0; i < 8; i++) ones[i] = Mma<T>::kOne;
     LinSource a, b;
-    a.init(dy, rows, m0, N, n0);
-    b.init(x, rows, m0, K, k0);
-    a.load(N), b.load(K);
-    for (long m = m0; m < last; m += kLinRows) {
-        __syncthreads();
-        a.store(lds[0]), b.store(lds[1]);
-        __syncthreads();
-        if (m + kLinRows < last) a.load(N), b.load(K);
+    a.init(dy, min(rows, max(last, m0)), m0, N, n0);
+    b.init(x, min(rows, max(last, m0)), m0, K, k0);
+    // a stage is multiplied while the next three travel (loads beyond the split's last row read nowhere)
+    auto stage = [&](uint16_t *sa, uint16_t *sb, uint16_t *na, uint16_t *nb) {
+        __builtin_amdgcn_s_waitcnt(0x0f78);  // vmcnt(8): this wave's part of the stage is there ..
+        asm volatile("s_barrier" ::: "memory");  // .. and the other waves'; nobody reads the one before any more
+        a.load(na, N), b.load(nb, K);
+        __builtin_amdgcn_sched_barrier(0);
+        mma_s8 fa[4], fb[4];
 #pragma unroll
-        for (int r = 0; r < kLinRows; r += 32) {
-            mma_s8 fa[4], fb[4];
+        for (int i = 0; i < 4; i++) fa[i] = lin_column(sa, ca[i]);
 #pragma unroll
-            for (int i = 0; i < 4; i++) fa[i] = lin_column(lds[0], r, wn + 16 * i);
+        for (int j = 0; j < 4; j++) fb[j] = lin_column(sb, cb[j]);
 #pragma unroll
-            for (int j = 0; j < 4; j++) fb[j] = lin_column(lds[1], r, wk + 16 * j);
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+            for (int j = 0; j < 4; j++) acc[i][j] = Mma<T>::run(fa[i], fb[j], acc[i][j]);
+        if (bias)
 #pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = Mma<T>::run(fa[i], fb[j], acc[i][j]);
-            if (bias)
-#pragma unroll
-                for (int i = 0; i < 4; i++) accb[i] = Mma<T>::run(fa[i], ones, accb[i]);
+            for (int i = 0; i < 4; i++) accb[i] = Mma<T>::run(fa[i], ones, accb[i]);
+    };
+    a.load(sa0, N), b.load(sb0, K);
+    a.load(sa1, N), b.load(sb1, K);
+    a.load(sa2, N), b.load(sb2, K);
+    const int pairs = (int)((max(last - m0, 0L) + 2 * kLinStage - 1) / (2 * kLinStage));
+    auto run = [&](int n) {
+        for (int p = 0; p < n; p++) {
+            stage(sa0, sb0, sa3, sb3), stage(sa1, sb1, sa0, sb0);
+            stage(sa2, sb2, sa1, sb1), stage(sa3, sb3, sa2, sb2);
         }
+    };
+    mma_f4 half[4][4], halfb[4];
+    if constexpr (HALVES) {
+        run(pairs / 4);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            halfb[i] = accb[i], accb[i] = mma_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 4; j++) half[i][j] = acc[i][j], acc[i][j] = mma_f4{0.f, 0.f, 0.f, 0.f};
+        }
+        run(pairs / 2 - pairs / 4);
+    } else {
+        run(pairs / 2);
     }
+    if (pairs % 2 != 0) stage(sa0, sb0, sa3, sb3), stage(sa1, sb1, sa0, sb0);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // (nothing may arrive in LDS behind the workgroup's end)
     const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    float *out = part + (size_t)split * ((size_t)N * K + N);
+    TO *out = dw + (size_t)split * stride;
+    if constexpr (HALVES)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            accb[i] += halfb[i];
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] += half[i][j];
+        }
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -164,67 +209,97 @@ __global__ __launch_bounds__(kLinThreads, 2) void linear_wgrad_kernel(const T *_
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int k = k0 + wk + 16 * j + c;
-                if (k < K) out[(size_t)n * K + k] = acc[i][j][r];
+                if (k < K) out[(size_t)n * K + k] = from_float<TO>(acc[i][j][r]);
             }
-            if (bias && c == 0) out[(size_t)N * K + n] = accb[i][r];
+            if (bias && c == 0) db[(size_t)split * stride + n] = from_float<TO>(accb[i][r]);
         }
 }
 
-// Sums over the splits, fixed order: eight threads share four outputs, each takes every eighth split.
-template <typename TO>
+// Sums over the splits, fixed order: SHARE threads share four outputs, each takes every SHARE-th split.
+template <typename TO, int SHARE>
 __global__ __launch_bounds__(kLinThreads) void linear_reduce_kernel(const float *__restrict__ part,
                                                                     TO *__restrict__ dw, TO *__restrict__ db, int N,
                                                                     int K, int splits) {
-    __shared__ mma_f4 red[kLinThreads];
+    constexpr int VECS = kLinThreads / SHARE;
+    __shared__ mma_f4 red[SHARE > 1 ? kLinThreads : 1];
     const size_t total = (size_t)N * K + N, first = (size_t)N * K;
-    const size_t i = ((size_t)blockIdx.x * 32 + threadIdx.x % 32) * 4;
+    const size_t i = ((size_t)blockIdx.x * VECS + threadIdx.x % VECS) * 4;
     mma_f4 s = mma_f4{0.f, 0.f, 0.f, 0.f};
     if (i < total)
-        for (int p = threadIdx.x / 32; p < splits; p += 8)
+#pragma unroll 4
+        for (int p = threadIdx.x / VECS; p < splits; p += SHARE)
             s += *reinterpret_cast<const mma_f4 *>(part + (size_t)p * total + i);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x >= 32 || i >= total || (i >= first && db == nullptr)) return;
+    if constexpr (SHARE > 1) {
+        red[threadIdx.x] = s;
+        __syncthreads();
+    }
+    if (threadIdx.x >= VECS || i >= total || (i >= first && db == nullptr)) return;
 #pragma unroll
-    for (int p = 1; p < 8; p++) s += red[threadIdx.x + 32 * p];
+    for (int p = 1; p < SHARE; p++) s += red[threadIdx.x + VECS * p];
     TO *out = i < first ? dw + i : db + (i - first);
 #pragma unroll
     for (int e = 0; e < 4; e++) out[e] = from_float<TO>(s[e]);
 }
 
-// Splits of the rows: two workgroups per CU (512), each with 256 rows where they were dealt evenly; a multiple of eight
-// where there are as many (whole splits per XCD).  A split holds whole steps of 64 rows, rounded up, so the last few may hold no
-// rows (10 of 168 for 131072 x 384 x 96): their sums are zeros.
-inline int linear_splits(size_t rows, int N, int K) {
-    const long tiles = (long)((N + kLinTile - 1) / kLinTile) * ((K + kLinTile - 1) / kLinTile);
-    const long steps = (long)((rows + kLinRows - 1) / kLinRows);
-    long s = 512 / tiles;
-    if (s > steps / 4) s = steps / 4;
-    if (s >= 8) s = s / 8 * 8;
-    return (int)(s < 1 ? 1 : s);
-}
+// Splits of the rows, each with 256 rows where they are dealt evenly; a multiple of eight where there are as many (whole splits
+// per XCD).  Two workgroups per CU (512), but
+//   one where the outputs are at most four tiles, memory binds, and the partial sums, 64 KB per workgroup both ways, are what can be
+//   saved (us with the sums, 512 / 256: 200704 x 512 x 128 64 / 58, 131072 x 384 x 96 40 / 33, 200704 x 128 x 64 36 / 23; eight tiles,
+//   50176 x 256 x 512, 31.5 / 32.2);
+//   no split where the tiles alone give each CU its workgroup (3136 x 4096 x 1024 53 / 44).
+// A split holds whole steps of 64 rows, rounded up, so the last few may hold no rows: their sums are zeros.
+struct LinearSplits {
+    int splits;
+    bool halves;
+    LinearSplits(size_t rows, int N, int K) {
+        const long tiles = (long)((N + kLinTile - 1) / kLinTile) * ((K + kLinTile - 1) / kLinTile);
+        const long steps = (long)((rows + kLinRows - 1) / kLinRows);
+        halves = tiles <= kLinFew || tiles >= kLinAlone;
+        long s = tiles >= kLinAlone ? 1 : (halves ? 256 : 512) / tiles;
+        if (s > steps / 4) s = steps / 4;
+        if (s >= 8) s = s / 8 * 8;
+        splits = (int)(s < 1 ? 1 : s);
+        halves = halves && steps >= 16;
+    }
+};
 inline size_t linear_wgrad_scratch(size_t rows, int N, int K) {
-    return (size_t)linear_splits(rows, N, K) * ((size_t)N * K + N) * sizeof(float);
+    return (size_t)LinearSplits(rows, N, K).splits * ((size_t)N * K + N) * sizeof(float);
 }
 
-template <typename T>
-int launch_linear_wgrad(const void *dy, const void *x, float *part, size_t rows, int N, int K, int splits,
-                        int with_bias, hipStream_t st) {
+template <typename T, typename TO>
+int launch_linear_products(const void *dy, const void *x, TO *dw, TO *db, size_t stride, size_t rows, int N, int K,
+                           const LinearSplits &s, hipStream_t st) {
+    const int splits = s.splits;
     const long steps = (long)((rows + kLinRows - 1) / kLinRows);
     const int per = (int)((steps + splits - 1) / splits);
     const unsigned tiles = (unsigned)((N + kLinTile - 1) / kLinTile) * ((K + kLinTile - 1) / kLinTile);
-    linear_wgrad_kernel<T><<<dim3(tiles * (unsigned)splits), dim3(kLinThreads), 0, st>>>(
-        (const T *)dy, (const T *)x, part, (long)rows, N, K, splits, per, with_bias);
+    const dim3 grid(tiles * (unsigned)splits), block(kLinThreads);
+    if (s.halves)
+        linear_wgrad_kernel<T, TO, true><<<grid, block, 0, st>>>((const T *)dy, (const T *)x, dw, db, stride, (long)rows, N, K,
+                                                                 splits, per);
+    else
+        linear_wgrad_kernel<T, TO, false><<<grid, block, 0, st>>>((const T *)dy, (const T *)x, dw, db, stride, (long)rows, N,
+                                                                  K, splits, per);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : (int)e;
 }
-template <typename TO>
-int launch_linear_reduce(const float *part, void *dw, void *db, int N, int K, int splits, hipStream_t st) {
-    const size_t vecs = ((size_t)N * K + N) / 4;
-    linear_reduce_kernel<TO><<<dim3((unsigned)((vecs + 31) / 32)), dim3(kLinThreads), 0, st>>>(part, (TO *)dw,
-                                                                                              (TO *)db, N, K, splits);
-    const hipError_t e = hipGetLastError();
-    return e == hipSuccess ? 0 : (int)e;
+template <typename T, typename TO>
+int launch_linear_wgrad(const void *dy, const void *x, void *dw, void *db, float *part, size_t rows, int N, int K,
+                        hipStream_t st) {
+    const LinearSplits s(rows, N, K);
+    const int splits = s.splits;
+    if (splits == 1) return launch_linear_products<T, TO>(dy, x, (TO *)dw, (TO *)db, 0, rows, N, K, s, st);
+    const size_t outputs = (size_t)N * K, stride = outputs + N;
+    const int e = launch_linear_products<T, float>(dy, x, part, db != nullptr ? part + outputs : nullptr, stride, rows, N, K,
+                                                   s, st);
+    if (e != 0) return e;
+    const size_t vecs = stride / 4;
+    const int share = splits < 8 ? 1 : 8, per = kLinThreads / share;
+    const dim3 grid((unsigned)((vecs + per - 1) / per)), block(kLinThreads);
+    if (share == 1) linear_reduce_kernel<TO, 1><<<grid, block, 0, st>>>(part, (TO *)dw, (TO *)db, N, K, splits);
+    else linear_reduce_kernel<TO, 8><<<grid, block, 0, st>>>(part, (TO *)dw, (TO *)db, N, K, splits);
+    const hipError_t err = hipGetLastError();
+    return err == hipSuccess ? 0 : (int)err;
 }
 
 // ------------------------------------------------------------------------------------------------- inference

@@ -19,21 +19,20 @@ int dwo_linear_wgrad(const void *dy, const void *x, void *dw, void *db, void *sc
     if (scratch_bytes < need) return DWO_ERR_SCRATCH_TOO_SMALL;
     hipStream_t st = (hipStream_t)stream;
     (void)hipGetLastError();  // (an earlier call's error is not this call's status)
-    const int splits = linear_splits(rows, N, K);
     float *part = (float *)scratch;
-    int e;
+#define DWO_TYPES(T)                                                                                    \
+    switch (grad_dtype) {                                                                               \
+        case DWO_F32: return launch_linear_wgrad<T, float>(dy, x, dw, db, part, rows, N, K, st);        \
+        case DWO_BF16: return launch_linear_wgrad<T, bf16_t>(dy, x, dw, db, part, rows, N, K, st);      \
+        case DWO_F16: return launch_linear_wgrad<T, f16_t>(dy, x, dw, db, part, rows, N, K, st);        \
+        default: return DWO_ERR_BAD_DTYPE;                                                              \
+    }
     switch (dtype) {
-        case DWO_BF16: e = launch_linear_wgrad<bf16_t>(dy, x, part, rows, N, K, splits, db != nullptr, st); break;
-        case DWO_F16: e = launch_linear_wgrad<f16_t>(dy, x, part, rows, N, K, splits, db != nullptr, st); break;
+        case DWO_BF16: DWO_TYPES(bf16_t)
+        case DWO_F16: DWO_TYPES(f16_t)
         default: return DWO_ERR_BAD_DTYPE;
     }
-    if (e != 0) return e;
-    switch (grad_dtype) {
-        case DWO_F32: return launch_linear_reduce<float>(part, dw, db, N, K, splits, st);
-        case DWO_BF16: return launch_linear_reduce<bf16_t>(part, dw, db, N, K, splits, st);
-        case DWO_F16: return launch_linear_reduce<f16_t>(part, dw, db, N, K, splits, st);
-        default: return DWO_ERR_BAD_DTYPE;
-    }
+#undef DWO_TYPES
 }
 
 // y = x w^T + b over 16-bit activations; x, w and out 16-byte aligned, N and K multiples of eight, offsets inside 31 bits

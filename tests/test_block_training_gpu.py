@@ -180,6 +180,25 @@ def test_linear_gradients(M, K, N, dtype):
     close(db, dy.double().sum(0), 1e-5, "db")
 
 
+# stages of 32 rows, four in flight: rows around a stage, a step of 64 and the four; outputs around a tile of 128; few tiles, whose
+# sums are kept in halves from 16 steps on; as many tiles as CUs, which write the gradients themselves in either type
+@pytest.mark.parametrize("grad", [F32, BF16])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (31, 128, 128), (33, 136, 120), (65, 256, 264), (127, 8, 1024), (129, 64, 72),
+                                   (1023, 128, 256), (1025, 120, 128), (4161, 256, 136), (20011, 128, 96), (97, 1920, 1920),
+                                   (1300, 1800, 2056)])
+def test_linear_wgrad_stages_and_splits(M, N, K, grad):
+    from oriented1d_amd import _lib
+    torch.manual_seed(M + N)
+    x, dy = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(M, N, device="cuda").bfloat16()
+    for bias in (True, False):
+        dw, db = _lib.host(0).linear_wgrad(dy, x, bias, grad)
+        tol = 1e-5 if grad == F32 else 2.0 ** -8
+        close(dw, dy.double().t() @ x.double(), tol, "dw")
+        assert (db is None) == (not bias)
+        if bias:
+            close(db, dy.double().sum(0), tol, "db")
+
+
 def test_linear_covers_batches_views_and_second_order():
     torch.manual_seed(0)
     m = fused.Linear(64, 128).cuda().bfloat16()
