@@ -302,6 +302,16 @@ int dwo_linear_planes(const void *x, const void *w, const void *bias, const void
 int dwo_block_mlp(const void *x, const void *w1, const void *b1, const void *w2, const void *b2, const void *scale,
                   const void *res, void *out, int images, int HW, int C, int dtype, void *stream);
 
+/*
+ * The stem's last layers at inference in one kernel (models/convnext.py:184-190), for 16-bit types, K = 64 and N = 96 or
+ * 128: out [images,N,HW] = LayerNorm over n of (bias[n] + sum_k w[n][k] z[image][p][k]), where z is GELU(LayerNorm over k of
+ * x) in x's type, x [images,HW,K].  x, w [N,K] and bias [N] (or null) have the activations' type, x, w and out are 16-byte
+ * aligned, images * HW is below 2^31; the norms' parameters (gamma_in, beta_in [K]; gamma, beta [N]) are fp32.
+ */
+int dwo_linear_norm_planes(const void *x, const float *gamma_in, const float *beta_in, float eps_in, const void *w,
+                           const void *bias, const float *gamma, const float *beta, float eps, void *out, int images, int HW,
+                           int N, int K, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -48,6 +48,7 @@ SIGNATURES = {
     "dwo_linear_rows": (_i, [_vp] * 4 + [_sz] + [_i] * 4 + [_vp]),
     "dwo_linear_planes": (_i, [_vp] * 6 + [_i] * 5 + [_vp]),
     "dwo_block_mlp": (_i, [_vp] * 8 + [_i] * 4 + [_vp]),
+    "dwo_linear_norm_planes": (_i, [_vp] * 3 + [ctypes.c_float] + [_vp] * 4 + [ctypes.c_float, _vp] + [_i] * 5 + [_vp]),
     "dwo_linear_wgrad": (_i, [_vp] * 5 + [_sz, _sz] + [_i] * 4 + [_vp]),
 }
 

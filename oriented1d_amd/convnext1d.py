@@ -135,7 +135,11 @@ class Stem1D(nn.Module):
             x = fused.pointwise_dwconv_nhwc(x, self.pw1, dw1)
             x = fused.layernorm_nhwc(x, self.norm1.weight, self.norm1.bias, self.norm1.eps,
                                      gelu=True)
-            x = fused.layernorm_nhwc(self.dw2(x), self.norm2.weight, self.norm2.bias,
+            x = self.dw2(x)
+            y = fused.norm_planes(x, self.norm2, self.pw2, self.norm3)
+            if y is not None:
+                return y
+            x = fused.layernorm_nhwc(x, self.norm2.weight, self.norm2.bias,
                                      self.norm2.eps, gelu=True)
             x = fused.layernorm_nhwc(self.pw2(x), self.norm3.weight, self.norm3.bias,
                                      self.norm3.eps)

@@ -52,6 +52,7 @@ struct Library {
     decltype(&::dwo_block_mlp) block_mlp;
     decltype(&::dwo_linear_rows) linear_rows;
     decltype(&::dwo_linear_planes) linear_planes;
+    decltype(&::dwo_linear_norm_planes) linear_norm_planes;
 } lib;
 
 [[noreturn]] void fail(const std::string &msg) { throw std::runtime_error(msg); }
@@ -89,6 +90,7 @@ void bind_library(const std::string &path) {
     find(lib.block_mlp, "dwo_block_mlp");
     find(lib.linear_rows, "dwo_linear_rows");
     find(lib.linear_planes, "dwo_linear_planes");
+    find(lib.linear_norm_planes, "dwo_linear_norm_planes");
 }
 
 void check(int status, const char *what) {
@@ -657,6 +659,27 @@ Tensor linear_planes(const Tensor &x_, const Tensor &w_, const OptTensor &b_, co
     return out;
 }
 
+// x [N,H,W,K] -> [N,C,H,W]: LayerNorm over C (fp32 g and beta) of z w^T + b with z = GELU(LayerNorm over K of x)
+Tensor linear_norm_planes(const Tensor &x_, const Tensor &g_in, const Tensor &beta_in, double eps_in, const Tensor &w_,
+                          const OptTensor &b_, const Tensor &g, const Tensor &beta, double eps) {
+    check_layer(x_, w_);
+    if (x_.dim() != 4) throw py::value_error("x must be a 4-d tensor");
+    const int64_t C = w_.size(0), K = w_.size(1);
+    check_norm(x_, g, beta, C);
+    check_norm(x_, g_in, beta_in, K);
+    const Dims d(x_, true);
+    py::gil_scoped_release nogil;
+    const Place at(x_);
+    const OptTensor b = dense_values(x_, b_, C, "bias");
+    const Tensor x = dense(x_), w = dense(w_);
+    Tensor out = at::empty({d.n, C, d.h, d.w}, x.options());
+    check(lib.linear_norm_planes(ptr(x), (const float *)ptr(g_in), (const float *)ptr(beta_in), (float)eps_in, ptr(w), optr(b), (const float *)ptr(g),
+                                 (const float *)ptr(beta), (float)eps, out.data_ptr(), as_int(d.n), as_int(d.h * d.w),
+                                 as_int(C), as_int(K), dtype_code(x), at.stream),
+          "dwo_linear_norm_planes");
+    return out;
+}
+
 // x [N,H,W,C], res [N,C,H,W] -> res + scale * (w2 gelu(w1 x + b1) + b2), planes
 Tensor block_mlp(const Tensor &x_, const Tensor &w1_, const Tensor &b1_, const Tensor &w2_, const Tensor &b2_,
                  const OptTensor &scale_, const Tensor &res_) {
@@ -709,6 +732,7 @@ PYBIND11_MODULE(_host, m) {
     m.def("conv_norm", &conv_norm);
     m.def("linear_rows", &linear_rows);
     m.def("linear_planes", &linear_planes);
+    m.def("linear_norm_planes", &linear_norm_planes);
     m.def("ln_rows", &ln_rows);
     m.def("ln_rows_backward", &ln_rows_backward);
     m.def("ln_tile", &ln_tile);

@@ -669,6 +669,133 @@ int launch_linear(const LinearArgs<T> &a, hipStream_t st) {
     return e == hipSuccess ? 0 : (int)e;
 }
 
+// ------------------------------------------------------------------------------------------------- norm behind a layer
+// out[image][n][p] = LayerNorm over n of (b[n] + sum_k w[n][k] z[image][p][k]) with z = GELU(LayerNorm over k of x), rounded as a layer
+// of its own would: the stem's last layers with the planes that follow (models/convnext.py:184-190), K = 64 and N = 16 NB <= 128.
+// A wave holds the weights as fragments and takes 32 pixels at a time with all their channels, so that a LayerNorm is a sum
+// over its registers and a few lanes.  GELU's vector instructions bound it: 401408 x 64 -> 96 in bf16 56 us (without the first norm
+// 38, which is reading x and writing the planes; as a norm pass, the library's product, a norm pass and a transposition 200), one
+// image 8 (20).
+constexpr int kNormK = 64, kNormGroups = 1024;
+struct NormArgs {
+    const float *gamma, *beta, *gamma_in, *beta_in;
+    float eps, eps_in;
+};
+template <typename T, int NB>
+__global__ __launch_bounds__(kLinThreads, 2) void linear_norm_kernel(LinearArgs<T> a, NormArgs na, long tiles) {
+    __shared__ __attribute__((aligned(16))) float affine[2 * kNormK];  // of the norm before
+    if (threadIdx.x < 2 * kNormK)
+        affine[threadIdx.x] = threadIdx.x < kNormK ? na.gamma_in[threadIdx.x] : na.beta_in[threadIdx.x - kNormK];
+    __syncthreads();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    mma_s8 fw[2][NB];
+    float bias[NB], gm[NB], bt[NB];
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        const int n = 16 * j + c;
+#pragma unroll
+        for (int k = 0; k < 2; k++) fw[k][j] = *reinterpret_cast<const mma_s8 *>(a.w + n * kNormK + k * 32 + g * 8);
+        bias[j] = a.bias != nullptr ? to_float(a.bias[n]) : 0.f, gm[j] = na.gamma[n], bt[j] = na.beta[n];
+    }
+    auto lanes = [](float v) {  // over the sixteen lanes of a row
+        auto add = [](float v, auto ctrl) {
+            return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value,
+                                                                             0xf, 0xf, true));
+        };
+        v = add(v, std::integral_constant<int, 0xB1>{});      // quad_perm [1,0,3,2]
+        v = add(v, std::integral_constant<int, 0x4E>{});      // quad_perm [2,3,0,1]
+        v = add(v, std::integral_constant<int, 0x141>{});     // row_half_mirror
+        return add(v, std::integral_constant<int, 0x140>{});  // row_mirror
+    };
+    mma_s8 fx[2][2], next[2][2];
+    auto fetch = [&](mma_s8 (&f)[2][2], long tile) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const long m = min(tile * 32 + 8 * (c >> 2) + 4 * i + (c & 3), a.M - 1);  // (pixels beyond the last are not written)
+#pragma unroll
+            for (int k = 0; k < 2; k++) f[k][i] = *reinterpret_cast<const mma_s8 *>(a.x + m * kNormK + k * 32 + g * 8);
+        }
+    };
+    const long step = (long)gridDim.x * (kLinThreads / 64);
+    long tile = (long)blockIdx.x * (kLinThreads / 64) + wave;
+    if (tile >= tiles) return;
+    fetch(next, tile);
+    for (; tile < tiles; tile += step) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) fx[k][0] = next[k][0], fx[k][1] = next[k][1];
+        if (tile + step < tiles) fetch(next, tile + step);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {  // a lane has 16 of its pixel's channels, the lanes 16, 32 and 48 on the others
+            float u[2][8], s = 0.f, q = 0.f;
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    u[k][e] = to_float(__builtin_bit_cast(T, (uint16_t)fx[k][i][e])), s += u[k][e];
+            s += __shfl_xor(s, 16, 64), s += __shfl_xor(s, 32, 64);
+            s *= 1.f / kNormK;
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) u[k][e] -= s, q = __builtin_fmaf(u[k][e], u[k][e], q);
+            q += __shfl_xor(q, 16, 64), q += __shfl_xor(q, 32, 64);
+            q = rsqrtf(q * (1.f / kNormK) + na.eps_in);
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const float *p = affine + 32 * k + 8 * g;
+                mma_u4 o;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const mma_f4 gi = *reinterpret_cast<const mma_f4 *>(p + 4 * h);
+                    const mma_f4 bi = *reinterpret_cast<const mma_f4 *>(p + kNormK + 4 * h);
+                    float w[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) w[e] = gelu_rounded(__builtin_fmaf(u[k][4 * h + e] * q, gi[e], bi[e]));
+                    o[2 * h] = lin_pack<T>(w[0], w[1]), o[2 * h + 1] = lin_pack<T>(w[2], w[3]);
+                }
+                fx[k][i] = __builtin_bit_cast(mma_s8, o);
+            }
+        }
+        mma_f4 v[2][NB];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            mma_f4 s = mma_f4{0.f, 0.f, 0.f, 0.f}, q = s;
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                v[i][j] = mma_f4{bias[j], bias[j], bias[j], bias[j]};
+#pragma unroll
+                for (int k = 0; k < 2; k++) v[i][j] = Mma<T>::run(fx[k][i], fw[k][j], v[i][j]);
+#pragma unroll
+                for (int r = 0; r < 4; r++) s[r] += v[i][j][r];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) s[r] = lanes(s[r]) * (1.f / (16 * NB));
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[i][j][r] -= s[r], q[r] = __builtin_fmaf(v[i][j][r], v[i][j][r], q[r]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) q[r] = rsqrtf(lanes(q[r]) / (float)(16 * NB) + na.eps);
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[i][j][r] = __builtin_fmaf(v[i][j][r] * q[r], gm[j], bt[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < NB; j++) lin_emit_pixels8(a, tile * 32 + 8 * g, 16 * j + c, v[0][j], v[1][j], 0.f, 1.f);
+    }
+}
+
+template <typename T>
+int launch_linear_norm(const LinearArgs<T> &a, const NormArgs &na, hipStream_t st) {
+    const long tiles = (a.M + 31) / 32, want = (tiles + 3) / 4;
+    const dim3 grid((unsigned)(want < kNormGroups ? want : kNormGroups)), block(kLinThreads);
+    if (a.N == 96) linear_norm_kernel<T, 6><<<grid, block, 0, st>>>(a, na, tiles);
+    else linear_norm_kernel<T, 8><<<grid, block, 0, st>>>(a, na, tiles);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : (int)e;
+}
+
 // ------------------------------------------------------------------------------------------------- few inputs
 // y[m][n] = b[n] + sum_k x[m][k] * w[n][k] for K <= 4 (the stem's first layer, models/convnext.py:143,177) and N a multiple of
 // 64.  Writing y bounds it (64 x 224 x 224 pixels of 64 channels in bf16: 411 MB; back to back 147 us, as a library product 330;

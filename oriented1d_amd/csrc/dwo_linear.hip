@@ -80,6 +80,28 @@ int dwo_linear_planes(const void *x, const void *w, const void *bias, const void
     }
 }
 
+int dwo_linear_norm_planes(const void *x, const float *gamma_in, const float *beta_in, float eps_in, const void *w,
+                           const void *bias, const float *gamma, const float *beta, float eps, void *out, int images, int HW,
+                           int N, int K, int dtype, void *stream) {
+    if (!x || !gamma_in || !beta_in || !w || !gamma || !beta || !out) return DWO_ERR_NULL_POINTER;
+    if (images < 1 || HW < 1 || (double)images * HW >= 2147483648.0 || K != kNormK || (N != 96 && N != 128) ||
+        ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 != 0)
+        return DWO_ERR_BAD_SHAPE;
+    (void)hipGetLastError();
+    hipStream_t st = (hipStream_t)stream;
+    const long M = (long)images * HW;
+    const NormArgs na{gamma, beta, gamma_in, beta_in, eps, eps_in};
+    switch (dtype) {
+        case DWO_BF16:
+            return launch_linear_norm<bf16_t>({(const bf16_t *)x, (const bf16_t *)w, (const bf16_t *)bias, nullptr, nullptr,
+                                               (bf16_t *)out, M, N, K, HW, 0}, na, st);
+        case DWO_F16:
+            return launch_linear_norm<f16_t>({(const f16_t *)x, (const f16_t *)w, (const f16_t *)bias, nullptr, nullptr,
+                                              (f16_t *)out, M, N, K, HW, 0}, na, st);
+        default: return DWO_ERR_BAD_DTYPE;
+    }
+}
+
 int dwo_pointwise_forward(const void *x, const void *w, const void *b, void *y, size_t rows, int Cin, int C, int dtype,
                           void *stream) {
     if (!x || !w || !y) return DWO_ERR_NULL_POINTER;

@@ -101,6 +101,20 @@ def linear_tail(x, linear, gamma, residual):
     return nhwc_scale_add_nchw(linear(x), gamma, residual)
 
 
+def norm_planes(x, before, linear, norm):
+    """``norm(linear(F.gelu(before(x)))).permute(0, 3, 1, 2)`` without gradients as one kernel where the library covers it (the stem's
+    64 inputs, 96 or 128 outputs), else None."""
+    w, b = linear.weight, linear.bias
+    if not (plain(linear, Linear) and x.dim() == 4 and w.shape[1] == 64 and w.shape[0] in (96, 128) and _layer16(x, w, b)
+            and x.numel() < 1 << 37):
+        return None
+    affine = before.weight, before.bias, norm.weight, norm.bias
+    if any(p is None or p.device != x.device or p.shape != (C,) for p, C in zip(affine, (64, 64, w.shape[0], w.shape[0]))):
+        return None
+    g0, b0, g1, b1 = map(_f32, affine)
+    return _lib.host(x.get_device()).linear_norm_planes(x, g0, b0, before.eps, w, b, g1, b1, norm.eps)
+
+
 # Rows from which both layers run as one kernel: enough workgroups of 128 pixels that its long chain is paid for (bf16, us, two
 # kernels / one: 12544 x 96 25 / 17, 8192 x 96 15.9 / 16.8; 16384 x 128 21 / 25, 17408 x 128, where the first product has more
 # tiles than the chip holds, 30 / 25; 29008 x 192 47 / 43, 25088 x 192 43 / 42 and in odd planes 67 / 70).  There is no instance for

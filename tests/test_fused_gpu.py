@@ -575,3 +575,32 @@ def test_inference_block_checked_once(C, plus_plus, hw, N, dtype, gamma, wrapped
         assert taken[-1] is None
         block.float()(x.float())
         assert taken[-1] is None
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("N,H,W,C,bias", [(1, 1, 1, 96, True), (3, 33, 31, 96, True), (2, 6, 10, 128, False), (5, 8, 12, 128, True),
+                                          (70, 56, 56, 96, True)])  # (pixels by eight, four and one; waves that take several tiles)
+def test_stem_tail_as_one_kernel(N, H, W, C, bias, dtype):
+    """LayerNorm + GELU + pointwise layer + LayerNorm as planes against the same layers in fp64, the value between them rounded as a
+    layer's output; tolerance: twice the type's rounding in the norm, its largest step relative to the largest value."""
+    import torch.nn.functional as F
+    from oriented1d_amd import fused
+    torch.manual_seed(H * W)
+    before, norm, linear = torch.nn.LayerNorm(64, eps=1e-6), torch.nn.LayerNorm(C, eps=1e-6), fused.Linear(64, C, bias=bias)
+    with torch.no_grad():
+        for m in (before, norm):
+            m.weight.add_(torch.randn(m.weight.shape) * 0.3), m.bias.add_(torch.randn(m.bias.shape) * 0.3)
+        before, norm, linear = (m.cuda().to(dtype) for m in (before, norm, linear))
+        x = (torch.randn(N, H, W, 64, device="cuda") * 3 + 1).to(dtype)
+        got = fused.norm_planes(x, before, linear, norm)
+        z = F.gelu(F.layer_norm(x.double(), (64,), before.weight.double(), before.bias.double(), 1e-6)).to(dtype).double()
+        y = F.linear(z, linear.weight.double(), None if not bias else linear.bias.double())
+        ref = F.layer_norm(y, (C,), norm.weight.double(), norm.bias.double(), 1e-6).permute(0, 3, 1, 2)
+        assert got.shape == ref.shape and got.is_contiguous() and got.dtype == dtype
+        ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+        assert (got.double() - ref).norm() <= ulp * ref.norm() and (got.double() - ref).abs().max() <= 2 * ulp * ref.abs().max()
+        handle = linear.register_forward_hook(lambda *_: None)
+        assert fused.norm_planes(x, before, linear, norm) is None
+        handle.remove()
+        assert fused.norm_planes(x.float(), before.float(), linear.float(), norm.float()) is None
+    assert fused.norm_planes(x, before.to(dtype), linear.to(dtype), norm.to(dtype)) is None  # (gradients are on)
