@@ -580,9 +580,9 @@ __global__ __launch_bounds__(kLinThreads, 2) void linear_kernel(LinearArgs<T> a,
     lin_emit<OUT, T, 2, QF>(a, (PLANES ? m0 : n0) + wp, (PLANES ? n0 : m0) + wq, acc);
 }
 
-// Fewer tiles than CUs: 64 x 64, and the four waves share the columns, a quarter of every 128 each (a chain half as long per
-// column, four times as many workgroups); their sums meet in LDS.  us, large tiles / these: 784 x 1536 x 384 9.7 / 6.8,
-// 196 x 768 x 3072 49 / 15.6, 3136 x 384 x 96 7.6 / 6.2; 3136 x 1536 x 384 (300 large tiles) 13.3 / 17.2.
+// Fewer tiles than CUs, but not few (launch_few_tiles): 64 x 64, and the four waves share the columns, a quarter of every 128 each
+// (a chain half as long per column, four times as many workgroups); their sums meet in LDS.  us, large tiles / these: 784 x
+// 1536 x 384 9.7 / 6.8, 3136 x 384 x 96 7.6 / 6.2; 3136 x 1536 x 384 (300 large tiles) 13.3 / 17.2.
 template <typename T, int OUT>
 __global__ __launch_bounds__(kLinThreads, 2) void linear_split_kernel(LinearArgs<T> a, int mtiles) {
     constexpr bool PLANES = OUT == LIN_PLANES;
@@ -644,6 +644,141 @@ __global__ __launch_bounds__(kLinThreads, 2) void linear_split_kernel(LinearArgs
     lin_emit<OUT, T, 1, 2>(a, (PLANES ? m0 : n0) + 32 * h, (PLANES ? n0 : m0) + 32 * x, sum);
 }
 
+// Fewer tiles still (launch_few_tiles): 32 rows of P and 16 * QF of Q.  No two waves read the same value (every fourth 64 columns are
+// a wave's), so each has its own four stages of LDS, three of them on their way, and no barrier until the sums meet: with the
+// kernel above two stages and few workgroups left the loads of a long row one after the other.  Through LDS and not straight to
+// registers, because a fragment's neighbouring lanes lie in different rows (196 x 384 x 1536 7.2, 49 x 768 x 3072 12.8).
+// bf16, us, 64 x 64 tiles / these: 49 x 3072 x 768 7.1 / 4.9, planes 196 x 384 x 1536 10.8 / 4.7, 784 x 192 x 768 7.2 / 4.2,
+// 98 x 1024 x 4096 24.0 / 8.5, 49 x 768 x 3072 19.3 / 7.5, rows 196 x 384 x 96 4.5 / 3.7 (an empty launch 3).
+template <typename T, int OUT, int QF>
+__global__ __launch_bounds__(kLinThreads, 1) void linear_wave_kernel(LinearArgs<T> a, int xtiles, int tiles) {
+    constexpr bool PLANES = OUT == LIN_PLANES;
+    constexpr int RP = 32, RQ = 16 * QF, BK = 64, WAVES = kLinThreads / 64, LP = RP / 8, LQ = RQ / 8;  // (a load is eight rows)
+    constexpr int SIZE = WAVES * (RP + RQ) * BK;
+    __shared__ __attribute__((aligned(16))) uint16_t s0[SIZE];
+    __shared__ __attribute__((aligned(16))) uint16_t s1[SIZE];
+    __shared__ __attribute__((aligned(16))) uint16_t s2[SIZE];
+    __shared__ __attribute__((aligned(16))) uint16_t s3[SIZE];
+    // an XCD (workgroup ids modulo eight) takes a run of tiles, those of x against the same weights next to each other
+    const int tile = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
+    if (tile >= tiles) return;
+    const long m0 = (long)(tile % xtiles) * (PLANES ? RP : RQ);
+    const int n0 = tile / xtiles * (PLANES ? RQ : RP);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const long pitch = (long)a.K * 2;
+    auto operand = [&](const T *p, long rows, long r0) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<const char *>(p) + r0 * pitch), 0,
+                                                 (unsigned)min((rows - r0) * pitch, 0x7fffffffL), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rp = PLANES ? operand(a.x, a.M, m0) : operand(a.w, a.N, n0);
+    const __amdgpu_buffer_rsrc_t rq = PLANES ? operand(a.w, a.N, n0) : operand(a.x, a.M, m0);
+    const int piece = (lane % 8) ^ (lane / 8);
+    unsigned op[LP], oq[LQ];  // (rows beyond the last lie beyond the operand's end: zeros)
+#pragma unroll
+    for (int u = 0; u < LP; u++) {
+        const int s = 8 * u + lane / 8;
+        const int row = OUT == LIN_PIXELS ? s : (s >> 2 & 3) * 8 + (s >> 4 & 1) * 4 + (s & 3);
+        op[u] = (unsigned)row * (unsigned)pitch + piece * 16;
+    }
+#pragma unroll
+    for (int u = 0; u < LQ; u++) oq[u] = (unsigned)(8 * u + lane / 8) * (unsigned)pitch + piece * 16;
+    int k0 = wave * BK;  // of the next load
+    auto load = [&](uint16_t *stage) {
+        typedef __attribute__((address_space(3))) void lds_void;
+        const unsigned kill = piece * 8 < a.K - k0 ? 0u : kLinNowhere;
+        uint16_t *at = stage + wave * (RP + RQ) * BK;
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+        for (int u = 0; u < LP; u++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rp, (lds_void *)(at + u * 8 * BK), 16, op[u] | kill, k0 * 2, 0, 0);
+#pragma unroll
+        for (int u = 0; u < LQ; u++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_void *)(at + (RP + u * 8) * BK), 16, oq[u] | kill, k0 * 2, 0, 0);
+#endif
+        k0 += WAVES * BK;
+    };
+    mma_f4 acc[2][QF];
+#pragma unroll
+    for (int i = 0; i < 2 * QF; i++) acc[i / QF][i % QF] = mma_f4{0.f, 0.f, 0.f, 0.f};
+    auto step = [&](const uint16_t *stage, uint16_t *next) {
+        // all but the next two stages' loads have arrived, and the reads of the one before, which `next` was
+        constexpr int N = 2 * (LP + LQ);
+        __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | N >> 4 << 14);  // vmcnt(N) lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        load(next);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint16_t *at = stage + wave * (RP + RQ) * BK;
+        mma_s8 fp[2][2], fq[2][QF];
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) fp[kk][i] = lin_fragment<BK>(at, 16 * i, kk);
+#pragma unroll
+            for (int j = 0; j < QF; j++) fq[kk][j] = lin_fragment<BK>(at + RP * BK, 16 * j, kk);
+        }
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < QF; j++) acc[i][j] = Mma<T>::run(fp[kk][i], fq[kk][j], acc[i][j]);
+    };
+    load(s0), load(s1), load(s2);
+    int left = (a.K + WAVES * BK - 1) / (WAVES * BK);
+    for (; left > 2; left -= 4) {
+        step(s0, s3), step(s1, s0), step(s2, s1);
+        if (left == 3) { left = 0; break; }
+        step(s3, s2);
+    }
+    if (left > 0) step(s0, s3);
+    if (left > 1) step(s1, s0);
+    __builtin_amdgcn_s_waitcnt(0x0070);  // (nothing may arrive behind the sums)
+    {
+        mma_f4 *mine = reinterpret_cast<mma_f4 *>(s0 + wave * (RP + RQ) * BK) + lane;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < QF; j++) mine[(2 * j + i) * 64] = acc[i][j];
+    }
+    __syncthreads();
+    if (wave >= QF) return;
+    mma_f4 sum[2][1];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        mma_f4 v[WAVES];
+#pragma unroll
+        for (int w = 0; w < WAVES; w++)
+            v[w] = reinterpret_cast<const mma_f4 *>(s0 + w * (RP + RQ) * BK)[(2 * wave + i) * 64 + lane];
+        sum[i][0] = (v[0] + v[1]) + (v[2] + v[3]);
+    }
+    lin_emit<OUT, T, 1, 1>(a, PLANES ? m0 : n0, (PLANES ? n0 : m0) + 16 * wave, sum);
+}
+
+// Workgroups of linear_wave_kernel, one per CU: the narrow tiles where they fit the chip at once, the others up to twice its CUs.
+// The second round pays where rows are long (us, 64 x 64 tiles / these: 300 tiles 784 x 384 x 1536 11.7 / 9.4, 400 tiles 784 x 512 x
+// 2048 15.6 / 10.6, 512 tiles 98 x 4096 x 1024 9.0 / 8.6; 392 tiles 3136 x 128 x 512 5.9 / 6.5, 448 tiles 220 x 2048 x 768 7.6 / 8.2,
+// 336 tiles 196 x 1536 x 384 5.9 / 7.2), the third does not (588 tiles 1568 x 384 x 1536 14.0 / 19.5).
+constexpr long kLinCus = 256;
+constexpr int kLinLongRow = 1024;
+template <typename T, int OUT, int QF>
+bool launch_wave_tiles(const LinearArgs<T> &a, long most, hipStream_t st) {
+    constexpr int X = OUT == LIN_PLANES ? 32 : 16 * QF, W = OUT == LIN_PLANES ? 16 * QF : 32;
+    const long xtiles = (a.M + X - 1) / X, tiles = xtiles * ((a.N + W - 1) / W);
+    if (tiles > most) return false;
+    linear_wave_kernel<T, OUT, QF><<<dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(kLinThreads), 0, st>>>(a, (int)xtiles, (int)tiles);
+    return true;
+}
+template <typename T, int OUT>
+int launch_few_tiles(const LinearArgs<T> &a, hipStream_t st) {
+    if (!launch_wave_tiles<T, OUT, 1>(a, kLinCus, st) &&
+        !launch_wave_tiles<T, OUT, 2>(a, a.K < kLinLongRow ? kLinCus : 2 * kLinCus, st)) {
+        const int mt = (int)((a.M + 63) / 64);
+        linear_split_kernel<T, OUT><<<dim3((unsigned)((long)mt * ((a.N + 63) / 64))), dim3(kLinThreads), 0, st>>>(a, mt);
+    }
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : (int)e;
+}
+
 constexpr long kLinLargeTiles = 160;
 template <typename T, bool PLANES>
 int launch_linear(const LinearArgs<T> &a, hipStream_t st) {
@@ -659,11 +794,10 @@ int launch_linear(const LinearArgs<T> &a, hipStream_t st) {
         else if (three) linear_kernel<T, LIN_PLANES, 3><<<grid, block, 0, st>>>(a, (int)mtiles, ntiles);
         else linear_kernel<T, LIN_PLANES, 4><<<grid, block, 0, st>>>(a, (int)mtiles, ntiles);
     } else {
-        const int mt = (int)((a.M + 63) / 64);
-        const dim3 grid((unsigned)((long)mt * ((a.N + 63) / 64))), block(kLinThreads);
-        if constexpr (!PLANES) linear_split_kernel<T, LIN_ROWS><<<grid, block, 0, st>>>(a, mt);
-        else if (a.HW % 4 != 0) linear_split_kernel<T, LIN_PIXELS><<<grid, block, 0, st>>>(a, mt);
-        else linear_split_kernel<T, LIN_PLANES><<<grid, block, 0, st>>>(a, mt);
+        constexpr int OUT = PLANES ? LIN_PLANES : LIN_ROWS;
+        if constexpr (PLANES)
+            if (a.HW % 4 != 0) return launch_few_tiles<T, LIN_PIXELS>(a, st);
+        return launch_few_tiles<T, OUT>(a, st);
     }
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : (int)e;

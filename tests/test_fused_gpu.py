@@ -374,6 +374,26 @@ def test_linear_rows_and_planes(shape, N, dtype):
     _close(host.linear_planes(x, w, b, None, None), y.permute(0, 3, 1, 2), dtype, "planes alone")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape,N", [((1, 1, 1, 1032), 8), ((2, 1, 1, 64), 16), ((1, 7, 7, 3072), 768), ((1, 14, 14, 264), 384),
+                                     ((1, 16, 16, 328), 512), ((1, 1, 257, 72), 512), ((2, 16, 16, 760), 512),
+                                     ((1, 1, 513, 760), 512), ((8, 8, 8, 1024), 1024), ((2, 2, 127, 1016), 1024),
+                                     ((1, 1, 513, 1024), 1024), ((98, 8, 4, 256), 24), ((5, 4, 5, 2056), 136)])
+def test_product_kernels_of_few_tiles(shape, N, dtype):
+    """Both sides of the lines between narrow, wide and 64 x 64 tiles (256 and 512 workgroups, rows of 1024), tails of the summed
+    index, tiles that no XCD's share divides; rows, even and odd planes."""
+    torch.manual_seed(N)
+    B, H, W, K = shape
+    x = torch.randn(*shape, device="cuda").to(dtype)
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).to(dtype)
+    b, s = torch.randn(N, device="cuda").to(dtype), torch.randn(N, device="cuda").to(dtype)
+    res = torch.randn(B, N, H, W, device="cuda").to(dtype)
+    host = fused._lib.host(0)
+    y = F.linear(x.double(), w.double(), b.double())
+    _close(host.linear_rows(x, w, b, True), F.gelu(y), dtype, "rows, gelu")
+    _close(host.linear_planes(x, w, b, s, res), res.double() + (s.double() * y).permute(0, 3, 1, 2), dtype, "planes")
+
+
 def test_product_kernels_keep_refusals():
     host = fused._lib.host(0)
     x = torch.zeros(1, 2, 2, 16, device="cuda", dtype=torch.bfloat16)
