@@ -322,20 +322,25 @@ struct LinearArgs {
     int N, K, HW, gelu;
 };
 
-// GELU of a sum that nothing has rounded, with erf from Abramowitz and Stegun, Handbook of Mathematical Functions, 7.1.26 (error
-// of erf below 1.5e-7): |u| (1/2 - q) + u / 2 with q = erfc(|u| / sqrt 2) / 2.  Two issue slots less than gelu_rounded, whose
-// tail is exact to the result's rounding; here a separate layer's rounding of u, which the tail magnifies by u^2, is gone, and is
-// worth five to nine times the difference (mean relative error on [-4, -3], separate layers / this, bf16 1.3e-2 / 1.4e-3, fp16
-// 1.7e-3 / 2.5e-4).  With gelu_rounded 401408 x 384 x 96 took 178 us instead of 174, a block of 100352 x 192 132 instead
-// of 127.  Infinities and NaN give what u * (1 + erf) gives.
+// GELU of a sum that nothing has rounded: |u| (1/2 - q) + u / 2 with q = Phi(-|u|) = 2^p(|u|), p the polynomial of degree eight for
+// log2 Phi(-t) on [0, 5] whose largest error, weighted with Phi(-t) + 1e-5, is least (from there on it falls, to -infinity).  The
+// logarithm is so smooth that no quotient is needed, and v_rcp_f32 takes four issue slots: 15 a value instead of 20
+// with erf from Abramowitz and Stegun 7.1.26 and further from 64 bits (in fp32, q off by 2.6e-7 at most, here 5.4e-8, GELU over N(0,1)
+// by 5.5e-8 and 2.2e-8 rms, mean relative error on [-4, -3] 2.1e-4 and 8e-5).  us, bf16, with that / this: both layers of a block
+// 401408 x 96 120 / 113, 100352 x 192 108.5 / 105; the first one 401408 x 384 x 96 173 / 167, 25088 x 1536 x 384 60 / 57.
+// gelu_rounded, whose tail is exact to the result's rounding, has no place here: a separate layer's rounding of u, which the
+// tail magnifies by u^2, is gone, and was worth five to nine times the difference.  Infinities and NaN give what u * (1 + erf) gives.
 __device__ __forceinline__ float lin_gelu(float u) {
-    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_fabsf(u), 0.3275911f * 0.70710678118654752f, 1.f));
-    float p = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
-    p = __builtin_fmaf(t, p, 0.5f * 1.421413741f);
-    p = __builtin_fmaf(t, p, 0.5f * -0.284496736f);
-    p = __builtin_fmaf(t, p, 0.5f * 0.254829592f);
-    const float q = p * t * __builtin_amdgcn_exp2f(u * u * -0.72134752044448170f);  // exp(-u^2 / 2)
-    return __builtin_fmaf(__builtin_fabsf(u), 0.5f - q, 0.5f * u);
+    const float t = __builtin_fabsf(u);
+    float p = __builtin_fmaf(t, -2.09645073e-06f, 3.15079535e-05f);
+    p = __builtin_fmaf(t, p, -0.000153187882f);
+    p = __builtin_fmaf(t, p, -0.000206634976f);
+    p = __builtin_fmaf(t, p, 0.00714238625f);
+    p = __builtin_fmaf(t, p, -0.0525433468f);
+    p = __builtin_fmaf(t, p, -0.459194624f);
+    p = __builtin_fmaf(t, p, -1.15110672f);
+    p = __builtin_fmaf(t, p, -0.999999963f);
+    return __builtin_fmaf(t, 0.5f - __builtin_amdgcn_exp2f(p), 0.5f * u);
 }
 
 typedef unsigned mma_u2 __attribute__((ext_vector_type(2)));
@@ -354,9 +359,10 @@ template <int Q, typename T>
 __device__ __forceinline__ void lin_emit_rows(const LinearArgs<T> &a, long m, int n, float (&v)[Q], const float (&b)[Q]) {
     if (m >= a.M || n >= a.N) return;
 #pragma unroll
-    for (int r = 0; r < Q; r++) {
-        v[r] += b[r];
-        if (a.gelu) v[r] = lin_gelu(v[r]);
+    for (int r = 0; r < Q; r++) v[r] += b[r];
+    if (a.gelu) {
+#pragma unroll
+        for (int r = 0; r < Q; r++) v[r] = lin_gelu(v[r]);
     }
     T *at = a.out + m * a.N + n;
     if constexpr (Q == 8)
@@ -516,8 +522,8 @@ __device__ __forceinline__ void lin_emit(const LinearArgs<T> &a, long p0, long q
 }
 
 // Large tiles: 128 rows of P, 32 * QF of Q, four waves of 64 x 16 QF products, two buffers: the next 64 columns travel
-// to LDS while these are multiplied, one barrier per step, two workgroups per CU.  bf16, us: 25088 x 1536 x 384 with GELU 60 (MFMA
-// 12, the GELU's vector instructions 30; library product and GELU kernel 92), 401408 x 384 x 96 172 (290); planes
+// to LDS while these are multiplied, one barrier per step, two workgroups per CU.  bf16, us: 25088 x 1536 x 384 with GELU 57 (MFMA
+// 12, the GELU's vector instructions 30; library product and GELU kernel 92), 401408 x 384 x 96 167 (290); planes
 // 25088 x 384 x 1536 58 (library and scale kernel 57), 401408 x 96 x 384 109 (193).  Tried: staging through registers
 // (the same; -20 % where few workgroups run), three buffers with one workgroup per CU (+30 %).
 template <typename T, int QF>

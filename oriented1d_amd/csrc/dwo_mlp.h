@@ -9,11 +9,12 @@
 // while the previous ones are used and are shared by the waves; 16 PF is what leaves two waves per SIMD, so that one's
 // GELU runs under the other's matrix instructions.
 //
-// What bounds it: at C = 96 the vector instructions, mostly of GELU (21 issue slots per hidden value), 63 % of the time by counters
-// (matrix cores 16 %, LDS 23 %); the share falls to 42 % at 192 and 31 % at 384, where the LDS reads of the weights, which
+// What bounds it: at C = 96 the vector instructions, mostly of GELU (16 issue slots per hidden value; counted with 21 of them 63 %
+// of the time, matrix cores 16 %, LDS 23 %); the share falls to 42 % at 192 and 31 % at 384, where the LDS reads of the weights, which
 // eight waves of 16 pixels share, lead with 40 % and no unit is busy for half the time.  us, bf16, two product kernels / this one: 401408 x 96
-// 316 / 142, 200704 x 128 200 / 114, 100352 x 192 160 / 124, 25088 x 384 120 / 105; slower from C = 512 (spills) and where its
-// workgroups of 128 pixels are few (its chain is 4 C / 32 steps of 1.5 to 1.9 us: 12544 x 384 65 / 100).
+// 269 / 113, 100352 x 192 159 / 105, 25088 x 384 119 / 100; slower from C = 512 (spills) and where its
+// workgroups of 128 pixels are few (its chain is 4 C / 32 steps of 1.5 to 1.9 us: 12544 x 384 60 / 90).  Tried at 384: four waves of 32 pixels, half the LDS reads
+// (one wave per SIMD overlaps nothing, 98 / 205).
 #pragma once
 
 #include "dwo_linear.h"

@@ -493,6 +493,20 @@ def test_parameters_that_are_not_dense(which, rows):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_gelu_of_a_product_far_out(dtype):
+    """Beyond the range of its polynomial: u or 0 as far as the type reaches, and what u * (1 + erf) gives for infinities and NaN."""
+    from oriented1d_amd import _lib
+    far = [8.5, 20.0, 300.0, torch.finfo(dtype).max]
+    u = torch.tensor(far + [-v for v in far[1:]] + [float("inf"), -float("inf"), float("nan"), 0.0, -0.0], device="cuda").to(dtype)
+    x, w = torch.zeros(u.numel(), 8, device="cuda", dtype=dtype), torch.zeros(8, 8, device="cuda", dtype=dtype)
+    x[:, 0], w[:, 0] = u, 1.0
+    ref = (0.5 * u.double() * (1 + torch.special.erf(u.double() * 0.5 ** 0.5))).to(dtype)
+    got = _lib.host(0).linear_rows(x, w, None, True)
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)[:, None].expand(-1, 8))
+    assert torch.equal(got.nan_to_num(1.5), ref.nan_to_num(1.5)[:, None].expand(-1, 8))
+
+
 @pytest.mark.parametrize("dtype,unit", [(torch.bfloat16, 2.0 ** -8), (torch.float16, 2.0 ** -11)], ids=["bf16", "f16"])
 def test_gelu_of_the_negative_tail(dtype, unit):
     """GELU value by value, as far as results are normal numbers.  Behind LayerNorm: the rounding of the result (``unit`` of it)
