@@ -149,7 +149,8 @@ __global__ __launch_bounds__(kLinThreads, 2) void linear_wgrad_kernel(const T *_
     b.init(x, min(rows, max(last, m0)), m0, K, k0);
     // a stage is multiplied while the next three travel (loads beyond the split's last row read nowhere)
     auto stage = [&](uint16_t *sa, uint16_t *sb, uint16_t *na, uint16_t *nb) {
-        __builtin_amdgcn_s_waitcnt(0x0f78);  // vmcnt(8): this wave's part of the stage is there ..
+        // vmcnt(8) lgkmcnt(0): this wave's part of the stage is there, and what it read of the one before ..
+        __builtin_amdgcn_s_waitcnt(0x0078);
         asm volatile("s_barrier" ::: "memory");  // .. and the other waves'; nobody reads the one before any more
         a.load(na, N), b.load(nb, K);
         __builtin_amdgcn_sched_barrier(0);
