@@ -526,7 +526,8 @@ __device__ __forceinline__ void lin_emit(const LinearArgs<T> &a, long p0, long q
 // to LDS while these are multiplied, one barrier per step, two workgroups per CU.  bf16, us: 25088 x 1536 x 384 with GELU 57 (MFMA
 // 12, the GELU's vector instructions 30; library product and GELU kernel 92), 401408 x 384 x 96 167 (290); planes
 // 25088 x 384 x 1536 58 (library and scale kernel 57), 401408 x 96 x 384 109 (193).  Tried: staging through registers
-// (the same; -20 % where few workgroups run), three buffers with one workgroup per CU (+30 %).
+// (the same; -20 % where few workgroups run), three buffers with one workgroup per CU (+30 %), stages of 32 columns, three ahead (half
+// lines; 6272 x 3072 x 768 52 / 63, planes 6272 x 768 x 3072 60 / 69).
 template <typename T, int QF>
 __device__ __forceinline__ void lin_products(const uint16_t *lp, const uint16_t *lq, int wp, int wq, mma_f4 (&acc)[4][QF]) {
 #pragma unroll
