@@ -166,7 +166,8 @@ def infer_block(x, block, conv, inner):
     bias, gamma = conv.bias, block.gamma
     module = conv.module_fp32_large if conv.arbitrary_size else conv.module_fp32
     if (w is None or theta is None or g is None or b is None or w1 is None or b1 is None or w2 is None or b2 is None
-            or conv.nhwc or conv.resid is not None or module.stride != 1 or C % 8 != 0 or C > MAX_C_TILE
+            or conv.nhwc or conv.resid is not None or type(module) is not KernelTuple or module.stride != 1
+            or C % 8 != 0 or C > MAX_C_TILE
             or 4 * rows * C >= _PRODUCT_MAX or w1.shape != (4 * C, C) or w2.shape != (C, 4 * C)
             or not _native_covers(x, w, theta, bias, None, module, False) or not ordinary(g, b, w1, b1, w2, b2, gamma)):
         return None

@@ -638,3 +638,24 @@ def test_stem_tail_as_one_kernel(N, H, W, C, bias, dtype):
         handle.remove()
         assert fused.norm_planes(x.float(), before.float(), linear.float(), norm.float()) is None
     assert fused.norm_planes(x, before.to(dtype), linear.to(dtype), norm.to(dtype)) is None  # (gradients are on)
+
+
+@pytest.mark.parametrize("plus_plus,which", [(False, "dwconv"), (True, "dwconv1"), (True, "dwconv2")])
+@pytest.mark.parametrize("arbitrary_size", [True, False])
+def test_inference_block_with_functions_of_the_caller(plus_plus, which, arbitrary_size, monkeypatch):
+    """A block whose operator holds five functions that are no ``KernelTuple`` runs layer by layer, through them."""
+    from oriented1d_amd.convnext1d import Block
+    torch.manual_seed(3)
+    block = Block(64, (15, 31) if plus_plus else (31,), plus_plus, layer_scale_init_value=0.1,
+                  arbitrary_size=arbitrary_size).cuda().bfloat16().eval()
+    conv, name, calls = getattr(block, which), "module_fp32_large" if arbitrary_size else "module_fp32", []
+    own = tuple(getattr(conv, name))
+    setattr(conv, name, (lambda *a: calls.append(1) or own[0](*a),) + own[1:])
+    taken, whole = [], fused.infer_block
+    monkeypatch.setattr(fused, "infer_block", lambda *a: taken.append(whole(*a)) or taken[-1])
+    x = torch.randn(2, 64, 9, 11, device="cuda").bfloat16()
+    with torch.no_grad():
+        got = block(x)
+        assert taken == [None] and calls == [1]
+        monkeypatch.setattr(fused, "infer_block", lambda *a: None)
+        assert torch.equal(got, block(x))
