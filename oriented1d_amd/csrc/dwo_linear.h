@@ -103,8 +103,9 @@ struct LinSource {
 
 // dw [split][stride] and db [split][stride]: partial sums, or with one split the gradients themselves (db may be null).
 // HALVES: the sums of the first half of a split's rows wait in registers of their own, so that no chain is longer than where
-// twice as many splits share the rows (error against 64 bits at 200704 x 512 x 128 with 256 workgroups 3.5e-7, like this 2.5e-7, with
-// 512 2.5e-7).
+// twice as many splits share the rows, but for 64 rows where these are an odd number of steps (error against 64 bits at 200704 x
+// 512 x 128 with 256 workgroups 3.5e-7, like this 2.5e-7, with 512 2.5e-7; 512 / 960 rows x 4096 x 1024 1.25e-7 / 1.78e-7 in
+// one chain, 9.0e-8 / 1.24e-7 like this and with two splits).
 template <typename T, typename TO, bool HALVES>
 __global__ __launch_bounds__(kLinThreads, 2) void linear_wgrad_kernel(const T *__restrict__ dy,
                                                                       const T *__restrict__ x, TO *__restrict__ dw,
@@ -179,14 +180,14 @@ __global__ __launch_bounds__(kLinThreads, 2) void linear_wgrad_kernel(const T *_
     };
     mma_f4 half[4][4], halfb[4];
     if constexpr (HALVES) {
-        run(pairs / 4);
+        run((pairs + 1) / 4);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             halfb[i] = accb[i], accb[i] = mma_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int j = 0; j < 4; j++) half[i][j] = acc[i][j], acc[i][j] = mma_f4{0.f, 0.f, 0.f, 0.f};
         }
-        run(pairs / 2 - pairs / 4);
+        run(pairs / 2 - (pairs + 1) / 4);
     } else {
         run(pairs / 2);
     }
@@ -260,7 +261,7 @@ struct LinearSplits {
         if (s > steps / 4) s = steps / 4;
         if (s >= 8) s = s / 8 * 8;
         splits = (int)(s < 1 ? 1 : s);
-        halves = halves && steps >= 16;
+        halves = halves && steps >= 8;
     }
 };
 inline size_t linear_wgrad_scratch(size_t rows, int N, int K) {

@@ -181,7 +181,7 @@ def test_linear_gradients(M, K, N, dtype):
 
 
 # stages of 32 rows, four in flight: rows around a stage, a step of 64 and the four; outputs around a tile of 128; few tiles, whose
-# sums are kept in halves from 16 steps on; as many tiles as CUs, which write the gradients themselves in either type
+# sums are kept in halves from eight steps on; as many tiles as CUs, which write the gradients themselves in either type
 @pytest.mark.parametrize("grad", [F32, BF16])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 8), (31, 128, 128), (33, 136, 120), (65, 256, 264), (127, 8, 1024), (129, 64, 72),
                                    (1023, 128, 256), (1025, 120, 128), (4161, 256, 136), (20011, 128, 96), (97, 1920, 1920),
@@ -197,6 +197,19 @@ def test_linear_wgrad_stages_and_splits(M, N, K, grad):
         assert (db is None) == (not bias)
         if bias:
             close(db, dy.double().sum(0), tol, "db")
+
+
+@pytest.mark.parametrize("rows", [449, 512, 576, 640, 700, 832, 960])
+def test_linear_wgrad_of_many_tiles_sums_in_chains_as_short_as_two_splits(rows):
+    """256 tiles (one workgroup per tile, whose sums are kept in halves) against 192 of the same columns (two splits of the
+    rows): the same error against 64 bits, within what a chain longer by 64 of 320 to 448 rows gives (sqrt(1.04)) and 2 %."""
+    from oriented1d_amd import _lib
+    torch.manual_seed(rows)
+    x, dy = torch.randn(rows, 1024, device="cuda").bfloat16(), torch.randn(rows, 4096, device="cuda").bfloat16()
+    ref = dy.double().t() @ x[:, :768].double()
+    err = [((dw[:, :768].double() - ref).norm() / ref.norm()).item()
+           for dw in (_lib.host(0).linear_wgrad(dy, v, False, F32)[0] for v in (x, x[:, :768].contiguous()))]
+    assert 0 < err[0] <= 1.04 * err[1] and err[1] < 2e-7, err
 
 
 def test_linear_covers_batches_views_and_second_order():
