@@ -20,6 +20,7 @@
 #pragma once
 
 #include "dwo_common.h"
+#include "dwo_linear_splits.h"
 
 namespace dwo {
 
@@ -51,9 +52,8 @@ struct Mma<f16_t> {
     }
 };
 
-constexpr int kLinThreads = 256, kLinTile = 128, kLinRows = 64;
+constexpr int kLinThreads = 256;
 constexpr int kLinStage = 32;  // rows that travel together
-constexpr long kLinFew = 4, kLinAlone = 224;  // tiles (LinearSplits)
 constexpr unsigned kLinNowhere = 0x80000000u;
 
 // Place of a fragment in a stage: columns [16 unit, 16 unit + 16) of rows 4 g + i / 4 and 16 rows on, as the transposing read
@@ -243,45 +243,17 @@ __global__ __launch_bounds__(kLinThreads) void linear_reduce_kernel(const float 
     for (int e = 0; e < 4; e++) out[e] = from_float<TO>(s[e]);
 }
 
-// Splits of the rows, each with 256 rows where they are dealt evenly; a multiple of eight where there are as many (whole splits
-// per XCD).  Two workgroups per CU (512), but
-//   one where the outputs are at most four tiles, memory binds, and the partial sums, 64 KB per workgroup both ways, are what can be
-//   saved (us with the sums, 512 / 256: 200704 x 512 x 128 64 / 58, 131072 x 384 x 96 40 / 33, 200704 x 128 x 64 36 / 23; eight tiles,
-//   50176 x 256 x 512, 31.5 / 32.2);
-//   no split where the tiles alone give each CU its workgroup (3136 x 4096 x 1024 53 / 44).
-// A split holds whole steps of 64 rows, rounded up, so the last few may hold no rows: their sums are zeros.
-struct LinearSplits {
-    int splits;
-    bool halves;
-    LinearSplits(size_t rows, int N, int K) {
-        const long tiles = (long)((N + kLinTile - 1) / kLinTile) * ((K + kLinTile - 1) / kLinTile);
-        const long steps = (long)((rows + kLinRows - 1) / kLinRows);
-        halves = tiles <= kLinFew || tiles >= kLinAlone;
-        long s = tiles >= kLinAlone ? 1 : (halves ? 256 : 512) / tiles;
-        if (s > steps / 4) s = steps / 4;
-        if (s >= 8) s = s / 8 * 8;
-        splits = (int)(s < 1 ? 1 : s);
-        halves = halves && steps >= 8;
-    }
-};
-inline size_t linear_wgrad_scratch(size_t rows, int N, int K) {
-    return (size_t)LinearSplits(rows, N, K).splits * ((size_t)N * K + N) * sizeof(float);
-}
-
 template <typename T, typename TO>
 int launch_linear_products(const void *dy, const void *x, TO *dw, TO *db, size_t stride, size_t rows, int N, int K,
                            const LinearSplits &s, hipStream_t st) {
-    const int splits = s.splits;
-    const long steps = (long)((rows + kLinRows - 1) / kLinRows);
-    const int per = (int)((steps + splits - 1) / splits);
     const unsigned tiles = (unsigned)((N + kLinTile - 1) / kLinTile) * ((K + kLinTile - 1) / kLinTile);
-    const dim3 grid(tiles * (unsigned)splits), block(kLinThreads);
+    const dim3 grid(tiles * (unsigned)s.splits), block(kLinThreads);
     if (s.halves)
         linear_wgrad_kernel<T, TO, true><<<grid, block, 0, st>>>((const T *)dy, (const T *)x, dw, db, stride, (long)rows, N, K,
-                                                                 splits, per);
+                                                                 s.splits, s.per);
     else
         linear_wgrad_kernel<T, TO, false><<<grid, block, 0, st>>>((const T *)dy, (const T *)x, dw, db, stride, (long)rows, N,
-                                                                  K, splits, per);
+                                                                  K, s.splits, s.per);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : (int)e;
 }

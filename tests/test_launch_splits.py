@@ -1,4 +1,4 @@
-"""CPU-only: the host code that cuts the window and grouped kernels' launches, compiled by itself and checked over
+"""CPU-only: the host code that cuts the window, grouped and product kernels' launches, compiled by itself and checked over
 the shapes that it accepts (tests/host)."""
 import os
 import subprocess
@@ -10,7 +10,7 @@ from oriented1d_amd import build
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-@pytest.mark.parametrize("program", ["window_units", "grouped_tasks"])
+@pytest.mark.parametrize("program", ["window_units", "grouped_tasks", "linear_splits"])
 def test_launch_splits(program, tmp_path):
     exe = str(tmp_path / program)
     subprocess.run([build.hipcc(), "-x", "hip", "--offload-host-only", "-O1", "-std=c++17", "-I" + build.CSRC,
