@@ -33,6 +33,7 @@ int main() {
                 const long chain = s.halves ? std::max((s.per + 1) / 4 * 2, s.per - (s.per + 1) / 4 * 2) : s.per;
                 const long before = (steps + two - 1) / two;
                 EXPECT(chain <= before + 1 + (tiles == 3 ? before / 20 : 0), "a longer chain of sums");
+                EXPECT(tiles > 256 || (K + 127) / 128 % 8 != 0 || s.splits > 1 || steps <= 128, "many rows in one workgroup per tile");
                 EXPECT(!s.halves || s.splits < two || tiles > 256, "halves without fewer splits");
             }
     return failures != 0;

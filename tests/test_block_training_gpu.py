@@ -181,11 +181,13 @@ def test_linear_gradients(M, K, N, dtype):
 
 
 # stages of 32 rows, four in flight: rows around a stage, a step of 64 and the four; outputs around a tile of 128; few tiles, whose
-# sums are kept in halves from eight steps on; as many tiles as CUs, which write the gradients themselves in either type
+# sums are kept in halves where there are fewer splits; as many tiles as CUs, which write the gradients themselves in either type
+# as long as the rows are few (54 or 128 steps)
 @pytest.mark.parametrize("grad", [F32, BF16])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 8), (31, 128, 128), (33, 136, 120), (65, 256, 264), (127, 8, 1024), (129, 64, 72),
                                    (1023, 128, 256), (1025, 120, 128), (4161, 256, 136), (20011, 128, 96), (97, 1920, 1920),
-                                   (1300, 1800, 2056)])
+                                   (1300, 1800, 2056), (3456, 1792, 2048), (3457, 1792, 2048), (8192, 3584, 1024),
+                                   (8193, 3584, 1024), (16640, 512, 128)])
 def test_linear_wgrad_stages_and_splits(M, N, K, grad):
     from oriented1d_amd import _lib
     torch.manual_seed(M + N)
