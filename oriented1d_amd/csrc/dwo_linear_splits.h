@@ -43,8 +43,10 @@ struct LinearSplits {
         halves = few || (alone && steps >= 8);
     }
 };
+// (one split writes the gradients themselves)
 inline size_t linear_wgrad_scratch(size_t rows, int N, int K) {
-    return (size_t)LinearSplits(rows, N, K).splits * ((size_t)N * K + N) * sizeof(float);
+    const int splits = LinearSplits(rows, N, K).splits;
+    return splits == 1 ? 16 : (size_t)splits * ((size_t)N * K + N) * sizeof(float);
 }
 
 }  // namespace dwo

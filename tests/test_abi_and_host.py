@@ -91,6 +91,14 @@ def test_tap_table_channel_order_cycles_through_classes(layout):
         assert all(sorted(r.tolist()) == [-1] + list(range(8)) for r in first)
 
 
+@pytest.mark.parametrize("rows,N,K,splits", [(3136, 4096, 1024, 1), (300, 1024, 264, 1), (64, 65536, 65536, 1),
+                                             (12544, 512, 2048, 8), (3457, 1024, 4096, 2)])
+def test_linear_wgrad_scratch_is_the_partial_sums(rows, N, K, splits):
+    """Calls whose workgroups write the gradients themselves ask for no more than a token."""
+    got = _lib.load().dwo_linear_wgrad_scratch_bytes(rows, N, K)
+    assert 0 < got <= 16 if splits == 1 else got == 4 * splits * (N * K + N)
+
+
 def test_module_contract():
     C, K = 16, 31
     angles = [math.pi * (c % 8) / 8 for c in range(C)]
