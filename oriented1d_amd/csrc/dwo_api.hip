@@ -468,9 +468,11 @@ int wgrad_t(const void *dy, const void *x, const void *taps, float *dw, float *d
     } else if (grouped_wgrad_covers(d, layout, sizeof(T)) && aligned16(x) && aligned16(dy)) {
         rc = try_grouped_wgrad<T>(x, dy, taps, part, &NG, d, st);
         if (rc != DWO_OK) return rc;
-        const long cells = (long)d.C * (d.K + 1);
-        wgrad_reduce_wide_kernel<<<dim3((unsigned)((cells + 15) / 16)), dim3(256), 0, st>>>(part, dw, db, d.C, d.K, NG);
-        return launch_status();
+        if (NG > kWideReduceGroups) {
+            const long cells = (long)d.C * (d.K + 1);
+            wgrad_reduce_wide_kernel<<<dim3((unsigned)((cells + 15) / 16)), dim3(256), 0, st>>>(part, dw, db, d.C, d.K, NG);
+            return launch_status();
+        }
     } else if (nhwc_plane_batch(d, layout) != 0) {
         unsigned *tickets = ticket_row(d.C / kSliceCh, st);
         rc = try_nhwc_plane_wgrad<T>(x, dy, taps, part, dw, db, tickets, &NG, d, st);

@@ -154,7 +154,9 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float *__restri
 
 // The same where no workgroup adds up in stage 1 (whose order this would have to be): 16 lanes share a cell and read its partial
 // sums side by side.  With a thread per cell the stem's 2048 cells of 128 sums were a chain of 32 loads on eight workgroups:
-// 16 us, now 4.4.
+// 16 us, now 4.2.  At most eight sums keep a thread per cell: two loads in a row there, half of the lanes idle here (us, thread /
+// lanes: 131072 cells of 8 4.1 / 6.5, 65536 of 8 4.1 / 4.4, 65536 of 16 4.2 / 4.3, 16384 of 16 4.3 / 4.2, 8192 of 32 5.8 / 4.3).
+constexpr int kWideReduceGroups = 8;
 __global__ __launch_bounds__(256) void wgrad_reduce_wide_kernel(const float *__restrict__ part, float *__restrict__ dw,
                                                                 float *__restrict__ db, int C, int K, int G) {
     const int idx = blockIdx.x * 16 + threadIdx.x / 16, lane = threadIdx.x % 16;

@@ -245,7 +245,9 @@ def test_window_kernels_unit_edges(oracle, N, C, H, W, K, dtype):
     (64, 64, 3, 70, 7, 1), (64, 64, 5, 70, 7, 2), (64, 64, 4, 65, 7, 1), (64, 64, 3, 64, 7, 1), (63, 64, 3, 70, 7, 1),
     # (wgrad: enough planes for the grouped kernel)
     (2, 1024, 28, 28, 31, 1), (2, 1024, 33, 65, 31, 1), (2, 1024, 17, 3, 13, 1), (2, 1024, 21, 18, 27, 1),
-    (2, 1024, 33, 67, 31, 2), (2, 1024, 5, 18, 7, 2), (2, 1024, 35, 31, 15, 2)])
+    (2, 1024, 33, 67, 31, 2), (2, 1024, 5, 18, 7, 2), (2, 1024, 35, 31, 15, 2),
+    # (wgrad: eight partial sums in fp32, sixteen in 16 bits, which are added up by another kernel)
+    (4, 512, 40, 36, 15, 1)])
 def test_grouped_nhwc_kernels(oracle, N, C, H, W, K, stride, dtype):
     """Channels grouped by angle, as the networks have them: whole 16-byte pieces per orientation."""
     for offset in (0.0, 0.5):
