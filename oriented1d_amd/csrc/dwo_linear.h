@@ -736,11 +736,13 @@ __global__ __launch_bounds__(kLinThreads, 1) void linear_wave_kernel(LinearArgs<
 }
 
 // Workgroups of linear_wave_kernel, one per CU: the narrow tiles where they fit the chip at once, the others up to twice its CUs.
-// The second round pays where rows are long (us, 64 x 64 tiles / these: 300 tiles 784 x 384 x 1536 11.7 / 9.4, 400 tiles 784 x 512 x
-// 2048 15.6 / 10.6, 512 tiles 98 x 4096 x 1024 9.0 / 8.6; 392 tiles 3136 x 128 x 512 5.9 / 6.5, 448 tiles 220 x 2048 x 768 7.6 / 8.2,
-// 336 tiles 196 x 1536 x 384 5.9 / 7.2), the third does not (588 tiles 1568 x 384 x 1536 14.0 / 19.5).
+// The second round pays where rows are long, as long as what it reads has to come from beyond the L2 (us, bf16, behind a pass over
+// other memory, 64 x 64 tiles / these: planes 300 tiles 784 x 384 x 1536 12.5 / 10.5, 484 x 320 x 1280 10.8 / 9.3, 784 x 512 x 2048 15.2 /
+// 11.6, 512 tiles 1024 x 512 x 2048 13.9 / 13.3, 512 x 1024 x 4096 24.3 / 17.5, 1024 x 320 x 1280 10.9 / 10.5); rows of 1024 gain nothing (1176 x
+// 256 x 1024 9.8 / 9.5, 1536 rows 8.7 / 9.1, 2048 rows 8.9 / 9.8, odd planes 15.0 / 15.9) and lose back to back (1176 x 256 x 1024 7.7 / 8.0, odd
+// planes 9.9 / 11.4), shorter ones lose (rows, 189 x 1536 x 384 5.7 / 7.1).  The third round does not pay (1056 x 512 x 2048 14.7 / 18.2).
 constexpr long kLinCus = 256;
-constexpr int kLinLongRow = 1024;
+constexpr int kLinLongRow = 1280;
 template <typename T, int OUT, int QF>
 bool launch_wave_tiles(const LinearArgs<T> &a, long most, hipStream_t st) {
     constexpr int X = OUT == LIN_PLANES ? 32 : 16 * QF, W = OUT == LIN_PLANES ? 16 * QF : 32;

@@ -378,9 +378,10 @@ def test_linear_rows_and_planes(shape, N, dtype):
 @pytest.mark.parametrize("shape,N", [((1, 1, 1, 1032), 8), ((2, 1, 1, 64), 16), ((1, 7, 7, 3072), 768), ((1, 14, 14, 264), 384),
                                      ((1, 16, 16, 328), 512), ((1, 1, 257, 72), 512), ((2, 16, 16, 760), 512),
                                      ((1, 1, 513, 760), 512), ((8, 8, 8, 1024), 1024), ((2, 2, 127, 1016), 1024),
-                                     ((1, 1, 513, 1024), 1024), ((98, 8, 4, 256), 24), ((5, 4, 5, 2056), 136)])
+                                     ((1, 1, 513, 1024), 1024), ((98, 8, 4, 256), 24), ((5, 4, 5, 2056), 136),
+                                     ((1, 1, 265, 1272), 1024), ((1, 1, 265, 1280), 1024)])
 def test_product_kernels_of_few_tiles(shape, N, dtype):
-    """Both sides of the lines between narrow, wide and 64 x 64 tiles (256 and 512 workgroups, rows of 1024), tails of the summed
+    """Both sides of the lines between narrow, wide and 64 x 64 tiles (256 and 512 workgroups, rows of 1280), tails of the summed
     index, tiles that no XCD's share divides; rows, even and odd planes."""
     torch.manual_seed(N)
     B, H, W, K = shape
