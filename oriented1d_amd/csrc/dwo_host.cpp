@@ -710,7 +710,7 @@ Tensor block_mlp(const Tensor &x_, const Tensor &w1_, const Tensor &b1_, const T
 // ln_tile)
 Tensor conv_norm(const Tensor &x, const Tensor &w, const OptTensor &bias, const Tensor &taps, const Tensor &g,
                  const Tensor &b, double eps, bool pieces) {
-    const Tensor y = fprop(x, w, taps, 1, bias, DWO_NCHW);
+    const Tensor y = fprop_entry(x, w, taps, 1, bias, DWO_NCHW);
     return pieces ? std::get<0>(ln_tile(y, g, b, eps, false, y.scalar_type(), false)) : nchw_layernorm_nhwc(y, g, b, eps);
 }
 

@@ -196,6 +196,37 @@ def test_specialized_import_name_and_tuple_contract():
         m.module_fp32[0](torch.zeros(1, 8, 4, 4), m.weight, m.theta)
 
 
+@pytest.mark.parametrize("call", ["fprop", "conv_norm"])
+def test_native_calls_let_other_threads_run(call):
+    """The operator's checks, allocations and launches run without the GIL: a thread that waits for it gets it while this one, which
+    nothing else makes let go of it, makes calls (refused ones, of CPU tensors)."""
+    import sys
+    import threading
+    import time
+    fn, x, w = getattr(_lib.host(-1), call), torch.zeros(1, 8, 4, 4), torch.zeros(8, 1, 1, 7)
+    taps, c = op.build_taps(torch.zeros(8), 8, 7), torch.zeros(8)
+    args = (x, w, taps, 1, None, 0) if call == "fprop" else (x, w, None, taps, c, c, 1e-6, True)
+    gate, ran = threading.Lock(), []
+    gate.acquire()
+    other = threading.Thread(target=lambda: gate.acquire() and ran.append(1))
+    other.start()
+    time.sleep(0.05)  # (the other thread stands at the gate)
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    try:
+        gate.release()
+        end = time.perf_counter() + 3.0
+        while not ran and time.perf_counter() < end:
+            try:
+                fn(*args)
+            except RuntimeError as e:
+                assert "must be a CUDA tensor" in str(e)
+        assert ran
+    finally:
+        sys.setswitchinterval(interval)
+        other.join()
+
+
 def test_state_dict_with_16_bit_theta_loads_as_fp32_values():
     """A checkpoint whose theta was saved in a 16-bit type loads into the fp32 parameter: the
     dtype stays fp32, the values are the rounded ones (the information is gone from the file)."""
