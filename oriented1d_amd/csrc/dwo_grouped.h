@@ -213,27 +213,20 @@ struct Word {
 struct GrpTile {
     int n, p, q, th, tw;  // image, corner, nominal extents
     int vh, vw;           // extents inside the image
-    // NEAR (stride 2, where a window is up to four times its tile's share of the image): neighbouring tiles on one XCD at about
-    // the same time, so that they find each other's lines in its L2.  grp_task deals units to the XCDs in turn; here XCD x
-    // gets the x-th eighth of them, in bands of two tile columns (a tile shares more with the rows below than with the columns
-    // beside).  Where the tile columns are a multiple of eight an XCD has whole columns as it is.  bf16, K = 31, us, in turn / like
-    // this: 64 x 64 x 224 x 224 fprop 318 / 307, dgrad 245 / 198, wgrad 451 / 367, at 112 x 112 81 / 73, 41 / 40, 117 / 98; without
-    // bands wgrad 381, and 8 x 512 x 512 fprop 190, in turn 176.  At stride 1 between 2 % more and 1 % less.
+    // NEAR: where tiles are dealt in runs (grp_run)
     template <bool NEAR>
     __device__ __forceinline__ void set(const ConvDims &d, const GrpTiles &t, int unit) {
-        const int per = t.nth * t.ntw;
+        int row, col;
         th = t.th, tw = t.tw;
         if (NEAR && t.run > 0) {
-            if (unit < 8 * t.run) unit = unit % 8 * t.run + unit / 8;
-            n = unit / per;
-            const int k = unit - n * per, b = k / (2 * t.nth), j = k - b * (2 * t.nth), two = 2 * b + 1 < t.ntw ? 1 : 0;
-            const int a = j >> two;
-            p = a * th, q = (2 * b + (j & two)) * tw;
+            grp_run_tile(t, unit, n, row, col);
         } else {
+            const int per = t.nth * t.ntw;
             n = unit / per;
-            const int k = unit - n * per, a = k / t.ntw;
-            p = a * th, q = (k - a * t.ntw) * tw;
+            const int k = unit - n * per;
+            row = k / t.ntw, col = k - row * t.ntw;
         }
+        p = row * th, q = col * tw;
         vh = min(th, d.P - p), vw = min(tw, d.Q - q);
     }
 };
@@ -534,7 +527,7 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
     if (!grp_task(blockIdx.x, d.N * tiles.nth * tiles.ntw, d.C / CG, unit, group)) return;
     const int c0 = group * CG;
     GrpTile t;
-    t.set<true>(d, tiles, unit);
+    t.set<false>(d, tiles, unit);  // (the image is small: in runs 0 to 2 % slower)
     const T *img = x + (size_t)t.n * d.H * d.W * CIN;
     T *yn = y + (size_t)t.n * d.P * d.Q * d.C + c0;
     if (threadIdx.x < CG * K) lw[threadIdx.x] = wt[(size_t)c0 * K + threadIdx.x];
@@ -859,16 +852,6 @@ GrpTiles grp_tiles(int P, int Q, long planes) {
     return t;
 }
 
-// Tiles of an XCD where they are dealt in runs (GrpTile::set): images cut into tiles, many more tasks than run at once (3 x 64 x
-// 200 x 300 with 840 of them: wgrad 47 us in turn, 49 in runs; 8 x 64 x 256 x 256 with 2048: 84 and 76), and windows whose halo
-// weighs: at K = 15 a tile shares half as much with its neighbours, and in fp32, where an XCD has half as many tiles under way, the
-// runs only spread its accesses (34 x 64 x 320 x 288 wgrad 539 / 594; bf16 64 x 64 x 224 x 224 298 / 269; K = 31 fp32 457 / 405).
-inline int grp_run(const GrpTiles &t, int N, int ngroups, int K, size_t esize) {
-    if (K <= 15 && esize == 4) return 0;
-    const long units = (long)N * t.nth * t.ntw;
-    return t.nth * t.ntw > 1 && t.ntw % 8 != 0 && units * ngroups >= 4 * kGrpSlots ? (int)(units / 8) : 0;
-}
-
 template <typename T, int K, int S>
 int launch_grouped_conv_s(const void *src, const float *w, const float *bias, const void *taps, void *dst,
                           const ConvDims &d, int flip, hipStream_t st) {
@@ -881,7 +864,7 @@ int launch_grouped_conv_s(const void *src, const float *w, const float *bias, co
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
     GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, (long)d.N * ngroups);
-    if (S == 2) t.run = grp_run(t, d.N, ngroups, K, sizeof(T));
+    if (S == 2) t.run = grp_run(t, d, sizeof(T), GRP_FPROP);
     const int pixels = grp_pixels<ConvSet<K, S>>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (!grp_grid_fits(grid)) return -100;
@@ -906,7 +889,7 @@ int launch_grouped_dgrad2(const void *dy, const float *w, const void *taps, void
     d.H = d.P, d.W = d.Q;
     const int ngroups = d.C / CG;
     GrpTiles t = grp_tiles<Set>(d.P, d.Q, (long)d.N * ngroups);
-    t.run = grp_run(t, d.N, ngroups, K, sizeof(T));
+    t.run = grp_run(t, d_, sizeof(T), GRP_DGRAD);
     const int pixels = grp_pixels<Set>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (!grp_grid_fits(grid)) return -100;
@@ -939,7 +922,7 @@ int launch_grouped_wgrad_s(const void *x, const void *dy, const void *taps, floa
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
     GrpTiles t = grp_tiles<ConvSet<K, S>>(d.P, d.Q, kGrpSlots);  // (lower tiles would cost more partial sums)
-    if (S == 2) t.run = grp_run(t, d.N, ngroups, K, sizeof(T));
+    if (S == 2) t.run = grp_run(t, d, sizeof(T), GRP_WGRAD);
     const size_t lds = cmax(grp_pixels<ConvSet<K, S>>(t.th) * 4, kRed) * sizeof(float);
     const dim3 grid((unsigned)grp_grid(NG, ngroups)), block(kGrpThreads);
     // (a kernel of its own where tiles are dealt in turn: finding a tile's place in its run costs scalar registers)
@@ -970,8 +953,7 @@ int launch_grouped_projected(const void *x, const float *pw_w, const float *pw_b
     });
     if (d.N == 0) return 0;  // set-up only
     const int ngroups = d.C / CG;
-    GrpTiles t = grp_tiles<ConvSet<K, 2>>(d.P, d.Q, (long)d.N * ngroups);
-    t.run = grp_run(t, d.N, ngroups, K, sizeof(T));
+    const GrpTiles t = grp_tiles<ConvSet<K, 2>>(d.P, d.Q, (long)d.N * ngroups);
     const int pixels = grp_pixels<ConvSet<K, 2>>(t.th);
     const long grid = grp_grid((long)d.N * t.nth * t.ntw, ngroups);
     if (!grp_grid_fits(grid)) return -100;

@@ -45,8 +45,43 @@ __host__ __device__ inline bool grp_task(unsigned block, int units, int ngroups,
 
 struct GrpTiles {
     int th, tw, nth, ntw;  // tile extents and counts
-    int run;               // tiles of an XCD where they are dealt in runs (GrpTile::set), else 0
+    int run;               // tiles of an XCD where they are dealt in runs, else 0
 };
+
+// Tiles in runs (stride 2, where a window is up to four times its tile's share of the image): neighbouring tiles on one XCD at about
+// the same time, so that they find each other's lines in its L2.  grp_task deals units to the XCDs in turn; in runs XCD x
+// gets the x-th eighth of them, in bands of two tile columns (a tile shares more with the rows below than with the columns
+// beside; without bands 64 x 64 x 224 x 224 wgrad in bf16 381 instead of 367).
+__host__ __device__ inline void grp_run_tile(const GrpTiles &t, int unit, int &n, int &row, int &col) {
+    const int per = t.nth * t.ntw;
+    if (unit < 8 * t.run) unit = unit % 8 * t.run + unit / 8;
+    n = unit / per;
+    const int k = unit - n * per, b = k / (2 * t.nth), j = k - b * (2 * t.nth), two = 2 * b + 1 < t.ntw ? 1 : 0;
+    row = j >> two, col = 2 * b + (j & two);
+}
+// Where that pays (us, in turn / in runs; NHWC, C = 64 unless noted, images N x H x W).  In general: images cut into tiles; tile columns
+// no multiple of eight, with which an XCD has whole columns as it is; many more tasks than run at once (3 x 200 x 300, K = 31, 840 of
+// them, wgrad fp32 47.5 / 50.0, bf16 40.9 / 43.0; 8 x 256 x 256, 2048, 119.6 / 112.0 and 74.7 / 63.9).
+//   fprop, wgrad: K = 27 and 31, whose halos weigh (fprop / wgrad bf16 64 x 224 x 224 312 / 300, 440 / 357; 48 x 320 x 288 422 / 413, 650 / 539; fp32
+//     64 x 112 x 112 150 / 127, 211 / 171, 64 x 224 x 224 611 / 595, 1002 / 966; the worst, fp32 128 x 112 x 112 with 128 channels, 804 / 855).  With smaller
+//     kernels as long as x and y fit the 256 MB of cache behind the L2s: beyond it eight places at a time only spread what is read
+//     (K = 15 bf16 fprop 32 x 224 x 224 106 / 95, 34 x 320 x 288 228 / 239; fp32 12 x 256 x 256 100 / 87, wgrad 127 / 106, 34 x 320 x 288 444 / 467,
+//     543 / 592; K = 7 bf16 32 x 224 x 224 94 / 83, 119 / 109, 64 images 216 / 221, 227 / 261, 48 x 320 x 288 293 / 323); wgrad in 16 bits from K = 13 on beyond
+//     that as well (K = 15 64 x 224 x 224 287 / 257, 48 x 320 x 288 456 / 404, 12 x 448 x 448 198 / 204).
+//   dgrad: whole bands, 16 bits or K = 27 and 31 (K = 31 bf16 64 x 224 x 224, two tile columns, 240 / 203, K = 15 265 / 242, K = 7 264 / 251, 48 x
+//     256 x 256 256 / 234; fp32 K = 31 506 / 490; three columns, 34 x 320 x 288, 270 / 290, K = 7 237 / 246, fp32 533 / 557; one column, 128 x
+//     112 x 112, 81 / 86; K = 15 fp32 64 x 224 x 224 506 / 506, 12 x 448 x 448 392 / 405).
+// Behind a projection the image is small and nothing is gained.
+enum GrpPass { GRP_FPROP, GRP_DGRAD, GRP_WGRAD };
+inline int grp_run(const GrpTiles &t, const ConvDims &d, size_t esize, GrpPass pass) {
+    const long units = (long)d.N * t.nth * t.ntw;
+    if (d.stride != 2 || t.nth * t.ntw == 1 || t.ntw % 8 == 0 || units * (d.C / grp_channels(esize)) < 4 * kGrpSlots) return 0;
+    const bool wide = d.K >= 27;
+    const double bytes = ((double)d.H * d.W + (double)d.P * d.Q) * d.C * d.N * esize;
+    const bool pays = pass == GRP_DGRAD ? t.ntw % 2 == 0 && (wide || esize == 2)
+                                        : wide || bytes <= 1 << 28 || (pass == GRP_WGRAD && esize == 2 && d.K >= 13);
+    return pays ? (int)(units / 8) : 0;
+}
 
 // Partial sums per (channel, tap): about two rounds of the chip's slots at most, and no more than there are tiles of
 // 16 x 32 outputs; a multiple of eight (unit u runs on XCD u % 8) where there are as many tiles.  A workgroup's sums

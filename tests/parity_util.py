@@ -8,6 +8,23 @@ import torch
 TOL = {torch.float32: 1e-5, torch.bfloat16: 1e-2, torch.float16: 1e-2}
 
 
+# NHWC layers at stride 2, (N, C, H, W, K), and which of their grouped kernels deal tiles in runs: pass and element size, tile rows x
+# columns
+TILES_IN_RUNS = {
+    (5, 256, 150, 150, 31): {"fprop 2": (5, 3), "wgrad 2": (5, 3), "fprop 4": (5, 3), "wgrad 4": (5, 3)},
+    (11, 256, 290, 38, 15): {"fprop 2": (7, 1), "wgrad 2": (7, 1), "fprop 4": (7, 1), "wgrad 4": (7, 1)},
+    (3, 256, 101, 301, 7): {},  # (960 tasks)
+    (7, 320, 97, 130, 13): {"fprop 2": (3, 3), "wgrad 2": (3, 3), "fprop 4": (3, 3), "wgrad 4": (3, 3)},
+    (17, 512, 40, 140, 31): {"fprop 2": (2, 3), "dgrad 2": (1, 2), "wgrad 2": (2, 3), "fprop 4": (2, 3), "dgrad 4": (1, 2),
+                             "wgrad 4": (2, 3)},
+    (8, 512, 150, 138, 31): {"fprop 2": (5, 3), "dgrad 2": (2, 2), "wgrad 2": (5, 3), "fprop 4": (5, 3), "dgrad 4": (2, 2),
+                             "wgrad 4": (5, 3)},
+    (17, 256, 20, 400, 13): {"fprop 2": (1, 7), "dgrad 2": (1, 4), "wgrad 2": (1, 7), "fprop 4": (1, 7), "wgrad 4": (1, 7)},
+    (11, 256, 60, 300, 7): {"fprop 2": (2, 5), "wgrad 2": (2, 5), "fprop 4": (2, 5), "wgrad 4": (2, 5)},
+    (9, 256, 50, 500, 27): {"dgrad 4": (1, 4)},
+}
+
+
 def canonical_theta(C):
     """theta_c = (c mod 8) * 22.5 degrees, round-robin (benchmark configurations)."""
     return np.array([(c % 8) * math.pi / 8 for c in range(C)], dtype=np.float32)

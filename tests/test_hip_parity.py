@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 import torch
 
-from parity_util import (TOL, assert_close, canonical_theta, dev, grouped_theta, host, rel_err,
+from parity_util import (TILES_IN_RUNS, TOL, assert_close, canonical_theta, dev, grouped_theta, host, rel_err,
                          rounded)
 
 pytestmark = pytest.mark.gpu
@@ -257,9 +257,10 @@ def test_grouped_nhwc_kernels(oracle, N, C, H, W, K, stride, dtype):
         _case(oracle, N, C, H, W, K, stride, dtype, 3, theta, seed=H + W + K)
 
 
-# stride-2 tiles dealt in runs: more than two thousand tasks, tile counts that eight does not divide, one to five tile columns
+# stride-2 tiles dealt in runs: every pass and element size, tile counts that eight does not divide, one to seven tile columns, whole
+# bands and a last one of one column (which shapes are is checked without a GPU, tests/test_launch_splits.py)
 @pytest.mark.parametrize("dtype", DTYPES, ids=["f32", "bf16", "f16"])
-@pytest.mark.parametrize("N,C,H,W,K", [(5, 256, 150, 150, 31), (11, 256, 290, 38, 15), (3, 256, 101, 301, 7), (7, 320, 97, 130, 13)])
+@pytest.mark.parametrize("N,C,H,W,K", list(TILES_IN_RUNS))
 def test_grouped_nhwc_tiles_in_runs(oracle, N, C, H, W, K, dtype):
     _case(oracle, N, C, H, W, K, 2, dtype, 3, grouped_theta(C, 0.5), seed=H + W)
 

@@ -5,19 +5,53 @@ import subprocess
 
 import pytest
 
+from parity_util import TILES_IN_RUNS
+
 from oriented1d_amd import build
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-@pytest.mark.parametrize("program", ["window_units", "grouped_tasks", "linear_splits"])
-def test_launch_splits(program, tmp_path):
-    exe = str(tmp_path / program)
+def _compiled(program, folder):
+    exe = str(folder / program)
     subprocess.run([build.hipcc(), "-x", "hip", "--offload-host-only", "-O1", "-std=c++17", "-I" + build.CSRC,
                     "-I" + os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "host", program + ".cpp"),
                     "-o", exe], check=True)
-    done = subprocess.run([exe], stdout=subprocess.PIPE, text=True)
+    return exe
+
+
+@pytest.mark.parametrize("program", ["window_units", "grouped_tasks", "grouped_runs", "linear_splits"])
+def test_launch_splits(program, tmp_path):
+    done = subprocess.run([_compiled(program, tmp_path)], stdout=subprocess.PIPE, text=True)
     assert done.returncode == 0, done.stdout
+
+
+def test_shapes_whose_tiles_go_in_runs(tmp_path):
+    """The layers that the GPU tests take for this reach it: every pass and element size, each with the tile columns that are stated."""
+    exe, seen = _compiled("grouped_runs", tmp_path), set()
+    for shape, want in TILES_IN_RUNS.items():
+        got = {}
+        for line in subprocess.run([exe, *map(str, shape)], stdout=subprocess.PIPE, text=True, check=True).stdout.splitlines():
+            name, size, run, rows, columns = line.split()
+            if int(run) > 0:
+                got[name + " " + size] = (int(rows), int(columns))
+        assert got == want, shape
+        seen.update((k, columns) for k, (_, columns) in got.items())
+    for size in ("2", "4"):
+        assert {("fprop " + size, c) for c in (1, 3, 5, 7)} | {("wgrad " + size, c) for c in (1, 3, 5, 7)} <= seen
+        assert {("dgrad " + size, c) for c in (2, 4)} <= seen
+
+
+@pytest.mark.parametrize("layer,runs", [
+    # x and y of 253 and 260 MB, or far more: K = 31 everywhere, smaller kernels by pass and type; three tile columns of dgrad; few tasks
+    ((64, 64, 224, 224, 31), {"fprop 2", "dgrad 2", "wgrad 2", "fprop 4", "dgrad 4", "wgrad 4"}),
+    ((64, 64, 224, 224, 15), {"dgrad 2", "wgrad 2"}), ((64, 64, 224, 224, 7), {"dgrad 2"}),
+    ((33, 64, 224, 224, 7), {"fprop 2", "wgrad 2"}), ((34, 64, 224, 224, 7), set()),
+    ((34, 64, 320, 288, 31), {"fprop 2", "wgrad 2", "fprop 4", "wgrad 4"}), ((8, 64, 512, 512, 31), {"dgrad 4"}),
+    ((3, 64, 200, 300, 31), set())])
+def test_rule_for_tiles_in_runs(layer, runs, tmp_path):
+    out = subprocess.run([_compiled("grouped_runs", tmp_path), *map(str, layer)], stdout=subprocess.PIPE, text=True, check=True).stdout
+    assert {" ".join(l.split()[:2]) for l in out.splitlines() if int(l.split()[2]) > 0} == runs
 
 
 def test_product_and_tail_launches_stay_below_two_to_the_32_threads():
