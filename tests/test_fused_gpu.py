@@ -641,6 +641,60 @@ def test_stem_tail_as_one_kernel(N, H, W, C, bias, dtype):
     assert fused.norm_planes(x, before.to(dtype), linear.to(dtype), norm.to(dtype)) is None  # (gradients are on)
 
 
+@pytest.mark.parametrize("plus_plus,wrapped", [(False, True), (False, False), (True, True)])
+def test_inference_block_leaves_what_watches_it_to_its_layers(plus_plus, wrapped, monkeypatch):
+    """Hooks on any layer, the operator or its wrapper, dispatch modes, dual tensors, subclasses and recorded gradients see the
+    layers one by one, with the same values but for roundings between them."""
+    import torch.autograd.forward_ad as fwd
+    import torch.nn.modules.module as modules
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from oriented1d_amd.convnext1d import Block
+    torch.manual_seed(5)
+    block = Block(64, (15, 31) if plus_plus else (31,), plus_plus, layer_scale_init_value=0.1, arbitrary_size=True,
+                  wrapped=wrapped).cuda().bfloat16().eval()
+    x, taken, whole = torch.randn(2, 64, 9, 11, device="cuda").bfloat16(), [], fused.infer_block
+    monkeypatch.setattr(fused, "infer_block", lambda *a: taken.append(whole(*a)) or taken[-1])
+
+    def refused(run):
+        del taken[:]
+        y = run()
+        assert taken and all(t is None for t in taken)
+        return y
+
+    class Watch(TorchDispatchMode):
+        ops = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Watch.ops += 1
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    with torch.no_grad():
+        ref = block(x)
+        assert taken[-1] is not None
+        for name, layer in block.named_modules():
+            if type(layer).__name__ in ("Linear", "ConvWrapper", "DepthwiseOrientedConv1d"):
+                seen = []
+                for register in (layer.register_forward_hook, layer.register_forward_pre_hook):
+                    handle = register(lambda *_: seen.append(1))
+                    _close(refused(lambda: block(x)), ref, x.dtype, name)
+                    assert seen, name
+                    handle.remove()
+        handle = modules.register_module_forward_hook(lambda *_: None)
+        _close(refused(lambda: block(x)), ref, x.dtype, "global hook")
+        handle.remove()
+        with Watch():
+            _close(refused(lambda: block(x)), ref, x.dtype, "dispatch mode")
+        assert Watch.ops > 0
+        with fwd.dual_level(), pytest.raises(NotImplementedError, match="jvp"):  # (no layer drops a tangent silently)
+            block(fwd.make_dual(x, torch.ones_like(x)))
+        _close(refused(lambda: block(x.as_subclass(Sub))).as_subclass(torch.Tensor), ref, x.dtype, "subclass")
+        assert torch.equal(block(x), ref) and taken[-1] is not None
+    assert refused(lambda: block(x.clone().requires_grad_())).requires_grad
+
+
 @pytest.mark.parametrize("plus_plus,which", [(False, "dwconv"), (True, "dwconv1"), (True, "dwconv2")])
 @pytest.mark.parametrize("arbitrary_size", [True, False])
 def test_inference_block_with_functions_of_the_caller(plus_plus, which, arbitrary_size, monkeypatch):
