@@ -115,14 +115,14 @@ def norm_planes(x, before, linear, norm):
     return _lib.host(x.get_device()).linear_norm_planes(x, g0, b0, before.eps, w, b, g1, b1, norm.eps)
 
 
-# Rows from which both layers run as one kernel: enough workgroups of 128 pixels that its long chain is paid for (bf16, us, two
-# kernels / one: 12544 x 96 25 / 17, 8192 x 96 15.9 / 16.8; 16384 x 128 21 / 25, 17408 x 128, where the first product has more
-# tiles than the chip holds, 30 / 25; 29008 x 192 47 / 43, 25088 x 192 43 / 42 and in odd planes 67 / 70).  There is no instance for
-# 256 channels.
+# Rows from which both layers run as one kernel: enough workgroups of 128 pixels that its long chain is paid for (bf16, us, behind a
+# pass over other memory, two kernels / one: 10240 x 96 16.1 / 17.8, 12288 x 96 18.4 / 18.0; 16384 x 128 20.9 / 25.3, 16640 x 128, where the
+# first product has more tiles than the chip holds, 30.8 / 25.4; 25088 x 192 44.3 / 43.9, 29008 x 192 47.7 / 45.0, in odd planes 29008 68 /
+# 75, 34300 99 / 90).  There is no instance for 256 channels.
 _MLP_ROWS = {96: 12288, 128: 16385, 192: 28672, 384: 21846}
-# At 384 channels a workgroup has a CU to itself (101 KB of LDS): its time goes in rounds of 256 workgroups, about 95 us each, and
-# the last round pays from two thirds on (20384 rows 85 / 98, 22540 115 / 97, 32732 151 / 109, 32928 155 / 191, 39984 186 / 192, 42924
-# 192 / 193, 43904 217 / 192, 66052 314 / 309)
+# At 384 channels a workgroup has a CU to itself (101 KB of LDS): its time goes in rounds of 256 workgroups, about 100 us each, and
+# the last round pays from two thirds on (20384 rows 82 / 101, 21952 112 / 102, 32732 148 / 112, 32928 151 / 199, 39200 171 / 199, 43120 201 /
+# 202, 49000 218 / 206, 65660 313 / 308; back to back the second round from three quarters on, 43904 181 / 199, 50960 216 / 197)
 _MLP_ROUND = 32768
 
 
