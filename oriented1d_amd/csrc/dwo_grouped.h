@@ -13,13 +13,14 @@
 // (two channels: 62), and two shifts or masks per read.
 //
 // What bounds them, from counters (K = 31): at stride 1 in bf16 the issue slots of the multiply-adds and those
-// unpacking instructions (64 x 512 x 56 x 56 fprop 151 of 233 us; L2 lookups 42 %, LDS 25 %); at stride 2 lines that cross
-// the fabric again, as the eight groups of a line come to it at different times, and the L1, which takes a line of 128 bytes in two
-// clocks whatever part of it is used (64 x 64 x 224 x 224).  Two workgroups per CU (80 KB of LDS,
+// unpacking instructions (64 x 512 x 56 x 56 fprop 151 of 233 us; L2 lookups 42 %, LDS 25 %); at stride 2 (64 x 64 x 224 x 224) no unit
+// is busy much more than half the time: fprop L2 lookups 52 %, vector instructions 38 %, x read 1.07 times; dgrad L2 lookups 56 %, dx
+// written 1.46 times, as a line leaves the L2 before its pieces are there; wgrad L2 lookups 44 %, x and dy read 3.2 times at 4.7 TB/s, as the
+// eight groups of a line come to it at different times.  Two workgroups per CU (80 KB of LDS,
 // 128 registers) overlap staging and evaluation.
 // Measured (us, fprop / wgrad, K = 31, angles of the networks): 64 x 512 x 56 x 56 bf16 233 / 264 (slice
 // kernels 335 / 428), 64 x 1024 x 28 x 28 bf16 114 / 121 (129 / 190), 64 x 384 x 56 x 56 fp32 298 / 355 (326 / 551);
-// stride 2, 64 x 64 x 224 x 224 bf16 307 / 367 (tile kernels 574 / 817).
+// stride 2, 64 x 64 x 224 x 224 bf16 298 / 357 (tile kernels 574 / 817).
 #pragma once
 
 #include "dwo_grouped_dispatch.h"
@@ -554,8 +555,8 @@ __global__ __launch_bounds__(kGrpThreads) __attribute__((amdgpu_waves_per_eu(4, 
 
 // ---------------------------------------------------------------------------------------------
 // dgrad at stride 2 (QuadPlan).  `d` describes dy as both the source and the plane of quads (H = P,
-// W = Q); dx is dxh x dxw.  64 x 64 x 224 x 224 bf16, K = 31: 198 us, bound by the writes in 16-byte
-// pieces, twice dx (the residue classes one after the other from a sorted tap table, dwo_nhwc_tile.h: 544).
+// W = Q); dx is dxh x dxw.  64 x 64 x 224 x 224 bf16, K = 31: 198 us, 1.46 times dx written in 16-byte
+// pieces (the residue classes one after the other from a sorted tap table, dwo_nhwc_tile.h: 544).
 template <int O, typename T, int K>
 __device__ __forceinline__ void grp_dgrad2_body(grp_u4 *lds, float *lw, const T *dyn, T *dxn, const ConvDims &d,
                                                 const GrpTile &t, int c0, int dxh, int dxw) {

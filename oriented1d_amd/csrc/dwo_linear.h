@@ -11,12 +11,14 @@
 // operands, hence free: a read takes rows 4 g .. 4 g + 3 for its lane group g.  The bias gradient is a product with
 // ones, in the workgroups of the first column of tiles.
 //
-// What binds it is the chain of a step, not a unit (by counters, with two barriers per 64 rows and staging through registers, at 12544 x
-// 512 x 2048 matrix cores and LDS 24 % each, no bank conflicts, 111 MB through memory at 2.6 TB/s): so the loads go straight to
-// LDS, three stages ahead, with one barrier per stage, and where the partial sums weigh more there are fewer of them (LinearSplits).
-// us with the reduction, before / so: 12544 x 512 x 2048 46.3 / 39.6, 3136 x 4096 x 1024 56 / 42.5, 8192 x 384 x 1536 30.4 / 25.0,
-// 131072 x 384 x 96 37.7 / 33.9, 200704 x 512 x 128 62 / 56.  Tried: three stages and three workgroups per CU (its partial sums
-// cost more than it gives, 200704 x 512 x 128 78).  Larger tiles would read less per product, but fewer tiles mean more splits.
+// What binds it is the chain of a step, not a unit: by counters matrix cores 25 %, vector instructions 12 %, LDS 12 %, no conflicts, waves
+// waiting 29 % of their cycles (12544 x 512 x 2048, 64 MB read; at 131072 x 384 x 96 129 MB in 31 us, 4.6 TB/s).  So the loads go straight to
+// LDS, three stages ahead, with one barrier per stage, and where the partial sums weigh more there are fewer of them
+// (LinearSplits).  us with the reduction, staging through registers with two barriers per 64 rows / so: 12544 x 512 x 2048 46.3 / 39.6,
+// 3136 x 4096 x 1024 56 / 42.5, 8192 x 384 x 1536 30.4 / 25.0, 131072 x 384 x 96 37.7 / 33.9, 200704 x 512 x 128 62 / 56; slower where few splits
+// or a K of one and a half tiles let workgroups that share lines drift apart, with many rows (75264 x 3072 x 768 581 / 602, 100352 x 768 x 192 73 / 79:
+// 12544 x 3072 x 768 reads 582 MB, its inputs six times).  Tried: three stages and three workgroups per CU (its partial sums cost more
+// than it gives, 200704 x 512 x 128 78).  Larger tiles would read less per product, but fewer tiles mean more splits.
 #pragma once
 
 #include "dwo_common.h"
@@ -629,8 +631,9 @@ __global__ __launch_bounds__(kLinThreads, 2) void linear_split_kernel(LinearArgs
 // a wave's), so each has its own four stages of LDS, three of them on their way, and no barrier until the sums meet: with the
 // kernel above two stages and few workgroups left the loads of a long row one after the other.  Through LDS and not straight to
 // registers, because a fragment's neighbouring lanes lie in different rows (196 x 384 x 1536 7.2, 49 x 768 x 3072 12.8).
-// bf16, us, 64 x 64 tiles / these: 49 x 3072 x 768 7.1 / 4.9, planes 196 x 384 x 1536 10.8 / 4.7, 784 x 192 x 768 7.2 / 4.2,
-// 98 x 1024 x 4096 24.0 / 8.5, 49 x 768 x 3072 19.3 / 7.5, rows 196 x 384 x 96 4.5 / 3.7 (an empty launch 3).
+// Waiting for memory bounds it (half of the waves' cycles by counters, no unit above 6 %).  bf16, us, 64 x 64 tiles / these, behind a
+// pass over other memory, as in a network, whose weights come from beyond the L2: 49 x 3072 x 768 7.1 / 4.7, planes 196 x 384 x 1536 12.6 / 5.0, 784 x
+// 192 x 768 7.8 / 4.8, 98 x 1024 x 4096 27.9 / 9.7, 49 x 768 x 3072 21.5 / 8.1, rows 196 x 384 x 96 4.3 / 4.3 (an empty launch 3).
 template <typename T, int OUT, int QF>
 __global__ __launch_bounds__(kLinThreads, 1) void linear_wave_kernel(LinearArgs<T> a, int xtiles, int tiles) {
     constexpr bool PLANES = OUT == LIN_PLANES;
@@ -790,9 +793,9 @@ int launch_linear(const LinearArgs<T> &a, hipStream_t st) {
 // out[image][n][p] = LayerNorm over n of (b[n] + sum_k w[n][k] z[image][p][k]) with z = GELU(LayerNorm over k of x), rounded as a layer
 // of its own would: the stem's last layers with the planes that follow (models/convnext.py:184-190), K = 64 and N = 16 NB <= 128.
 // A wave holds the weights as fragments and takes 32 pixels at a time with all their channels, so that a LayerNorm is a sum
-// over its registers and a few lanes.  GELU's vector instructions bound it: 401408 x 64 -> 96 in bf16 56 us (without the first norm
-// 38, which is reading x and writing the planes; as a norm pass, the library's product, a norm pass and a transposition 200), one
-// image 8 (20).
+// over its registers and a few lanes.  GELU's vector instructions bound it, 68 % of the time by counters: 401408 x 64 -> 96 in bf16 56
+// us (without the first norm 38, which is reading x and writing the planes; as a norm pass, the library's product, a norm pass and a
+// transposition 200), one image 9.6 behind other work (back to back 8, 20), waiting for its one tile per wave.
 constexpr int kNormK = 64, kNormGroups = 1024;
 struct NormArgs {
     const float *gamma, *beta, *gamma_in, *beta_in;

@@ -9,9 +9,9 @@
 // while the previous ones are used and are shared by the waves; 16 PF is what leaves two waves per SIMD, so that one's
 // GELU runs under the other's matrix instructions.
 //
-// What bounds it: at C = 96 the vector instructions, mostly of GELU (16 issue slots per hidden value; counted with 21 of them 63 %
-// of the time, matrix cores 16 %, LDS 23 %); the share falls to 42 % at 192 and 31 % at 384, where the LDS reads of the weights, which
-// eight waves of 16 pixels share, lead with 40 % and no unit is busy for half the time.  us, bf16, two product kernels / this
+// What bounds it, by counters: at C = 96 the vector instructions, mostly of GELU (16 issue slots per hidden value), 66 % of the time
+// (matrix cores 19 %, LDS 27 %); the share falls to 40 % at 192 and 29 % at 384, where the LDS reads of the weights, which
+// eight waves of 16 pixels share, lead with 39 % and no unit is busy for half the time.  us, bf16, two product kernels / this
 // one: 401408 x 96 269 / 113, 100352 x 192 159 / 105, 25088 x 384 119 / 100; slower from C = 512 (spills) and where its
 // workgroups of 128 pixels are few (its chain is 4 C / 32 steps of 1.5 to 1.9 us: 12544 x 384 60 / 90).  Tried: at 384 four waves
 // of 32 pixels, half the LDS reads (one wave per SIMD overlaps nothing, 98 / 205); GELU of a step under the first products of the
