@@ -62,24 +62,26 @@ __host__ __device__ inline void grp_run_tile(const GrpTiles &t, int unit, int &n
 // Where that pays (us, in turn / in runs; NHWC, C = 64 unless noted, images N x H x W).  In general: images cut into tiles; tile columns
 // no multiple of eight, with which an XCD has whole columns as it is; many more tasks than run at once (3 x 200 x 300, K = 31, 840 of
 // them, wgrad fp32 47.5 / 50.0, bf16 40.9 / 43.0; 8 x 256 x 256, 2048, 119.6 / 112.0 and 74.7 / 63.9).
-//   fprop, wgrad: K = 27 and 31, whose halos weigh (fprop / wgrad bf16 64 x 224 x 224 312 / 300, 440 / 357; 48 x 320 x 288 422 / 413, 650 / 539; fp32
-//     64 x 112 x 112 150 / 127, 211 / 171, 64 x 224 x 224 611 / 595, 1002 / 966; the worst, fp32 128 x 112 x 112 with 128 channels, 804 / 855).  With smaller
-//     kernels as long as x and y fit the 256 MB of cache behind the L2s: beyond it eight places at a time only spread what is read
-//     (K = 15 bf16 fprop 32 x 224 x 224 106 / 95, 34 x 320 x 288 228 / 239; fp32 12 x 256 x 256 100 / 87, wgrad 127 / 106, 34 x 320 x 288 444 / 467,
-//     543 / 592; K = 7 bf16 32 x 224 x 224 94 / 83, 119 / 109, 64 images 216 / 221, 227 / 261, 48 x 320 x 288 293 / 323); wgrad in 16 bits from K = 13 on beyond
-//     that as well (K = 15 64 x 224 x 224 287 / 257, 48 x 320 x 288 456 / 404, 12 x 448 x 448 198 / 204).
-//   dgrad: whole bands, 16 bits or K = 27 and 31 (K = 31 bf16 64 x 224 x 224, two tile columns, 240 / 203, K = 15 265 / 242, K = 7 264 / 251, 48 x
-//     256 x 256 256 / 234; fp32 K = 31 506 / 490; three columns, 34 x 320 x 288, 270 / 290, K = 7 237 / 246, fp32 533 / 557; one column, 128 x
-//     112 x 112, 81 / 86; K = 15 fp32 64 x 224 x 224 506 / 506, 12 x 448 x 448 392 / 405).
+//   fprop, wgrad: always while x and y fit the 256 MB of cache behind the L2s (K = 31 64 x 112 x 112 fp32 150 / 127, 211 / 171, K = 15 fp32 12 x
+//     256 x 256 100 / 87, 127 / 106, K = 7 bf16 32 x 224 x 224 94 / 83, 119 / 109).  Beyond it eight places at a time spread what is read, and
+//     the halos have to weigh more:
+//     fprop with K = 27 and 31 (bf16 64 x 224 x 224 312 / 300, fp32 611 / 595, 128 x 112 x 112 with 128 channels 621 / 572; K = 15 bf16 34 x 320 x 288
+//     228 / 239, K = 7 293 / 323);
+//     wgrad with these, in 16 bits from K = 13 on, of at most 384 bytes per pixel (bf16 64 x 224 x 224 440 / 357, K = 15 287 / 257, 12 x 448 x 448 198 /
+//     204, K = 7 227 / 261; fp32 1002 / 966, K = 15 34 x 320 x 288 543 / 592; bf16 80 x 112 x 112 with 192 channels 464 / 426, 64 with 256 403 / 430; fp32 32 x
+//     224 x 224 with 96 824 / 841, with 128 775 / 886).
+//   dgrad: whole bands, 16 bits or K = 27 and 31, 64 channels at most beyond that cache (K = 31 bf16 64 x 224 x 224, two tile columns, 240 /
+//     203, K = 15 265 / 242, K = 7 264 / 251; fp32 K = 31 506 / 490, K = 15 506 / 506; three columns, bf16 34 x 320 x 288, 270 / 290; one column, 128 x 112 x
+//     112, 81 / 86; 24 x 224 x 224 with 192 channels 262 / 291).
 // Behind a projection the image is small and nothing is gained.
 enum GrpPass { GRP_FPROP, GRP_DGRAD, GRP_WGRAD };
 inline int grp_run(const GrpTiles &t, const ConvDims &d, size_t esize, GrpPass pass) {
     const long units = (long)d.N * t.nth * t.ntw;
     if (d.stride != 2 || t.nth * t.ntw == 1 || t.ntw % 8 == 0 || units * (d.C / grp_channels(esize)) < 4 * kGrpSlots) return 0;
-    const bool wide = d.K >= 27;
-    const double bytes = ((double)d.H * d.W + (double)d.P * d.Q) * d.C * d.N * esize;
-    const bool pays = pass == GRP_DGRAD ? t.ntw % 2 == 0 && (wide || esize == 2)
-                                        : wide || bytes <= 1 << 28 || (pass == GRP_WGRAD && esize == 2 && d.K >= 13);
+    const bool wide = d.K >= 27, cached = ((double)d.H * d.W + (double)d.P * d.Q) * d.C * d.N * esize <= 1 << 28;
+    bool pays = wide || cached;
+    if (pass == GRP_WGRAD) pays = cached || ((wide || (esize == 2 && d.K >= 13)) && d.C * esize <= 384);
+    if (pass == GRP_DGRAD) pays = t.ntw % 2 == 0 && (wide || esize == 2) && (cached || d.C <= 64);
     return pays ? (int)(units / 8) : 0;
 }
 

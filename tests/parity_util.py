@@ -17,11 +17,10 @@ TILES_IN_RUNS = {
     (7, 320, 97, 130, 13): {"fprop 2": (3, 3), "wgrad 2": (3, 3), "fprop 4": (3, 3), "wgrad 4": (3, 3)},
     (17, 512, 40, 140, 31): {"fprop 2": (2, 3), "dgrad 2": (1, 2), "wgrad 2": (2, 3), "fprop 4": (2, 3), "dgrad 4": (1, 2),
                              "wgrad 4": (2, 3)},
-    (8, 512, 150, 138, 31): {"fprop 2": (5, 3), "dgrad 2": (2, 2), "wgrad 2": (5, 3), "fprop 4": (5, 3), "dgrad 4": (2, 2),
-                             "wgrad 4": (5, 3)},
+    (8, 512, 150, 138, 31): {"fprop 2": (5, 3), "dgrad 2": (2, 2), "wgrad 2": (5, 3), "fprop 4": (5, 3)},
     (17, 256, 20, 400, 13): {"fprop 2": (1, 7), "dgrad 2": (1, 4), "wgrad 2": (1, 7), "fprop 4": (1, 7), "wgrad 4": (1, 7)},
     (11, 256, 60, 300, 7): {"fprop 2": (2, 5), "wgrad 2": (2, 5), "fprop 4": (2, 5), "wgrad 4": (2, 5)},
-    (9, 256, 50, 500, 27): {"dgrad 4": (1, 4)},
+    (8, 256, 50, 500, 27): {"dgrad 4": (1, 4)},
 }
 
 

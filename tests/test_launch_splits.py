@@ -26,12 +26,17 @@ def test_launch_splits(program, tmp_path):
     assert done.returncode == 0, done.stdout
 
 
-def test_shapes_whose_tiles_go_in_runs(tmp_path):
+@pytest.fixture(scope="module")
+def grouped_runs(tmp_path_factory):
+    return _compiled("grouped_runs", tmp_path_factory.mktemp("host"))
+
+
+def test_shapes_whose_tiles_go_in_runs(grouped_runs):
     """The layers that the GPU tests take for this reach it: every pass and element size, each with the tile columns that are stated."""
-    exe, seen = _compiled("grouped_runs", tmp_path), set()
+    seen = set()
     for shape, want in TILES_IN_RUNS.items():
         got = {}
-        for line in subprocess.run([exe, *map(str, shape)], stdout=subprocess.PIPE, text=True, check=True).stdout.splitlines():
+        for line in subprocess.run([grouped_runs, *map(str, shape)], stdout=subprocess.PIPE, text=True, check=True).stdout.splitlines():
             name, size, run, rows, columns = line.split()
             if int(run) > 0:
                 got[name + " " + size] = (int(rows), int(columns))
@@ -43,14 +48,17 @@ def test_shapes_whose_tiles_go_in_runs(tmp_path):
 
 
 @pytest.mark.parametrize("layer,runs", [
-    # x and y of 253 and 260 MB, or far more: K = 31 everywhere, smaller kernels by pass and type; three tile columns of dgrad; few tasks
+    # x and y of 253 and 260 MB, or far more: K = 31 everywhere, smaller kernels by pass and type; three tile columns of dgrad;
+    # many channels; few tasks
     ((64, 64, 224, 224, 31), {"fprop 2", "dgrad 2", "wgrad 2", "fprop 4", "dgrad 4", "wgrad 4"}),
     ((64, 64, 224, 224, 15), {"dgrad 2", "wgrad 2"}), ((64, 64, 224, 224, 7), {"dgrad 2"}),
     ((33, 64, 224, 224, 7), {"fprop 2", "wgrad 2"}), ((34, 64, 224, 224, 7), set()),
     ((34, 64, 320, 288, 31), {"fprop 2", "wgrad 2", "fprop 4", "wgrad 4"}), ((8, 64, 512, 512, 31), {"dgrad 4"}),
-    ((3, 64, 200, 300, 31), set())])
-def test_rule_for_tiles_in_runs(layer, runs, tmp_path):
-    out = subprocess.run([_compiled("grouped_runs", tmp_path), *map(str, layer)], stdout=subprocess.PIPE, text=True, check=True).stdout
+    ((128, 128, 112, 112, 31), {"fprop 2", "wgrad 2", "fprop 4"}), ((40, 192, 224, 224, 31), {"fprop 2", "wgrad 2", "fprop 4"}),
+    ((40, 256, 224, 224, 31), {"fprop 2", "fprop 4"}),
+    ((16, 128, 224, 224, 15), {"fprop 2", "wgrad 2"}), ((3, 64, 200, 300, 31), set())])
+def test_rule_for_tiles_in_runs(layer, runs, grouped_runs):
+    out = subprocess.run([grouped_runs, *map(str, layer)], stdout=subprocess.PIPE, text=True, check=True).stdout
     assert {" ".join(l.split()[:2]) for l in out.splitlines() if int(l.split()[2]) > 0} == runs
 
 
